@@ -255,11 +255,15 @@ struct GemmArgs {
     const float *norm_w = nullptr;
     float eps = 0.0f;
     const float *gate = nullptr;
+    // W is the gate projection, W_more[0] the up projection (N columns each, end[0] == N): Y becomes silu(X gate^T) * (X up^T), as
+    // launch_silu_mul forms it.  Only where gemm_gates() says so.
+    bool gated = false;
 };
 int32_t launch_gemm(nh_device *d, const GemmArgs &args);
 // whether launch_gemm takes a product of this element and depth with matrices stacked along N at these boundaries, or with
 // activations the launch before packed
 bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, const void *W1, const void *W2, uint32_t end0, uint32_t end1);
+bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up);
 // device scratch a Q4_K wide product over M rows of K activations packs them into
 size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows);
 

@@ -5,6 +5,7 @@
 // activation rows; each thread owns a 4 x 4 patch of the output in registers.
 #include "blocks.hpp"
 #include "common.hpp"
+#include "gemm_few.hpp"
 
 #include <cstdlib>
 
@@ -109,12 +110,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint8_t *__restrict__ W
 // per eight weights, and stages step s + 1 into the other half of LDS while the matrix cores
 // walk step s: one barrier per step.
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int GT = 128;           // tile edge (rows of A' and rows of W)
 constexpr int GK = 64;            // k per step
 constexpr int GS = GK + 8;        // LDS row stride in halves: 144 B keeps 128-bit reads of 8 neighbouring rows on distinct banks
@@ -140,14 +135,16 @@ __device__ __forceinline__ void fetch_parameters(const GemmQ4Params &p) {
 }
 
 // Four neighbouring numbers of a row (`hi`: as halves; `lo`, with SPLIT: their residues * 2^11) into the packed rows, and their
-// share of the sub-block sums: eight neighbouring lanes hold the 32 numbers of a sub-block.
-template <bool SPLIT>
+// share of the sub-block sums: eight neighbouring lanes hold the 32 numbers of a sub-block.  FEW: in the operand order of the
+// product of few rows (few_operand_at), not row by row.
+template <bool SPLIT, bool FEW>
 __device__ __forceinline__ void pack_piece(const _Float16 (&hi)[4], const _Float16 (&lo)[4], uint32_t row, uint32_t k, uint32_t K, uint32_t nsb,
                                            _Float16 *__restrict__ A, _Float16 *__restrict__ S) {
     // the nibbles of four weight bytes unpack as bytes 0, 2, 1, 3
     const half4_t out_hi = {hi[0], hi[2], hi[1], hi[3]}, out_lo = {lo[0], lo[2], lo[1], lo[3]};
-    *reinterpret_cast<half4_t *>(A + (size_t)row * K + k) = out_hi;
-    if (SPLIT) *reinterpret_cast<half4_t *>(A + (size_t)(row + 1u) * K + k) = out_lo;
+    const size_t place = FEW ? few_operand_at(row, k, K) : (size_t)row * K + k;
+    *reinterpret_cast<half4_t *>(A + place) = out_hi;
+    if (SPLIT) *reinterpret_cast<half4_t *>(A + place + (FEW ? 8u : K)) = out_lo;  // (a residue row is its value row's neighbour in a tile)
     // sums of the 32 halves of a sub-block: eight neighbouring lanes
     float sum_hi = ((float)hi[0] + (float)hi[1]) + ((float)hi[2] + (float)hi[3]);
     float sum_lo = ((float)lo[0] + (float)lo[1]) + ((float)lo[2] + (float)lo[3]);
@@ -161,16 +158,16 @@ __device__ __forceinline__ void pack_piece(const _Float16 (&hi)[4], const _Float
         {
             const float v = sum_hi * 0.015625f;
             const _Float16 h = (_Float16)v;
-            _Float16 *dst = S + ((size_t)row * nsb + sb) * 16u;
+            _Float16 *dst = S + (FEW ? few_sums_at(row, sb, nsb, 0) : ((size_t)row * nsb + sb) * 16u);
             dst[slot] = h;
-            dst[8u + slot] = (_Float16)((v - (float)h) * 2048.0f);
+            dst[(FEW ? 256u : 8u) + slot] = (_Float16)((v - (float)h) * 2048.0f);
         }
         if (SPLIT) {
             const float v = sum_lo * 0.015625f;
             const _Float16 h = (_Float16)v;
-            _Float16 *dst = S + ((size_t)(row + 1u) * nsb + sb) * 16u;
+            _Float16 *dst = S + (FEW ? few_sums_at(row + 1u, sb, nsb, 0) : ((size_t)(row + 1u) * nsb + sb) * 16u);
             dst[slot] = h;
-            dst[8u + slot] = (_Float16)((v - (float)h) * 2048.0f);
+            dst[(FEW ? 256u : 8u) + slot] = (_Float16)((v - (float)h) * 2048.0f);
         }
     }
 }
@@ -180,10 +177,10 @@ __device__ __forceinline__ void pack_piece(const _Float16 (&hi)[4], const _Float
 // fp32 numbers: thread t adds the squares of columns t, t + 256, ..., then a 256-wide tree); 2: silu(gate) * X as
 // silu_mul_kernel forms it.  `aux` is the norm's weight vector or the gate rows.
 constexpr int PACK_PLAIN = 0, PACK_NORM = 1, PACK_SWIGLU = 2;
-template <bool HALF_IN, int PRELUDE = PACK_PLAIN>
+template <bool HALF_IN, int PRELUDE, bool FEW>
 __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
                                                              _Float16 *__restrict__ S, float *__restrict__ unscale,
-                                                             const float *__restrict__ aux = nullptr, float eps = 0.0f) {
+                                                             const float *__restrict__ aux, float eps) {
     static_assert(!(HALF_IN && PRELUDE != PACK_PLAIN), "half rows are packed as they lie");
     __shared__ uint32_t wave_top[4];
     __shared__ float red[256];
@@ -249,7 +246,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
                 lo[e] = (_Float16)((t[e] - (float)hi[e]) * 2048.0f);
             }
         }
-        pack_piece<!HALF_IN>(hi, lo, row, k, K, nsb, A, S);
+        pack_piece<!HALF_IN, FEW>(hi, lo, row, k, K, nsb, A, S);
     }
 }
 
@@ -258,7 +255,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
 // with the norm, 37 on an 18944-wide gated one.  Here a row crosses memory once, four 16-byte loads a thread in flight at a
 // time, and waits in LDS as the prelude left it: the squares are added from LDS in the same thread order, the packing reads
 // LDS.  The same arithmetic on the same numbers: the packed rows are the kernel above's bit for bit.  K is a multiple of 4.
-template <int PRELUDE>
+template <int PRELUDE, bool FEW>
 __global__ __launch_bounds__(256) void gemm_pack_rows_staged_kernel(const float *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
                                                                     _Float16 *__restrict__ S, float *__restrict__ unscale,
                                                                     const float *__restrict__ aux, float eps) {
@@ -335,7 +332,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_staged_kernel(const float 
             hi[e] = (_Float16)t[e];
             lo[e] = (_Float16)((t[e] - (float)hi[e]) * 2048.0f);
         }
-        pack_piece<true>(hi, lo, 2u * m, k, K, nsb, A, S);
+        pack_piece<true, FEW>(hi, lo, 2u * m, k, K, nsb, A, S);
     }
 }
 
@@ -1197,8 +1194,38 @@ __global__ __launch_bounds__(512) void gemm_q3k_mfma_kernel(GemmQ4Params p) {
 
 // bytes of device scratch a Q4_K wide product over M activation rows of K numbers packs into
 size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows) {
-    const size_t rows = half_rows ? M : (size_t)2 * M;
+    const size_t rows = ((half_rows ? M : (size_t)2 * M) + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;  // (whole tiles: few_operand_at)
     return rows * K * sizeof(_Float16) + rows * ((K + 255u) / 256u) * 16u * sizeof(_Float16) + (size_t)M * sizeof(float);
+}
+
+template <bool FEW>
+static int32_t pack_rows(nh_device *d, const GemmArgs &a, bool half_rows, _Float16 *A, _Float16 *S, float *unscale) {
+    const float *none = nullptr, *rows = static_cast<const float *>(a.X);
+    const dim3 grid(a.M), block(256);
+    if (half_rows) {
+        hipLaunchKernelGGL((gemm_pack_rows_kernel<true, PACK_PLAIN, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f);
+    } else if (a.K % 4u == 0 && a.K >= 4u && (size_t)a.K * sizeof(float) <= PACK_STAGED_LDS_MOST && !pack_unstaged()) {
+        // a row of fp32 numbers crosses memory once and waits in LDS
+        const size_t lds = (size_t)a.K * sizeof(float);
+        static bool roomy = false;
+        if (!roomy) {
+            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_PLAIN, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
+            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_NORM, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
+            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_SWIGLU, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
+            roomy = true;
+        }
+        if (a.norm_w) hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_NORM, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, a.norm_w, a.eps);
+        else if (a.gate) hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_SWIGLU, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, a.gate, 0.0f);
+        else hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_PLAIN, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, none, 0.0f);
+    } else if (a.norm_w) {
+        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_NORM, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, a.norm_w, a.eps);
+    } else if (a.gate) {
+        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_SWIGLU, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, a.gate, 0.0f);
+    } else {
+        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_PLAIN, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f);
+    }
+    NH_HIP(hipGetLastError());
+    return NH_OK;
 }
 
 static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
@@ -1218,41 +1245,24 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const bool half_rows = a.x_element == NH_F16;
     p.rows = half_rows ? a.M : 2 * a.M;
     p.split = half_rows ? 0 : 1;
-    // scratch: [rows][K] halves, [rows][K / 256][16] sums, M row scales
-    const size_t halves = (size_t)p.rows * a.K * sizeof(_Float16), sums = (size_t)p.rows * ((a.K + 255u) / 256u) * 16u * sizeof(_Float16);
+    const bool few = gemm_few_takes(a.element, a.N, a.K, p.rows);
+    if (a.gated && (!few || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
+        return fail(NH_E_ARGUMENT, "this wide product gates no outputs (ask gemm_gates first)");
+    // scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row scales
+    const size_t held = (size_t)(p.rows + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;
+    const size_t halves = held * a.K * sizeof(_Float16), sums = held * ((a.K + 255u) / 256u) * 16u * sizeof(_Float16);
     uint8_t *room = static_cast<uint8_t *>(scratch(d, gemm_q4k_scratch_bytes(a.M, a.K, half_rows)));
     if (!room) return NH_E_MEMORY;
     _Float16 *A = reinterpret_cast<_Float16 *>(room), *S = reinterpret_cast<_Float16 *>(room + halves);
     float *unscale = reinterpret_cast<float *>(room + halves + sums);
     if ((a.norm_w || a.gate) && (half_rows || (a.norm_w && a.gate) || ((uintptr_t)(a.norm_w ? a.norm_w : a.gate) & 15u)))
         return fail(NH_E_ARGUMENT, "a wide product normalises or gates fp32 rows read from 16-byte aligned addresses, one of the two");
-    if (a.packed) {
-        // what the launch before left in the scratch is this launch's operand
-    } else if (half_rows) {
-        hipLaunchKernelGGL(gemm_pack_rows_kernel<true>, dim3(a.M), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, nullptr, 0.0f);
-    } else if (a.K % 4u == 0 && a.K >= 4u && (size_t)a.K * sizeof(float) <= PACK_STAGED_LDS_MOST && !pack_unstaged()) {
-        // a row of fp32 numbers crosses memory once and waits in LDS
-        const size_t lds = (size_t)a.K * sizeof(float);
-        static bool roomy = false;
-        if (!roomy) {
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_PLAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_SWIGLU>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            roomy = true;
-        }
-        const float *rows = static_cast<const float *>(a.X);
-        if (a.norm_w) hipLaunchKernelGGL(gemm_pack_rows_staged_kernel<PACK_NORM>, dim3(a.M), dim3(256), lds, d->stream, rows, a.K, A, S, unscale, a.norm_w, a.eps);
-        else if (a.gate) hipLaunchKernelGGL(gemm_pack_rows_staged_kernel<PACK_SWIGLU>, dim3(a.M), dim3(256), lds, d->stream, rows, a.K, A, S, unscale, a.gate, 0.0f);
-        else hipLaunchKernelGGL(gemm_pack_rows_staged_kernel<PACK_PLAIN>, dim3(a.M), dim3(256), lds, d->stream, rows, a.K, A, S, unscale, static_cast<const float *>(nullptr), 0.0f);
-    } else if (a.norm_w) {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_NORM>), dim3(a.M), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, a.norm_w, a.eps);
-    } else if (a.gate) {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_SWIGLU>), dim3(a.M), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, a.gate, 0.0f);
-    } else {
-        hipLaunchKernelGGL(gemm_pack_rows_kernel<false>, dim3(a.M), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, nullptr, 0.0f);
-    }
-    NH_HIP(hipGetLastError());
+    // (rows packed by the launch before are this launch's operand)
+    if (const int32_t status = a.packed ? NH_OK : few ? pack_rows<true>(d, a, half_rows, A, S, unscale) : pack_rows<false>(d, a, half_rows, A, S, unscale); status != NH_OK)
+        return status;
     p.A = A, p.S = S, p.unscale = unscale;
+    if (few)
+        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale, 1u, 1u}, a.gated);
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
@@ -1293,10 +1303,16 @@ bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, con
     return true;
 }
 
+// one launch for the gate and the up projection, silu(gate) * up leaving it: the product of few rows
+bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up) {
+    return N % GT == 0 && gemm_stacks(element, K, X, gate, nullptr, nullptr, 0, 0) && gemm_stacks(element, K, X, up, nullptr, nullptr, 0, 0) &&
+           2u * M <= FEW_TILE && gemm_few_takes(element, N, K, 2u * M);
+}
+
 int32_t launch_gemm(nh_device *d, const GemmArgs &a) {
     if (!a.M || !a.N) return NH_OK;
     if (mfma_takes(a.element, a.K, a.X, a.W)) return launch_gemm_mfma(d, a);
-    if (a.W_more[0] || a.W_more[1] || a.packed || a.norm_w || a.gate)
+    if (a.W_more[0] || a.W_more[1] || a.packed || a.norm_w || a.gate || a.gated)
         return fail(NH_E_ARGUMENT, "this wide product stacks no matrices, reuses no packed activations and packs rows as they lie (ask gemm_stacks first)");
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM), block(256);
     uint32_t row_bytes = (uint32_t)payload_bytes(a.element, a.K);

@@ -1,0 +1,45 @@
+// The wide product of few activation rows (gemm_few.hip), as the wide products' launcher (gemm.hip) reaches it.
+#pragma once
+#include "common.hpp"
+
+namespace nh {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t FEW_TILE = 32;  // weight rows and packed activation rows of a tile
+
+// Where four neighbouring numbers (k a multiple of 4) of packed row `row` lie, in halves, when the rows are packed as the
+// operands of v_mfma_f32_32x32x16_f16: [row / 32][k / 64][depth 0..3][part 0..1][row % 32][8], the eight numbers at
+// k = 64 step + 8 chunk being depth 2 (chunk / 4) + chunk % 2 of part (chunk / 2) % 2 -- a wave reads an operand as 1 KB in a row.
+__host__ __device__ inline size_t few_operand_at(uint32_t row, uint32_t k, uint32_t K) {
+    const uint32_t chunk = (k >> 3) & 7u, depth = 2u * (chunk >> 2) + (chunk & 1u), part = (chunk >> 1) & 1u;
+    return (((((size_t)(row >> 5) * (K >> 6) + (k >> 6)) * 4u + depth) * 2u + part) * 32u + (row & 31u)) * 8u + (k & 4u);
+}
+// and where the eight sub-block sums (part 0) or their residues (part 1) of a super-block lie: [row / 32][super-block][part][row % 32][8]
+__host__ __device__ inline size_t few_sums_at(uint32_t row, uint32_t sb, uint32_t nsb, uint32_t part) {
+    return ((((size_t)(row >> 5) * nsb + sb) * 2u + part) * 32u + (row & 31u)) * 8u;
+}
+
+struct FewParams {
+    const uint8_t *W, *W1, *W2;  // matrices stacked along N, column ends end0 and end1 (multiples of the tile); gated: gate and up, N columns each
+    uint32_t end0, end1;
+    uint32_t N, K, row_bytes;
+    const _Float16 *A, *S;  // packed rows and sums, in operand order
+    uint32_t rows;          // rows of A: twice M where an activation row is a value and a residue row
+    float *Y;
+    const float *residual;
+    uint32_t ldy, M;
+    int32_t split;
+    const float *unscale;
+    uint32_t across, deep;  // the waves of a workgroup: tiles of columns x shares of K
+};
+
+// whether the product of `rows` packed rows is this kernel's, and its launch (the rows are packed)
+bool gemm_few_takes(int32_t element, uint32_t N, uint32_t K, uint32_t rows);
+int32_t launch_gemm_few(nh_device *d, int32_t element, FewParams p, bool gated);
+
+}  // namespace nh

@@ -259,19 +259,21 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             GemmArgs o{element_at(m, L, O), m->attn_o[L], H, QW, m->att, NH_F32, T, m->h, m->h, H};
             if ((status = launch_gemm(d, o)) != NH_OK) return status;
             // where the matrix cores take both projections the norm rides in the pass that packs the rows for the gate
-            // projection, and the up projection multiplies those same packed rows
-            const bool paired = element_at(m, L, GATE) == element_at(m, L, UP) &&
-                                gemm_stacks(element_at(m, L, GATE), H, m->h, m->ffn_gate[L], nullptr, nullptr, 0, 0) &&
+            // projection, and the up projection multiplies those same packed rows -- in the same launch where the rows are few
+            const bool alike = element_at(m, L, GATE) == element_at(m, L, UP);
+            const bool both = alike && gemm_gates(element_at(m, L, GATE), F, H, T, m->h, m->ffn_gate[L], m->ffn_up[L]);
+            const bool paired = alike && !both && gemm_stacks(element_at(m, L, GATE), H, m->h, m->ffn_gate[L], nullptr, nullptr, 0, 0) &&
                                 gemm_stacks(element_at(m, L, UP), H, m->h, m->ffn_up[L], nullptr, nullptr, 0, 0);
-            if (!paired && (status = launch_rmsnorm(d, m->h, nullptr, m->ffn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
-            GemmArgs g{element_at(m, L, GATE), m->ffn_gate[L], F, H, paired ? m->h : m->xn, NH_F32, T, m->act, nullptr, F};
+            if (!paired && !both && (status = launch_rmsnorm(d, m->h, nullptr, m->ffn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
+            GemmArgs g{element_at(m, L, GATE), m->ffn_gate[L], F, H, paired || both ? m->h : m->xn, NH_F32, T, m->act, nullptr, F};
             GemmArgs u{element_at(m, L, UP), m->ffn_up[L], F, H, paired ? m->h : m->xn, NH_F32, T, m->up, nullptr, F};
-            if (paired) g.norm_w = m->ffn_norm[L], g.eps = c.eps, u.packed = true;
+            if (paired || both) g.norm_w = m->ffn_norm[L], g.eps = c.eps, u.packed = true;
+            if (both) g.gated = true, g.W_more[0] = m->ffn_up[L], g.end[0] = g.end[1] = F;
             if ((status = launch_gemm(d, g)) != NH_OK) return status;
-            if ((status = launch_gemm(d, u)) != NH_OK) return status;
-            // silu(gate) * up is formed as the down projection packs its rows, or by a kernel of its own
-            const bool gated = gemm_stacks(element_at(m, L, DOWN), F, m->up, m->ffn_down[L], nullptr, nullptr, 0, 0);
-            if (!gated && (status = launch_silu_mul(d, m->act, m->up, (uint64_t)T * F, m->act)) != NH_OK) return status;
+            if (!both && (status = launch_gemm(d, u)) != NH_OK) return status;
+            // silu(gate) * up is formed by the product itself, as the down projection packs its rows, or by a kernel of its own
+            const bool gated = !both && gemm_stacks(element_at(m, L, DOWN), F, m->up, m->ffn_down[L], nullptr, nullptr, 0, 0);
+            if (!gated && !both && (status = launch_silu_mul(d, m->act, m->up, (uint64_t)T * F, m->act)) != NH_OK) return status;
             GemmArgs dn{element_at(m, L, DOWN), m->ffn_down[L], H, F, gated ? m->up : m->act, NH_F32, T, m->h, m->h, H};
             if (gated) dn.gate = m->act;
             if ((status = launch_gemm(d, dn)) != NH_OK) return status;
@@ -342,7 +344,15 @@ int32_t decode_kernels(nh_model *m, bool any_inactive, bool sampled) {
     if ((status = forward(m, 1, any_inactive)) != NH_OK) return status;
     GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
     head.norm_w = m->output_norm, head.eps = m->c.eps;
-    if ((status = launch_gemv(m->d, head)) != NH_OK) return status;
+    if (m->c.batch > 8u && gemm_stacks(head.element, head.K, m->h, m->output, nullptr, nullptr, 0, 0)) {
+        // more rows than a narrow product takes at once: the wide one walks the vocabulary once for all of them
+        GemmArgs wide{head.element, m->output, head.N, head.K, m->h, NH_F32, m->c.batch, m->logits, nullptr, head.N};
+        wide.norm_w = m->output_norm, wide.eps = m->c.eps;
+        status = launch_gemm(m->d, wide);
+    } else {
+        status = launch_gemv(m->d, head);
+    }
+    if (status != NH_OK) return status;
     // the choices and the refusal word go to the host's pinned words from a kernel of the step (part of the recorded graph): the
     // two device-to-host copies they would otherwise take are two more operations behind every step.  The greedy choice's
     // last kernel writes them itself; a sampled step has a kernel for it.

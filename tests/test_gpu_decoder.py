@@ -55,6 +55,26 @@ def test_decode_steps_match_oracle_logits_and_tokens(device, shape, element):
     model.release(), weights.release()
 
 
+@pytest.mark.parametrize("planes", [9, 16, 21])
+@pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K), (SMALL_Q4, NH_Q6_K)], ids=["q8_0", "q4_k", "q6_k"])
+def test_steps_of_more_planes_than_a_narrow_product_takes(device, shape, element, planes):
+    """Every product of a step runs as the wide product of few rows, the head over the whole vocabulary too; up to sixteen planes the
+    gate and the up projection share a launch that gates its outputs.  Eager, recorded and replayed steps at cursors of their own."""
+    model, ref, weights = build(device, shape, element, batch=planes, context=40, seed=planes)
+    rng = np.random.default_rng(planes)
+    first = rng.integers(0, 30, planes)
+    tokens = rng.integers(0, shape["vocab"], planes)
+    for step in range(5):
+        cursors = [int(at) + step for at in first]
+        want_logits, want = ref.forward(tokens, 1, cursors)
+        got = model.decode_step(tokens, cursors)
+        assert np.abs(model.logits() - want_logits).max() <= 1e-3 * np.abs(want_logits).max(), step
+        clear = margins(want_logits) > 2e-3 * np.abs(want_logits).max()
+        assert (np.asarray(got)[clear] == np.asarray(want)[clear]).all(), (step, margins(want_logits))
+        tokens = np.asarray(want)
+    model.release(), weights.release()
+
+
 @pytest.mark.parametrize("cache_element", [0, 30], ids=["single", "bfloat16"])
 @pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K)])
 def test_decoders_keep_their_states_in_single_or_bfloat16(device, shape, element, cache_element):

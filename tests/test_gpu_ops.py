@@ -593,6 +593,29 @@ def test_q6_k_q5_k_and_q3_k_wide_products_on_the_matrix_cores(device, element, M
     close(device.gemm(element, raw, N, K, X, residual=r), want + r)
 
 
+@pytest.mark.parametrize("form", ["0", "1"])
+@pytest.mark.parametrize("element,M,N,K,half", [
+    (NH_Q4_K, 1, 256, 256, False), (NH_Q4_K, 16, 96, 1536, False), (NH_Q4_K, 17, 130, 512, False), (NH_Q4_K, 48, 100, 2304, False), (NH_Q4_K, 100, 640, 1024, True),
+    (NH_Q5_K, 33, 33, 768, True), (NH_Q5_K, 9, 2080, 512, False), (NH_Q6_K, 5, 64, 2816, False), (NH_Q6_K, 65, 129, 1024, True), (NH_Q6_K, 49, 160, 256, False),
+    (NH_Q3_K, 12, 65, 2816, False), (NH_Q3_K, 97, 96, 512, True), (NH_Q8_0, 9, 77, 64, False), (NH_Q8_0, 40, 500, 192, False), (NH_Q8_0, 33, 300, 4864, False),
+    (NH_Q8_0, 130, 33, 320, True)])
+def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, K, half):
+    """The wide product of few rows (operands in registers, the K shares of a workgroup's waves meeting in LDS) and the one of 128 x 128
+    tiles, each forced: single tiles, ragged columns and rows, one to three row tiles a wave and more, K of one unit, of fewer units than
+    waves and of half a Q8_0 unit -- against the exact product.  Bar: 22 bits of every activation take part and fp32 sums of K terms
+    in any order stay within a few rounding errors of the sum of magnitudes' root (1e-6 of the outputs' scale at these depths)."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_FEW", form)
+    rng = np.random.default_rng(M + N + K + element)
+    raw = synth.RANDOM[element](rng, N * K)
+    X = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    exact = X.astype(np.float64) @ weights.T
+    scale = np.sqrt((X.astype(np.float64) ** 2) @ (weights.T ** 2))  # a random product's own size, whatever its columns weigh
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    assert (np.abs(device.gemm(element, raw, N, K, X) - exact) <= 4e-6 * scale + 1e-30).all()
+    assert (np.abs(device.gemm(element, raw, N, K, X, residual=r) - (exact + r)) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r)) + 1e-30).all()
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
