@@ -78,6 +78,7 @@ struct nh_device {
     // recorded again when this no longer matches the count at its capture
     uint64_t moved = 0;
     uint32_t *refusal = nullptr;  // device word: 0 = none, else a refusal code
+    uint32_t *meets = nullptr;  // device words, zero between launches: where workgroups that share a product's K count each other (gemm_few.hip)
     uint32_t *tick = nullptr;  // device word that launch_tick moves on at the start of every pass over a decoder's layers: part of every tag word
     uint8_t *static_scratch = nullptr;  // this device's copy of the file-scope array nh_argmax_static works in (argmax.hip)
     struct RopeTable {

@@ -6,6 +6,7 @@
 #include "blocks.hpp"
 #include "common.hpp"
 #include "gemm_few.hpp"
+#include "gemv_shared.hpp"
 
 #include <cstdlib>
 
@@ -155,15 +156,20 @@ __device__ __forceinline__ void pack_piece(const _Float16 (&hi)[4], const _Float
     }
     if ((threadIdx.x & 7u) == 0) {
         const uint32_t sb = k >> 8, slot = (k >> 5) & 7u;
+        float left;
         {
             const float v = sum_hi * 0.015625f;
             const _Float16 h = (_Float16)v;
             _Float16 *dst = S + (FEW ? few_sums_at(row, sb, nsb, 0) : ((size_t)row * nsb + sb) * 16u);
+            const float rest = (v - (float)h) * 2048.0f;
+            const _Float16 residue = (_Float16)rest;
             dst[slot] = h;
-            dst[(FEW ? 256u : 8u) + slot] = (_Float16)((v - (float)h) * 2048.0f);
+            dst[(FEW ? 256u : 8u) + slot] = residue;
+            left = rest - (float)residue;
         }
         if (SPLIT) {
-            const float v = sum_lo * 0.015625f;
+            // (a sum of 32 is longer than 22 bits, and the minimums' part largely cancels: what the value row's sum drops goes in here)
+            const float v = fmaf(sum_lo, 0.015625f, left);
             const _Float16 h = (_Float16)v;
             _Float16 *dst = S + (FEW ? few_sums_at(row + 1u, sb, nsb, 0) : ((size_t)(row + 1u) * nsb + sb) * 16u);
             dst[slot] = h;
@@ -255,12 +261,13 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
 // with the norm, 37 on an 18944-wide gated one.  Here a row crosses memory once, four 16-byte loads a thread in flight at a
 // time, and waits in LDS as the prelude left it: the squares are added from LDS in the same thread order, the packing reads
 // LDS.  The same arithmetic on the same numbers: the packed rows are the kernel above's bit for bit.  K is a multiple of 4.
-template <int PRELUDE, bool FEW>
-__global__ __launch_bounds__(256) void gemm_pack_rows_staged_kernel(const float *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
+// THREADS: 256, or 1024 where the rows are too few to fill the chip -- the loads of a wide row are then all in flight at once.
+template <int PRELUDE, bool FEW, uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void gemm_pack_rows_staged_kernel(const float *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
                                                                     _Float16 *__restrict__ S, float *__restrict__ unscale,
                                                                     const float *__restrict__ aux, float eps) {
     extern __shared__ __attribute__((aligned(16))) float staged_row[];  // [K]
-    __shared__ uint32_t wave_top[4];
+    __shared__ uint32_t wave_top[THREADS / 64u];
     __shared__ float red[256];
     const uint32_t m = blockIdx.x, tid = threadIdx.x;
     const uint32_t nsb = (K + 255u) / 256u;
@@ -268,37 +275,46 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_staged_kernel(const float 
     const float *other = PRELUDE == PACK_NORM ? aux : (PRELUDE == PACK_SWIGLU ? aux + (size_t)m * K : nullptr);
     float norm = 1.0f;
     if (PRELUDE == PACK_NORM) {
-        for (uint32_t k0 = tid * 4u; k0 < K; k0 += 4096u) {
+        for (uint32_t k0 = tid * 4u; k0 < K; k0 += 16u * THREADS) {
             float4 held[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) held[j] = *reinterpret_cast<const float4 *>(xr + min(k0 + 1024u * j, K - 4u));
+            for (int j = 0; j < 4; j++) held[j] = *reinterpret_cast<const float4 *>(xr + min(k0 + 4u * THREADS * j, K - 4u));
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (k0 + 1024u * j < K) *reinterpret_cast<float4 *>(staged_row + k0 + 1024u * j) = held[j];
+                if (k0 + 4u * THREADS * j < K) *reinterpret_cast<float4 *>(staged_row + k0 + 4u * THREADS * j) = held[j];
         }
         __syncthreads();
-        float square = 0.0f;  // thread t adds the squares of columns t, t + 256, ... as rmsnorm_kernel does
-        for (uint32_t c = tid; c < K; c += 256) square = __fadd_rn(square, __fmul_rn(staged_row[c], staged_row[c]));
-        red[tid] = square;
-        __syncthreads();
-        for (uint32_t stride = 128; stride > 0; stride >>= 1) {
-            if (tid < stride) red[tid] = __fadd_rn(red[tid], red[tid + stride]);
-            __syncthreads();
+        // thread t of the first 256 adds the squares of columns t, t + 256, ... as rmsnorm_kernel does, and so does the tree above them
+        // (its last six levels within a wave)
+        if (THREADS == 256u || tid < 256u) {
+            float square = 0.0f;
+            for (uint32_t c = tid; c < K; c += 256) square = __fadd_rn(square, __fmul_rn(staged_row[c], staged_row[c]));
+            red[tid] = square;
         }
+        __syncthreads();
+        if (tid < 128u) red[tid] = __fadd_rn(red[tid], red[tid + 128u]);
+        __syncthreads();
+        if (tid < 64u) {
+            float square = __fadd_rn(red[tid], red[tid + 64u]);
+#pragma unroll
+            for (int stride = 32; stride > 0; stride >>= 1) square = __fadd_rn(square, __shfl_down(square, stride, 64));
+            if (tid == 0) red[0] = square;
+        }
+        __syncthreads();
         norm = rms_scale_of(red[0], K, eps);
     }
     uint32_t top = 0;
-    for (uint32_t k0 = tid * 4u; k0 < K; k0 += 4096u) {
+    for (uint32_t k0 = tid * 4u; k0 < K; k0 += 16u * THREADS) {
         float4 held[4], with[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const uint32_t k = min(k0 + 1024u * j, K - 4u);
+            const uint32_t k = min(k0 + 4u * THREADS * j, K - 4u);
             held[j] = PRELUDE == PACK_NORM ? *reinterpret_cast<const float4 *>(staged_row + k) : *reinterpret_cast<const float4 *>(xr + k);
             if (PRELUDE != PACK_PLAIN) with[j] = *reinterpret_cast<const float4 *>(other + k);
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if (k0 + 1024u * j >= K) continue;
+            if (k0 + 4u * THREADS * j >= K) continue;
             float4 v = held[j];
             if (PRELUDE == PACK_NORM) {
                 const float4 w = with[j];
@@ -311,19 +327,21 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_staged_kernel(const float 
             }
             top = max(max(top, __builtin_bit_cast(uint32_t, v.x) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.y) & 0x7fffffffu);
             top = max(max(top, __builtin_bit_cast(uint32_t, v.z) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.w) & 0x7fffffffu);
-            *reinterpret_cast<float4 *>(staged_row + k0 + 1024u * j) = v;  // the thread that packs these four wrote them
+            *reinterpret_cast<float4 *>(staged_row + k0 + 4u * THREADS * j) = v;  // the thread that packs these four wrote them
         }
     }
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, offset, 64));
     if ((tid & 63u) == 0) wave_top[tid >> 6] = top;
     __syncthreads();
-    top = max(max(wave_top[0], wave_top[1]), max(wave_top[2], wave_top[3]));
+    top = wave_top[0];
+#pragma unroll
+    for (uint32_t w = 1; w < THREADS / 64u; w++) top = max(top, wave_top[w]);
     // a power of two that puts the largest magnitude in [2^13, 2^14)
     const uint32_t raw = top >> 23, exponent = min(max(raw, 27u), 254u);
     const float scale = __builtin_bit_cast(float, (267u - exponent) << 23);
     if (tid == 0) unscale[m] = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
-    for (uint32_t k = tid * 4u; k < K; k += 1024u) {
+    for (uint32_t k = tid * 4u; k < K; k += 4u * THREADS) {
         const float4 v = *reinterpret_cast<const float4 *>(staged_row + k);
         const float t[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
         _Float16 hi[4], lo[4];
@@ -1195,28 +1213,34 @@ __global__ __launch_bounds__(512) void gemm_q3k_mfma_kernel(GemmQ4Params p) {
 // bytes of device scratch a Q4_K wide product over M activation rows of K numbers packs into
 size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows) {
     const size_t rows = ((half_rows ? M : (size_t)2 * M) + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;  // (whole tiles: few_operand_at)
-    return rows * K * sizeof(_Float16) + rows * ((K + 255u) / 256u) * 16u * sizeof(_Float16) + (size_t)M * sizeof(float);
+    return rows * K * sizeof(_Float16) + rows * ((K + 255u) / 256u) * 16u * sizeof(_Float16) + ((size_t)M * sizeof(float) + 15u) / 16u * 16u + FEW_PARTIAL_BYTES;
+}
+
+template <int PRELUDE, bool FEW, uint32_t THREADS>
+static int32_t pack_staged(nh_device *d, const GemmArgs &a, size_t lds, _Float16 *A, _Float16 *S, float *unscale, const float *aux, float eps) {
+    static bool roomy = false;
+    if (!roomy) {
+        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PRELUDE, FEW, THREADS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
+        roomy = true;
+    }
+    hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PRELUDE, FEW, THREADS>), dim3(a.M), dim3(THREADS), lds, d->stream, static_cast<const float *>(a.X), a.K, A, S, unscale, aux, eps);
+    NH_HIP(hipGetLastError());
+    return NH_OK;
 }
 
 template <bool FEW>
 static int32_t pack_rows(nh_device *d, const GemmArgs &a, bool half_rows, _Float16 *A, _Float16 *S, float *unscale) {
-    const float *none = nullptr, *rows = static_cast<const float *>(a.X);
+    const float *none = nullptr;
     const dim3 grid(a.M), block(256);
     if (half_rows) {
         hipLaunchKernelGGL((gemm_pack_rows_kernel<true, PACK_PLAIN, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f);
     } else if (a.K % 4u == 0 && a.K >= 4u && (size_t)a.K * sizeof(float) <= PACK_STAGED_LDS_MOST && !pack_unstaged()) {
         // a row of fp32 numbers crosses memory once and waits in LDS
         const size_t lds = (size_t)a.K * sizeof(float);
-        static bool roomy = false;
-        if (!roomy) {
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_PLAIN, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_NORM, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PACK_SWIGLU, FEW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-            roomy = true;
-        }
-        if (a.norm_w) hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_NORM, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, a.norm_w, a.eps);
-        else if (a.gate) hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_SWIGLU, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, a.gate, 0.0f);
-        else hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PACK_PLAIN, FEW>), grid, block, lds, d->stream, rows, a.K, A, S, unscale, none, 0.0f);
+        const bool many = a.M > 2u * (uint32_t)d->compute_units;
+        if (a.norm_w) return many ? pack_staged<PACK_NORM, FEW, 256>(d, a, lds, A, S, unscale, a.norm_w, a.eps) : pack_staged<PACK_NORM, FEW, 1024>(d, a, lds, A, S, unscale, a.norm_w, a.eps);
+        if (a.gate) return many ? pack_staged<PACK_SWIGLU, FEW, 256>(d, a, lds, A, S, unscale, a.gate, 0.0f) : pack_staged<PACK_SWIGLU, FEW, 1024>(d, a, lds, A, S, unscale, a.gate, 0.0f);
+        return many ? pack_staged<PACK_PLAIN, FEW, 256>(d, a, lds, A, S, unscale, none, 0.0f) : pack_staged<PACK_PLAIN, FEW, 1024>(d, a, lds, A, S, unscale, none, 0.0f);
     } else if (a.norm_w) {
         hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_NORM, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, a.norm_w, a.eps);
     } else if (a.gate) {
@@ -1248,7 +1272,8 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const bool few = gemm_few_takes(a.element, a.N, a.K, p.rows);
     if (a.gated && (!few || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
         return fail(NH_E_ARGUMENT, "this wide product gates no outputs (ask gemm_gates first)");
-    // scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row scales
+    // scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row scales, the sums workgroups of the product of few
+    // rows leave each other (the same for every product over the same rows: `packed` ones find them where they were)
     const size_t held = (size_t)(p.rows + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;
     const size_t halves = held * a.K * sizeof(_Float16), sums = held * ((a.K + 255u) / 256u) * 16u * sizeof(_Float16);
     uint8_t *room = static_cast<uint8_t *>(scratch(d, gemm_q4k_scratch_bytes(a.M, a.K, half_rows)));
@@ -1262,7 +1287,8 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
         return status;
     p.A = A, p.S = S, p.unscale = unscale;
     if (few)
-        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale, 1u, 1u}, a.gated);
+        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale, 1u, 1u, 1u,
+                                                        unscale + ((size_t)a.M + 3u) / 4u * 4u, d->meets}, a.gated);
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));

@@ -58,8 +58,9 @@ struct FewQ45 {
     static constexpr int STEPS = 4, PLANES = 1, CLOSED = 4;
     static constexpr uint32_t BYTES = FIFTH ? 176u : 144u;
     static constexpr bool FLOORS = true;
+    static constexpr float CENTRE = FIFTH ? 16.0f : 8.0f;
     u32x4 header, fifth, runs[4];
-    half2_t low_scale, high_scale;
+    half2_t low_scale, high_scale, low_centre, high_centre;
     __device__ __forceinline__ void fetch(const uint8_t *row, uint32_t unit, uint32_t, uint32_t part) {
         const uint8_t *block = row + (size_t)unit * BYTES;
         header = *(global_uint4)(uintptr_t)block;
@@ -69,10 +70,12 @@ struct FewQ45 {
     }
     __device__ __forceinline__ float scale() const { return (float)as_halves(header.x).x * 16384.0f; }  // operands are code * sc * 2^-14
     __device__ __forceinline__ float floor_scale() const { return (float)as_halves(header.x).y * -64.0f; }  // the sums are packed / 64
-    // the eight minimums as halves; k 8..15 meet the sums' residues * 2^11
-    __device__ __forceinline__ half8_t floors(uint32_t part) const {
+    __device__ __forceinline__ float centre_scale() const { return (float)as_halves(header.x).x * (64.0f * CENTRE); }
+    // the eight minimums (`scales`: the eight scales) as halves; k 8..15 meet the sums' residues * 2^11
+    __device__ __forceinline__ half8_t floors(uint32_t part, bool scales) const {
         const half2_t offset = {(_Float16)1024.0f, (_Float16)1024.0f};
-        const uint32_t lo4 = header.z & 0x3f3f3f3fu, hi4 = ((header.w >> 4) & 0x0f0f0f0fu) | ((header.z >> 2) & 0x30303030u);
+        const uint32_t first = scales ? header.y : header.z, more = scales ? header.w : header.w >> 4;
+        const uint32_t lo4 = first & 0x3f3f3f3fu, hi4 = (more & 0x0f0f0f0fu) | ((first >> 2) & 0x30303030u);
         half2_t m[4] = {as_halves(__builtin_amdgcn_perm(0u, lo4, 0x0c010c00u) | 0x64006400u) - offset,
                         as_halves(__builtin_amdgcn_perm(0u, lo4, 0x0c030c02u) | 0x64006400u) - offset,
                         as_halves(__builtin_amdgcn_perm(0u, hi4, 0x0c010c00u) | 0x64006400u) - offset,
@@ -89,6 +92,12 @@ struct FewQ45 {
         const uint32_t sc = g < 2 ? (ya & 0x3f3fu) : ((wa & 0x0f0fu) | ((ya >> 2) & 0x3030u));
         const half2_t scales = (as_halves(__builtin_amdgcn_perm(0u, sc, 0x0c010c00u) | 0x64006400u) - offset) * powers;  // (sc0 * 2^10, sc1 * 2^6)
         low_scale = half2_t{scales.x, scales.x}, high_scale = half2_t{scales.y, scales.y};
+        // a code enters less CENTRE: the products then add up to sums of the output's own size, and not to ones that the minimums
+        // take most of off again (2-norm from the exact products, eight rows of the 7B shapes: 2.2e-7 -> 1.1e-7); CENTRE times
+        // the scales comes back with the minimums.  (code - CENTRE) * sc * 2^-14 is exact: one rounding, of a whole number below 2^11
+        const half2_t down = {(_Float16)(-CENTRE * 0.000000059604644775390625f), (_Float16)(-CENTRE * 0.00000095367431640625f)};
+        const half2_t centres = scales * down;
+        low_centre = half2_t{centres.x, centres.x}, high_centre = half2_t{centres.y, centres.y};
     }
     __device__ __forceinline__ void operand(int g, int depth, half8_t (&b)[PLANES]) const {
         const uint32_t words[4] = {runs[g].x, runs[g].y, runs[g].z, runs[g].w}, fifths[4] = {fifth.x, fifth.y, fifth.z, fifth.w};
@@ -103,8 +112,8 @@ struct FewQ45 {
                 const uint32_t bits = fifths[at] >> (2 * g + (depth < 2 ? 0 : 1));
                 even |= (bits & 0x00010001u) << (depth < 2 ? 4 : 8), odd |= ((bits >> 8) & 0x00010001u) << (depth < 2 ? 4 : 8);
             }
-            const half2_t scale = depth < 2 ? low_scale : high_scale;
-            out[2 * w] = as_word(as_halves(even) * scale), out[2 * w + 1] = as_word(as_halves(odd) * scale);
+            const half2_t scale = depth < 2 ? low_scale : high_scale, centre = depth < 2 ? low_centre : high_centre;
+            out[2 * w] = as_word(__builtin_elementwise_fma(as_halves(even), scale, centre)), out[2 * w + 1] = as_word(__builtin_elementwise_fma(as_halves(odd), scale, centre));
         }
         b[0] = __builtin_bit_cast(half8_t, u32x4{out[0], out[1], out[2], out[3]});
     }
@@ -277,6 +286,8 @@ template <> struct FewOf<NH_Q6_K> { typedef FewQ6 type; };
 template <> struct FewOf<NH_Q3_K> { typedef FewQ3 type; };
 template <> struct FewOf<NH_Q8_0> { typedef FewQ8 type; };
 
+constexpr uint32_t FEW_SLICES_MOST = 8;
+
 // MT: tiles of 32 packed rows a wave multiplies its weights by; GATED: a wave walks the same 32 columns of the gate and of the up
 // matrix, and what leaves is silu(gate) * up; AHEAD: steps the activation operands are read ahead (the loads of a wave come
 // back in order: an operand asked for after the next super-block's weights waits for them, so they are asked for
@@ -292,7 +303,7 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
     float4 *parts = reinterpret_cast<float4 *>(few_lds);  // [wave][NT][MT][4][64]
     const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, part = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t share = wave % p.deep, beside = wave / p.deep;
+    const uint32_t within = wave % p.deep, beside = wave / p.deep, shares = p.deep * p.slices, share = blockIdx.z * p.deep + within;
     const uint32_t n0 = (blockIdx.x * p.across + beside) * FEW_TILE, tile0 = blockIdx.y * MT;
     const uint32_t steps = p.K / 64u, units = (steps + STEPS - 1u) / STEPS;
     const uint32_t nsb = p.K / 256u;
@@ -340,10 +351,10 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
         for (int s = 0; s < SLOTS; s++)
 #pragma unroll
             for (int depth = 0; depth < 4; depth++) fetch_rows(s, depth, share * STEPS + s);
-        for (uint32_t unit = share; unit < units; unit += p.deep) {
+        for (uint32_t unit = share; unit < units; unit += shares) {
             Weights w[NT];
             half8_t sums[MT];
-            const uint32_t after = min(unit + p.deep, units - 1u);  // past the end the last unit again, dropped
+            const uint32_t after = min(unit + shares, units - 1u);  // past the end the last unit again, dropped
 #pragma unroll
             for (int t = 0; t < NT; t++) w[t] = next[t];
             if (Weights::FLOORS) {
@@ -410,13 +421,14 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
             if constexpr (Weights::FLOORS) {
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    const half8_t b = w[t].floors(part);
-                    const float floor_scale = w[t].floor_scale();
+                    const half8_t b = w[t].floors(part, false), c = w[t].floors(part, true);
+                    const float floor_scale = w[t].floor_scale(), centre_scale = w[t].centre_scale();
 #pragma unroll
                     for (int i = 0; i < MT; i++) {
                         const f32x16 floors = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], b, zero, 0, 0, 0);
+                        const f32x16 centres = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], c, zero, 0, 0, 0);
 #pragma unroll
-                        for (int e = 0; e < 16; e++) acc[t][i][e] = fmaf(floor_scale, floors[e], acc[t][i][e]);
+                        for (int e = 0; e < 16; e++) acc[t][i][e] += fmaf(floor_scale, floors[e], centre_scale * centres[e]);
                     }
                 }
             }
@@ -431,20 +443,72 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
                 parts[(((wave * NT + t) * MT + i) * 4u + q) * 64u + lane] = float4{acc[t][i][4 * q], acc[t][i][4 * q + 1], acc[t][i][4 * q + 2], acc[t][i][4 * q + 3]};
     __syncthreads();
     // ---- out: an item is column l32 and rows 8q + 4 part .. + 3 of a 32 x 32 block; the shares of K are added in their order
-    for (uint32_t item = threadIdx.x; item < p.across * MT * 256u; item += blockDim.x) {
+    const uint32_t items = p.across * MT * 256u;
+    auto own_sum = [&](uint32_t item, int t) {
         const uint32_t at = item & 63u, q = (item >> 6) & 3u, i = (item >> 8) % MT, b = (item >> 8) / MT;
+        float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t s = 0; s < p.deep; s++) {
+            const float4 add = parts[((((b * p.deep + s) * NT + t) * MT + i) * 4u + q) * 64u + at];
+            v.x += add.x, v.y += add.y, v.z += add.z, v.w += add.w;
+        }
+        return v;
+    };
+    auto row_of = [&](uint32_t item) { return (tile0 + (item >> 8) % MT) * FEW_TILE + 8u * ((item >> 6) & 3u) + 4u * ((item >> 5) & 1u); };
+    // with more workgroups over the same outputs: each leaves its sums in memory and the last to arrive adds them, in the order of
+    // the slices, so the sums do not depend on who that is.  Nobody waits for another.
+    typedef unsigned long long pair_word;
+    auto place_of = [&](uint32_t slice, uint32_t item, int t) {
+        const size_t place = ((size_t)slice * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        return reinterpret_cast<pair_word *>(p.partial) + ((place * items + item) * NT + t) * 2u;
+    };
+    if (p.slices > 1u) {
+        for (uint32_t item = threadIdx.x; item < items; item += blockDim.x) {
+            if (row_of(item) >= p.rows) continue;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const float4 v = own_sum(item, t);
+                pair_word *to = place_of(blockIdx.z, item, t);
+                __hip_atomic_store(to, __builtin_bit_cast(pair_word, float2{v.x, v.y}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(to + 1, __builtin_bit_cast(pair_word, float2{v.z, v.w}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        // the stores go past the caches that other workgroups do not share, and the loads below come from there: what is left to
+        // order is their completion (a fence would write back and drop whole caches: 20 to 90 us a launch)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // (every wave's sums are out, and the last word of LDS read)
+        uint32_t *arrived = reinterpret_cast<uint32_t *>(few_lds), *meet = p.meets + blockIdx.y * gridDim.x + blockIdx.x;
+        if (threadIdx.x == 0) arrived[0] = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (arrived[0] != p.slices - 1u) return;
+        asm volatile("" ::: "memory");
+        if (threadIdx.x == 0) __hip_atomic_store(meet, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // as the next launch expects it
+    }
+    for (uint32_t item = threadIdx.x; item < items; item += blockDim.x) {
+        const uint32_t row = row_of(item), n = (blockIdx.x * p.across + (item >> 8) / MT) * FEW_TILE + (item & 31u);
+        if (n >= p.N || row >= p.rows) continue;
         float v[NT][4];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             v[t][0] = v[t][1] = v[t][2] = v[t][3] = 0.0f;
-            for (uint32_t s = 0; s < p.deep; s++) {
-                const float4 add = parts[((((b * p.deep + s) * NT + t) * MT + i) * 4u + q) * 64u + at];
-                v[t][0] += add.x, v[t][1] += add.y, v[t][2] += add.z, v[t][3] += add.w;
+            if (p.slices == 1u) {
+                const float4 sum = own_sum(item, t);
+                v[t][0] = sum.x, v[t][1] = sum.y, v[t][2] = sum.z, v[t][3] = sum.w;
+            } else {
+                pair_word held[FEW_SLICES_MOST][2];
+#pragma unroll
+                for (uint32_t s = 0; s < FEW_SLICES_MOST; s++) {
+                    const pair_word *from = place_of(min(s, p.slices - 1u), item, t);
+                    held[s][0] = __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    held[s][1] = __hip_atomic_load(from + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (uint32_t s = 0; s < FEW_SLICES_MOST; s++) {
+                    if (s >= p.slices) break;
+                    const float2 low = __builtin_bit_cast(float2, held[s][0]), high = __builtin_bit_cast(float2, held[s][1]);
+                    v[t][0] += low.x, v[t][1] += low.y, v[t][2] += high.x, v[t][3] += high.y;
+                }
             }
         }
-        const uint32_t n = (blockIdx.x * p.across + b) * FEW_TILE + (at & 31u);
-        const uint32_t row = (tile0 + i) * FEW_TILE + 8u * q + 4u * (at >> 5);
-        if (n >= p.N) continue;
         auto leave = [&](uint32_t m, float value, float up) {
             if (m >= p.M) return;
             if (GATED) value = value * (1.0f / (1.0f + expf(-value))) * up;
@@ -465,6 +529,8 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
     }
 }
 
+constexpr uint32_t slice_list[] = {1, 2, 3, 4, 6, 8};
+
 template <int ELEMENT, int MT, bool GATED>
 int32_t launch_few(nh_device *d, FewParams p) {
     constexpr int STEPS = FewOf<ELEMENT>::type::STEPS;
@@ -472,21 +538,27 @@ int32_t launch_few(nh_device *d, FewParams p) {
     constexpr int AHEAD = MT * NT > 2 ? 1 : (STEPS < 4 || MT * NT > 1 ? 2 : 4);
     const uint32_t units = (p.K / 64u + STEPS - 1u) / STEPS, tiles = (p.N + FEW_TILE - 1u) / FEW_TILE, row_tiles = (p.rows + FEW_TILE - 1u) / FEW_TILE;
     // the split of a workgroup's waves that walks the fewest units: rounds of workgroups times the units of a wave (and what a
-    // workgroup takes before its first and after its last, about two units' time)
+    // workgroup takes before its first and after its last, about two units' time).  A matrix of few tiles and deep rows leaves most
+    // of the chip idle that way, so K may be shared among workgroups too: their meeting costs a unit's time and the passage of
+    // their sums, 2.5 MB in another (eight rows of fp32, with the packing: ffn_down of the 7B shape Q8_0 55 -> 37 us, Q6_K
+    // 45 -> 34, Q5_K 37 -> 29, of the 1.5B shape Q8_0 28 -> 18; gate|up of the 7B shape, 592 tiles, is better left alone: Q4_K 34, not 38)
     uint32_t best = ~0u;
     for (uint32_t across = 1; across <= 4u; across *= 2u)
-        for (uint32_t deep = 1; deep * across <= 8u; deep++) {
-            const uint32_t groups = ((tiles + across - 1u) / across) * ((row_tiles + MT - 1u) / MT), resident = 256u * (8u / (deep * across));
-            const uint32_t cost = ((groups + resident - 1u) / resident) * ((units + deep - 1u) / deep + 2u) * 64u + across * deep;
-            if (cost < best) best = cost, p.across = across, p.deep = deep;
-        }
+        for (uint32_t deep = 1; deep * across <= 8u; deep++)
+            for (uint32_t slices : slice_list) {
+                const uint32_t places = ((tiles + across - 1u) / across) * ((row_tiles + MT - 1u) / MT), resident = 256u * (8u / (deep * across));
+                if (slices > 1u && (places > FEW_MEETS || deep * slices > units || (size_t)slices * places * across * MT * NT * 4096u > FEW_PARTIAL_BYTES)) continue;
+                const uint32_t meeting = slices > 1u ? 64u + (uint32_t)((uint64_t)slices * p.N * NT * p.rows * 4u * 64u / 2500000u) : 0u;
+                const uint32_t cost = ((places * slices + resident - 1u) / resident) * ((units + deep * slices - 1u) / (deep * slices) + 2u) * 64u + meeting + across * deep;
+                if (cost < best) best = cost, p.across = across, p.deep = deep, p.slices = slices;
+            }
     const size_t lds = (size_t)p.across * p.deep * NT * MT * 4096u;
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), hipFuncAttributeMaxDynamicSharedMemorySize, 8 * NT * MT * 4096));
         sized = true;
     }
-    const dim3 grid((tiles + p.across - 1u) / p.across, (row_tiles + MT - 1u) / MT);
+    const dim3 grid((tiles + p.across - 1u) / p.across, (row_tiles + MT - 1u) / MT, p.slices);
     hipLaunchKernelGGL((gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), grid, dim3(64u * p.across * p.deep), lds, d->stream, p);
     NH_HIP(hipGetLastError());
     return NH_OK;

@@ -24,6 +24,10 @@ __host__ __device__ inline size_t few_sums_at(uint32_t row, uint32_t sb, uint32_
     return ((((size_t)(row >> 5) * nsb + sb) * 2u + part) * 32u + (row & 31u)) * 8u;
 }
 
+// where K is shared among workgroups: the most their sums may take, and the most places they may meet at
+constexpr size_t FEW_PARTIAL_BYTES = 16u << 20;
+constexpr uint32_t FEW_MEETS = 1024;
+
 struct FewParams {
     const uint8_t *W, *W1, *W2;  // matrices stacked along N, column ends end0 and end1 (multiples of the tile); gated: gate and up, N columns each
     uint32_t end0, end1;
@@ -36,6 +40,9 @@ struct FewParams {
     int32_t split;
     const float *unscale;
     uint32_t across, deep;  // the waves of a workgroup: tiles of columns x shares of K
+    uint32_t slices;        // workgroups (blockIdx.z) that share the K of the same tiles
+    float *partial;         // FEW_PARTIAL_BYTES of scratch for their sums
+    uint32_t *meets;        // FEW_MEETS words, zero between launches: workgroups of a place that have left their sums
 };
 
 // whether the product of `rows` packed rows is this kernel's, and its launch (the rows are packed)

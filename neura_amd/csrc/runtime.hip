@@ -1,6 +1,7 @@
 // Device handle, memory, timing and the weight arena: the part of the library that stands
 // where the reference's GPU abstraction (device / queue / buffer / submission) stands.
 #include "common.hpp"
+#include "gemm_few.hpp"
 
 #include <cmath>
 #include <cstdlib>
@@ -123,7 +124,9 @@ nh_device *nh_open(int32_t device_index) {
     bool ok = hipStreamCreateWithFlags(&device->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&device->started) == hipSuccess && hipEventCreate(&device->stopped) == hipSuccess &&
               hipMalloc((void **)&device->refusal, 256) == hipSuccess && hipMemset(device->refusal, 0, 256) == hipSuccess &&
-              hipMalloc((void **)&device->tick, 256) == hipSuccess && hipMemset(device->tick, 0, 256) == hipSuccess;
+              hipMalloc((void **)&device->tick, 256) == hipSuccess && hipMemset(device->tick, 0, 256) == hipSuccess &&
+              hipMalloc((void **)&device->meets, FEW_MEETS * sizeof(uint32_t)) == hipSuccess &&
+              hipMemset(device->meets, 0, FEW_MEETS * sizeof(uint32_t)) == hipSuccess && hipStreamSynchronize(nullptr) == hipSuccess;
     if (!ok) {
         fail(NH_E_DEVICE, "device %d opens no stream, events or refusal word", device_index);
         nh_close(device);
@@ -144,6 +147,7 @@ void nh_close(nh_device *device) {
     for (void *block : device->retired) (void)hipFree(block);
     if (device->refusal) (void)hipFree(device->refusal);
     if (device->tick) (void)hipFree(device->tick);
+    if (device->meets) (void)hipFree(device->meets);
     for (const nh_device::RopeTable &known : device->rope_tables) (void)hipFree(known.table);
     for (hipEvent_t event : device->profile_events) (void)hipEventDestroy(event);
     if (device->started) (void)hipEventDestroy(device->started);

@@ -616,6 +616,28 @@ def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, 
     assert (np.abs(device.gemm(element, raw, N, K, X, residual=r) - (exact + r)) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r)) + 1e-30).all()
 
 
+@pytest.mark.parametrize("element,M,N,K", [
+    (NH_Q4_K, 8, 96, 8960), (NH_Q4_K, 48, 33, 18944), (NH_Q5_K, 5, 160, 4608), (NH_Q5_K, 17, 64, 2560), (NH_Q6_K, 16, 130, 8960), (NH_Q3_K, 3, 32, 18944),
+    (NH_Q3_K, 100, 96, 8960), (NH_Q8_0, 9, 77, 4864), (NH_Q8_0, 33, 256, 8960), (NH_Q8_0, 2, 31, 18944)])
+def test_wide_products_whose_depth_is_shared_among_workgroups(device, monkeypatch, element, M, N, K):
+    """Few tiles of deep rows: several workgroups share K and the last to arrive adds their sums, in one order -- the same bits on every
+    run, whatever ran between, and within the bar of test_both_forms_of_a_wide_product of the exact product (a K of 18944: sqrt(K)
+    rounding errors of 2^-24 each are 8e-6 of one term's size, 1e-7 of the outputs' scale, and the bar stands)."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_FEW", "1")
+    rng = np.random.default_rng(M + N + K + element)
+    raw = synth.RANDOM[element](rng, N * K)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    exact = X.astype(np.float64) @ weights.T
+    scale = np.sqrt((X.astype(np.float64) ** 2) @ (weights.T ** 2))
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    first = device.gemm(element, raw, N, K, X)
+    assert (np.abs(first - exact) <= 4e-6 * scale + 1e-30).all()
+    assert (np.abs(device.gemm(element, raw, N, K, X, residual=r) - (exact + r)) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r)) + 1e-30).all()
+    for _ in range(3):
+        assert np.array_equal(device.gemm(element, raw, N, K, X), first)
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
