@@ -265,6 +265,8 @@ int32_t launch_gemm(nh_device *d, const GemmArgs &args);
 // activations the launch before packed
 bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, const void *W1, const void *W2, uint32_t end0, uint32_t end1);
 bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up);
+// whether three products over the same M rows of K numbers pack them alike: the second and third may be `packed`
+bool gemm_shares_rows(const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M);
 // device scratch a Q4_K wide product over M rows of K activations packs them into
 size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows);
 
@@ -300,13 +302,14 @@ int32_t launch_attention(nh_device *d, const AttentionArgs &args);
 int32_t launch_rope_angles(nh_device *d, float base, uint32_t width, uint32_t positions, float *cosines, float *sines);
 int32_t launch_rope_append(nh_device *d, float *qkv, uint32_t heads, uint32_t kv_heads, uint32_t width, uint32_t batch, uint32_t rows,
                            void *cache_k, void *cache_v, uint32_t capacity, uint32_t window, const uint32_t *cursor,
-                           const uint8_t *mask, float base, bool ring, int32_t cache_element = NH_F16, const float *cosines = nullptr,
-                           const float *sines = nullptr, uint32_t positions = 0);  // (a model's table of cosines and sines, where it has one)
+                           const uint8_t *mask, float base, bool ring, int32_t cache_element, const float *cosines,
+                           const float *sines, uint32_t positions,  // (a model's table of cosines and sines; may be null)
+                           const float *const *biases);             // of q, k and v, added first; any may be null
 
 // one token of one plane: v (+ bias) as halves into the value state at cursor[0] (at cursor[0] % ring when the cache is a ring)
 int32_t launch_value_append(nh_device *d, const float *v, const float *bias, void *cache_v, uint32_t kv_heads, uint32_t width, uint32_t capacity,
                             const uint32_t *cursor, uint32_t ring, int32_t cache_element = NH_F16);
-int32_t launch_columns(nh_device *d, const float *src, uint32_t lds, const float *bias, float *dst, uint32_t ldd, uint32_t rows, uint32_t n);
+int32_t launch_columns(nh_device *d, const float *src, uint32_t lds, float *dst, uint32_t ldd, uint32_t rows, uint32_t n);
 
 int32_t launch_pack_q8_0(nh_device *d, const float *src, uint64_t elements, uint8_t *dst);
 int32_t launch_gather(nh_device *d, int32_t element, const void *table, uint32_t vocab, uint32_t width, const uint32_t *tokens,

@@ -1335,6 +1335,51 @@ bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void 
            2u * M <= FEW_TILE && gemm_few_takes(element, N, K, 2u * M);
 }
 
+bool gemm_shares_rows(const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M) {
+    for (int s = 0; s < 3; s++)
+        if (!mfma_takes(elements[s], K, X, W[s]) || gemm_few_takes(elements[s], N[s], K, 2u * M) != gemm_few_takes(elements[0], N[0], K, 2u * M)) return false;
+    return true;
+}
+
+// Where the line lies (us, the vector and staged kernels, which walk the weights once for every two or four rows, -> here).  Q4_K has
+// tiles of its own and stays (7B shape, eight rows: gate|up 26 against 34, ffn_down 24 against 27).  Of the others five rows are three passes or
+// two and always lose, three rows are two (7B shape, eight rows: Q8_0 gate|up 307 -> 60, Q6_K ffn_down 103 -> 34; 0.5B shape: Q8_0
+// q|k|v 19 -> 8).  Four and two rows are one pass, and the packing (4 to 5 us) wants a matrix to be worth it: four rows Q8_0 always (1.5B
+// q|k|v 11 -> 9), the staged formats from 6 M numbers on (7B attn_output, 12.8 M: Q6_K 18 -> 16, Q3_K 18 -> 12; 1.5B q|k|v, 3.1 M: 7.4 against
+// 9.4); two rows Q8_0 from 12 M (7B attn_output 19 -> 14; 0.5B gate|up, 8.7 M: 10 against 11), Q5_K and Q3_K from 13 M (1.5B ffn_down,
+// 13.8 M: Q5_K 19 -> 15; 7B attn_output: 11 against 12), Q6_K from 60 M (7B ffn_down, 67.9 M: 34 -> 33; 1.5B gate|up, 27.5 M: 21 against 22).
+// The error against 64 bits is no larger (2-norm, those shapes: Q8_0 2.3..4e-7 -> 1.0..2.3e-7, Q6_K 1.5..2.3e-7 -> 1.2..1.9e-7, Q5_K
+// 1.5..2.4e-7 -> 1.3..2.1e-7, Q3_K 1.4..2.2e-7 -> 1.0..1.6e-7).
+bool gemv_wide_takes(const GemvArgs &a) {
+    const int held = env_int("NEURA_HIP_GEMV_WIDE", 1);  // 0 never, 2 wherever it can
+    if (held == 0 || a.rows < 2u || a.rows > 8u || a.rope || a.append_value || a.merge || a.digits_in || a.digits_out || a.pairs_out) return false;
+    if (held != 2) {
+        if (a.element == NH_Q4_K) return false;
+        const uint64_t numbers = (uint64_t)a.N * a.K;
+        const uint64_t two = a.element == NH_Q8_0 ? 12000000u : a.element == NH_Q6_K ? 60000000u : 13000000u;
+        if (a.rows == 4u && a.element != NH_Q8_0 && numbers < 6000000u) return false;
+        if (a.rows == 2u && numbers < two) return false;
+    }
+    if ((uintptr_t)a.norm_w & 15u) return false;
+    const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
+    if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(a.element, outputs, a.K, a.rows, a.x, a.W[0], a.W[1]);
+    if (!gemm_few_takes(a.element, a.N, a.K, 2u * a.rows)) return false;
+    return gemm_stacks(a.element, a.K, a.x, a.W[0], a.W[1], a.W[2], a.end[0], a.end[1]);
+}
+
+int32_t launch_gemv_wide(nh_device *d, const GemvArgs &a) {
+    const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
+    GemmArgs g{a.element, a.W[0], outputs, a.K, a.x, NH_F32, a.rows, a.y, a.residual, outputs};
+    g.W_more[0] = a.W[1], g.W_more[1] = a.W[2], g.end[0] = a.end[0], g.end[1] = a.end[1];
+    g.norm_w = a.norm_w, g.eps = a.eps;
+    if (a.swiglu) g.gated = true, g.W_more[1] = nullptr;
+    profile_mark(d);
+    if (const int32_t status = launch_gemm_mfma(d, g); status != NH_OK) return status;
+    profile_mark(d);
+    if (d->profile) d->profile_bytes += (uint64_t)a.N * payload_bytes(a.element, a.K);
+    return NH_OK;
+}
+
 int32_t launch_gemm(nh_device *d, const GemmArgs &a) {
     if (!a.M || !a.N) return NH_OK;
     if (mfma_takes(a.element, a.K, a.X, a.W)) return launch_gemm_mfma(d, a);

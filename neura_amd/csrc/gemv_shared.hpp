@@ -237,6 +237,9 @@ int32_t launch_tile16(nh_device *d, const GemvArgs &args);
 // the same for two to eight activation rows, four rows to an MFMA
 bool rows4_takes(const GemvArgs &args);
 int32_t launch_rows4(nh_device *d, const GemvArgs &args);
+// several activation rows as a wide product of few rows (gemm.hip)
+bool gemv_wide_takes(const GemvArgs &args);
+int32_t launch_gemv_wide(nh_device *d, const GemvArgs &args);
 // one activation row against a Q6_K matrix on the same tiles (gemv_q6k_tile16.hip)
 bool q6k_tile16_takes(const GemvArgs &args);
 int32_t launch_q6k_tile16(nh_device *d, const GemvArgs &args);

@@ -142,14 +142,19 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
     const float scale = 1.0f / sqrtf((float)hd);
     for (uint32_t L = 0; L < c.layers; L++) {
         bool roped = false;
-        if (wide) {
+        const float *biases[3] = {m->bias_q[L], m->bias_k[L], m->bias_v[L]};  // added by the rotation, in the product or behind it
+        const bool alike = element_at(m, L, Q) == element_at(m, L, K_) && element_at(m, L, Q) == element_at(m, L, V);
+        const int32_t elements[3] = {element_at(m, L, Q), element_at(m, L, K_), element_at(m, L, V)};
+        const bool shares_rows = !alike && T > 1 && gemm_shares_rows(elements, {m->attn_q[L], m->attn_k[L], m->attn_v[L]}, {QW, KW, KW}, H, m->h, T);
+        if (wide || shares_rows) {
             const uint8_t *mats[3] = {m->attn_q[L], m->attn_k[L], m->attn_v[L]};
-            const float *biases[3] = {m->bias_q[L], m->bias_k[L], m->bias_v[L]};
             const uint32_t widths[3] = {QW, KW, KW};
-            const bool alike = element_at(m, L, Q) == element_at(m, L, K_) && element_at(m, L, Q) == element_at(m, L, V);
             const bool stacked = alike && gemm_stacks(element_at(m, L, Q), H, m->h, mats[0], mats[1], mats[2], QW, QW + KW);
             uint32_t column = 0;
-            if (!stacked && (status = launch_rmsnorm(d, m->h, nullptr, m->attn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
+            // matrices of different elements: the norm still rides in a pass that packs the rows, once for the three products (the
+            // Q4_K_M mix of the 7B shape at five planes: 68 us of products and columns in such a layer -> 32)
+            const bool shared = !stacked && shares_rows;
+            if (!stacked && !shared && (status = launch_rmsnorm(d, m->h, nullptr, m->attn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
             if (stacked) {
                 // q|k|v as one product (the key and value projections alone are a few dozen workgroups each), the norm
                 // done by the pass that packs the rows
@@ -157,21 +162,15 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
                 g.W_more[0] = mats[1], g.W_more[1] = mats[2], g.end[0] = QW, g.end[1] = QW + KW;
                 g.norm_w = m->attn_norm[L], g.eps = c.eps;
                 if ((status = launch_gemm(d, g)) != NH_OK) return status;
-                for (int s = 0; s < 3; s++) {
-                    if (biases[s] && (status = launch_columns(d, m->qkv + column, QKV, biases[s], m->qkv + column, QKV, T, widths[s])) != NH_OK) return status;
-                    column += widths[s];
-                }
             } else {
                 for (int s = 0; s < 3; s++) {
-                    GemmArgs g{element_at(m, L, Q + s), mats[s], widths[s], H, m->xn, NH_F32, T, m->qkv + column, nullptr, QKV};
+                    GemmArgs g{element_at(m, L, Q + s), mats[s], widths[s], H, shared ? m->h : m->xn, NH_F32, T, m->qkv + column, nullptr, QKV};
+                    if (shared) g.norm_w = m->attn_norm[L], g.eps = c.eps, g.packed = s > 0;
                     if ((status = launch_gemm(d, g)) != NH_OK) return status;
-                    if (biases[s] && (status = launch_columns(d, m->qkv + column, QKV, biases[s], m->qkv + column, QKV, T, widths[s])) != NH_OK) return status;
                     column += widths[s];
                 }
             }
         } else {
-            const bool biased = m->bias_q[L] || m->bias_k[L] || m->bias_v[L];
-            const bool alike = element_at(m, L, Q) == element_at(m, L, K_) && element_at(m, L, Q) == element_at(m, L, V);
             GemvArgs a = narrow(m, element_at(m, L, Q), m->attn_q[L], QKV, H, m->h, T, m->qkv);
             a.W[1] = m->attn_k[L], a.W[2] = m->attn_v[L];
             a.end[0] = QW, a.end[1] = QW + KW, a.end[2] = QKV;
@@ -196,7 +195,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             RopeFusion rope_qk = rope;
             const bool split_value = halves && !alike && element_at(m, L, Q) == element_at(m, L, K_) && !products_only && T == 1 && !mask &&
                                      gemv_fuses_rope(qk, rope_qk);
-            if (roped || (alike && (!biased || products_only))) {
+            if (alike) {
                 if ((status = launch_gemv(d, a)) != NH_OK) return status;
             } else if (split_value) {
                 qk.rope = &rope_qk;
@@ -219,23 +218,22 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
                     return status;
                 roped = true;
             } else {
-                // matrices of different elements, or biases outside the folded rotation: one product each, placed side by side
+                // matrices of different elements: one product each, placed side by side
                 const uint8_t *mats[3] = {m->attn_q[L], m->attn_k[L], m->attn_v[L]};
-                const float *biases[3] = {m->bias_q[L], m->bias_k[L], m->bias_v[L]};
                 const uint32_t widths[3] = {QW, KW, KW};
                 uint32_t column = 0;
                 for (int s = 0; s < 3; s++) {
                     GemvArgs one = narrow(m, element_at(m, L, Q + s), mats[s], widths[s], H, m->h, T, m->xn);
                     one.norm_w = m->attn_norm[L], one.eps = c.eps;
                     if ((status = launch_gemv(d, one)) != NH_OK) return status;
-                    if ((status = launch_columns(d, m->xn, widths[s], products_only ? nullptr : biases[s], m->qkv + column, QKV, T, widths[s])) != NH_OK) return status;
+                    if ((status = launch_columns(d, m->xn, widths[s], m->qkv + column, QKV, T, widths[s])) != NH_OK) return status;
                     column += widths[s];
                 }
             }
         }
         if (!products_only && !roped && (status = launch_rope_append(d, m->qkv, c.heads, c.kv_heads, hd, B, rows, m->cache_k[L], m->cache_v[L],
                                                            m->capacity, m->window, dev_cursor(m), mask, c.rope_base, m->ring, c.cache_element, m->rope_cos, m->rope_sin,
-                                                           m->positions)) != NH_OK)
+                                                           m->positions, biases)) != NH_OK)
             return status;
         AttentionArgs at{};
         at.q = m->qkv, at.out = m->att;
@@ -517,7 +515,7 @@ nh_model *nh_model_create(nh_device *device, const nh_model_config *config, nh_w
         // the wide product packs its fp32 activations as two half rows each, with their sub-block sums and a scale per row
         size_t deepest = (size_t)(F > QW ? F : QW);
         if (H > deepest) deepest = H;
-        size_t split_rows = T > 8 ? gemm_q4k_scratch_bytes(T, (uint32_t)deepest, false) : 0;
+        size_t split_rows = T > 1 ? gemm_q4k_scratch_bytes(T, (uint32_t)deepest, false) : 0;
         size_t wanted = products > sections ? products : sections;
         if (choice > wanted) wanted = choice;
         if (split_rows > wanted) wanted = split_rows;

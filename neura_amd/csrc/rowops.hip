@@ -188,15 +188,17 @@ int32_t launch_rope_angles(nh_device *d, float base, uint32_t width, uint32_t po
 // A token a blockIdx.y, its (vector, channel pair) items over blockIdx.x: no 64-bit division on the way to an item.  `cosines` /
 // `sines` [positions][width / 2] (may be null): what rotate() would compute for (position, channel pair), tabulated by
 // rope_angles_kernel with the same instructions, so a table entry is bit for bit the cosine and sine formed on the spot;
-// positions past the table are formed on the spot.
+// positions past the table are formed on the spot.  The projections' biases (any may be null; head by head behind each other) are
+// added as the values arrive: a pass of their own for each of the three was 4 to 5 us of latency a launch.
 template <int CE>
 __global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ qkv, uint32_t heads, uint32_t kv_heads, uint32_t width,
                                                           uint32_t batch, uint32_t rows, void *__restrict__ cache_k,
                                                           void *__restrict__ cache_v, uint32_t capacity, uint32_t window,
                                                           const uint32_t *__restrict__ cursor, const uint8_t *__restrict__ mask,
                                                           const float *__restrict__ table, uint32_t *refusal, bool ring,
-                                                          const float *__restrict__ cosines, const float *__restrict__ sines, uint32_t positions) {
-    NH_FETCH(qkv, heads, kv_heads, width, batch, rows, cache_k, cache_v, capacity, window, cursor, mask, table, refusal, cosines, sines, positions);
+                                                          const float *__restrict__ cosines, const float *__restrict__ sines, uint32_t positions,
+                                                          const float *__restrict__ bias_q, const float *__restrict__ bias_k, const float *__restrict__ bias_v) {
+    NH_FETCH(qkv, heads, kv_heads, width, batch, rows, cache_k, cache_v, capacity, window, cursor, mask, table, refusal, cosines, sines, positions, bias_q, bias_k, bias_v);
     const uint32_t half = width / 2;
     const uint32_t vectors = heads + 2 * kv_heads;  // per token: q heads, k heads, v heads
     const uint32_t stride = vectors * width;
@@ -204,12 +206,19 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ qk
     const uint32_t item = blockIdx.x * blockDim.x + threadIdx.x;
     if (item >= items) return;
     const uint32_t c = item % half, vector = item / half;
+    const float *bias = vector < heads ? bias_q : vector < heads + kv_heads ? bias_k : bias_v;
+    float low_bias = 0.0f, high_bias = 0.0f;
+    if (bias) {
+        bias += (size_t)(vector < heads ? vector : vector < heads + kv_heads ? vector - heads : vector - heads - kv_heads) * width;
+        low_bias = bias[c], high_bias = bias[c + half];
+    }
     for (uint32_t t = blockIdx.y; t < tokens; t += gridDim.y) {
         const uint32_t row = t / batch, b = t % batch;
         float *src = qkv + (size_t)t * stride + (size_t)vector * width;
         const uint32_t position = cursor[b] + row;
         const bool key = vector >= heads && vector < heads + kv_heads;
         float low = src[c], high = src[c + half];
+        if (bias) low += low_bias, high += high_bias;
         if (vector < heads || key) {
             if (cosines && position < positions) {
                 const float cosine = cosines[(size_t)position * half + c], sine = sines[(size_t)position * half + c];
@@ -241,14 +250,14 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ qk
 int32_t launch_rope_append(nh_device *d, float *qkv, uint32_t heads, uint32_t kv_heads, uint32_t width, uint32_t batch, uint32_t rows,
                            void *cache_k, void *cache_v, uint32_t capacity, uint32_t window, const uint32_t *cursor,
                            const uint8_t *mask, float base, bool ring, int32_t cache_element, const float *cosines, const float *sines,
-                           uint32_t positions) {
+                           uint32_t positions, const float *const *biases) {
     const float *table = rope_frequencies(d, base, width);
     if (!table) return NH_E_DEVICE;
     const uint32_t items = (heads + 2 * kv_heads) * (width / 2), tokens = batch * rows;
     if (!items || !tokens) return NH_OK;
     const dim3 grid((items + 255u) / 256u, tokens < 65535u ? tokens : 65535u);
 #define NH_ROPE(CE) hipLaunchKernelGGL(rope_append_kernel<CE>, grid, dim3(256), 0, d->stream, qkv, heads, kv_heads, width, batch, rows, cache_k, \
-                                       cache_v, capacity, window, cursor, mask, table, d->refusal, ring, cosines, sines, positions)
+                                       cache_v, capacity, window, cursor, mask, table, d->refusal, ring, cosines, sines, positions, biases[0], biases[1], biases[2])
     if (cache_element == NH_F32) NH_ROPE(NH_F32);
     else if (cache_element == NH_BF16) NH_ROPE(NH_BF16);
     else NH_ROPE(NH_F16);
@@ -258,20 +267,18 @@ int32_t launch_rope_append(nh_device *d, float *qkv, uint32_t heads, uint32_t kv
 }
 
 // silu(gate) * up (examples/qwen/mlp.rs:33; crates/neura-pointwise/src/op.rs:163)
-// dst[r][c] = src[r][c] + bias[c]: places the columns of one projection in a wider row, or adds a bias where it stands
-__global__ __launch_bounds__(256) void columns_kernel(const float *__restrict__ src, uint32_t lds, const float *__restrict__ bias,
-                                                      float *__restrict__ dst, uint32_t ldd, uint32_t rows, uint32_t n) {
+// dst[r][c] = src[r][c]: places the columns of one projection in a wider row
+__global__ __launch_bounds__(256) void columns_kernel(const float *__restrict__ src, uint32_t lds, float *__restrict__ dst, uint32_t ldd, uint32_t rows, uint32_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (uint64_t)rows * n; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t r = (uint32_t)(i / n), c = (uint32_t)(i % n);
-        const float value = src[(size_t)r * lds + c];
-        dst[(size_t)r * ldd + c] = bias ? value + bias[c] : value;
+        dst[(size_t)r * ldd + c] = src[(size_t)r * lds + c];
     }
 }
 
-int32_t launch_columns(nh_device *d, const float *src, uint32_t lds, const float *bias, float *dst, uint32_t ldd, uint32_t rows, uint32_t n) {
+int32_t launch_columns(nh_device *d, const float *src, uint32_t lds, float *dst, uint32_t ldd, uint32_t rows, uint32_t n) {
     if (!rows || !n) return NH_OK;
     const uint64_t wanted = ((uint64_t)rows * n + 255) / 256, most = (uint64_t)d->compute_units * 8;
-    hipLaunchKernelGGL(columns_kernel, dim3((uint32_t)(wanted < most ? wanted : most)), dim3(256), 0, d->stream, src, lds, bias, dst, ldd, rows, n);
+    hipLaunchKernelGGL(columns_kernel, dim3((uint32_t)(wanted < most ? wanted : most)), dim3(256), 0, d->stream, src, lds, dst, ldd, rows, n);
     NH_HIP(hipGetLastError());
     return NH_OK;
 }

@@ -638,6 +638,33 @@ def test_wide_products_whose_depth_is_shared_among_workgroups(device, monkeypatc
         assert np.array_equal(device.gemm(element, raw, N, K, X), first)
 
 
+@pytest.mark.parametrize("wide", ["0", "1", "2"])
+@pytest.mark.parametrize("element,N,K", [(NH_Q8_0, 256, 64), (NH_Q8_0, 512, 4864), (NH_Q6_K, 256, 256), (NH_Q6_K, 2048, 2816), (NH_Q6_K, 130, 2048), (NH_Q5_K, 256, 8960),
+                                         (NH_Q3_K, 1024, 5888), (NH_Q3_K, 66, 768), (NH_Q4_K, 256, 2304)])
+def test_narrow_products_of_several_rows_in_both_forms(device, monkeypatch, wide, element, N, K):
+    """Two to eight activation rows through the vector and staged kernels (0), through the wide product of few rows wherever it can (2) and
+    as the rule on sizes has it (1): plain, with a residual and gated, against the exact product, at the bar of
+    test_both_forms_of_a_wide_product (Q4_K: its own kernels' digits cost 8e-6)."""
+    monkeypatch.setenv("NEURA_HIP_GEMV_WIDE", wide)
+    rng = np.random.default_rng(N + K + element)
+    raw = synth.RANDOM[element](rng, N * K)
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    bar = 8e-6 if element == NH_Q4_K else 4e-6
+    for rows in (2, 3, 4, 5, 8):
+        x = rng.standard_normal((rows, K)).astype(np.float32)
+        r = rng.standard_normal((rows, N)).astype(np.float32)
+        exact = x.astype(np.float64) @ weights.T
+        scale = np.sqrt((x.astype(np.float64) ** 2) @ (weights.T ** 2))
+        assert (np.abs(device.gemv(element, raw, N, K, x) - exact) <= bar * scale).all(), rows
+        assert (np.abs(device.gemv(element, raw, N, K, x, residual=r) - (exact + r)) <= bar * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r))).all(), rows
+        gate, up = exact[:, : N // 2], exact[:, N // 2:]
+        with np.errstate(over="ignore"):
+            want = gate / (1.0 + np.exp(-gate)) * up
+        # the gate's and the up half's errors, each weighed by the other (silu's slope stays below 1.1), and four roundings of silu
+        room = bar * (1.1 * scale[:, : N // 2] * np.abs(up) + np.abs(gate) * scale[:, N // 2:]) + 2.0 ** -21 * np.abs(want) + 1e-30
+        assert (np.abs(device.gemv(element, raw, N, K, x, swiglu=True) - want) <= 2 * room).all(), rows
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
