@@ -665,6 +665,31 @@ def test_narrow_products_of_several_rows_in_both_forms(device, monkeypatch, wide
         assert (np.abs(device.gemv(element, raw, N, K, x, swiglu=True) - want) <= 2 * room).all(), rows
 
 
+@pytest.mark.parametrize("wide", ["0", "2"])
+@pytest.mark.parametrize("element,N,K", [(NH_Q8_0, 130, 4864), (NH_Q6_K, 256, 2816), (NH_Q5_K, 96, 8960), (NH_Q3_K, 66, 5888)])
+def test_narrow_products_of_several_rows_over_wide_ranges(device, monkeypatch, wide, element, N, K):
+    """Rows of many orders of magnitude with outliers at any seat, and rows that hold an infinity, a NaN or zeros alone, in both forms.
+    A rounding error is one of an activation times a column's typical weight (an outlier may meet a weight that its minimum cancels), so
+    the bar of test_both_forms_of_a_wide_product is taken of the row's 2-norm times the matrix's largest column deviation.  An infinity
+    or a NaN stays visible in its own row and leaves the others as they were; zeros give zeros."""
+    monkeypatch.setenv("NEURA_HIP_GEMV_WIDE", wide)
+    rng = np.random.default_rng(N * K + element)
+    raw = synth.RANDOM[element](rng, N * K)
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    x = (rng.standard_normal((5, K)) * np.exp(rng.uniform(-6, 6, (5, K)))).astype(np.float32)
+    x[1, rng.integers(0, K, 24)] *= 1e4
+    x[2], x[3] = x[2] * np.float32(1e-30), x[3] * np.float32(1e20)
+    got = device.gemv(element, raw, N, K, x)
+    scale = np.sqrt((x.astype(np.float64) ** 2).sum(1, keepdims=True)) * np.sqrt((weights ** 2).mean(0).max())
+    assert (np.abs(got - x.astype(np.float64) @ weights.T) <= 4e-6 * scale).all()
+    bad = x.copy()
+    bad[0, 5], bad[2, 77] = np.inf, np.nan
+    bad[4] = 0.0
+    seen = device.gemv(element, raw, N, K, bad)
+    assert not np.isfinite(seen[0]).any() and not np.isfinite(seen[2]).any()
+    assert np.array_equal(seen[[1, 3]], got[[1, 3]]) and np.array_equal(seen[4], np.zeros(N, np.float32))
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
