@@ -264,9 +264,9 @@ int32_t launch_gemm(nh_device *d, const GemmArgs &args);
 // whether launch_gemm takes a product of this element and depth with matrices stacked along N at these boundaries, or with
 // activations the launch before packed
 bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, const void *W1, const void *W2, uint32_t end0, uint32_t end1);
-bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up);
+bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up);
 // whether three products over the same M rows of K numbers pack them alike: the second and third may be `packed`
-bool gemm_shares_rows(const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M);
+bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M);
 // device scratch a Q4_K wide product over M rows of K activations packs them into
 size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows);
 

@@ -1269,7 +1269,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const bool half_rows = a.x_element == NH_F16;
     p.rows = half_rows ? a.M : 2 * a.M;
     p.split = half_rows ? 0 : 1;
-    const bool few = gemm_few_takes(a.element, a.N, a.K, p.rows);
+    const bool few = gemm_few_takes(d, a.element, a.N, a.K, p.rows);
     if (a.gated && (!few || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
         return fail(NH_E_ARGUMENT, "this wide product gates no outputs (ask gemm_gates first)");
     // scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row scales, the sums workgroups of the product of few
@@ -1330,14 +1330,14 @@ bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, con
 }
 
 // one launch for the gate and the up projection, silu(gate) * up leaving it: the product of few rows
-bool gemm_gates(int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up) {
+bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up) {
     return N % GT == 0 && gemm_stacks(element, K, X, gate, nullptr, nullptr, 0, 0) && gemm_stacks(element, K, X, up, nullptr, nullptr, 0, 0) &&
-           2u * M <= FEW_TILE && gemm_few_takes(element, N, K, 2u * M);
+           2u * M <= FEW_TILE && gemm_few_takes(d, element, N, K, 2u * M);
 }
 
-bool gemm_shares_rows(const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M) {
+bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M) {
     for (int s = 0; s < 3; s++)
-        if (!mfma_takes(elements[s], K, X, W[s]) || gemm_few_takes(elements[s], N[s], K, 2u * M) != gemm_few_takes(elements[0], N[0], K, 2u * M)) return false;
+        if (!mfma_takes(elements[s], K, X, W[s]) || gemm_few_takes(d, elements[s], N[s], K, 2u * M) != gemm_few_takes(d, elements[0], N[0], K, 2u * M)) return false;
     return true;
 }
 
@@ -1350,7 +1350,7 @@ bool gemm_shares_rows(const int32_t (&elements)[3], const uint8_t *const (&W)[3]
 // 13.8 M: Q5_K 19 -> 15; 7B attn_output: 11 against 12), Q6_K from 60 M (7B ffn_down, 67.9 M: 34 -> 33; 1.5B gate|up, 27.5 M: 21 against 22).
 // The error against 64 bits is no larger (2-norm, those shapes: Q8_0 2.3..4e-7 -> 1.0..2.3e-7, Q6_K 1.5..2.3e-7 -> 1.2..1.9e-7, Q5_K
 // 1.5..2.4e-7 -> 1.3..2.1e-7, Q3_K 1.4..2.2e-7 -> 1.0..1.6e-7).
-bool gemv_wide_takes(const GemvArgs &a) {
+bool gemv_wide_takes(const nh_device *d, const GemvArgs &a) {
     const int held = env_int("NEURA_HIP_GEMV_WIDE", 1);  // 0 never, 2 wherever it can
     if (held == 0 || a.rows < 2u || a.rows > 8u || a.rope || a.append_value || a.merge || a.digits_in || a.digits_out || a.pairs_out) return false;
     if (held != 2) {
@@ -1362,8 +1362,8 @@ bool gemv_wide_takes(const GemvArgs &a) {
     }
     if ((uintptr_t)a.norm_w & 15u) return false;
     const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
-    if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(a.element, outputs, a.K, a.rows, a.x, a.W[0], a.W[1]);
-    if (!gemm_few_takes(a.element, a.N, a.K, 2u * a.rows)) return false;
+    if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(d, a.element, outputs, a.K, a.rows, a.x, a.W[0], a.W[1]);
+    if (!gemm_few_takes(d, a.element, a.N, a.K, 2u * a.rows)) return false;
     return gemm_stacks(a.element, a.K, a.x, a.W[0], a.W[1], a.W[2], a.end[0], a.end[1]);
 }
 

@@ -13,6 +13,7 @@
 // of the 128 x 128 kernels: exact half operands code * sub-scale, fp32 sums weighed by d a super-block (Q8_0: a block), the
 // minimums off with one more MFMA a super-block.  Rows past the last are read as the last (the same lines again) and never stored.
 #include "blocks.hpp"
+#include "few_rule.hpp"
 #include "gemm_few.hpp"
 
 #include <cstdlib>
@@ -546,7 +547,7 @@ int32_t launch_few(nh_device *d, FewParams p) {
     for (uint32_t across = 1; across <= 4u; across *= 2u)
         for (uint32_t deep = 1; deep * across <= 8u; deep++)
             for (uint32_t slices : slice_list) {
-                const uint32_t places = ((tiles + across - 1u) / across) * ((row_tiles + MT - 1u) / MT), resident = 256u * (8u / (deep * across));
+                const uint32_t places = ((tiles + across - 1u) / across) * ((row_tiles + MT - 1u) / MT), resident = (uint32_t)d->compute_units * (8u / (deep * across));
                 if (slices > 1u && (places > FEW_MEETS || deep * slices > units || (size_t)slices * places * across * MT * NT * 4096u > FEW_PARTIAL_BYTES)) continue;
                 const uint32_t meeting = slices > 1u ? 64u + (uint32_t)((uint64_t)slices * p.N * NT * p.rows * 4u * 64u / 2500000u) : 0u;
                 const uint32_t cost = ((places * slices + resident - 1u) / resident) * ((units + deep * slices - 1u) / (deep * slices) + 2u) * 64u + meeting + across * deep;
@@ -566,32 +567,19 @@ int32_t launch_few(nh_device *d, FewParams p) {
 
 template <int ELEMENT>
 int32_t launch_element(nh_device *d, const FewParams &p, bool gated) {
-    const uint32_t row_tiles = (p.rows + FEW_TILE - 1u) / FEW_TILE;
     if (gated) return launch_few<ELEMENT, 1, true>(d, p);
-    if (row_tiles == 1u) return launch_few<ELEMENT, 1, false>(d, p);
-    // two or three tiles of rows a wave: passes over the weights, each the time of its row tiles and of one more for the weights;
-    // a matrix of few column tiles is bound by how much is in flight and takes twos (attn_output of the 7B shape: 48 rows in
-    // threes 18.6 us, 64 rows in twos 16.7; gate: 22.4 and 26.0)
-    const uint32_t tiles = (p.N + FEW_TILE - 1u) / FEW_TILE, twos = (row_tiles + 1u) / 2u * 3u, threes = (row_tiles + 2u) / 3u * 4u;
-    if (tiles <= 128u) return launch_few<ELEMENT, 2, false>(d, p);
-    return twos <= threes ? launch_few<ELEMENT, 2, false>(d, p) : launch_few<ELEMENT, 3, false>(d, p);
+    switch (few_row_tiles(p.N, p.rows, (uint32_t)d->compute_units)) {
+        case 1: return launch_few<ELEMENT, 1, false>(d, p);
+        case 2: return launch_few<ELEMENT, 2, false>(d, p);
+        default: return launch_few<ELEMENT, 3, false>(d, p);
+    }
 }
 
 }  // namespace
 
-// Where the line lies (us with the packing, 128 x 128 tiles -> here).  Up to 96 packed rows most of a tile of 128 is padding (7B shape,
-// Q4_K, 16 rows of fp32: gate|up 74 -> 36; 1.5B shape, 48 rows: 24 -> 22).  Past that the tiles lose where their workgroups leave
-// half of the compute units idle, in one round (7B attn_output at 128 rows: 43 -> 24; ffn_down 193 -> 87; at 512 rows 214 -> 265, and
-// 50 -> 64) or in the last of more (1.5B gate|up at 128 rows, 280 workgroups: 43 -> 37; 7B q|k|v at 512, 288: 82 -> 73).  Where both fill
-// the chip the Q4_K tiles win (gate|up at 128 rows: 120 against 140) and the formats unpacked through LDS lose (Q6_K ffn_down at
-// 512 rows 431 -> 352, Q8_0 4864 x 896 46 -> 35, Q3_K gate 254 -> 239), Q5_K from 256 rows on excepted (235 against 248).
-bool gemm_few_takes(int32_t element, uint32_t N, uint32_t K, uint32_t rows) {
-    (void)K;
+bool gemm_few_takes(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows) {
     if (const char *held = getenv("NEURA_HIP_GEMM_FEW"); held && (held[0] == '0' || held[0] == '1')) return held[0] == '1';  // never, always
-    if (rows <= 96u) return true;
-    if (element != NH_Q4_K && rows <= (element == NH_Q5_K ? 256u : 1024u)) return true;
-    const uint64_t groups = (uint64_t)((N + 127u) / 128u) * ((rows + 127u) / 128u), rounds = (groups + 255u) / 256u;
-    return rounds == 1u ? groups <= 128u : groups * 5u <= rounds * 256u * 3u;
+    return few_rows_win(element, N, K, rows, (uint32_t)d->compute_units);
 }
 
 int32_t launch_gemm_few(nh_device *d, int32_t element, FewParams p, bool gated) {

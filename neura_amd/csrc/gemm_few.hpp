@@ -46,7 +46,7 @@ struct FewParams {
 };
 
 // whether the product of `rows` packed rows is this kernel's, and its launch (the rows are packed)
-bool gemm_few_takes(int32_t element, uint32_t N, uint32_t K, uint32_t rows);
+bool gemm_few_takes(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows);
 int32_t launch_gemm_few(nh_device *d, int32_t element, FewParams p, bool gated);
 
 }  // namespace nh

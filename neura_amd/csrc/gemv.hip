@@ -2734,7 +2734,7 @@ int32_t launch_gemv(nh_device *d, const GemvArgs &a) {
         if (!mfma32_takes(d, a)) return fail(NH_E_ARGUMENT, "this product cannot fold the rotation in (ask gemv_fuses_rope first)");
         return launch_mfma32(d, a);
     }
-    if (gemv_wide_takes(a)) return launch_gemv_wide(d, a);
+    if (gemv_wide_takes(d, a)) return launch_gemv_wide(d, a);
     if (a.rope && mfma_takes(a)) return fail(NH_E_ARGUMENT, "this product cannot fold the rotation in (ask gemv_fuses_rope first)");
     if (f16_tiles_take(d, a)) return launch_f16_tiles(d, a);
     if (mfma32_takes(d, a)) return launch_mfma32(d, a);

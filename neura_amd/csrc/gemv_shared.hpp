@@ -238,7 +238,7 @@ int32_t launch_tile16(nh_device *d, const GemvArgs &args);
 bool rows4_takes(const GemvArgs &args);
 int32_t launch_rows4(nh_device *d, const GemvArgs &args);
 // several activation rows as a wide product of few rows (gemm.hip)
-bool gemv_wide_takes(const GemvArgs &args);
+bool gemv_wide_takes(const nh_device *d, const GemvArgs &args);
 int32_t launch_gemv_wide(nh_device *d, const GemvArgs &args);
 // one activation row against a Q6_K matrix on the same tiles (gemv_q6k_tile16.hip)
 bool q6k_tile16_takes(const GemvArgs &args);

@@ -151,7 +151,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
                           gemm_stacks(elements[0], H, m->xn, m->attn_q[L], m->attn_k[L], nullptr, QW, 0);
         const uint32_t first = pair ? QW + KW : QW;
         const bool shares_rows =
-            !alike && T > 1 && gemm_shares_rows(elements, {m->attn_q[L], m->attn_k[L], m->attn_v[L]}, {first, pair ? first : KW, KW}, H, m->h, T);
+            !alike && T > 1 && gemm_shares_rows(d, elements, {m->attn_q[L], m->attn_k[L], m->attn_v[L]}, {first, pair ? first : KW, KW}, H, m->h, T);
         if (wide || shares_rows) {
             const uint8_t *mats[3] = {m->attn_q[L], m->attn_k[L], m->attn_v[L]};
             const uint32_t widths[3] = {QW, KW, KW};
@@ -267,7 +267,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             // where the matrix cores take both projections the norm rides in the pass that packs the rows for the gate
             // projection, and the up projection multiplies those same packed rows -- in the same launch where the rows are few
             const bool alike = element_at(m, L, GATE) == element_at(m, L, UP);
-            const bool both = alike && gemm_gates(element_at(m, L, GATE), F, H, T, m->h, m->ffn_gate[L], m->ffn_up[L]);
+            const bool both = alike && gemm_gates(d, element_at(m, L, GATE), F, H, T, m->h, m->ffn_gate[L], m->ffn_up[L]);
             const bool paired = alike && !both && gemm_stacks(element_at(m, L, GATE), H, m->h, m->ffn_gate[L], nullptr, nullptr, 0, 0) &&
                                 gemm_stacks(element_at(m, L, UP), H, m->h, m->ffn_up[L], nullptr, nullptr, 0, 0);
             if (!paired && !both && (status = launch_rmsnorm(d, m->h, nullptr, m->ffn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
