@@ -259,16 +259,24 @@ struct GemmArgs {
     // W is the gate projection, W_more[0] the up projection (N columns each, end[0] == N): Y becomes silu(X gate^T) * (X up^T), as
     // launch_silu_mul forms it.  Only where gemm_gates() says so.
     bool gated = false;
+    // fp32 rows with every bit of every number, whatever their ranges (three half rows each and a list, where the wide product's two
+    // hold 22 bits).  Only where gemm_takes_whole() says so.
+    bool whole = false;
+    // another matrix, of whatever element, meets the rows this launch packs (with `packed`)
+    bool shared = false;
 };
 int32_t launch_gemm(nh_device *d, const GemmArgs &args);
 // whether launch_gemm takes a product of this element and depth with matrices stacked along N at these boundaries, or with
 // activations the launch before packed
 bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, const void *W1, const void *W2, uint32_t end0, uint32_t end1);
-bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up);
-// whether three products over the same M rows of K numbers pack them alike: the second and third may be `packed`
-bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M);
-// device scratch a Q4_K wide product over M rows of K activations packs them into
-size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows);
+// rows: packed rows, two of every fp32 row or (GemmArgs::whole) three
+bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, const void *X, const void *gate, const void *up);
+bool gemm_takes_whole(int32_t element, uint32_t K, const void *X, const void *W);
+// whether three products over the same M rows of K numbers pack them alike (whole: as GemmArgs::whole has it): the second and third may
+// be `packed`
+bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M, bool whole);
+// device scratch a wide product over M rows of K activations packs them into, `pieces` half rows each
+size_t gemm_scratch_bytes(uint32_t M, uint32_t K, uint32_t pieces);
 
 int32_t launch_rmsnorm(nh_device *d, const float *x, const float *residual, const float *w, float eps, uint32_t rows, uint32_t C,
                        float *out, float *sum_out);

@@ -135,64 +135,110 @@ __device__ __forceinline__ void fetch_parameters(const GemmQ4Params &p) {
     NH_FETCH(p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale);
 }
 
-// Four neighbouring numbers of a row (`hi`: as halves; `lo`, with SPLIT: their residues * 2^11) into the packed rows, and their
-// share of the sub-block sums: eight neighbouring lanes hold the 32 numbers of a sub-block.  FEW: in the operand order of the
-// product of few rows (few_operand_at), not row by row.
-template <bool SPLIT, bool FEW>
-__device__ __forceinline__ void pack_piece(const _Float16 (&hi)[4], const _Float16 (&lo)[4], uint32_t row, uint32_t k, uint32_t K, uint32_t nsb,
-                                           _Float16 *__restrict__ A, _Float16 *__restrict__ S) {
-    // the nibbles of four weight bytes unpack as bytes 0, 2, 1, 3
-    const half4_t out_hi = {hi[0], hi[2], hi[1], hi[3]}, out_lo = {lo[0], lo[2], lo[1], lo[3]};
-    const size_t place = FEW ? few_operand_at(row, k, K) : (size_t)row * K + k;
-    *reinterpret_cast<half4_t *>(A + place) = out_hi;
-    if (SPLIT) *reinterpret_cast<half4_t *>(A + place + (FEW ? 8u : K)) = out_lo;  // (a residue row is its value row's neighbour in a tile)
-    // sums of the 32 halves of a sub-block: eight neighbouring lanes
-    float sum_hi = ((float)hi[0] + (float)hi[1]) + ((float)hi[2] + (float)hi[3]);
-    float sum_lo = ((float)lo[0] + (float)lo[1]) + ((float)lo[2] + (float)lo[3]);
+// A number (times its row's scale) as PIECES halves whose weights fall by 2^11: two hold 22 of an fp32 number's bits; three hold all 24
+// of every number down to 2^-36 of the row's largest.  Returns what is left over.
+template <int PIECES>
+__device__ __forceinline__ float cut(float t, _Float16 (&pieces)[PIECES][4], int at) {
 #pragma unroll
-    for (int offset = 1; offset < 8; offset <<= 1) {
-        sum_hi += __shfl_xor(sum_hi, offset, 64);
-        sum_lo += __shfl_xor(sum_lo, offset, 64);
+    for (int j = 0; j < PIECES; j++) {
+        pieces[j][at] = (_Float16)t;
+        t = (t - (float)pieces[j][at]) * 2048.0f;  // (exact)
+    }
+    return t;
+}
+
+// Four neighbouring numbers of a row, cut into PIECES, into as many packed rows from `row` on, and their share of the sub-block sums:
+// eight neighbouring lanes hold the 32 numbers of a sub-block.  FEW: in the operand order of the product of few rows
+// (few_operand_at), not row by row.
+template <int PIECES, bool FEW>
+__device__ __forceinline__ void pack_piece(const _Float16 (&pieces)[PIECES][4], uint32_t row, uint32_t k, uint32_t K, uint32_t nsb,
+                                           _Float16 *__restrict__ A, _Float16 *__restrict__ S) {
+    const size_t place = FEW ? few_operand_at(row, k, K) : (size_t)row * K + k;
+    float sums[PIECES];
+#pragma unroll
+    for (int j = 0; j < PIECES; j++) {
+        // the nibbles of four weight bytes unpack as bytes 0, 2, 1, 3; (the rows of an activation row are neighbours in a tile)
+        *reinterpret_cast<half4_t *>(A + place + (size_t)j * (FEW ? 8u : K)) = half4_t{pieces[j][0], pieces[j][2], pieces[j][1], pieces[j][3]};
+        // sums of the 32 halves of a sub-block: eight neighbouring lanes
+        sums[j] = ((float)pieces[j][0] + (float)pieces[j][1]) + ((float)pieces[j][2] + (float)pieces[j][3]);
+    }
+    if (!S) return;  // (weights without minimums)
+#pragma unroll
+    for (int j = 0; j < PIECES; j++) {
+        sums[j] += dpp<DPP_QUAD_XOR1>(sums[j]);
+        sums[j] += dpp<DPP_QUAD_XOR2>(sums[j]);
+        sums[j] += dpp<DPP_ROW_HALF_MIRROR>(sums[j]);  // (a quad's lanes hold the same sum: the mirrored lane's is the other quad's)
     }
     if ((threadIdx.x & 7u) == 0) {
         const uint32_t sb = k >> 8, slot = (k >> 5) & 7u;
-        float left;
-        {
-            const float v = sum_hi * 0.015625f;
+        float left = 0.0f;
+#pragma unroll
+        for (int j = 0; j < PIECES; j++) {
+            // (a sum of 32 is longer than 22 bits, and the minimums' part largely cancels: what a row's sum drops goes into the next's)
+            const float v = j ? fmaf(sums[j], 0.015625f, left) : sums[j] * 0.015625f;
             const _Float16 h = (_Float16)v;
-            _Float16 *dst = S + (FEW ? few_sums_at(row, sb, nsb, 0) : ((size_t)row * nsb + sb) * 16u);
             const float rest = (v - (float)h) * 2048.0f;
             const _Float16 residue = (_Float16)rest;
+            _Float16 *dst = S + (FEW ? few_sums_at(row + j, sb, nsb, 0) : ((size_t)(row + j) * nsb + sb) * 16u);
             dst[slot] = h;
             dst[(FEW ? 256u : 8u) + slot] = residue;
             left = rest - (float)residue;
         }
-        if (SPLIT) {
-            // (a sum of 32 is longer than 22 bits, and the minimums' part largely cancels: what the value row's sum drops goes in here)
-            const float v = fmaf(sum_lo, 0.015625f, left);
-            const _Float16 h = (_Float16)v;
-            _Float16 *dst = S + (FEW ? few_sums_at(row + 1u, sb, nsb, 0) : ((size_t)(row + 1u) * nsb + sb) * 16u);
-            dst[slot] = h;
-            dst[(FEW ? 256u : 8u) + slot] = (_Float16)((v - (float)h) * 2048.0f);
-        }
     }
 }
 
-// One workgroup per activation row: the row as MFMA-ready halves (and, for fp32 rows, its residue row and scale).
+// the bits of a number's magnitude; FINITE: zero for an infinity or a NaN
+template <bool FINITE>
+__device__ __forceinline__ uint32_t magnitude(float v) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+    return FINITE && bits >= 0x7f800000u ? 0u : bits;
+}
+
+// What a whole row's packing leaves (WholeRow), for share blockIdx.y of the row: cutting a row in three is most of the packing's work
+// (some 40 operations a number), and a few rows leave the chip idle, so WHOLE_PARTS workgroups take one each -- every one of them
+// having read and measured the whole row by itself, which costs no time (7B ffn_down, eight rows: one workgroup a row 8 us).
+template <class Get>
+__device__ __forceinline__ void pack_whole(Get get, uint32_t K, uint32_t nsb, float scale, float back, _Float16 *__restrict__ A, _Float16 *__restrict__ S, WholeRow *__restrict__ whole,
+                                           float *__restrict__ outside, uint32_t &listed) {
+    const uint32_t m = blockIdx.x, part = blockIdx.y;
+    const uint32_t quads = K / 4u, share = ((quads + WHOLE_PARTS - 1u) / WHOLE_PARTS + 7u) / 8u * 8u, end = min((part + 1u) * share, quads);  // whole sub-blocks
+    for (uint32_t quad = part * share + threadIdx.x; quad < end; quad += blockDim.x) {
+        const float4 v = get(4u * quad);
+        const float held[4] = {v.x, v.y, v.z, v.w};
+        _Float16 pieces[WHOLE_PIECES][4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float left = cut(held[e] * scale, pieces, e);
+            if (!(left == 0.0f) || (held[e] != 0.0f && held[e] * scale == 0.0f)) {
+#pragma unroll
+                for (uint32_t j = 0; j < WHOLE_PIECES; j++) pieces[j][e] = (_Float16)0.0f;
+                const uint32_t at = atomicAdd(&listed, 1u);
+                if (at < WHOLE_LISTED) whole[m].list[part][at].k = 4u * quad + e, whole[m].list[part][at].value = held[e];
+            }
+        }
+        *reinterpret_cast<float4 *>(outside + (size_t)m * K + 4u * quad) = v;
+        pack_piece<WHOLE_PIECES, true>(pieces, whole_row(m), 4u * quad, K, nsb, A, S);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) whole[m].unscale = back, whole[m].listed[part] = (uint8_t)min(listed, 255u);  // (the scale: the same word from every share)
+}
+
+// One workgroup per activation row (whole ones: WHOLE_PARTS): the row as MFMA-ready halves (fp32 rows: in PIECES rows, and a scale).
 // PRELUDE: what a row is before it is packed -- 0: X as it lies; 1: X normalised (rmsnorm_kernel's arithmetic, so the same
 // fp32 numbers: thread t adds the squares of columns t, t + 256, ..., then a 256-wide tree); 2: silu(gate) * X as
 // silu_mul_kernel forms it.  `aux` is the norm's weight vector or the gate rows.
 constexpr int PACK_PLAIN = 0, PACK_NORM = 1, PACK_SWIGLU = 2;
-template <bool HALF_IN, int PRELUDE, bool FEW>
+template <int PIECES, int PRELUDE, bool FEW>
 __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
                                                              _Float16 *__restrict__ S, float *__restrict__ unscale,
-                                                             const float *__restrict__ aux, float eps) {
+                                                             const float *__restrict__ aux, float eps, WholeRow *__restrict__ whole, float *__restrict__ outside) {
+    constexpr bool HALF_IN = PIECES == 1, WHOLE = PIECES == WHOLE_PIECES;
     static_assert(!(HALF_IN && PRELUDE != PACK_PLAIN), "half rows are packed as they lie");
-    __shared__ uint32_t wave_top[4];
+    __shared__ uint32_t wave_top[4], listed;
     __shared__ float red[256];
     const uint32_t m = blockIdx.x, tid = threadIdx.x;
     const uint32_t nsb = (K + 255u) / 256u;
-    float scale = 1.0f, norm = 1.0f;
+    float scale = 1.0f, norm = 1.0f, back = 1.0f;
     if (PRELUDE == PACK_NORM) {
         const float *xr = static_cast<const float *>(X) + (size_t)m * K;
         float square = 0.0f;
@@ -223,36 +269,38 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         uint32_t top = 0;
         for (uint32_t k = tid * 4u; k < K; k += 1024u) {
             const float4 v = fetch(k);
-            top = max(max(top, __builtin_bit_cast(uint32_t, v.x) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.y) & 0x7fffffffu);
-            top = max(max(top, __builtin_bit_cast(uint32_t, v.z) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.w) & 0x7fffffffu);
+            top = max(max(top, magnitude<WHOLE>(v.x)), magnitude<WHOLE>(v.y));
+            top = max(max(top, magnitude<WHOLE>(v.z)), magnitude<WHOLE>(v.w));
         }
 #pragma unroll
         for (int offset = 32; offset > 0; offset >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, offset, 64));
         if ((tid & 63u) == 0) wave_top[tid >> 6] = top;
+        if (WHOLE && tid == 0) listed = 0;
         __syncthreads();
         top = max(max(wave_top[0], wave_top[1]), max(wave_top[2], wave_top[3]));
         // a power of two that puts the largest magnitude in [2^13, 2^14)
         const uint32_t raw = top >> 23, exponent = min(max(raw, 27u), 254u);
         scale = __builtin_bit_cast(float, (267u - exponent) << 23);
-        if (tid == 0) unscale[m] = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
+        back = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
+        if (!WHOLE && tid == 0) unscale[m] = back;
     }
-    const uint32_t row = HALF_IN ? m : 2u * m;
+    if constexpr (WHOLE) {
+        pack_whole(fetch, K, nsb, scale, back, A, S, whole, outside, listed);
+        return;
+    }
     for (uint32_t k = tid * 4u; k < K; k += 1024u) {
-        _Float16 hi[4], lo[4];
+        _Float16 pieces[PIECES][4];
         if (HALF_IN) {
             const half4_t v = *reinterpret_cast<const half4_t *>(static_cast<const _Float16 *>(X) + (size_t)m * K + k);
 #pragma unroll
-            for (int e = 0; e < 4; e++) hi[e] = v[e], lo[e] = (_Float16)0.0f;
+            for (int e = 0; e < 4; e++) pieces[0][e] = v[e];
         } else {
             const float4 v = fetch(k);
-            const float t[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
+            const float held[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                hi[e] = (_Float16)t[e];
-                lo[e] = (_Float16)((t[e] - (float)hi[e]) * 2048.0f);
-            }
+            for (int e = 0; e < 4; e++) cut(held[e] * scale, pieces, e);
         }
-        pack_piece<!HALF_IN, FEW>(hi, lo, row, k, K, nsb, A, S);
+        pack_piece<PIECES, FEW>(pieces, PIECES * m, k, K, nsb, A, S);
     }
 }
 
@@ -262,12 +310,13 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
 // time, and waits in LDS as the prelude left it: the squares are added from LDS in the same thread order, the packing reads
 // LDS.  The same arithmetic on the same numbers: the packed rows are the kernel above's bit for bit.  K is a multiple of 4.
 // THREADS: 256, or 1024 where the rows are too few to fill the chip -- the loads of a wide row are then all in flight at once.
-template <int PRELUDE, bool FEW, uint32_t THREADS>
+template <int PIECES, int PRELUDE, bool FEW, uint32_t THREADS>
 __global__ __launch_bounds__(THREADS) void gemm_pack_rows_staged_kernel(const float *__restrict__ X, uint32_t K, _Float16 *__restrict__ A,
                                                                     _Float16 *__restrict__ S, float *__restrict__ unscale,
-                                                                    const float *__restrict__ aux, float eps) {
+                                                                    const float *__restrict__ aux, float eps, WholeRow *__restrict__ whole, float *__restrict__ outside) {
+    constexpr bool WHOLE = PIECES == WHOLE_PIECES;
     extern __shared__ __attribute__((aligned(16))) float staged_row[];  // [K]
-    __shared__ uint32_t wave_top[THREADS / 64u];
+    __shared__ uint32_t wave_top[THREADS / 64u], listed;
     __shared__ float red[256];
     const uint32_t m = blockIdx.x, tid = threadIdx.x;
     const uint32_t nsb = (K + 255u) / 256u;
@@ -325,14 +374,15 @@ __global__ __launch_bounds__(THREADS) void gemm_pack_rows_staged_kernel(const fl
                 v.x = g.x * (1.0f / (1.0f + expf(-g.x))) * v.x, v.y = g.y * (1.0f / (1.0f + expf(-g.y))) * v.y;
                 v.z = g.z * (1.0f / (1.0f + expf(-g.z))) * v.z, v.w = g.w * (1.0f / (1.0f + expf(-g.w))) * v.w;
             }
-            top = max(max(top, __builtin_bit_cast(uint32_t, v.x) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.y) & 0x7fffffffu);
-            top = max(max(top, __builtin_bit_cast(uint32_t, v.z) & 0x7fffffffu), __builtin_bit_cast(uint32_t, v.w) & 0x7fffffffu);
+            top = max(max(top, magnitude<WHOLE>(v.x)), magnitude<WHOLE>(v.y));
+            top = max(max(top, magnitude<WHOLE>(v.z)), magnitude<WHOLE>(v.w));
             *reinterpret_cast<float4 *>(staged_row + k0 + 4u * THREADS * j) = v;  // the thread that packs these four wrote them
         }
     }
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, offset, 64));
     if ((tid & 63u) == 0) wave_top[tid >> 6] = top;
+    if (WHOLE && tid == 0) listed = 0;
     __syncthreads();
     top = wave_top[0];
 #pragma unroll
@@ -340,17 +390,20 @@ __global__ __launch_bounds__(THREADS) void gemm_pack_rows_staged_kernel(const fl
     // a power of two that puts the largest magnitude in [2^13, 2^14)
     const uint32_t raw = top >> 23, exponent = min(max(raw, 27u), 254u);
     const float scale = __builtin_bit_cast(float, (267u - exponent) << 23);
-    if (tid == 0) unscale[m] = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
+    const float back = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
+    if constexpr (WHOLE) {
+        // (the share's numbers may be other threads': the barrier behind wave_top stands between)
+        pack_whole([&](uint32_t k) { return *reinterpret_cast<const float4 *>(staged_row + k); }, K, nsb, scale, back, A, S, whole, outside, listed);
+        return;
+    }
+    if (tid == 0) unscale[m] = back;
     for (uint32_t k = tid * 4u; k < K; k += 4u * THREADS) {
         const float4 v = *reinterpret_cast<const float4 *>(staged_row + k);
-        const float t[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
-        _Float16 hi[4], lo[4];
+        const float held[4] = {v.x, v.y, v.z, v.w};
+        _Float16 pieces[PIECES][4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            hi[e] = (_Float16)t[e];
-            lo[e] = (_Float16)((t[e] - (float)hi[e]) * 2048.0f);
-        }
-        pack_piece<true, FEW>(hi, lo, 2u * m, k, K, nsb, A, S);
+        for (int e = 0; e < 4; e++) cut(held[e] * scale, pieces, e);
+        pack_piece<PIECES, FEW>(pieces, PIECES * m, k, K, nsb, A, S);
     }
 }
 
@@ -1210,46 +1263,61 @@ __global__ __launch_bounds__(512) void gemm_q3k_mfma_kernel(GemmQ4Params p) {
     gemm_multiply<false>(p, As, Bs, mns, dds, wave, lane, n0, m0, steps, 1.0f);
 }
 
-// bytes of device scratch a Q4_K wide product over M activation rows of K numbers packs into
-size_t gemm_q4k_scratch_bytes(uint32_t M, uint32_t K, bool half_rows) {
-    const size_t rows = ((half_rows ? M : (size_t)2 * M) + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;  // (whole tiles: few_operand_at)
-    return rows * K * sizeof(_Float16) + rows * ((K + 255u) / 256u) * 16u * sizeof(_Float16) + ((size_t)M * sizeof(float) + 15u) / 16u * 16u + FEW_PARTIAL_BYTES;
-}
+// Where a wide product's packed rows lie in the device's scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row
+// scales (whole rows: WholeRow, and the rows themselves), the sums workgroups of the product of few rows leave each other (the same for
+// every product over the same rows: `packed` ones find them where they were).
+struct PackedRows {
+    size_t sums, unscale, outside, partial, bytes;
+    PackedRows(uint32_t M, uint32_t K, uint32_t pieces) {
+        const bool whole = pieces == WHOLE_PIECES;
+        const size_t rows = ((whole ? (size_t)whole_rows(M) : (size_t)M * pieces) + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;  // (whole tiles: few_operand_at)
+        sums = rows * K * sizeof(_Float16);
+        unscale = sums + rows * ((K + 255u) / 256u) * 16u * sizeof(_Float16);
+        outside = unscale + ((size_t)M * (whole ? sizeof(WholeRow) : sizeof(float)) + 15u) / 16u * 16u;
+        partial = outside + (whole ? (size_t)M * K * sizeof(float) : 0u);
+        bytes = partial + FEW_PARTIAL_BYTES;
+    }
+};
+size_t gemm_scratch_bytes(uint32_t M, uint32_t K, uint32_t pieces) { return PackedRows(M, K, pieces).bytes; }
 
-template <int PRELUDE, bool FEW, uint32_t THREADS>
-static int32_t pack_staged(nh_device *d, const GemmArgs &a, size_t lds, _Float16 *A, _Float16 *S, float *unscale, const float *aux, float eps) {
+template <int PIECES, int PRELUDE, bool FEW, uint32_t THREADS>
+static int32_t pack_staged(nh_device *d, const GemmArgs &a, size_t lds, _Float16 *A, _Float16 *S, float *unscale, const float *aux, float *outside) {
     static bool roomy = false;
     if (!roomy) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PRELUDE, FEW, THREADS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
+        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PIECES, PRELUDE, FEW, THREADS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
         roomy = true;
     }
-    hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PRELUDE, FEW, THREADS>), dim3(a.M), dim3(THREADS), lds, d->stream, static_cast<const float *>(a.X), a.K, A, S, unscale, aux, eps);
+    hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PIECES, PRELUDE, FEW, THREADS>), dim3(a.M, PIECES == WHOLE_PIECES ? WHOLE_PARTS : 1u), dim3(THREADS), lds, d->stream, static_cast<const float *>(a.X), a.K, A, S, unscale, aux, a.eps, reinterpret_cast<WholeRow *>(unscale), outside);
     NH_HIP(hipGetLastError());
     return NH_OK;
 }
 
-template <bool FEW>
-static int32_t pack_rows(nh_device *d, const GemmArgs &a, bool half_rows, _Float16 *A, _Float16 *S, float *unscale) {
-    const float *none = nullptr;
-    const dim3 grid(a.M), block(256);
-    if (half_rows) {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<true, PACK_PLAIN, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f);
-    } else if (a.K % 4u == 0 && a.K >= 4u && (size_t)a.K * sizeof(float) <= PACK_STAGED_LDS_MOST && !pack_unstaged()) {
+template <int PIECES, int PRELUDE, bool FEW>
+static int32_t pack_fp32(nh_device *d, const GemmArgs &a, _Float16 *A, _Float16 *S, float *unscale, const float *aux, float *outside) {
+    if (a.K % 4u == 0 && a.K >= 4u && (size_t)a.K * sizeof(float) <= PACK_STAGED_LDS_MOST && !pack_unstaged()) {
         // a row of fp32 numbers crosses memory once and waits in LDS
         const size_t lds = (size_t)a.K * sizeof(float);
-        const bool many = a.M > 2u * (uint32_t)d->compute_units;
-        if (a.norm_w) return many ? pack_staged<PACK_NORM, FEW, 256>(d, a, lds, A, S, unscale, a.norm_w, a.eps) : pack_staged<PACK_NORM, FEW, 1024>(d, a, lds, A, S, unscale, a.norm_w, a.eps);
-        if (a.gate) return many ? pack_staged<PACK_SWIGLU, FEW, 256>(d, a, lds, A, S, unscale, a.gate, 0.0f) : pack_staged<PACK_SWIGLU, FEW, 1024>(d, a, lds, A, S, unscale, a.gate, 0.0f);
-        return many ? pack_staged<PACK_PLAIN, FEW, 256>(d, a, lds, A, S, unscale, none, 0.0f) : pack_staged<PACK_PLAIN, FEW, 1024>(d, a, lds, A, S, unscale, none, 0.0f);
-    } else if (a.norm_w) {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_NORM, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, a.norm_w, a.eps);
-    } else if (a.gate) {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_SWIGLU, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, a.gate, 0.0f);
-    } else {
-        hipLaunchKernelGGL((gemm_pack_rows_kernel<false, PACK_PLAIN, FEW>), grid, block, 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f);
+        if (a.M > 2u * (uint32_t)d->compute_units) return pack_staged<PIECES, PRELUDE, FEW, 256>(d, a, lds, A, S, unscale, aux, outside);
+        return pack_staged<PIECES, PRELUDE, FEW, 1024>(d, a, lds, A, S, unscale, aux, outside);
     }
+    hipLaunchKernelGGL((gemm_pack_rows_kernel<PIECES, PRELUDE, FEW>), dim3(a.M, PIECES == WHOLE_PIECES ? WHOLE_PARTS : 1u), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, aux, a.eps,
+                       reinterpret_cast<WholeRow *>(unscale), outside);
     NH_HIP(hipGetLastError());
     return NH_OK;
+}
+
+template <int PIECES, bool FEW>
+static int32_t pack_rows(nh_device *d, const GemmArgs &a, _Float16 *A, _Float16 *S, float *unscale, float *outside) {
+    const float *none = nullptr;
+    if constexpr (PIECES == 1) {
+        hipLaunchKernelGGL((gemm_pack_rows_kernel<1, PACK_PLAIN, FEW>), dim3(a.M), dim3(256), 0, d->stream, a.X, a.K, A, S, unscale, none, 0.0f, nullptr, outside);
+        NH_HIP(hipGetLastError());
+        return NH_OK;
+    } else {
+        if (a.norm_w) return pack_fp32<PIECES, PACK_NORM, FEW>(d, a, A, S, unscale, a.norm_w, outside);
+        if (a.gate) return pack_fp32<PIECES, PACK_SWIGLU, FEW>(d, a, A, S, unscale, a.gate, outside);
+        return pack_fp32<PIECES, PACK_PLAIN, FEW>(d, a, A, S, unscale, none, outside);
+    }
 }
 
 static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
@@ -1267,28 +1335,33 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     p.ldy = a.ldy;
     p.M = a.M;
     const bool half_rows = a.x_element == NH_F16;
-    p.rows = half_rows ? a.M : 2 * a.M;
+    const uint32_t pieces = half_rows ? 1u : a.whole ? WHOLE_PIECES : 2u;
+    p.rows = a.whole ? whole_rows(a.M) : pieces * a.M;
     p.split = half_rows ? 0 : 1;
-    const bool few = gemm_few_takes(d, a.element, a.N, a.K, p.rows);
+    const bool few = a.whole || gemm_few_takes(d, a.element, a.N, a.K, p.rows);
+    if (a.whole && (half_rows || gemm_few_held() == 0 || a.M > 65535u * WHOLE_TILE))
+        return fail(NH_E_ARGUMENT, "this wide product takes no fp32 rows whole (ask gemm_takes_whole first)");
     if (a.gated && (!few || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
         return fail(NH_E_ARGUMENT, "this wide product gates no outputs (ask gemm_gates first)");
-    // scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row scales, the sums workgroups of the product of few
-    // rows leave each other (the same for every product over the same rows: `packed` ones find them where they were)
-    const size_t held = (size_t)(p.rows + FEW_TILE - 1u) / FEW_TILE * FEW_TILE;
-    const size_t halves = held * a.K * sizeof(_Float16), sums = held * ((a.K + 255u) / 256u) * 16u * sizeof(_Float16);
-    uint8_t *room = static_cast<uint8_t *>(scratch(d, gemm_q4k_scratch_bytes(a.M, a.K, half_rows)));
+    const PackedRows at(a.M, a.K, pieces);
+    uint8_t *room = static_cast<uint8_t *>(scratch(d, at.bytes));
     if (!room) return NH_E_MEMORY;
-    _Float16 *A = reinterpret_cast<_Float16 *>(room), *S = reinterpret_cast<_Float16 *>(room + halves);
-    float *unscale = reinterpret_cast<float *>(room + halves + sums);
+    _Float16 *A = reinterpret_cast<_Float16 *>(room), *S = reinterpret_cast<_Float16 *>(room + at.sums);
+    float *unscale = reinterpret_cast<float *>(room + at.unscale), *outside = reinterpret_cast<float *>(room + at.outside);
     if ((a.norm_w || a.gate) && (half_rows || (a.norm_w && a.gate) || ((uintptr_t)(a.norm_w ? a.norm_w : a.gate) & 15u)))
         return fail(NH_E_ARGUMENT, "a wide product normalises or gates fp32 rows read from 16-byte aligned addresses, one of the two");
-    // (rows packed by the launch before are this launch's operand)
-    if (const int32_t status = a.packed ? NH_OK : few ? pack_rows<true>(d, a, half_rows, A, S, unscale) : pack_rows<false>(d, a, half_rows, A, S, unscale); status != NH_OK)
-        return status;
+    const bool sums = a.shared || a.element == NH_Q4_K || a.element == NH_Q5_K;  // whether weights with minimums meet these rows
+    if (!a.packed) {  // (rows packed by the launch before are this launch's operand)
+        const int32_t status = half_rows ? (few ? pack_rows<1, true>(d, a, A, S, unscale, outside) : pack_rows<1, false>(d, a, A, S, unscale, outside))
+                               : a.whole ? pack_rows<WHOLE_PIECES, true>(d, a, A, sums ? S : nullptr, unscale, outside)
+                               : few     ? pack_rows<2, true>(d, a, A, S, unscale, outside)
+                                         : pack_rows<2, false>(d, a, A, S, unscale, outside);
+        if (status != NH_OK) return status;
+    }
     p.A = A, p.S = S, p.unscale = unscale;
     if (few)
-        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale, 1u, 1u, 1u,
-                                                        unscale + ((size_t)a.M + 3u) / 4u * 4u, d->meets}, a.gated);
+        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, pieces, p.unscale, reinterpret_cast<const WholeRow *>(unscale), outside,
+                                                       1u, 1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets}, a.gated);
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
@@ -1329,13 +1402,22 @@ bool gemm_stacks(int32_t element, uint32_t K, const void *X, const void *W0, con
     return true;
 }
 
-// one launch for the gate and the up projection, silu(gate) * up leaving it: the product of few rows
-bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t M, const void *X, const void *gate, const void *up) {
-    return N % GT == 0 && gemm_stacks(element, K, X, gate, nullptr, nullptr, 0, 0) && gemm_stacks(element, K, X, up, nullptr, nullptr, 0, 0) &&
-           2u * M <= FEW_TILE && gemm_few_takes(d, element, N, K, 2u * M);
+bool gemm_takes_whole(int32_t element, uint32_t K, const void *X, const void *W) {
+    return gemm_few_held() != 0 && mfma_takes(element, K, X, W);
 }
 
-bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M) {
+// one launch for the gate and the up projection, silu(gate) * up leaving it: the product of few rows
+bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, const void *X, const void *gate, const void *up) {
+    return N % GT == 0 && gemm_stacks(element, K, X, gate, nullptr, nullptr, 0, 0) && gemm_stacks(element, K, X, up, nullptr, nullptr, 0, 0) &&
+           rows <= FEW_TILE && gemm_few_takes(d, element, N, K, rows);
+}
+
+bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M, bool whole) {
+    if (whole) {
+        for (int s = 0; s < 3; s++)
+            if (!gemm_takes_whole(elements[s], K, X, W[s])) return false;
+        return true;
+    }
     for (int s = 0; s < 3; s++)
         if (!mfma_takes(elements[s], K, X, W[s]) || gemm_few_takes(d, elements[s], N[s], K, 2u * M) != gemm_few_takes(d, elements[0], N[0], K, 2u * M)) return false;
     return true;
@@ -1362,16 +1444,15 @@ bool gemv_wide_takes(const nh_device *d, const GemvArgs &a) {
     }
     if ((uintptr_t)a.norm_w & 15u) return false;
     const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
-    if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(d, a.element, outputs, a.K, a.rows, a.x, a.W[0], a.W[1]);
-    if (!gemm_few_takes(d, a.element, a.N, a.K, 2u * a.rows)) return false;
-    return gemm_stacks(a.element, a.K, a.x, a.W[0], a.W[1], a.W[2], a.end[0], a.end[1]);
+    if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(d, a.element, outputs, a.K, whole_rows(a.rows), a.x, a.W[0], a.W[1]);
+    return gemm_takes_whole(a.element, a.K, a.x, a.W[0]) && gemm_stacks(a.element, a.K, a.x, a.W[0], a.W[1], a.W[2], a.end[0], a.end[1]);
 }
 
 int32_t launch_gemv_wide(nh_device *d, const GemvArgs &a) {
     const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
     GemmArgs g{a.element, a.W[0], outputs, a.K, a.x, NH_F32, a.rows, a.y, a.residual, outputs};
     g.W_more[0] = a.W[1], g.W_more[1] = a.W[2], g.end[0] = a.end[0], g.end[1] = a.end[1];
-    g.norm_w = a.norm_w, g.eps = a.eps;
+    g.norm_w = a.norm_w, g.eps = a.eps, g.whole = true;
     if (a.swiglu) g.gated = true, g.W_more[1] = nullptr;
     profile_mark(d);
     if (const int32_t status = launch_gemm_mfma(d, g); status != NH_OK) return status;

@@ -16,6 +16,7 @@
 #include "few_rule.hpp"
 #include "gemm_few.hpp"
 
+#include <cmath>
 #include <cstdlib>
 
 namespace nh {
@@ -289,6 +290,22 @@ template <> struct FewOf<NH_Q8_0> { typedef FewQ8 type; };
 
 constexpr uint32_t FEW_SLICES_MOST = 8;
 
+// what an activation row's numbers beyond its packed pieces add to an output -- or, where they are too many, take its place: numbers
+// and weights as they are stored, added in 64 bits
+template <int ELEMENT>
+__device__ __forceinline__ float beyond_pieces(float value, const WholeRow &held, const float *outside, const uint8_t *row, uint32_t K) {
+    bool all = false;
+    for (uint32_t part = 0; part < WHOLE_PARTS; part++) all |= held.listed[part] > WHOLE_LISTED;
+    double sum = all ? 0.0 : (double)value;
+    if (all) {
+        for (uint32_t k = 0; k < K; k++) sum = fma((double)outside[k], (double)stored_element<ELEMENT>(row, k), sum);
+    } else {
+        for (uint32_t part = 0; part < WHOLE_PARTS; part++)
+            for (uint32_t i = 0; i < held.listed[part]; i++) sum = fma((double)held.list[part][i].value, (double)stored_element<ELEMENT>(row, held.list[part][i].k), sum);
+    }
+    return (float)sum;
+}
+
 // MT: tiles of 32 packed rows a wave multiplies its weights by; GATED: a wave walks the same 32 columns of the gate and of the up
 // matrix, and what leaves is silu(gate) * up; AHEAD: steps the activation operands are read ahead (the loads of a wave come
 // back in order: an operand asked for after the next super-block's weights waits for them, so they are asked for
@@ -484,6 +501,55 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
         asm volatile("" ::: "memory");
         if (threadIdx.x == 0) __hip_atomic_store(meet, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // as the next launch expects it
     }
+    auto leave = [&](uint32_t m, uint32_t n, float value, float up) {
+        if (m >= p.M) return;
+        if (GATED) value = value * (1.0f / (1.0f + expf(-value))) * up;
+        const size_t to = (size_t)m * p.ldy + n;
+        p.Y[to] = p.residual ? p.residual[to] + value : value;
+    };
+    if (p.pieces == WHOLE_PIECES) {
+        // an item is a column and one of a tile's ten activation rows, whose pieces lie wherever rows 3r .. 3r + 2 do
+        const uint32_t rows = min(p.M, WHOLE_TILE), outputs = p.across * MT * rows * 32u;
+        for (uint32_t item = threadIdx.x; item < outputs; item += blockDim.x) {
+            const uint32_t at = item & 31u, bi = (item >> 5) / rows, r = (item >> 5) - bi * rows, i = bi % MT, b = bi / MT;
+            const uint32_t m = (tile0 + i) * WHOLE_TILE + r, n = (blockIdx.x * p.across + b) * FEW_TILE + at;
+            if (n >= p.N || m >= p.M) continue;
+            const u32x4 head = *(global_uint4)(uintptr_t)(p.whole + m);  // the scale, and how many numbers are listed
+            float out[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                float v[WHOLE_PIECES];
+#pragma unroll
+                for (uint32_t j = 0; j < WHOLE_PIECES; j++) {
+                    const uint32_t row = WHOLE_PIECES * r + j, seat = (((row >> 2) & 1u) * 32u + at) * 4u + (row & 3u), q = row >> 3;
+                    v[j] = 0.0f;
+                    if (p.slices == 1u) {
+                        const float *sums = reinterpret_cast<const float *>(few_lds);
+                        for (uint32_t s = 0; s < p.deep; s++) v[j] += sums[((((b * p.deep + s) * NT + t) * MT + i) * 4u + q) * 256u + seat];
+                    } else {
+                        uint32_t held[FEW_SLICES_MOST];
+#pragma unroll
+                        for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
+                            held[s] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(place_of(min(s, p.slices - 1u), bi * 256u + q * 64u + seat / 4u, t)) + (row & 3u), __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                        for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
+                            if (s < p.slices) v[j] += __builtin_bit_cast(float, held[s]);
+                    }
+                }
+                out[t] = fmaf(fmaf(v[2], 0.00048828125f, v[1]), 0.00048828125f, v[0]) * __builtin_bit_cast(float, head.x);
+                if (head.z | head.w) {
+                    const uint8_t *from = GATED        ? (t ? p.W1 : p.W) + (size_t)n * p.row_bytes
+                                          : n < p.end0 ? p.W + (size_t)n * p.row_bytes
+                                          : n < p.end1 ? p.W1 + (size_t)(n - p.end0) * p.row_bytes
+                                                       : p.W2 + (size_t)(n - p.end1) * p.row_bytes;
+                    out[t] = beyond_pieces<ELEMENT>(out[t], p.whole[m], p.outside + (size_t)m * p.K, from, p.K);
+                }
+            }
+            leave(m, n, out[0], out[NT - 1]);
+        }
+        return;
+    }
     for (uint32_t item = threadIdx.x; item < items; item += blockDim.x) {
         const uint32_t row = row_of(item), n = (blockIdx.x * p.across + (item >> 8) / MT) * FEW_TILE + (item & 31u);
         if (n >= p.N || row >= p.rows) continue;
@@ -510,22 +576,16 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
                 }
             }
         }
-        auto leave = [&](uint32_t m, float value, float up) {
-            if (m >= p.M) return;
-            if (GATED) value = value * (1.0f / (1.0f + expf(-value))) * up;
-            const size_t to = (size_t)m * p.ldy + n;
-            p.Y[to] = p.residual ? p.residual[to] + value : value;
-        };
-        if (p.split) {
+        if (p.pieces == 2u) {
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const uint32_t m = (row >> 1) + e;
                 const float unscale = p.unscale[min(m, p.M - 1u)];
-                leave(m, fmaf(v[0][2 * e + 1], 0.00048828125f, v[0][2 * e]) * unscale, fmaf(v[NT - 1][2 * e + 1], 0.00048828125f, v[NT - 1][2 * e]) * unscale);
+                leave(m, n, fmaf(v[0][2 * e + 1], 0.00048828125f, v[0][2 * e]) * unscale, fmaf(v[NT - 1][2 * e + 1], 0.00048828125f, v[NT - 1][2 * e]) * unscale);
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; e++) leave(row + e, v[0][e], v[NT - 1][e]);
+            for (int e = 0; e < 4; e++) leave(row + e, n, v[0][e], v[NT - 1][e]);
         }
     }
 }
@@ -577,8 +637,13 @@ int32_t launch_element(nh_device *d, const FewParams &p, bool gated) {
 
 }  // namespace
 
+int gemm_few_held() {
+    const char *held = getenv("NEURA_HIP_GEMM_FEW");
+    return held && (held[0] == '0' || held[0] == '1') ? held[0] - '0' : -1;
+}
+
 bool gemm_few_takes(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows) {
-    if (const char *held = getenv("NEURA_HIP_GEMM_FEW"); held && (held[0] == '0' || held[0] == '1')) return held[0] == '1';  // never, always
+    if (const int held = gemm_few_held(); held >= 0) return held == 1;
     return few_rows_win(element, N, K, rows, (uint32_t)d->compute_units);
 }
 

@@ -89,7 +89,7 @@ __device__ __forceinline__ float dpp(float v) {
 }
 constexpr int DPP_QUAD_XOR1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int DPP_QUAD_XOR2 = 0x4E;  // quad_perm [2,3,0,1]
-constexpr int DPP_ROW_ROR4 = 0x124, DPP_ROW_ROR8 = 0x128;
+constexpr int DPP_ROW_ROR4 = 0x124, DPP_ROW_ROR8 = 0x128, DPP_ROW_HALF_MIRROR = 0x141;
 
 // Per-lane constants of the branch-free scale decode (they depend on the lane's group only).
 struct ScaleLane {

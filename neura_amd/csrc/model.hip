@@ -151,7 +151,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
                           gemm_stacks(elements[0], H, m->xn, m->attn_q[L], m->attn_k[L], nullptr, QW, 0);
         const uint32_t first = pair ? QW + KW : QW;
         const bool shares_rows =
-            !alike && T > 1 && gemm_shares_rows(d, elements, {m->attn_q[L], m->attn_k[L], m->attn_v[L]}, {first, pair ? first : KW, KW}, H, m->h, T);
+            !alike && T > 1 && gemm_shares_rows(d, elements, {m->attn_q[L], m->attn_k[L], m->attn_v[L]}, {first, pair ? first : KW, KW}, H, m->h, T, !wide);
         if (wide || shares_rows) {
             const uint8_t *mats[3] = {m->attn_q[L], m->attn_k[L], m->attn_v[L]};
             const uint32_t widths[3] = {QW, KW, KW};
@@ -173,7 +173,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
                     if (pair && s == 1) continue;
                     GemmArgs g{elements[s], mats[s], s ? widths[s] : first, H, shared ? m->h : m->xn, NH_F32, T, m->qkv + column, nullptr, QKV};
                     if (pair && s == 0) g.W_more[0] = mats[1], g.end[0] = QW;
-                    if (shared) g.norm_w = m->attn_norm[L], g.eps = c.eps, g.packed = s > 0;
+                    if (shared) g.norm_w = m->attn_norm[L], g.eps = c.eps, g.packed = s > 0, g.whole = !wide, g.shared = s == 0;
                     if ((status = launch_gemm(d, g)) != NH_OK) return status;
                     column += g.N;
                 }
@@ -267,7 +267,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             // where the matrix cores take both projections the norm rides in the pass that packs the rows for the gate
             // projection, and the up projection multiplies those same packed rows -- in the same launch where the rows are few
             const bool alike = element_at(m, L, GATE) == element_at(m, L, UP);
-            const bool both = alike && gemm_gates(d, element_at(m, L, GATE), F, H, T, m->h, m->ffn_gate[L], m->ffn_up[L]);
+            const bool both = alike && gemm_gates(d, element_at(m, L, GATE), F, H, 2u * T, m->h, m->ffn_gate[L], m->ffn_up[L]);
             const bool paired = alike && !both && gemm_stacks(element_at(m, L, GATE), H, m->h, m->ffn_gate[L], nullptr, nullptr, 0, 0) &&
                                 gemm_stacks(element_at(m, L, UP), H, m->h, m->ffn_up[L], nullptr, nullptr, 0, 0);
             if (!paired && !both && (status = launch_rmsnorm(d, m->h, nullptr, m->ffn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
@@ -350,10 +350,10 @@ int32_t decode_kernels(nh_model *m, bool any_inactive, bool sampled) {
     if ((status = forward(m, 1, any_inactive)) != NH_OK) return status;
     GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
     head.norm_w = m->output_norm, head.eps = m->c.eps;
-    if (m->c.batch > 8u && gemm_stacks(head.element, head.K, m->h, m->output, nullptr, nullptr, 0, 0)) {
+    if (m->c.batch > 8u && gemm_takes_whole(head.element, head.K, m->h, m->output)) {
         // more rows than a narrow product takes at once: the wide one walks the vocabulary once for all of them
         GemmArgs wide{head.element, m->output, head.N, head.K, m->h, NH_F32, m->c.batch, m->logits, nullptr, head.N};
-        wide.norm_w = m->output_norm, wide.eps = m->c.eps;
+        wide.norm_w = m->output_norm, wide.eps = m->c.eps, wide.whole = true;
         status = launch_gemm(m->d, wide);
     } else {
         status = launch_gemv(m->d, head);
@@ -520,11 +520,16 @@ nh_model *nh_model_create(nh_device *device, const nh_model_config *config, nh_w
         size_t products = 8 * 4 * widest * sizeof(float);
         size_t sections = (size_t)256 * c.heads * T * (c.head_dim + 2) * sizeof(float);
         size_t choice = (size_t)c.batch * 1024 * 8;
-        // the wide product packs its fp32 activations as two half rows each, with their sub-block sums and a scale per row
+        // the wide product packs its fp32 activations as two half rows each, with their sub-block sums and a scale per row; the narrow
+        // products' rows and the output projection's as three
         size_t deepest = (size_t)(F > QW ? F : QW);
         if (H > deepest) deepest = H;
-        size_t split_rows = T > 1 ? gemm_q4k_scratch_bytes(T, (uint32_t)deepest, false) : 0;
+        size_t split_rows = T > 1 ? gemm_scratch_bytes(T, (uint32_t)deepest, 2) : 0;
+        size_t whole_rows = T > 1 ? gemm_scratch_bytes(T < 8 ? T : 8, (uint32_t)deepest, 3) : 0;
+        size_t head_rows = c.batch > 8 ? gemm_scratch_bytes(c.batch, H, 3) : 0;
         size_t wanted = products > sections ? products : sections;
+        if (whole_rows > wanted) wanted = whole_rows;
+        if (head_rows > wanted) wanted = head_rows;
         if (choice > wanted) wanted = choice;
         if (split_rows > wanted) wanted = split_rows;
         ok = ok && scratch(device, wanted) != nullptr && rope_frequencies(device, c.rope_base, c.head_dim) != nullptr &&

@@ -690,6 +690,47 @@ def test_narrow_products_of_several_rows_over_wide_ranges(device, monkeypatch, w
     assert np.array_equal(seen[[1, 3]], got[[1, 3]]) and np.array_equal(seen[4], np.zeros(N, np.float32))
 
 
+@pytest.mark.parametrize("element,N,K", [(NH_Q8_0, 130, 4864), (NH_Q6_K, 256, 2816), (NH_Q5_K, 96, 8960), (NH_Q3_K, 66, 5888), (NH_Q8_0, 96, 64)])
+@pytest.mark.parametrize("staged", ["1", "0"])
+def test_narrow_products_of_several_rows_hold_every_number(device, monkeypatch, staged, element, N, K):
+    """Several rows as the product of few rows multiplies them: every fp32 number takes part with all of its bits, whatever stands beside
+    it in its row.  The weights of the first 32 (256) numbers are zeros, so an outlier there adds nothing and the bar is one of the other
+    numbers alone (4e-6 of the outputs' scale, as in test_both_forms_of_a_wide_product): outliers of 1e6 to 1e30, one number, a few and
+    most of a row below what three half pieces reach (2^-36 of the largest), the smallest fp32 numbers.  An infinity gives what its weights
+    make of it, as fp32 multiplies.  Both packings."""
+    monkeypatch.setenv("NEURA_HIP_GEMV_WIDE", "2")
+    monkeypatch.setenv("NEURA_HIP_PACK_STAGED", staged)
+    rng = np.random.default_rng(N * K + element)
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    per, size = synth.BLOCK_BYTES[element]
+    halves = {NH_Q8_0: (0,), NH_Q5_K: (0, 2), NH_Q6_K: (208,), NH_Q3_K: (108,)}[element]
+    blocks = raw.reshape(N, K // per, size)
+    for at in halves:
+        blocks[:, 0, at:at + 2] = 0
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    assert (weights[:, :per] == 0).all()
+    for outlier in (1e6, 1e12, 1e18, 1e30):
+        x = rng.standard_normal((5, K)).astype(np.float32)
+        x[0, 3] = outlier
+        x[1, :per] *= np.float32(outlier)
+        x[2, per:] *= np.float32(1e-30)  # every number that counts is tiny
+        x[2, 5] = outlier
+        x[3, rng.integers(0, K, 40)] *= np.float32(1.0 / outlier)  # some are
+        x[4] = 0.0
+        x[4, -1], x[4, per + 1], x[4, 1] = 1.5, 2.0 ** -140, outlier
+        exact = x.astype(np.float64) @ weights.T
+        scale = np.sqrt((x.astype(np.float64) ** 2) @ (weights.T ** 2))
+        got = device.gemv(element, raw, N, K, x)
+        assert (np.abs(got - exact) <= 4e-6 * scale + 1e-37).all(), outlier
+    x = rng.standard_normal((3, K)).astype(np.float32)
+    clean = device.gemv(element, raw, N, K, x)
+    x[1, per + 5], x[2, per + 7] = np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        want = np.where(weights[:, per + 5] == 0, np.nan, np.inf * weights[:, per + 5])
+    got = device.gemv(element, raw, N, K, x)
+    assert np.array_equal(got[0], clean[0]) and np.array_equal(got[1], want.astype(np.float32), equal_nan=True) and np.isnan(got[2]).all()
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
