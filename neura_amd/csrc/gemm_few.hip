@@ -70,14 +70,22 @@ struct FewQ45 {
 #pragma unroll
         for (int g = 0; g < 4; g++) runs[g] = *(global_uint4)(uintptr_t)(block + (FIFTH ? 48u : 16u) + 32u * g + 16u * part);
     }
+    // A sub-block whose minimum is zero is left as it lies: its weights may be exact zeros, and beside a large activation that
+    // meets one, the centre's share and what takes it off again would swallow the other numbers' products (0x3f + 0x7f stays below 0x100:
+    // no carry crosses a byte)
+    __device__ __forceinline__ uint32_t centred(int high) const {  // 0xff where a sub-block's codes are centred, of four sub-blocks
+        const uint32_t minimums = high ? ((header.w >> 4) & 0x0f0f0f0fu) | ((header.z >> 2) & 0x30303030u) : header.z & 0x3f3f3f3fu;
+        const uint32_t some = (minimums + 0x7f7f7f7fu) & 0x80808080u;
+        return some | (some - (some >> 7));
+    }
     __device__ __forceinline__ float scale() const { return (float)as_halves(header.x).x * 16384.0f; }  // operands are code * sc * 2^-14
     __device__ __forceinline__ float floor_scale() const { return (float)as_halves(header.x).y * -64.0f; }  // the sums are packed / 64
     __device__ __forceinline__ float centre_scale() const { return (float)as_halves(header.x).x * (64.0f * CENTRE); }
-    // the eight minimums (`scales`: the eight scales) as halves; k 8..15 meet the sums' residues * 2^11
+    // the eight minimums (`scales`: the eight scales where the codes are centred) as halves; k 8..15 meet the sums' residues * 2^11
     __device__ __forceinline__ half8_t floors(uint32_t part, bool scales) const {
         const half2_t offset = {(_Float16)1024.0f, (_Float16)1024.0f};
         const uint32_t first = scales ? header.y : header.z, more = scales ? header.w : header.w >> 4;
-        const uint32_t lo4 = first & 0x3f3f3f3fu, hi4 = (more & 0x0f0f0f0fu) | ((first >> 2) & 0x30303030u);
+        const uint32_t lo4 = first & 0x3f3f3f3fu & (scales ? centred(0) : ~0u), hi4 = ((more & 0x0f0f0f0fu) | ((first >> 2) & 0x30303030u)) & (scales ? centred(1) : ~0u);
         half2_t m[4] = {as_halves(__builtin_amdgcn_perm(0u, lo4, 0x0c010c00u) | 0x64006400u) - offset,
                         as_halves(__builtin_amdgcn_perm(0u, lo4, 0x0c030c02u) | 0x64006400u) - offset,
                         as_halves(__builtin_amdgcn_perm(0u, hi4, 0x0c010c00u) | 0x64006400u) - offset,
@@ -97,8 +105,9 @@ struct FewQ45 {
         // a code enters less CENTRE: the products then add up to sums of the output's own size, and not to ones that the minimums
         // take most of off again (2-norm from the exact products, eight rows of the 7B shapes: 2.2e-7 -> 1.1e-7); CENTRE times
         // the scales comes back with the minimums.  (code - CENTRE) * sc * 2^-14 is exact: one rounding, of a whole number below 2^11
-        const half2_t down = {(_Float16)(-CENTRE * 0.000000059604644775390625f), (_Float16)(-CENTRE * 0.00000095367431640625f)};
-        const half2_t centres = scales * down;
+        const half2_t down = {(_Float16)(-CENTRE * 0.00006103515625f), (_Float16)(-CENTRE * 0.00006103515625f)};
+        const uint32_t some = sc & (centred(g >> 1) >> shift);
+        const half2_t centres = (as_halves(__builtin_amdgcn_perm(0u, some, 0x0c010c00u) | 0x64006400u) - offset) * down;
         low_centre = half2_t{centres.x, centres.x}, high_centre = half2_t{centres.y, centres.y};
     }
     __device__ __forceinline__ void operand(int g, int depth, half8_t (&b)[PLANES]) const {

@@ -731,6 +731,39 @@ def test_narrow_products_of_several_rows_hold_every_number(device, monkeypatch, 
     assert np.array_equal(got[0], clean[0]) and np.array_equal(got[1], want.astype(np.float32), equal_nan=True) and np.isnan(got[2]).all()
 
 
+@pytest.mark.parametrize("element", [NH_Q4_K, NH_Q5_K])
+@pytest.mark.parametrize("rows", [4, 16, 40])
+def test_outliers_on_zero_weights_of_a_sub_block_without_a_minimum(device, monkeypatch, element, rows):
+    """Sub-blocks whose minimum is zero hold exact zeros (code 0): a large activation there adds nothing, so the other numbers' products
+    stay what they are -- no centre may be taken off such codes first and put back later.  Bar: that of test_both_forms_of_a_wide_product,
+    of the numbers that count.  Four rows of Q5_K as a narrow product of whole rows, the others as a wide product of few rows."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_FEW", "1")
+    monkeypatch.setenv("NEURA_HIP_GEMV_WIDE", "2")
+    rng = np.random.default_rng(rows + element)
+    N, K = 160, 1536
+    per, size = synth.BLOCK_BYTES[element]
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    blocks = raw.reshape(N, K // per, size)
+    codes = 16 if element == NH_Q4_K else 48
+    blocks[:, :, 4 + 4] &= 0xC0  # the minimum of sub-block 0
+    blocks[:, :, 4 + 8 + 2] &= 0x0F  # and of sub-block 6: its low four bits here,
+    blocks[:, :, 4 + 6] &= 0x3F  # its high two there
+    blocks[:, :, codes + 5] &= 0xF0  # codes of numbers 5 and 201 (group 3, low, lane 9)
+    blocks[:, :, codes + 96 + 9] &= 0xF0
+    if element == NH_Q5_K:
+        blocks[:, :, 16 + 5] &= 0xFE
+        blocks[:, :, 16 + 9] &= 0xBF
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    assert (weights[:, 5::per] == 0).all() and (weights[:, 201::per] == 0).all()
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    x[:, 5] *= 1e6
+    x[:, per + 201] *= 1e5
+    exact = x.astype(np.float64) @ weights.T
+    scale = np.sqrt((x.astype(np.float64) ** 2) @ (weights.T ** 2))
+    got = device.gemv(element, raw, N, K, x) if rows <= 8 and element == NH_Q5_K else device.gemm(element, raw, N, K, x)
+    assert (np.abs(got - exact) <= 4e-6 * scale).all()
+
+
 def test_q8_0_wide_product_of_the_small_decoder_s_shapes(device):
     """The Q8_0 products of a 512-token fill of the 0.5B-shape decoder (hidden 896, FFN 4864, 14 heads of 64, 2 key heads), weights
     N(0, 0.02) quantised as a checkpoint's are, fp32 activations over a few orders of magnitude: every output against fp32
