@@ -1414,6 +1414,7 @@ bool gemm_gates(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uin
 
 bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const uint8_t *const (&W)[3], const uint32_t (&N)[3], uint32_t K, const void *X, uint32_t M, bool whole) {
     if (whole) {
+        if (env_int("NEURA_HIP_GEMV_WIDE", 1) == 0) return false;  // one narrow product a matrix
         for (int s = 0; s < 3; s++)
             if (!gemm_takes_whole(elements[s], K, X, W[s])) return false;
         return true;

@@ -157,8 +157,10 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             const uint32_t widths[3] = {QW, KW, KW};
             const bool stacked = alike && gemm_stacks(element_at(m, L, Q), H, m->h, mats[0], mats[1], mats[2], QW, QW + KW);
             uint32_t column = 0;
-            // matrices of different elements: the norm still rides in a pass that packs the rows, once for the three products (the
-            // Q4_K_M mix of the 7B shape at five planes: 68 us of products and columns in such a layer -> 32)
+            // matrices of different elements: the norm still rides in a pass that packs the rows, once for the three products (a step of
+            // the 7B Q4_K_M mix at two, three, four, five and eight planes, one narrow product a matrix -> here: 2.49 -> 2.43, 3.09 -> 2.87,
+            // 3.20 -> 2.93, 3.41 -> 3.06, 3.48 -> 3.14 ms; of the Q3_K_M mix 3.46 -> 3.17, 4.11 -> 3.47, 4.56 -> 3.49, 4.32 -> 3.61, 4.42 ->
+            // 3.70; of the 1.5B Q4_K_M mix at two planes 1.64 -> 1.58)
             const bool shared = !stacked && shares_rows;
             if (!stacked && !shared && (status = launch_rmsnorm(d, m->h, nullptr, m->attn_norm[L], c.eps, T, H, m->xn, nullptr)) != NH_OK) return status;
             if (stacked) {

@@ -229,6 +229,36 @@ def test_mixed_elements_and_projection_biases(device, batch, base, mixed):
     model.release(), weights.release()
 
 
+@pytest.mark.parametrize("base,mixed", [(NH_Q4_K, MIXED), (NH_Q3_K, MIXED_3)], ids=["q4_k_m", "q3_k_m"])
+@pytest.mark.parametrize("batch", [2, 5])
+def test_the_switches_send_a_mixed_layer_s_products_back(device, monkeypatch, batch, base, mixed):
+    """NEURA_HIP_GEMV_WIDE=0: q, k and v of a layer of mixed elements are narrow products at up to eight planes, one a matrix, so the wide
+    product's own switch has no say in them: the same bits whatever it holds.  NEURA_HIP_GEMM_FEW=0 alone takes the product of few rows
+    away, which is what the default multiplies those matrices with: never the 128 x 128 tiles, so the same bits as with both.  All of
+    it within the decoder's bar of the oracle."""
+    monkeypatch.setenv("NEURA_HIP_GRAPH", "0")  # eager steps read the switches every time
+    shape = SMALL_Q4
+    tensors = list(synth.model_tensors(shape, base, np.random.default_rng(77), mode="normal", elements=mixed, biases=(0, 1)))
+    host = {name: (raw.view(np.float32) if name.endswith(".bias") else raw) for name, _, _, raw in tensors}
+    ref = oracle.Model(shape, base, host, batch, 40, 1, elements=mixed)
+    tokens = [5 + 3 * plane for plane in range(batch)]
+    want, _ = ref.forward(tokens, 1, [0] * batch)
+    weights = Weights(device, tensors)
+    seen = {}
+    for wide, few in ((None, None), ("0", None), ("0", "0"), ("0", "1"), (None, "0")):
+        for name, held in (("NEURA_HIP_GEMV_WIDE", wide), ("NEURA_HIP_GEMM_FEW", few)):
+            monkeypatch.setenv(name, held) if held else monkeypatch.delenv(name, raising=False)
+        model = Model(device, weights, shape, base, batch, 40, 1)
+        model.decode_step(tokens, [0] * batch)
+        seen[wide, few] = model.logits()
+        assert np.abs(seen[wide, few] - want).max() <= 1e-3 * np.abs(want).max(), (wide, few)
+        model.release()
+    for few in ("0", "1"):
+        assert np.array_equal(seen["0", few], seen["0", None])
+    assert np.array_equal(seen[None, "0"], seen["0", None])
+    weights.release()
+
+
 def test_sampled_decode_steps_draw_as_the_oracle_draws(device):
     """A sampled answer program: the same forward pass, the choice drawn per plane with its own seed, temperature,
     candidate count and nucleus, all written by the host before each step (the recorded graph is replayed with new
