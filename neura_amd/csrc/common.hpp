@@ -89,6 +89,7 @@ struct nh_device {
     std::vector<RopeTable> rope_tables;  // one per (base, width) met so far; entries never move
     // per-launch timing of the narrow products (nh_profile_*): event pairs on the stream
     bool profile = false;
+    bool profile_wide = false;               // the wide products too (nh_model_time_products)
     std::vector<hipEvent_t> profile_events;  // start, stop, start, stop, ...
     size_t profile_used = 0;
     uint64_t profile_bytes = 0;              // weight bytes the timed launches walked

@@ -1455,17 +1455,12 @@ int32_t launch_gemv_wide(nh_device *d, const GemvArgs &a) {
     g.W_more[0] = a.W[1], g.W_more[1] = a.W[2], g.end[0] = a.end[0], g.end[1] = a.end[1];
     g.norm_w = a.norm_w, g.eps = a.eps, g.whole = true;
     if (a.swiglu) g.gated = true, g.W_more[1] = nullptr;
-    profile_mark(d);
-    if (const int32_t status = launch_gemm_mfma(d, g); status != NH_OK) return status;
-    profile_mark(d);
-    if (d->profile) d->profile_bytes += (uint64_t)a.N * payload_bytes(a.element, a.K);
-    return NH_OK;
+    return launch_gemm(d, g);
 }
 
-int32_t launch_gemm(nh_device *d, const GemmArgs &a) {
-    if (!a.M || !a.N) return NH_OK;
+static int32_t launch_gemm_any(nh_device *d, const GemmArgs &a) {
     if (mfma_takes(a.element, a.K, a.X, a.W)) return launch_gemm_mfma(d, a);
-    if (a.W_more[0] || a.W_more[1] || a.packed || a.norm_w || a.gate || a.gated)
+    if (a.W_more[0] || a.W_more[1] || a.packed || a.norm_w || a.gate || a.gated || a.whole)
         return fail(NH_E_ARGUMENT, "this wide product stacks no matrices, reuses no packed activations and packs rows as they lie (ask gemm_stacks first)");
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM), block(256);
     uint32_t row_bytes = (uint32_t)payload_bytes(a.element, a.K);
@@ -1492,6 +1487,17 @@ int32_t launch_gemm(nh_device *d, const GemmArgs &a) {
     }
 #undef NH_GEMM
     NH_HIP(hipGetLastError());
+    return NH_OK;
+}
+
+int32_t launch_gemm(nh_device *d, const GemmArgs &a) {
+    if (!a.M || !a.N) return NH_OK;
+    // a narrow product's rows, or a step's products as nh_model_time_products counts them: one launch, its packing within
+    const bool counted = a.whole || d->profile_wide;
+    if (counted) profile_mark(d);
+    if (const int32_t status = launch_gemm_any(d, a); status != NH_OK) return status;
+    if (counted) profile_mark(d);
+    if (counted && d->profile) d->profile_bytes += (uint64_t)a.N * (a.gated ? 2u : 1u) * payload_bytes(a.element, a.K);
     return NH_OK;
 }
 

@@ -345,22 +345,23 @@ __global__ __launch_bounds__(64) void publish_kernel(const uint32_t *chosen, con
     for (uint32_t i = threadIdx.x; i <= batch; i += 64u) host[i] = i < batch ? chosen[i] : *refusal;
 }
 
+// logits = rms(hidden) . head^T
+int32_t output_product(nh_model *m) {
+    GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
+    head.norm_w = m->output_norm, head.eps = m->c.eps;
+    if (m->c.batch <= 8u || !gemm_takes_whole(head.element, head.K, m->h, m->output)) return launch_gemv(m->d, head);
+    // more rows than a narrow product takes at once: the wide one walks the vocabulary once for all of them
+    GemmArgs wide{head.element, m->output, head.N, head.K, m->h, NH_F32, m->c.batch, m->logits, nullptr, head.N};
+    wide.norm_w = m->output_norm, wide.eps = m->c.eps, wide.whole = true;
+    return launch_gemm(m->d, wide);
+}
+
 // every kernel of one decode step: the layers, then logits = rms(hidden) . head^T and the greedy
 // choice (examples/qwen/model.rs:81-84, crates/neura-generate/src/sampling.rs:69-71)
 int32_t decode_kernels(nh_model *m, bool any_inactive, bool sampled) {
     int32_t status;
     if ((status = forward(m, 1, any_inactive)) != NH_OK) return status;
-    GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
-    head.norm_w = m->output_norm, head.eps = m->c.eps;
-    if (m->c.batch > 8u && gemm_takes_whole(head.element, head.K, m->h, m->output)) {
-        // more rows than a narrow product takes at once: the wide one walks the vocabulary once for all of them
-        GemmArgs wide{head.element, m->output, head.N, head.K, m->h, NH_F32, m->c.batch, m->logits, nullptr, head.N};
-        wide.norm_w = m->output_norm, wide.eps = m->c.eps, wide.whole = true;
-        status = launch_gemm(m->d, wide);
-    } else {
-        status = launch_gemv(m->d, head);
-    }
-    if (status != NH_OK) return status;
+    if ((status = output_product(m)) != NH_OK) return status;
     // the choices and the refusal word go to the host's pinned words from a kernel of the step (part of the recorded graph): the
     // two device-to-host copies they would otherwise take are two more operations behind every step.  The greedy choice's
     // last kernel writes them itself; a sampled step has a kernel for it.
@@ -684,12 +685,10 @@ int32_t nh_model_time_products(nh_model *m, uint32_t steps, double *seconds_out,
     // `steps` passes of the same launches between one pair of events
     int32_t status;
     if ((status = nh_profile_begin(d)) != NH_OK) return status;
+    d->profile_wide = true;
     status = forward(m, 1, false, true);
-    if (status == NH_OK) {
-        GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
-        head.norm_w = m->output_norm, head.eps = m->c.eps;
-        status = launch_gemv(d, head);
-    }
+    if (status == NH_OK) status = output_product(m);
+    d->profile_wide = false;
     double ignored = 0.0;
     int32_t ended = nh_profile_end(d, &ignored, launches_out, bytes_out);
     if (status != NH_OK) return status;
@@ -697,9 +696,7 @@ int32_t nh_model_time_products(nh_model *m, uint32_t steps, double *seconds_out,
     if ((status = nh_timer_start(d)) != NH_OK) return status;
     for (uint32_t step = 0; step < steps; step++) {
         if ((status = forward(m, 1, false, true)) != NH_OK) return status;
-        GemvArgs head = narrow(m, m->output == m->token_embd ? m->elements[EMBD] : m->elements[HEAD], m->output, m->c.vocab, m->c.hidden, m->h, m->c.batch, m->logits);
-        head.norm_w = m->output_norm, head.eps = m->c.eps;
-        if ((status = launch_gemv(d, head)) != NH_OK) return status;
+        if ((status = output_product(m)) != NH_OK) return status;
     }
     if ((status = nh_timer_stop(d, seconds_out)) != NH_OK) return status;
     *launches_out *= steps;

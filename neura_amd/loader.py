@@ -140,7 +140,7 @@ class Model:
                                    self.batch))
 
     def time_products(self, steps):
-        """(device seconds, launches, weight bytes) of `steps` back-to-back passes over the narrow products of a decode step"""
+        """(device seconds, launches, weight bytes) of `steps` back-to-back passes over the products of a decode step"""
         seconds, launches, nbytes = ctypes.c_double(), ctypes.c_uint64(), ctypes.c_uint64()
         _check(self.lib.nh_model_time_products(self.handle, steps, ctypes.byref(seconds), ctypes.byref(launches), ctypes.byref(nbytes)))
         return seconds.value, launches.value, nbytes.value

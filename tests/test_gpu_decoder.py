@@ -259,6 +259,25 @@ def test_the_switches_send_a_mixed_layer_s_products_back(device, monkeypatch, ba
     weights.release()
 
 
+@pytest.mark.parametrize("base,mixed", [(NH_Q4_K, MIXED), (NH_Q3_K, MIXED_3), (NH_Q8_0, {})], ids=["q4_k_m", "q3_k_m", "q8_0"])
+@pytest.mark.parametrize("batch", [1, 2, 8, 9, 16])
+def test_timed_products_are_those_of_a_step(device, batch, base, mixed):
+    """nh_model_time_products counts every product that a step launches, whatever form it takes at this many planes: where each walks its
+    weights once, the bytes are those of all matrices."""
+    shape = SMALL_Q4
+    tensors = list(synth.model_tensors(shape, base, np.random.default_rng(4), mode="blocks", elements=mixed))
+    weights = Weights(device, tensors)
+    model = Model(device, weights, shape, base, batch, 40, 1)
+    matrices = {name: len(raw) for name, element, _, raw in tensors if element in synth.BLOCK_BYTES}
+    if not shape["tied"]:
+        matrices.pop("token_embd.weight")
+    for steps in (1, 3):
+        seconds, launches, walked = model.time_products(steps)
+        assert seconds > 0.0 and walked == steps * sum(matrices.values())
+        assert steps * (3 * shape["layers"] + 1) <= launches <= steps * len(matrices) and launches % steps == 0
+    model.release(), weights.release()
+
+
 def test_sampled_decode_steps_draw_as_the_oracle_draws(device):
     """A sampled answer program: the same forward pass, the choice drawn per plane with its own seed, temperature,
     candidate count and nucleus, all written by the host before each step (the recorded graph is replayed with new
