@@ -5,6 +5,7 @@
 // activation rows; each thread owns a 4 x 4 patch of the output in registers.
 #include "blocks.hpp"
 #include "common.hpp"
+#include "few_rule.hpp"
 #include "gemm_few.hpp"
 #include "gemv_shared.hpp"
 
@@ -1424,25 +1425,12 @@ bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const ui
     return true;
 }
 
-// Where the line lies (us, the vector and staged kernels, which walk the weights once for every two or four rows, -> here).  Q4_K has
-// tiles of its own and stays (7B shape, eight rows: gate|up 26 against 34, ffn_down 24 against 27).  Of the others five rows are three passes or
-// two and always lose, three rows are two (7B shape, eight rows: Q8_0 gate|up 307 -> 60, Q6_K ffn_down 103 -> 34; 0.5B shape: Q8_0
-// q|k|v 19 -> 8).  Four and two rows are one pass, and the packing (4 to 5 us) wants a matrix to be worth it: four rows Q8_0 always (1.5B
-// q|k|v 11 -> 9), the staged formats from 6 M numbers on (7B attn_output, 12.8 M: Q6_K 18 -> 16, Q3_K 18 -> 12; 1.5B q|k|v, 3.1 M: 7.4 against
-// 9.4); two rows Q8_0 from 12 M (7B attn_output 19 -> 14; 0.5B gate|up, 8.7 M: 10 against 11), Q5_K and Q3_K from 13 M (1.5B ffn_down,
-// 13.8 M: Q5_K 19 -> 15; 7B attn_output: 11 against 12), Q6_K from 60 M (7B ffn_down, 67.9 M: 34 -> 33; 1.5B gate|up, 27.5 M: 21 against 22).
-// The error against 64 bits is no larger (2-norm, those shapes: Q8_0 2.3..4e-7 -> 1.0..2.3e-7, Q6_K 1.5..2.3e-7 -> 1.2..1.9e-7, Q5_K
-// 1.5..2.4e-7 -> 1.3..2.1e-7, Q3_K 1.4..2.2e-7 -> 1.0..1.6e-7).
+// (the rule's measurements are beside it; the error against 64 bits is no larger -- N(0, 1) rows, 2-norm, the decoder shapes: Q8_0
+// 2.3..3.1e-7 -> 0.8..1.3e-7, Q6_K 1.5..1.6e-7 -> 1.1..1.2e-7, Q5_K 1.5..1.8e-7 -> 1.3..1.4e-7, Q3_K 1.5..1.6e-7 -> 0.9..1.0e-7)
 bool gemv_wide_takes(const nh_device *d, const GemvArgs &a) {
     const int held = env_int("NEURA_HIP_GEMV_WIDE", 1);  // 0 never, 2 wherever it can
     if (held == 0 || a.rows < 2u || a.rows > 8u || a.rope || a.append_value || a.merge || a.digits_in || a.digits_out || a.pairs_out) return false;
-    if (held != 2) {
-        if (a.element == NH_Q4_K) return false;
-        const uint64_t numbers = (uint64_t)a.N * a.K;
-        const uint64_t two = a.element == NH_Q8_0 ? 12000000u : a.element == NH_Q6_K ? 60000000u : 13000000u;
-        if (a.rows == 4u && a.element != NH_Q8_0 && numbers < 6000000u) return false;
-        if (a.rows == 2u && numbers < two) return false;
-    }
+    if (held != 2 && !few_narrow_rows_win(a.element, a.N, a.K, a.rows, a.swiglu, (uint32_t)d->compute_units)) return false;
     if ((uintptr_t)a.norm_w & 15u) return false;
     const uint32_t outputs = a.swiglu ? a.N / 2u : a.N;
     if (a.swiglu) return !a.residual && a.N % 2u == 0 && a.end[0] == outputs && a.W[1] && gemm_gates(d, a.element, outputs, a.K, whole_rows(a.rows), a.x, a.W[0], a.W[1]);
