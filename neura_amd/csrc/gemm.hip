@@ -1362,7 +1362,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     p.A = A, p.S = S, p.unscale = unscale;
     if (few)
         return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, pieces, p.unscale, reinterpret_cast<const WholeRow *>(unscale), outside,
-                                                       1u, 1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets}, a.gated);
+                                                       1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets}, a.gated);
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));

@@ -2,10 +2,12 @@
 // workgroups (a chunk of a short prompt, a step of more planes than the narrow products take).
 //
 // What bounds it is weight bytes in flight: a wave walks weight rows of 32 columns, a super-block of k at a time, the next
-// super-block's blocks on their way while it unpacks and multiplies this one's.  A workgroup is up to eight waves over `across`
-// tiles of columns and `deep` shares of K (wave `share` takes super-blocks share, share + deep, ...); they meet once, in LDS, at
-// the end of the walk, so nothing in the walk waits for another wave.  As many workgroups fill the chip as the matrix has column
-// tiles, and the K shares make up for narrow matrices -- no partial sums cross memory.
+// super-block's blocks on their way while it unpacks and multiplies this one's.  A workgroup is up to eight waves over one tile of
+// columns that share K (wave `share` takes super-blocks share, share + deep, ...); they meet once, in LDS, at the end of the walk, so
+// nothing in the walk waits for another wave.  Where a matrix has too few column tiles for the chip, `slices` workgroups share the K
+// of a tile as well: each leaves its sums in memory (`partial`, past the caches that workgroups do not share) and counts itself in
+// the tile's word of `meets`; the last to arrive adds them in the order of the slices and sets the word back to zero.  That
+// rests on the launches of a device following each other on its one stream and on the words being zero between them.
 //
 // v_mfma_f32_32x32x16_f16: the weights are B (lane l32 + 32 part unpacks the numbers of ITS column in registers: runs of 16
 // stored numbers at 32 i + 16 part, which for every format are the pieces its blocks are stored in), the packed activation rows
@@ -330,8 +332,8 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
     float4 *parts = reinterpret_cast<float4 *>(few_lds);  // [wave][NT][MT][4][64]
     const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, part = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t within = wave % p.deep, beside = wave / p.deep, shares = p.deep * p.slices, share = blockIdx.z * p.deep + within;
-    const uint32_t n0 = (blockIdx.x * p.across + beside) * FEW_TILE, tile0 = blockIdx.y * MT;
+    const uint32_t shares = p.deep * p.slices, share = blockIdx.z * p.deep + wave;
+    const uint32_t n0 = blockIdx.x * FEW_TILE, tile0 = blockIdx.y * MT;
     const uint32_t steps = p.K / 64u, units = (steps + STEPS - 1u) / STEPS;
     const uint32_t nsb = p.K / 256u;
 
@@ -470,17 +472,17 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
                 parts[(((wave * NT + t) * MT + i) * 4u + q) * 64u + lane] = float4{acc[t][i][4 * q], acc[t][i][4 * q + 1], acc[t][i][4 * q + 2], acc[t][i][4 * q + 3]};
     __syncthreads();
     // ---- out: an item is column l32 and rows 8q + 4 part .. + 3 of a 32 x 32 block; the shares of K are added in their order
-    const uint32_t items = p.across * MT * 256u;
+    constexpr uint32_t items = MT * 256u;
     auto own_sum = [&](uint32_t item, int t) {
-        const uint32_t at = item & 63u, q = (item >> 6) & 3u, i = (item >> 8) % MT, b = (item >> 8) / MT;
+        const uint32_t at = item & 63u, q = (item >> 6) & 3u, i = item >> 8;
         float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         for (uint32_t s = 0; s < p.deep; s++) {
-            const float4 add = parts[((((b * p.deep + s) * NT + t) * MT + i) * 4u + q) * 64u + at];
+            const float4 add = parts[(((s * NT + t) * MT + i) * 4u + q) * 64u + at];
             v.x += add.x, v.y += add.y, v.z += add.z, v.w += add.w;
         }
         return v;
     };
-    auto row_of = [&](uint32_t item) { return (tile0 + (item >> 8) % MT) * FEW_TILE + 8u * ((item >> 6) & 3u) + 4u * ((item >> 5) & 1u); };
+    auto row_of = [&](uint32_t item) { return (tile0 + (item >> 8)) * FEW_TILE + 8u * ((item >> 6) & 3u) + 4u * ((item >> 5) & 1u); };
     // with more workgroups over the same outputs: each leaves its sums in memory and the last to arrive adds them, in the order of
     // the slices, so the sums do not depend on who that is.  Nobody waits for another.
     typedef unsigned long long pair_word;
@@ -518,10 +520,10 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
     };
     if (p.pieces == WHOLE_PIECES) {
         // an item is a column and one of a tile's ten activation rows, whose pieces lie wherever rows 3r .. 3r + 2 do
-        const uint32_t rows = min(p.M, WHOLE_TILE), outputs = p.across * MT * rows * 32u;
+        const uint32_t rows = min(p.M, WHOLE_TILE), outputs = MT * rows * 32u;
         for (uint32_t item = threadIdx.x; item < outputs; item += blockDim.x) {
-            const uint32_t at = item & 31u, bi = (item >> 5) / rows, r = (item >> 5) - bi * rows, i = bi % MT, b = bi / MT;
-            const uint32_t m = (tile0 + i) * WHOLE_TILE + r, n = (blockIdx.x * p.across + b) * FEW_TILE + at;
+            const uint32_t at = item & 31u, i = (item >> 5) / rows, r = (item >> 5) - i * rows;
+            const uint32_t m = (tile0 + i) * WHOLE_TILE + r, n = n0 + at;
             if (n >= p.N || m >= p.M) continue;
             const u32x4 head = *(global_uint4)(uintptr_t)(p.whole + m);  // the scale, and how many numbers are listed
             float out[NT];
@@ -534,12 +536,12 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
                     v[j] = 0.0f;
                     if (p.slices == 1u) {
                         const float *sums = reinterpret_cast<const float *>(few_lds);
-                        for (uint32_t s = 0; s < p.deep; s++) v[j] += sums[((((b * p.deep + s) * NT + t) * MT + i) * 4u + q) * 256u + seat];
+                        for (uint32_t s = 0; s < p.deep; s++) v[j] += sums[(((s * NT + t) * MT + i) * 4u + q) * 256u + seat];
                     } else {
                         uint32_t held[FEW_SLICES_MOST];
 #pragma unroll
                         for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
-                            held[s] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(place_of(min(s, p.slices - 1u), bi * 256u + q * 64u + seat / 4u, t)) + (row & 3u), __ATOMIC_RELAXED,
+                            held[s] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(place_of(min(s, p.slices - 1u), i * 256u + q * 64u + seat / 4u, t)) + (row & 3u), __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
                         for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
@@ -560,7 +562,7 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
         return;
     }
     for (uint32_t item = threadIdx.x; item < items; item += blockDim.x) {
-        const uint32_t row = row_of(item), n = (blockIdx.x * p.across + (item >> 8) / MT) * FEW_TILE + (item & 31u);
+        const uint32_t row = row_of(item), n = n0 + (item & 31u);
         if (n >= p.N || row >= p.rows) continue;
         float v[NT][4];
 #pragma unroll
@@ -613,23 +615,23 @@ int32_t launch_few(nh_device *d, FewParams p) {
     // their sums, 2.5 MB in another (eight rows of fp32, with the packing: ffn_down of the 7B shape Q8_0 55 -> 37 us, Q6_K
     // 45 -> 34, Q5_K 37 -> 29, of the 1.5B shape Q8_0 28 -> 18; gate|up of the 7B shape, 592 tiles, is better left alone: Q4_K 34, not 38)
     uint32_t best = ~0u;
-    for (uint32_t across = 1; across <= 4u; across *= 2u)
-        for (uint32_t deep = 1; deep * across <= 8u; deep++)
-            for (uint32_t slices : slice_list) {
-                const uint32_t places = ((tiles + across - 1u) / across) * ((row_tiles + MT - 1u) / MT), resident = (uint32_t)d->compute_units * (8u / (deep * across));
-                if (slices > 1u && (places > FEW_MEETS || deep * slices > units || (size_t)slices * places * across * MT * NT * 4096u > FEW_PARTIAL_BYTES)) continue;
-                const uint32_t meeting = slices > 1u ? 64u + (uint32_t)((uint64_t)slices * p.N * NT * p.rows * 4u * 64u / 2500000u) : 0u;
-                const uint32_t cost = ((places * slices + resident - 1u) / resident) * ((units + deep * slices - 1u) / (deep * slices) + 2u) * 64u + meeting + across * deep;
-                if (cost < best) best = cost, p.across = across, p.deep = deep, p.slices = slices;
-            }
-    const size_t lds = (size_t)p.across * p.deep * NT * MT * 4096u;
+    const uint32_t places = tiles * ((row_tiles + MT - 1u) / MT);
+    for (uint32_t deep = 1; deep <= 8u; deep++)
+        for (uint32_t slices : slice_list) {
+            const uint32_t resident = (uint32_t)d->compute_units * (8u / deep);
+            if (slices > 1u && (places > FEW_MEETS || deep * slices > units || (size_t)slices * places * MT * NT * 4096u > FEW_PARTIAL_BYTES)) continue;
+            const uint32_t meeting = slices > 1u ? 64u + (uint32_t)((uint64_t)slices * p.N * NT * p.rows * 4u * 64u / 2500000u) : 0u;
+            const uint32_t cost = ((places * slices + resident - 1u) / resident) * ((units + deep * slices - 1u) / (deep * slices) + 2u) * 64u + meeting + deep;
+            if (cost < best) best = cost, p.deep = deep, p.slices = slices;
+        }
+    const size_t lds = (size_t)p.deep * NT * MT * 4096u;
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), hipFuncAttributeMaxDynamicSharedMemorySize, 8 * NT * MT * 4096));
         sized = true;
     }
-    const dim3 grid((tiles + p.across - 1u) / p.across, (row_tiles + MT - 1u) / MT, p.slices);
-    hipLaunchKernelGGL((gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), grid, dim3(64u * p.across * p.deep), lds, d->stream, p);
+    const dim3 grid(tiles, (row_tiles + MT - 1u) / MT, p.slices);
+    hipLaunchKernelGGL((gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), grid, dim3(64u * p.deep), lds, d->stream, p);
     NH_HIP(hipGetLastError());
     return NH_OK;
 }

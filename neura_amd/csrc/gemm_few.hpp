@@ -60,7 +60,7 @@ struct FewParams {
     const float *unscale;   // [M], with two pieces
     const WholeRow *whole;  // [M], with three
     const float *outside;   // [M][K], with three: the rows as fp32 numbers
-    uint32_t across, deep;  // the waves of a workgroup: tiles of columns x shares of K
+    uint32_t deep;          // the waves of a workgroup: shares of K
     uint32_t slices;        // workgroups (blockIdx.z) that share the K of the same tiles
     float *partial;         // FEW_PARTIAL_BYTES of scratch for their sums
     uint32_t *meets;        // FEW_MEETS words, zero between launches: workgroups of a place that have left their sums
