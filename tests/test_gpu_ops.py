@@ -598,10 +598,12 @@ def test_q6_k_q5_k_and_q3_k_wide_products_on_the_matrix_cores(device, element, M
     (NH_Q4_K, 1, 256, 256, False), (NH_Q4_K, 16, 96, 1536, False), (NH_Q4_K, 17, 130, 512, False), (NH_Q4_K, 48, 100, 2304, False), (NH_Q4_K, 100, 640, 1024, True),
     (NH_Q5_K, 33, 33, 768, True), (NH_Q5_K, 9, 2080, 512, False), (NH_Q6_K, 5, 64, 2816, False), (NH_Q6_K, 65, 129, 1024, True), (NH_Q6_K, 49, 160, 256, False),
     (NH_Q3_K, 12, 65, 2816, False), (NH_Q3_K, 97, 96, 512, True), (NH_Q8_0, 9, 77, 64, False), (NH_Q8_0, 40, 500, 192, False), (NH_Q8_0, 33, 300, 4864, False),
-    (NH_Q8_0, 130, 33, 320, True)])
+    (NH_Q8_0, 130, 33, 320, True), (NH_Q4_K, 33, 4130, 512, False), (NH_Q5_K, 48, 4130, 512, False), (NH_Q6_K, 33, 4130, 512, False), (NH_Q6_K, 70, 4130, 256, False),
+    (NH_Q3_K, 42, 4130, 512, False), (NH_Q3_K, 65, 4130, 768, True), (NH_Q8_0, 48, 4130, 192, False), (NH_Q5_K, 33, 4224, 1280, False)])
 def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, K, half):
     """The wide product of few rows (operands in registers, the K shares of a workgroup's waves meeting in LDS) and the one of 128 x 128
-    tiles, each forced: single tiles, ragged columns and rows, one to three row tiles a wave and more, K of one unit, of fewer units than
+    tiles, each forced: single tiles, ragged columns and rows, one and two row tiles a wave, three (more than 128 column
+    tiles, three row tiles or five of them, the last ones ragged) and more passes, K of one unit, of fewer units than
     waves and of half a Q8_0 unit -- against the exact product.  Bar: 22 bits of every activation take part and fp32 sums of K terms
     in any order stay within a few rounding errors of the sum of magnitudes' root (1e-6 of the outputs' scale at these depths)."""
     monkeypatch.setenv("NEURA_HIP_GEMM_FEW", form)
