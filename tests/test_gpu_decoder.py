@@ -197,9 +197,10 @@ MIXED_3 = {"output.weight": NH_Q6_K, "blk.0.attn_v.weight": NH_Q5_K, "blk.1.attn
 @pytest.mark.parametrize("batch", [1, 2, 8])
 def test_mixed_elements_and_projection_biases(device, batch, base, mixed):
     """A decoder stored the way Q4_K_M files are (Q6_K for some matrices, Q4_K for the rest) whose q, k and v projections
-    carry Qwen2's biases: layer 0 (a Q6_K value projection, biases) takes one product per matrix, layer 1 (one element,
-    biases) folds rotation and biases into the stacked product at batch 1, layer 2 (gate and up stored differently) runs
-    the two halves apart.  Decode steps, a 16-row fill and the caches against the oracle.  The same for decoders stored in
+    carry Qwen2's biases: layer 0 (a Q6_K value projection, biases) rotates q|k in one product and appends v from another at
+    batch 1, and at batch 2 and 8 and in the fill multiplies rows packed once by q|k and by v, the biases added by the rotation; layer
+    1 (one element, biases) folds rotation and biases into the stacked product at batch 1 and 8; layer 2 (gate and up stored
+    differently) runs the two halves apart.  Decode steps, a 16-row fill and the caches against the oracle.  The same for decoders stored in
     one K-quant throughout (the fill's q|k|v is then one stacked wide product of that element on the matrix cores).  In the
     Q3_K_M mix layers 0 and 1 rotate q|k in a Q3_K product and cast the rows of a Q5_K and a Q4_K value projection into the
     value state from those products' own epilogues."""
@@ -275,6 +276,35 @@ def test_timed_products_are_those_of_a_step(device, batch, base, mixed):
         seconds, launches, walked = model.time_products(steps)
         assert seconds > 0.0 and walked == steps * sum(matrices.values())
         assert steps * (3 * shape["layers"] + 1) <= launches <= steps * len(matrices) and launches % steps == 0
+    model.release(), weights.release()
+
+
+@pytest.mark.parametrize("few", [None, "0", "1"])
+def test_a_fill_whose_projections_take_different_forms(device, monkeypatch, few):
+    """256 rows of a layer whose value projection is stored otherwise: q|k, 5120 columns stacked, fill the chip as 128 x 128 tiles and v, 1024 of
+    them, is a product of few rows, so they pack the rows apart and the norm runs before (the default); with either form forced the three
+    share them.  Caches and the next step's logits against the oracle."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_FEW", few) if few else monkeypatch.delenv("NEURA_HIP_GEMM_FEW", raising=False)
+    shape = dict(layers=2, hidden=512, heads=32, kv_heads=8, head_dim=128, ffn=1024, vocab=1000, tied=False)
+    mixed = {"blk.0.attn_v.weight": NH_Q6_K, "blk.1.attn_v.weight": NH_Q5_K}
+    rng = np.random.default_rng(43)
+    tensors = list(synth.model_tensors(shape, NH_Q4_K, rng, mode="normal", elements=mixed, biases=(0, 1)))
+    host = {name: (raw.view(np.float32) if name.endswith(".bias") else raw) for name, _, _, raw in tensors}
+    weights = Weights(device, tensors)
+    model = Model(device, weights, shape, NH_Q4_K, 1, 260, 256)
+    ref = oracle.Model(shape, NH_Q4_K, host, 1, 260, 256, elements=mixed)
+    prompt = rng.integers(0, shape["vocab"], 256)
+    model.prefill(prompt, 256, [0])
+    ref.forward(prompt, 256, [0], want_logits=False, threads=16)
+    want_logits, want = ref.forward([7], 1, [256])
+    got = model.decode_step([7], [256])
+    assert np.abs(model.logits() - want_logits).max() <= 1e-3 * np.abs(want_logits).max()
+    assert list(got) == list(want), margins(want_logits)
+    for layer in range(shape["layers"]):
+        for which, held in ((0, ref.cache_k), (1, ref.cache_v)):
+            got_cache = oracle.f16_to_f32(model.cache_read(layer, which).reshape(-1))
+            want_cache = oracle.f16_to_f32(held[layer])
+            assert np.abs(got_cache - want_cache).max() <= 2e-3 * max(1.0, np.abs(want_cache).max())
     model.release(), weights.release()
 
 
@@ -754,8 +784,8 @@ def test_rotation_folded_into_the_product_of_several_planes(device, monkeypatch,
     """Five to eight planes of one token each: the q|k|v product of a Q4_K decoder (the 32-row integer tiles) rotates q and k
     and appends k and v in its epilogue, every plane at its own cursor.  The twin with the rotation as a kernel of its own runs
     the same product kernel and the same table of cosines and sines, so logits and caches agree bit for bit; both are held to
-    the oracle (logits, tokens, and the rows the steps appended).  With q, k and v biases the twin multiplies the three
-    matrices one by one: each row's sums are the same, and so are the bits."""
+    the oracle (logits, tokens, and the rows the steps appended).  With q, k and v biases the twin's stacked product leaves
+    them to the rotation's kernel, which adds them first as the folded epilogue does: the same sums, and the same bits."""
     monkeypatch.setenv("NEURA_HIP_GRAPH", "0")  # both twins launch eagerly, so the switch below is read at every step
     layers = list(range(shape["layers"])) if biased else []
 

@@ -485,7 +485,7 @@ def test_gemv_is_linear_and_matches_at_full_size(device, element):
     both = device.gemv(element, raw, N, K, np.float32(0.5) * x - np.float32(2.0) * z)[0]
     tight(both, 0.5 * yx - 2.0 * yz, 1e-5)
     batched = device.gemv(element, raw, N, K, np.stack([x, z]))
-    tight(batched[0], yx, 3e-6)  # (two rows of a K-quant other than Q4_K run the staged kernel: another order of the sums)
+    tight(batched[0], yx, 3e-6)  # (two rows of a K-quant other than Q4_K run the product of few rows at this size: another order of the sums)
     tight(batched[1], yz, 3e-6)
     assert np.array_equal(yx, device.gemv(element, raw, N, K, x)[0])  # deterministic
     # and a handful of rows against the exact product of the unpacked weights
