@@ -42,24 +42,24 @@ inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows,
 }
 
 // The same for two to eight rows of a narrow product, against the vector and staged kernels (gemv.hip), which walk the weights once for
-// every four, two or one rows.  Q4_K has tiles of its own and stays (7B shape, eight rows: gate|up 25 against 38 us, ffn_down 23 against
-// 29).  Of the others three rows and five are two passes or more and go (7B shape, eight rows: Q8_0 gate|up 303 -> 64, Q6_K ffn_down 101 ->
-// 34; the worst of 53 shapes at three rows: 1.12 times).  Two and four rows are one pass.  The staged kernel takes eight columns and a
+// every four, two or one rows.  Q4_K has tiles of its own and stays (7B shape, eight rows: gate|up 25 against 36 us, ffn_down 23 against
+// 30).  Of the others three rows and five are two passes or more and go (7B shape, eight rows: Q8_0 gate|up 304 -> 62, Q6_K ffn_down 101 ->
+// 34; the worst of 53 shapes at three rows: 1.06 times).  Two and four rows are one pass.  The staged kernel takes eight columns and a
 // slice of K a workgroup: up to two workgroups a compute unit it is one round of latency, which the packing launch alone does not
-// beat (4096 x 3584, 512 of them, two rows: Q3_K 8.9 against 12.4, Q5_K 10.2 against 13.0, Q6_K 9.8 against 15.7), and a second
-// round costs more than all of the product here (4608 x 3584, 576: Q3_K 14.4 -> 12.6, Q5_K 16.6 -> 13.2; 4 rows of 3584 x 3584, 896:
-// Q3_K 18.4 -> 12.8, Q6_K 18.5 -> 16.2).  Four rows of Q5_K fill a compute unit's LDS with one.  Two rows of Q6_K, two planes of MFMAs,
-// are worth it later (4608 x 3584 15.3 against 16.3, 1536 x 8960 16.6 against 17.5, 16768 x 1024 18 -> 15), gated ones, two matrices, later
-// still (17920 x 1536 20.5 against 22.7, 37888 x 3584 57 -> 54).  Q8_0 streams on the vector
-// kernel without rounds; two rows of it go where the walk outweighs the packing, 46 K numbers a compute unit (3584 x 3584 18.6 ->
-// 14.1, 2688 x 4096 12.9 against 16.0).  Over 1245 products timed in both forms the pick takes 1.002 times the faster one's time on average.
+// beat (4096 x 3584, 512 of them, two rows: Q3_K 8.9 against 11.7, Q5_K 10.2 against 12.4, Q6_K 9.8 against 15.3), and a second
+// round costs more than all of the product here (4608 x 3584, 576: Q3_K 14.3 -> 11.9, Q5_K 16.4 -> 12.5; four rows of 3584 x 3584, 896:
+// Q3_K 18.3 -> 12.2, Q6_K 18.4 -> 15.8).  Four rows of Q5_K fill a compute unit's LDS with one (2048 x 1536, 256: 8.0 against 8.7; 3584 x
+// 3584 27 -> 13).  Two gated rows of Q6_K, two planes of MFMAs over two matrices, are worth it later (17920 x 1536 20.3 against 21.3,
+// 37888 x 3584 57 -> 52).  Q8_0 streams on the vector kernel without rounds; two rows of it go where the walk outweighs the packing, 46 K
+// numbers a compute unit (3584 x 3584 18.5 -> 13.5, 2688 x 4096 13.0 against 15.1).  Over 1245 products timed in both forms the pick takes
+// 1.003 times the faster one's time on average.
 inline bool few_narrow_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows, bool gated, uint32_t compute_units) {
     if (element == NH_Q4_K) return false;
     if (rows == 3u || rows >= 5u) return true;
     if (element == NH_Q8_0) return rows == 4u || (uint64_t)N * K >= 46000u * (uint64_t)compute_units;
     const uint64_t blocks = K / 256u, most = rows == 4u ? 8u : 16u, workgroups = (N + 7u) / 8u * ((blocks + most - 1u) / most);
     if (element == NH_Q5_K && rows == 4u) return workgroups > compute_units;
-    if (element == NH_Q6_K && rows == 2u) return workgroups > (gated ? 12u : 3u) * (uint64_t)compute_units;
+    if (element == NH_Q6_K && rows == 2u && gated) return workgroups > 12u * (uint64_t)compute_units;
     return workgroups > 2u * (uint64_t)compute_units;
 }
 

@@ -317,6 +317,15 @@ __device__ __forceinline__ float beyond_pieces(float value, const WholeRow &held
     return (float)sum;
 }
 
+// where piece j of a tile's activation row r lies among the sums of a 32 x 32 block, [q][part][column][4]: q and the rest at column 0
+struct PieceRow {
+    uint32_t q, seat;
+};
+__device__ __forceinline__ PieceRow piece_row(uint32_t r, uint32_t j) {
+    const uint32_t row = WHOLE_PIECES * r + j;
+    return {row >> 3, ((row >> 2) & 1u) * 128u + (row & 3u)};
+}
+
 // MT: tiles of 32 packed rows a wave multiplies its weights by; GATED: a wave walks the same 32 columns of the gate and of the up
 // matrix, and what leaves is silu(gate) * up; AHEAD: steps the activation operands are read ahead (the loads of a wave come
 // back in order: an operand asked for after the next super-block's weights waits for them, so they are asked for
@@ -371,6 +380,12 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
 #pragma unroll
         for (int i = 0; i < MT; i++) a[slot][depth][i] = __builtin_bit_cast(half8_t, *(global_uint4)(uintptr_t)(arow[i] + at));
     };
+    // a whole row's scale and whether it lists numbers: asked for before the weights and put by for the end
+    __shared__ float2 heads[MT * WHOLE_TILE];
+    if (p.pieces == WHOLE_PIECES && threadIdx.x < MT * WHOLE_TILE) {
+        const u32x4 head = *(global_uint4)(uintptr_t)(p.whole + min(tile0 * WHOLE_TILE + threadIdx.x, p.M - 1u));
+        heads[threadIdx.x] = float2{__builtin_bit_cast(float, head.x), __builtin_bit_cast(float, head.z | head.w)};
+    }
     if (share < units) {
         Weights next[NT];
 #pragma unroll
@@ -525,31 +540,41 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
             const uint32_t at = item & 31u, i = (item >> 5) / rows, r = (item >> 5) - i * rows;
             const uint32_t m = (tile0 + i) * WHOLE_TILE + r, n = n0 + at;
             if (n >= p.N || m >= p.M) continue;
-            const u32x4 head = *(global_uint4)(uintptr_t)(p.whole + m);  // the scale, and how many numbers are listed
-            float out[NT];
+            const float2 head = heads[i * WHOLE_TILE + r];
+            float out[NT], v[NT][WHOLE_PIECES];
+            // (every load of a share's sums before any is added: a chain of them is an LDS latency each)
+            if (p.slices == 1u) {
+                const float *sums = reinterpret_cast<const float *>(few_lds);
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                float v[WHOLE_PIECES];
+                for (int t = 0; t < NT; t++)
 #pragma unroll
-                for (uint32_t j = 0; j < WHOLE_PIECES; j++) {
-                    const uint32_t row = WHOLE_PIECES * r + j, seat = (((row >> 2) & 1u) * 32u + at) * 4u + (row & 3u), q = row >> 3;
-                    v[j] = 0.0f;
-                    if (p.slices == 1u) {
-                        const float *sums = reinterpret_cast<const float *>(few_lds);
-                        for (uint32_t s = 0; s < p.deep; s++) v[j] += sums[(((s * NT + t) * MT + i) * 4u + q) * 256u + seat];
-                    } else {
+                    for (uint32_t j = 0; j < WHOLE_PIECES; j++) v[t][j] = 0.0f;
+                for (uint32_t s = 0; s < p.deep; s++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+#pragma unroll
+                        for (uint32_t j = 0; j < WHOLE_PIECES; j++) v[t][j] += sums[(((s * NT + t) * MT + i) * 4u + piece_row(r, j).q) * 256u + piece_row(r, j).seat + at * 4u];
+            } else {
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (uint32_t j = 0; j < WHOLE_PIECES; j++) {
                         uint32_t held[FEW_SLICES_MOST];
 #pragma unroll
                         for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
-                            held[s] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(place_of(min(s, p.slices - 1u), i * 256u + q * 64u + seat / 4u, t)) + (row & 3u), __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT);
+                            held[s] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(place_of(min(s, p.slices - 1u), i * 256u + piece_row(r, j).q * 64u + piece_row(r, j).seat / 4u + at, t)) +
+                                                            piece_row(r, j).seat % 4u,
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        v[t][j] = 0.0f;
 #pragma unroll
                         for (uint32_t s = 0; s < FEW_SLICES_MOST; s++)
-                            if (s < p.slices) v[j] += __builtin_bit_cast(float, held[s]);
+                            if (s < p.slices) v[t][j] += __builtin_bit_cast(float, held[s]);
                     }
-                }
-                out[t] = fmaf(fmaf(v[2], 0.00048828125f, v[1]), 0.00048828125f, v[0]) * __builtin_bit_cast(float, head.x);
-                if (head.z | head.w) {
+            }
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                out[t] = fmaf(fmaf(v[t][2], 0.00048828125f, v[t][1]), 0.00048828125f, v[t][0]) * head.x;
+                if (__builtin_bit_cast(uint32_t, head.y)) {
                     const uint8_t *from = GATED        ? (t ? p.W1 : p.W) + (size_t)n * p.row_bytes
                                           : n < p.end0 ? p.W + (size_t)n * p.row_bytes
                                           : n < p.end1 ? p.W1 + (size_t)(n - p.end0) * p.row_bytes

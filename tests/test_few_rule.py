@@ -25,55 +25,55 @@ MEASURED = [
     (Q4_K, 8960, 1536, 768, 46.3, 56.9), (Q4_K, 896, 4864, 2048, 60.9, 54.7), (Q4_K, 3584, 3584, 1024, 47.9, 61.3)]
 
 NARROW = [
-    (Q8_0, 4608, 3584, 2, False, 19.8, 16.2), (Q8_0, 4608, 3584, 4, False, 31.9, 16.4), (Q3_K, 4608, 3584, 2, False, 14.4, 12.6),
-    (Q3_K, 4608, 3584, 4, False, 19.9, 12.9), (Q5_K, 4608, 3584, 2, False, 16.6, 13.2), (Q5_K, 4608, 3584, 4, False, 30.7, 13.6),
-    (Q6_K, 4608, 3584, 2, False, 15.3, 16.3), (Q6_K, 4608, 3584, 4, False, 20.2, 16.5), (Q8_0, 3584, 3584, 2, False, 18.6, 14.1),
-    (Q8_0, 3584, 3584, 3, False, 26.3, 14.5), (Q8_0, 3584, 3584, 4, False, 25.1, 14.5), (Q3_K, 3584, 3584, 2, False, 8.8, 12.4),
-    (Q3_K, 3584, 3584, 3, False, 15.6, 12.8), (Q3_K, 3584, 3584, 4, False, 18.2, 12.8), (Q5_K, 3584, 3584, 2, False, 10.0, 13.0),
-    (Q5_K, 3584, 3584, 3, False, 17.3, 13.3), (Q5_K, 3584, 3584, 4, False, 27.1, 13.4), (Q6_K, 3584, 3584, 2, False, 9.5, 15.8),
-    (Q6_K, 3584, 3584, 3, False, 15.9, 16.3), (Q6_K, 3584, 3584, 4, False, 18.4, 16.2), (Q8_0, 37888, 3584, 2, True, 110.0, 56.3),
-    (Q8_0, 37888, 3584, 4, True, 154.9, 63.6), (Q3_K, 37888, 3584, 2, True, 55.9, 39.9), (Q3_K, 37888, 3584, 4, True, 91.6, 40.6),
-    (Q5_K, 37888, 3584, 2, True, 69.4, 41.0), (Q5_K, 37888, 3584, 4, True, 146.8, 42.1), (Q6_K, 37888, 3584, 2, True, 57.4, 54.0),
-    (Q6_K, 37888, 3584, 4, True, 94.2, 55.0), (Q8_0, 3584, 18944, 2, False, 61.0, 32.7), (Q8_0, 3584, 18944, 4, False, 89.0, 34.4),
-    (Q3_K, 3584, 18944, 2, False, 32.9, 23.7), (Q3_K, 3584, 18944, 4, False, 50.5, 24.1), (Q5_K, 3584, 18944, 2, False, 38.8, 25.8),
-    (Q5_K, 3584, 18944, 4, False, 77.5, 26.9), (Q6_K, 3584, 18944, 2, False, 34.2, 30.9), (Q6_K, 3584, 18944, 4, False, 51.5, 31.6),
-    (Q8_0, 512, 3584, 2, False, 9.8, 11.4), (Q8_0, 512, 3584, 3, False, 13.8, 11.6), (Q8_0, 512, 3584, 4, False, 13.1, 11.6),
-    (Q3_K, 512, 3584, 2, False, 7.2, 11.8), (Q3_K, 512, 3584, 3, False, 13.0, 11.9), (Q3_K, 512, 3584, 4, False, 9.6, 11.9),
-    (Q5_K, 512, 3584, 2, False, 8.2, 11.9), (Q5_K, 512, 3584, 3, False, 14.8, 12.2), (Q5_K, 512, 3584, 4, False, 10.2, 12.2),
-    (Q6_K, 512, 3584, 2, False, 7.1, 14.0), (Q6_K, 512, 3584, 3, False, 12.7, 14.3), (Q6_K, 512, 3584, 4, False, 9.5, 14.3),
-    (Q8_0, 2048, 1536, 2, False, 8.0, 9.8), (Q8_0, 2048, 1536, 3, False, 11.2, 9.9), (Q8_0, 2048, 1536, 4, False, 11.1, 10.0),
-    (Q3_K, 2048, 1536, 2, False, 5.5, 8.7), (Q3_K, 2048, 1536, 3, False, 10.0, 8.9), (Q3_K, 2048, 1536, 4, False, 7.5, 8.8),
-    (Q5_K, 2048, 1536, 2, False, 6.0, 9.1), (Q5_K, 2048, 1536, 3, False, 10.8, 9.1), (Q5_K, 2048, 1536, 4, False, 8.0, 9.1),
-    (Q6_K, 2048, 1536, 2, False, 5.5, 9.9), (Q6_K, 2048, 1536, 3, False, 9.7, 10.0), (Q6_K, 2048, 1536, 4, False, 7.4, 10.0),
-    (Q8_0, 1536, 1536, 2, False, 8.1, 9.8), (Q8_0, 1536, 1536, 4, False, 11.1, 9.9), (Q3_K, 1536, 1536, 2, False, 5.5, 8.7),
-    (Q3_K, 1536, 1536, 4, False, 7.4, 8.8), (Q5_K, 1536, 1536, 2, False, 5.9, 9.0), (Q5_K, 1536, 1536, 4, False, 7.9, 9.1),
-    (Q6_K, 1536, 1536, 2, False, 5.4, 9.9), (Q6_K, 1536, 1536, 4, False, 7.4, 9.9), (Q8_0, 17920, 1536, 2, True, 29.8, 22.8),
-    (Q8_0, 17920, 1536, 4, True, 45.3, 23.1), (Q3_K, 17920, 1536, 2, True, 19.6, 17.2), (Q3_K, 17920, 1536, 4, True, 27.2, 17.8),
-    (Q5_K, 17920, 1536, 2, True, 22.9, 18.2), (Q5_K, 17920, 1536, 4, True, 43.9, 18.8), (Q6_K, 17920, 1536, 2, True, 20.3, 22.6),
-    (Q6_K, 17920, 1536, 4, True, 27.6, 23.2), (Q8_0, 1536, 8960, 2, False, 18.6, 16.7), (Q8_0, 1536, 8960, 4, False, 25.6, 15.9),
-    (Q3_K, 1536, 8960, 2, False, 16.2, 14.6), (Q3_K, 1536, 8960, 4, False, 19.8, 15.0), (Q5_K, 1536, 8960, 2, False, 18.2, 15.3),
-    (Q5_K, 1536, 8960, 4, False, 30.4, 15.8), (Q6_K, 1536, 8960, 2, False, 16.6, 17.5), (Q6_K, 1536, 8960, 4, False, 20.1, 17.8),
-    (Q8_0, 256, 1536, 2, False, 7.6, 9.0), (Q8_0, 256, 1536, 4, False, 10.7, 9.0), (Q3_K, 256, 1536, 2, False, 5.3, 8.8),
-    (Q3_K, 256, 1536, 4, False, 7.3, 8.9), (Q5_K, 256, 1536, 2, False, 5.8, 9.0), (Q5_K, 256, 1536, 4, False, 7.7, 9.1),
-    (Q6_K, 256, 1536, 2, False, 5.3, 9.7), (Q6_K, 256, 1536, 4, False, 7.1, 9.8), (Q8_0, 1152, 896, 2, False, 7.4, 8.6),
-    (Q8_0, 1152, 896, 4, False, 9.9, 8.7), (Q8_0, 896, 896, 2, False, 7.5, 8.7), (Q8_0, 896, 896, 4, False, 9.8, 8.7),
-    (Q8_0, 9728, 896, 2, True, 10.2, 12.9), (Q8_0, 9728, 896, 3, True, 13.8, 13.1), (Q8_0, 9728, 896, 4, True, 20.6, 13.0),
-    (Q8_0, 896, 4864, 2, False, 11.3, 11.0), (Q8_0, 896, 4864, 4, False, 14.4, 12.5), (Q8_0, 4096, 3584, 2, False, 18.9, 14.3),
-    (Q3_K, 4096, 3584, 2, False, 8.9, 12.4), (Q5_K, 4096, 3584, 2, False, 10.2, 13.0), (Q6_K, 4096, 3584, 2, False, 9.8, 16.0),
-    (Q8_0, 14592, 1280, 2, False, 24.9, 13.4), (Q5_K, 2944, 256, 2, False, 6.1, 7.0), (Q5_K, 2688, 4096, 4, False, 23.5, 14.2),
-    (Q8_0, 2816, 14336, 2, False, 39.6, 29.2), (Q5_K, 20864, 512, 4, False, 45.6, 10.2), (Q6_K, 384, 16384, 4, False, 10.9, 16.1),
-    (Q6_K, 3712, 1280, 2, False, 5.9, 9.7), (Q5_K, 384, 5120, 4, False, 10.0, 11.7), (Q5_K, 5376, 16384, 2, False, 45.7, 28.7),
-    (Q5_K, 1408, 2048, 4, False, 8.1, 10.2), (Q6_K, 384, 5120, 2, False, 9.1, 12.4), (Q6_K, 5504, 4096, 2, False, 15.4, 16.5),
-    (Q6_K, 384, 3072, 2, False, 7.0, 10.3), (Q6_K, 14592, 1280, 2, False, 17.4, 14.3), (Q5_K, 1280, 2048, 2, False, 6.1, 10.1),
-    (Q3_K, 2048, 11264, 2, False, 16.7, 15.6), (Q8_0, 640, 14336, 4, False, 25.3, 16.5), (Q3_K, 5760, 1280, 2, False, 9.5, 8.6),
-    (Q5_K, 2816, 256, 4, False, 13.6, 7.7), (Q8_0, 384, 256, 2, False, 6.2, 6.7), (Q6_K, 1536, 2048, 4, False, 7.5, 10.4),
-    (Q6_K, 6912, 11264, 2, False, 37.0, 29.1), (Q8_0, 20864, 512, 4, False, 19.8, 11.1), (Q5_K, 20864, 512, 2, False, 25.2, 9.8),
-    (Q3_K, 768, 256, 4, False, 8.1, 7.3), (Q3_K, 384, 11264, 2, False, 9.4, 12.0), (Q6_K, 2944, 256, 4, False, 7.0, 7.7),
-    (Q6_K, 16768, 1024, 4, False, 24.0, 15.1), (Q3_K, 3840, 1280, 4, False, 8.3, 8.6), (Q6_K, 2816, 14336, 2, False, 24.6, 24.8),
-    (Q8_0, 768, 256, 2, False, 6.1, 6.8), (Q5_K, 20992, 256, 2, False, 25.8, 7.4), (Q8_0, 1280, 4096, 2, False, 12.1, 13.3),
-    (Q3_K, 1152, 8192, 4, False, 16.2, 12.9), (Q6_K, 2816, 256, 2, False, 5.3, 7.0), (Q3_K, 14592, 1280, 2, False, 17.1, 11.2),
-    (Q6_K, 640, 14336, 2, False, 11.2, 15.5), (Q6_K, 20864, 512, 2, False, 20.7, 11.2), (Q3_K, 4864, 512, 2, False, 8.6, 6.8),
-    (Q8_0, 256, 6144, 4, False, 13.4, 12.2)]
+    (Q8_0, 4608, 3584, 2, False, 19.8, 15.5), (Q8_0, 4608, 3584, 4, False, 31.9, 15.8), (Q3_K, 4608, 3584, 2, False, 14.3, 11.9),
+    (Q3_K, 4608, 3584, 4, False, 19.9, 12.2), (Q5_K, 4608, 3584, 2, False, 16.4, 12.5), (Q5_K, 4608, 3584, 4, False, 30.8, 13.0),
+    (Q6_K, 4608, 3584, 2, False, 15.2, 15.6), (Q6_K, 4608, 3584, 4, False, 20.1, 16.0), (Q8_0, 3584, 3584, 2, False, 18.5, 13.5),
+    (Q8_0, 3584, 3584, 3, False, 26.2, 14.2), (Q8_0, 3584, 3584, 4, False, 25.1, 14.2), (Q3_K, 3584, 3584, 2, False, 8.8, 11.7),
+    (Q3_K, 3584, 3584, 3, False, 15.5, 12.2), (Q3_K, 3584, 3584, 4, False, 18.3, 12.2), (Q5_K, 3584, 3584, 2, False, 10.0, 12.3),
+    (Q5_K, 3584, 3584, 3, False, 17.2, 12.7), (Q5_K, 3584, 3584, 4, False, 27.2, 12.8), (Q6_K, 3584, 3584, 2, False, 9.5, 15.2),
+    (Q6_K, 3584, 3584, 3, False, 15.9, 15.8), (Q6_K, 3584, 3584, 4, False, 18.4, 15.8), (Q8_0, 37888, 3584, 2, True, 110.3, 55.1),
+    (Q8_0, 37888, 3584, 4, True, 154.8, 62.6), (Q3_K, 37888, 3584, 2, True, 55.8, 38.3), (Q3_K, 37888, 3584, 4, True, 91.4, 38.7),
+    (Q5_K, 37888, 3584, 2, True, 69.5, 39.0), (Q5_K, 37888, 3584, 4, True, 147.7, 40.1), (Q6_K, 37888, 3584, 2, True, 57.0, 52.4),
+    (Q6_K, 37888, 3584, 4, True, 94.4, 53.1), (Q8_0, 3584, 18944, 2, False, 60.9, 32.2), (Q8_0, 3584, 18944, 4, False, 89.5, 34.1),
+    (Q3_K, 3584, 18944, 2, False, 32.7, 22.5), (Q3_K, 3584, 18944, 4, False, 50.5, 23.7), (Q5_K, 3584, 18944, 2, False, 38.7, 25.1),
+    (Q5_K, 3584, 18944, 4, False, 77.6, 26.3), (Q6_K, 3584, 18944, 2, False, 34.1, 29.9), (Q6_K, 3584, 18944, 4, False, 51.5, 31.1),
+    (Q8_0, 512, 3584, 2, False, 9.9, 10.6), (Q8_0, 512, 3584, 3, False, 13.7, 11.0), (Q8_0, 512, 3584, 4, False, 13.0, 11.1),
+    (Q3_K, 512, 3584, 2, False, 7.2, 11.0), (Q3_K, 512, 3584, 3, False, 13.0, 11.3), (Q3_K, 512, 3584, 4, False, 9.4, 11.3),
+    (Q5_K, 512, 3584, 2, False, 8.2, 11.2), (Q5_K, 512, 3584, 3, False, 14.8, 11.4), (Q5_K, 512, 3584, 4, False, 10.0, 11.5),
+    (Q6_K, 512, 3584, 2, False, 7.2, 13.3), (Q6_K, 512, 3584, 3, False, 12.8, 13.5), (Q6_K, 512, 3584, 4, False, 9.4, 13.5),
+    (Q8_0, 2048, 1536, 2, False, 8.1, 9.3), (Q8_0, 2048, 1536, 3, False, 11.1, 9.5), (Q8_0, 2048, 1536, 4, False, 11.1, 9.4),
+    (Q3_K, 2048, 1536, 2, False, 5.5, 8.2), (Q3_K, 2048, 1536, 3, False, 9.8, 8.3), (Q3_K, 2048, 1536, 4, False, 7.4, 8.3),
+    (Q5_K, 2048, 1536, 2, False, 6.0, 8.5), (Q5_K, 2048, 1536, 3, False, 10.7, 8.6), (Q5_K, 2048, 1536, 4, False, 8.0, 8.7),
+    (Q6_K, 2048, 1536, 2, False, 5.4, 9.5), (Q6_K, 2048, 1536, 3, False, 9.7, 9.6), (Q6_K, 2048, 1536, 4, False, 7.4, 9.7),
+    (Q8_0, 1536, 1536, 2, False, 8.1, 9.1), (Q8_0, 1536, 1536, 4, False, 11.2, 9.4), (Q3_K, 1536, 1536, 2, False, 5.4, 8.2),
+    (Q3_K, 1536, 1536, 4, False, 7.4, 8.3), (Q5_K, 1536, 1536, 2, False, 6.0, 8.4), (Q5_K, 1536, 1536, 4, False, 7.9, 8.6),
+    (Q6_K, 1536, 1536, 2, False, 5.4, 9.4), (Q6_K, 1536, 1536, 4, False, 7.4, 9.7), (Q8_0, 17920, 1536, 2, True, 29.7, 21.4),
+    (Q8_0, 17920, 1536, 4, True, 45.3, 21.9), (Q3_K, 17920, 1536, 2, True, 19.6, 15.9), (Q3_K, 17920, 1536, 4, True, 27.3, 16.2),
+    (Q5_K, 17920, 1536, 2, True, 23.0, 16.9), (Q5_K, 17920, 1536, 4, True, 44.2, 17.5), (Q6_K, 17920, 1536, 2, True, 20.3, 21.3),
+    (Q6_K, 17920, 1536, 4, True, 27.5, 21.9), (Q8_0, 1536, 8960, 2, False, 18.7, 16.1), (Q8_0, 1536, 8960, 4, False, 25.9, 15.5),
+    (Q3_K, 1536, 8960, 2, False, 16.0, 13.6), (Q3_K, 1536, 8960, 4, False, 19.7, 14.4), (Q5_K, 1536, 8960, 2, False, 18.2, 14.4),
+    (Q5_K, 1536, 8960, 4, False, 30.5, 15.4), (Q6_K, 1536, 8960, 2, False, 16.6, 16.3), (Q6_K, 1536, 8960, 4, False, 20.2, 17.6),
+    (Q8_0, 256, 1536, 2, False, 7.6, 8.1), (Q8_0, 256, 1536, 4, False, 10.6, 8.7), (Q3_K, 256, 1536, 2, False, 5.3, 8.1),
+    (Q3_K, 256, 1536, 4, False, 7.2, 8.3), (Q5_K, 256, 1536, 2, False, 5.8, 8.3), (Q5_K, 256, 1536, 4, False, 7.8, 8.5),
+    (Q6_K, 256, 1536, 2, False, 5.3, 9.1), (Q6_K, 256, 1536, 4, False, 7.2, 9.2), (Q8_0, 1152, 896, 2, False, 7.5, 7.9),
+    (Q8_0, 1152, 896, 4, False, 9.9, 8.2), (Q8_0, 896, 896, 2, False, 7.5, 7.9), (Q8_0, 896, 896, 4, False, 9.9, 8.3),
+    (Q8_0, 9728, 896, 2, True, 10.3, 11.6), (Q8_0, 9728, 896, 3, True, 13.8, 11.7), (Q8_0, 9728, 896, 4, True, 20.5, 11.7),
+    (Q8_0, 896, 4864, 2, False, 11.4, 10.1), (Q8_0, 896, 4864, 4, False, 14.4, 12.1), (Q8_0, 4096, 3584, 2, False, 18.9, 13.8),
+    (Q3_K, 4096, 3584, 2, False, 8.9, 11.7), (Q5_K, 4096, 3584, 2, False, 10.2, 12.4), (Q6_K, 4096, 3584, 2, False, 9.8, 15.3),
+    (Q8_0, 14592, 1280, 2, False, 25.0, 13.2), (Q5_K, 2944, 256, 2, False, 6.1, 6.8), (Q5_K, 2688, 4096, 4, False, 23.6, 14.1),
+    (Q8_0, 2816, 14336, 2, False, 39.8, 28.7), (Q5_K, 20864, 512, 4, False, 45.7, 9.7), (Q6_K, 384, 16384, 4, False, 10.7, 15.5),
+    (Q6_K, 3712, 1280, 2, False, 6.0, 9.4), (Q5_K, 384, 5120, 4, False, 10.1, 11.2), (Q5_K, 5376, 16384, 2, False, 45.9, 28.2),
+    (Q5_K, 1408, 2048, 4, False, 8.1, 9.9), (Q6_K, 384, 5120, 2, False, 9.1, 11.8), (Q6_K, 5504, 4096, 2, False, 15.4, 16.4),
+    (Q6_K, 384, 3072, 2, False, 7.1, 9.5), (Q6_K, 14592, 1280, 2, False, 17.3, 13.8), (Q5_K, 1280, 2048, 2, False, 6.1, 9.7),
+    (Q3_K, 2048, 11264, 2, False, 16.7, 14.7), (Q8_0, 640, 14336, 4, False, 25.3, 16.1), (Q3_K, 5760, 1280, 2, False, 9.4, 8.1),
+    (Q5_K, 2816, 256, 4, False, 13.8, 7.1), (Q8_0, 384, 256, 2, False, 6.2, 6.9), (Q6_K, 1536, 2048, 4, False, 7.5, 10.2),
+    (Q6_K, 6912, 11264, 2, False, 37.1, 28.8), (Q8_0, 20864, 512, 4, False, 19.9, 10.7), (Q5_K, 20864, 512, 2, False, 25.2, 9.4),
+    (Q3_K, 768, 256, 4, False, 8.3, 7.0), (Q3_K, 384, 11264, 2, False, 9.4, 10.9), (Q6_K, 2944, 256, 4, False, 7.0, 7.2),
+    (Q6_K, 16768, 1024, 4, False, 24.1, 14.6), (Q3_K, 3840, 1280, 4, False, 8.3, 8.1), (Q6_K, 2816, 14336, 2, False, 24.8, 24.2),
+    (Q8_0, 768, 256, 2, False, 6.2, 6.8), (Q5_K, 20992, 256, 2, False, 25.8, 7.4), (Q8_0, 1280, 4096, 2, False, 12.1, 12.3),
+    (Q3_K, 1152, 8192, 4, False, 16.2, 12.0), (Q6_K, 2816, 256, 2, False, 5.3, 6.9), (Q3_K, 14592, 1280, 2, False, 17.1, 10.7),
+    (Q6_K, 640, 14336, 2, False, 11.4, 14.8), (Q6_K, 20864, 512, 2, False, 20.7, 10.7), (Q3_K, 4864, 512, 2, False, 8.6, 6.8),
+    (Q8_0, 256, 6144, 4, False, 13.5, 11.6)]
 
 
 @pytest.fixture(scope="module")
