@@ -42,8 +42,8 @@ inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows,
 }
 
 // The same for two to eight rows of a narrow product, against the vector and staged kernels (gemv.hip), which walk the weights once for
-// every four, two or one rows.  Q4_K has tiles of its own and stays (7B shape, eight rows: gate|up 25 against 36 us, ffn_down 23 against
-// 30).  Of the others three rows and five are two passes or more and go (7B shape, eight rows: Q8_0 gate|up 304 -> 62, Q6_K ffn_down 101 ->
+// every four, two or one rows.  Q4_K has tiles of its own and stays (7B shape, eight rows: gate|up 26 against 36 us, ffn_down 23 against
+// 27).  Of the others three rows and five are two passes or more and go (7B shape, eight rows: Q8_0 gate|up 304 -> 62, Q6_K ffn_down 101 ->
 // 34; the worst of 53 shapes at three rows: 1.06 times).  Two and four rows are one pass.  The staged kernel takes eight columns and a
 // slice of K a workgroup: up to two workgroups a compute unit it is one round of latency, which the packing launch alone does not
 // beat (4096 x 3584, 512 of them, two rows: Q3_K 8.9 against 11.7, Q5_K 10.2 against 12.4, Q6_K 9.8 against 15.3), and a second
