@@ -123,7 +123,8 @@ int32_t nh_convert_half(nh_device *device, const float *dev_src, uint64_t elemen
 int32_t nh_pack_q8_0(nh_device *device, const float *dev_src, uint64_t elements, void *dev_dst);
 /* narrow product, rows <= 8 (template_run_matmul_folded{,_fused,_quad},
  * crates/neura-kernel/src/task/matmul.rs:376-803): y[r][n] = sum_k x[r][k]·W[n][k], fp32; W in NH_Q8_0, NH_Q3_K, NH_Q4_K,
- * NH_Q5_K or NH_Q6_K blocks (the dots of crates/neura-kernel/src/dot.rs:471-797) */
+ * NH_Q5_K or NH_Q6_K blocks (the dots of crates/neura-kernel/src/dot.rs:471-797).  An infinity or a NaN in a row of x shows in
+ * that row of y alone, as infinities or NaN */
 int32_t nh_gemv(nh_device *device, int32_t element, const void *dev_W, uint32_t N, uint32_t K, const float *dev_x, uint32_t rows,
                 float *dev_y, const nh_epilogue *epilogue);
 /* wide product (template_run_matmul_codes / _run, crates/neura-kernel/src/task/matmul.rs:943-1221):
@@ -253,7 +254,7 @@ int32_t nh_decode_step_sampled(nh_model *model, const uint32_t *tokens, const ui
  * tokens[row * batch + plane]; no logits, no readback. */
 int32_t nh_prefill(nh_model *model, const uint32_t *tokens, uint32_t rows, const uint32_t *cursors, const uint8_t *mask, uint32_t batch);
 /* Runtime::measure restricted to the products (crates/neura-runtime/src/runtime.rs:807-816,
- * examples/benchmark/product.rs:19-107): launches every narrow product of one decode step
+ * examples/benchmark/product.rs:19-107): launches every product of one decode step
  * (same matrices, shapes and buffers, nothing else) `steps` times back to back on the device's
  * stream between one pair of HIP events.  Returns the device seconds, the number of product
  * launches and the weight payload bytes they walked. */
