@@ -56,10 +56,12 @@ def test_decode_steps_match_oracle_logits_and_tokens(device, shape, element):
 
 
 @pytest.mark.parametrize("planes", [9, 16, 21])
-@pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K), (SMALL_Q4, NH_Q6_K)], ids=["q8_0", "q4_k", "q6_k"])
+@pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K), (SMALL_Q4, NH_Q6_K), (dict(SMALL_Q4, layers=1, vocab=4400), NH_Q5_K)],
+                         ids=["q8_0", "q4_k", "q6_k", "q5_k-more-than-128-tiles"])
 def test_steps_of_more_planes_than_a_narrow_product_takes(device, shape, element, planes):
     """Every product of a step runs as the wide product of few rows, the head over the whole vocabulary too; up to sixteen planes the
-    gate and the up projection share a launch that gates its outputs.  Eager, recorded and replayed steps at cursors of their own."""
+    gate and the up projection share a launch that gates its outputs.  The head's rows are whole: ten to a tile, one, two and three tiles of
+    them (three a wave over more than 128 column tiles).  Eager, recorded and replayed steps at cursors of their own."""
     model, ref, weights = build(device, shape, element, batch=planes, context=40, seed=planes)
     rng = np.random.default_rng(planes)
     first = rng.integers(0, 30, planes)
