@@ -381,6 +381,11 @@ __device__ __forceinline__ void states_as_halves(const u32x4 (&raw)[WORDS], u32x
 // The running maximum, sum and the 32 x 64 accumulators of a column live in its two lanes; nothing is folded afterwards.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float float4_loose __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr uint32_t FILL_SECTIONS_MOST = 32;
+// two rounds of staged keys and values, a tile of 32 a set of waves (rows padded by eight halves to spread the banks), residues beside single states
+__host__ __device__ constexpr size_t fill_lds_bytes(int width, int element, bool split) { return 2u * 2u * (split ? 2u : 1u) * (element == NH_F32 ? 2u : 1u) * 32u * (width + 8u) * 2u; }
 
 // CE: what the states hold (states_as_halves above); single states stage a second plane of key and value residues and cost
 // one more MFMA a product.
@@ -395,20 +400,19 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     constexpr int TK = 32;                       // keys per tile
     constexpr int STEPS = WIDTH / 16;            // MFMA steps over the channels of a score
     constexpr int BLOCKS = WIDTH / 32;           // 32-channel blocks of the output
-    constexpr int KPITCH = WIDTH + 8;            // halves per staged key row (the pad spreads the banks)
-    constexpr int VPITCH = TK + 4;               // halves per staged value channel
+    constexpr int KPITCH = WIDTH + 8;            // halves per staged key or value row (the pad spreads the banks)
     constexpr int PLANES = CE == NH_F32 ? 2 : 1;  // values, and for single states their residues * 2^11
     constexpr int WORDS = CE == NH_F32 ? 2 : 1;   // 16-byte loads that hold eight stored numbers
     constexpr uint32_t STORED = CE == NH_F32 ? 4u : 2u;
-    constexpr size_t KT_BYTES = sizeof(uint16_t) * SETS * PLANES * TK * KPITCH, VT_BYTES = sizeof(uint16_t) * SETS * PLANES * WIDTH * VPITCH;
-    __shared__ __attribute__((aligned(16))) uint8_t tile_lds[KT_BYTES + VT_BYTES];  // the staged key tiles, then the value tiles
-    uint16_t(*const kt_planes)[PLANES][TK][KPITCH] = reinterpret_cast<uint16_t(*)[PLANES][TK][KPITCH]>(tile_lds);
-    uint16_t(*const vt_planes)[PLANES][WIDTH][VPITCH] = reinterpret_cast<uint16_t(*)[PLANES][WIDTH][VPITCH]>(tile_lds + KT_BYTES);
+    // two rounds' key and value tiles: a round is staged while the one before is multiplied, one barrier a round
+    constexpr size_t PLANE = sizeof(uint16_t) * TK * KPITCH, ROUND = 2 * SETS * PLANES * PLANE;
+    static_assert(2 * ROUND == fill_lds_bytes(WIDTH, CE, SPLIT), "what the launch asks for");
+    extern __shared__ __attribute__((aligned(16))) uint8_t tile_lds[];
     const uint32_t set = SPLIT ? threadIdx.x >> 8 : 0u;  // which of the two sets of waves; tid, wave: within the set
-    uint16_t(*const kt)[KPITCH] = kt_planes[set][0];
-    uint16_t(*const vt)[VPITCH] = vt_planes[set][0];
-    uint16_t(*const kt_fine)[KPITCH] = kt_planes[set][PLANES - 1];
-    uint16_t(*const vt_fine)[VPITCH] = vt_planes[set][PLANES - 1];
+    typedef uint16_t (*tile_rows)[KPITCH];
+    auto staged = [&](uint32_t round, int value, int plane) {
+        return reinterpret_cast<tile_rows>(tile_lds + (round & 1u) * ROUND + ((value * SETS + set) * PLANES + plane) * PLANE);
+    };
     const uint32_t tid = threadIdx.x & 255u, lane = tid & 63u, wave = tid >> 6;
     const uint32_t n = lane & 31u, h = lane >> 5;
     const uint32_t G = p.groups;
@@ -429,18 +433,27 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     // the workgroup walks up to the last key its last row sees; a ring is walked whole, every slot asked what it holds
     const uint32_t last_row = min(p.rows, block_row + 4u * rows_per_wave) - 1u;
     const uint32_t span = min(p.keys, p.reach ? origin + p.rows : origin + last_row + 1u);
+    // a section of the walk: whole rounds of tiles, the same number for every section of a block (the last ones may be left without)
+    const uint32_t rounds = (span + SETS * TK - 1u) / (SETS * TK), share = (rounds + p.sections - 1u) / p.sections * (SETS * TK);
+    const uint32_t begin = blockIdx.z * share, stop = min(span, begin + share);
     const uint32_t wave_first = block_row + wave * rows_per_wave;
+    // keys below this are seen by every row of the wave (a column that is not held may weigh what it likes: it leaves nothing)
+    const uint32_t all_see = min(p.keys, origin + wave_first + 1u);
     const uint32_t wave_span = wave_first >= p.rows ? 0u : (p.reach ? span : min(p.keys, origin + min(p.rows, wave_first + rows_per_wave)));
 
     // queries as two half planes: q = value + residue, both halves
     half8_t q_value[STEPS], q_residue[STEPS];
     {
+        // (every load whatever the column: under a condition each waits for the one before, 10 us of a fill of few tiles)
         const float *src = p.q + (uint64_t)(kvh * G + g) * p.q_sh + (uint64_t)b * p.q_sb + (uint64_t)min(row, p.rows - 1u) * p.q_sr;
+        float4_loose raw[STEPS][2];
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) raw[s][0] = *reinterpret_cast<const float4_loose *>(src + 16 * s + 8 * h), raw[s][1] = *reinterpret_cast<const float4_loose *>(src + 16 * s + 8 * h + 4);
 #pragma unroll
         for (int s = 0; s < STEPS; s++) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float value = held ? src[16 * s + 8 * h + i] : 0.0f;
+                const float value = held ? raw[s][i >> 2][i & 3] : 0.0f;
                 const _Float16 high = (_Float16)value;
                 q_value[s][i] = high;
                 q_residue[s][i] = (_Float16)((value - (float)high) * 2048.0f);  // scaled up, clear of the subnormal halves
@@ -471,11 +484,12 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
         }
     };
     // set s walks tiles s, s + SETS, ...; both sets meet every barrier of every round
-    if (set * TK < span) fetch(set * TK);
-    for (uint32_t first = 0; first < span; first += SETS * TK) {
+    if (begin + set * TK < stop) fetch(begin + set * TK);
+    uint32_t round = 0;
+    for (uint32_t first = begin; first < stop; first += SETS * TK, round++) {
         const uint32_t tile = first + set * TK;
-        const bool have = tile < span;
-        __syncthreads();  // the last tile's readers are done
+        const bool have = tile < stop;
+        const tile_rows kt = staged(round, 0, 0), vt = staged(round, 1, 0), kt_fine = staged(round, 0, PLANES - 1), vt_fine = staged(round, 1, PLANES - 1);
 #pragma unroll
         for (int k = 0; k < PIECES; k++) {
             if (!have) break;
@@ -487,21 +501,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
             if constexpr (CE == NH_F32) *reinterpret_cast<u32x4 *>(&kt_fine[key][chunk * 8u]) = k_fine;
             // rows past the written keys may hold anything, and a weight of zero does not silence a NaN
             const uint32_t keep = tile + key < span ? 0xffffffffu : 0u;
-            // groups of four keys change places by the channel block (chunk / 4), or the chunks a store instruction touches share four banks
-            const uint32_t column = (((key >> 2) ^ (chunk >> 2)) << 2) | (key & 3u);
-            {
-                const uint32_t words[4] = {v_words.x & keep, v_words.y & keep, v_words.z & keep, v_words.w & keep};
-#pragma unroll
-                for (int i = 0; i < 8; i++) vt[chunk * 8u + i][column] = (uint16_t)(words[i >> 1] >> (16 * (i & 1)));
-            }
-            if constexpr (CE == NH_F32) {
-                const uint32_t words[4] = {v_fine.x & keep, v_fine.y & keep, v_fine.z & keep, v_fine.w & keep};
-#pragma unroll
-                for (int i = 0; i < 8; i++) vt_fine[chunk * 8u + i][column] = (uint16_t)(words[i >> 1] >> (16 * (i & 1)));
-            }
+            *reinterpret_cast<u32x4 *>(&vt[key][chunk * 8u]) = u32x4{v_words.x & keep, v_words.y & keep, v_words.z & keep, v_words.w & keep};
+            if constexpr (CE == NH_F32) *reinterpret_cast<u32x4 *>(&vt_fine[key][chunk * 8u]) = u32x4{v_fine.x & keep, v_fine.y & keep, v_fine.z & keep, v_fine.w & keep};
         }
-        if (tile + SETS * TK < span) fetch(tile + SETS * TK);  // in flight while this tile is multiplied
-        __syncthreads();
+        if (tile + SETS * TK < stop) fetch(tile + SETS * TK);  // in flight while this tile is multiplied
+        __syncthreads();  // the round is staged; every wave is done with the round before, whose LDS the next one takes
         if (!have || tile >= wave_span) continue;  // keys none of this wave's rows see (every wave still meets the barriers)
 
         // ---- scores
@@ -518,12 +522,20 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
         }
         // ---- weights: register 4j + e of lane (column, h) is key 8j + 4h + e of the tile
         float tile_top = -INFINITY;
+        if (!p.reach && tile + TK <= all_see) {  // every row of the wave sees the whole tile
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t key = tile + 8u * (r >> 2) + 4u * h + (r & 3);
-            const bool seen = held && key < p.keys && (p.reach ? ring.seen(key, limit) : key <= limit);
-            scores[r] = seen ? fmaf(fine[r], 1.0f / 2048.0f, scores[r]) * p.scale : -INFINITY;
-            tile_top = fmaxf(tile_top, scores[r]);
+            for (int r = 0; r < 16; r++) {
+                scores[r] = fmaf(fine[r], 1.0f / 2048.0f, scores[r]) * p.scale;
+                tile_top = fmaxf(tile_top, scores[r]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const uint32_t key = tile + 8u * (r >> 2) + 4u * h + (r & 3);
+                const bool seen = held && key < p.keys && (p.reach ? ring.seen(key, limit) : key <= limit);
+                scores[r] = seen ? fmaf(fine[r], 1.0f / 2048.0f, scores[r]) * p.scale : -INFINITY;
+                tile_top = fmaxf(tile_top, scores[r]);
+            }
         }
         tile_top = fmaxf(tile_top, __shfl_xor(tile_top, 32, 64));
         const float next = fmaxf(top, tile_top);
@@ -546,24 +558,32 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
         mass = fmaf(mass, rescale, tile_mass);
         top = next;
         // ---- values
+        if (__any(rescale != 1.0f)) {  // (most tiles past a row's first few raise no maximum)
+#pragma unroll
+            for (int d = 0; d < BLOCKS; d++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[d][r] *= rescale;
+        }
+        // ds_read_b64_tr_b16 hands lane 4 k + a of a group of sixteen, which points at four halves of key k, channels 4 a .., the
+        // channel of its own number of the four keys
+        typedef short short4_t __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) short4_t *lds_short4;
+        auto transposed = [&](const tile_rows rows, int first_key, int d) -> uint2 {
+            return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)&rows[first_key + 4u * h + ((lane & 15u) >> 2)][32 * d + 16u * ((lane >> 4) & 1u) + 4u * (lane & 3u)]));
+        };
 #pragma unroll
         for (int d = 0; d < BLOCKS; d++) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[d][r] *= rescale;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 // slots 8h + i of step t: keys 16t + 4h + i (i < 4) and 16t + 8 + 4h + (i - 4), as the weights lie
                 half8_t values;
-                // channels 32 d + n lie in chunks 4 d .. 4 d + 3: their key groups sit d places off
-                const uint2 low = *reinterpret_cast<const uint2 *>(&vt[32 * d + n][4 * ((4 * t + h) ^ d)]);
-                const uint2 high = *reinterpret_cast<const uint2 *>(&vt[32 * d + n][4 * ((4 * t + 2 + h) ^ d)]);
+                const uint2 low = transposed(vt, 16 * t, d), high = transposed(vt, 16 * t + 8, d);
                 const u32x4 joined = {low.x, low.y, high.x, high.y};
                 values = __builtin_bit_cast(half8_t, joined);
                 acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(values, w_value[t], acc[d], 0, 0, 0);
                 acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(values, w_residue[t], acc[d], 0, 0, 0);
                 if constexpr (CE == NH_F32) {
-                    const uint2 low_fine = *reinterpret_cast<const uint2 *>(&vt_fine[32 * d + n][4 * ((4 * t + h) ^ d)]);
-                    const uint2 high_fine = *reinterpret_cast<const uint2 *>(&vt_fine[32 * d + n][4 * ((4 * t + 2 + h) ^ d)]);
+                    const uint2 low_fine = transposed(vt_fine, 16 * t, d), high_fine = transposed(vt_fine, 16 * t + 8, d);
                     const half8_t residues = __builtin_bit_cast(half8_t, u32x4{low_fine.x, low_fine.y, high_fine.x, high_fine.y});
                     acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(residues, w_small[t], acc[d], 0, 0, 0);
                 }
@@ -573,7 +593,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     if constexpr (SPLIT) {
         // ---- the two sets meet lane by lane: the second leaves its maximum, its mass and its sums (a 32-channel block a
         // round) where the tiles were staged, the first joins them as two partial softmaxes join
-        static_assert(KT_BYTES + VT_BYTES >= sizeof(float) * 256 * 18, "the staged tiles' LDS holds a round of the meeting");
+        static_assert(2 * ROUND >= sizeof(float) * 256 * 18, "the staged tiles' LDS holds a round of the meeting");
         float *const meet = reinterpret_cast<float *>(tile_lds);
         float mine = 1.0f, theirs = 0.0f;
 #pragma unroll
@@ -602,8 +622,16 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     }
     if (!held) return;
     // register 4j + e of block d is channel 32d + 8j + 4h + e of this lane's column
-    const float normalized = mass > 0.0f ? 1.0f / (mass * 1024.0f) : 0.0f;
+    float normalized = mass > 0.0f ? 1.0f / (mass * 1024.0f) : 0.0f;
     float *dst = p.out + (uint64_t)(kvh * G + g) * p.o_sh + (uint64_t)b * p.o_sb + (uint64_t)row * p.o_sr;
+    if (p.sections > 1u) {
+        // sums, maximum and mass as they stand; the sums of a section no key of which was seen are left out (attention_fill_fold_kernel)
+        const uint64_t place = (((uint64_t)(kvh * p.batch + b) * p.rows + row) * p.sections + blockIdx.z) * G + g;
+        if (h == 0u) reinterpret_cast<float2 *>(p.partial + (uint64_t)p.kv_heads * p.batch * p.rows * p.sections * G * WIDTH)[place] = float2{top, mass};
+        if (top == -INFINITY && mass == 0.0f) return;
+        normalized = 1.0f / 1024.0f;
+        dst = p.partial + place * WIDTH;
+    }
 #pragma unroll
     for (int d = 0; d < BLOCKS; d++)
 #pragma unroll
@@ -613,6 +641,49 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
         }
 }
 
+
+// The sections of a fill's rows, one (row, query head) a wave: lane s < sections turns section s's maximum and mass into its weight,
+// then the lanes of a stripe take four channels each over every second section (fourth at width 64), eight loads in flight.
+template <int WIDTH>
+__global__ __launch_bounds__(256) void attention_fill_fold_kernel(AttentionParams p) {
+    constexpr uint32_t LANES = WIDTH / 4, STRIPES = 64 / LANES;
+    static_assert(FILL_SECTIONS_MOST <= 64, "a lane a section");
+    const uint32_t lane = threadIdx.x & 63u, G = p.groups, S = p.sections;
+    const uint32_t count = p.kv_heads * p.batch * p.rows * G, row_head = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (row_head >= count) return;  // (a whole wave: nothing below meets another)
+    const uint32_t unit = row_head / G, g = row_head - unit * G;
+    const uint64_t place = (uint64_t)unit * S * G + g;  // of section 0; a section further is G further
+    const float2 held = reinterpret_cast<const float2 *>(p.partial + (uint64_t)count * S * WIDTH)[place + (uint64_t)min(lane, S - 1u) * G];
+    const float top = lane < S ? held.x : -INFINITY;
+    const bool empty = lane >= S || (held.x == -INFINITY && held.y == 0.0f);
+    const float largest = wave_max(top);
+    const float weight = top == -INFINITY ? 0.0f : softmax_exp(top - largest);
+    const float total = wave_sum(empty ? 0.0f : held.y * weight);
+    const float normalized = total > 0.0f ? 1.0f / (total) : 0.0f;
+    const uint32_t c = lane % LANES * 4u, stripe = lane / LANES;
+    const float *from = p.partial + place * WIDTH + c;
+    float4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t s0 = 0; s0 < S; s0 += 8u * STRIPES) {
+        float4 v[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) v[j] = *reinterpret_cast<const float4 *>(from + (uint64_t)min(s0 + stripe + STRIPES * j, S - 1u) * G * WIDTH);
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) {
+            const uint32_t s = s0 + stripe + STRIPES * j;
+            const float w = __shfl(weight, (int)min(s, 63u), 64);
+            // (a section left out holds whatever the scratch held)
+            if (__shfl((int)empty, (int)min(s, 63u), 64) || s >= S) continue;
+            sum.x = fmaf(v[j].x, w, sum.x), sum.y = fmaf(v[j].y, w, sum.y), sum.z = fmaf(v[j].z, w, sum.z), sum.w = fmaf(v[j].w, w, sum.w);
+        }
+    }
+#pragma unroll
+    for (uint32_t hop = LANES; hop < 64u; hop <<= 1)
+        sum.x += __shfl_xor(sum.x, (int)hop, 64), sum.y += __shfl_xor(sum.y, (int)hop, 64), sum.z += __shfl_xor(sum.z, (int)hop, 64), sum.w += __shfl_xor(sum.w, (int)hop, 64);
+    if (stripe != 0u) return;
+    const uint32_t row = unit % p.rows, b = unit / p.rows % p.batch, kvh = unit / p.rows / p.batch;
+    *reinterpret_cast<float4 *>(p.out + (uint64_t)(kvh * G + g) * p.o_sh + (uint64_t)b * p.o_sb + (uint64_t)row * p.o_sr + c) =
+        float4{sum.x * normalized, sum.y * normalized, sum.z * normalized, sum.w * normalized};
+}
 
 // ---------------------------------------------------------------- one query row, many planes: the matrix cores ------
 //
@@ -978,6 +1049,39 @@ static void launch_fold(uint32_t sections, dim3 grid, dim3 block, size_t lds, hi
     else hipLaunchKernelGGL(attention_fold_kernel<32>, grid, block, lds, stream, args...);
 }
 
+// How many workgroups share the walk of a block of query rows in a fill.  A block's walk is a chain of rounds (a tile a set of waves:
+// 2.35 us at width 128, 1.85 at 64) behind some 10 us (6.5) of queries, first tile and meeting; one workgroup runs on a compute unit
+// at a time, so blocks times sections come in turns of the chip; sections leave their sums in memory for a fold of 4 us and
+// more (480 rows of 28 heads in two: 10 us).  In hundredths of a microsecond; over 40 shapes of 5 to 480 rows behind 0 to 1500 kept
+// positions the pick takes 1.005 times the best one's time.  28 heads of 128, one workgroup a block -> here: 37 rows behind 700 kept
+// positions 41 -> 18 us, 100 behind 1500 72 -> 29, 480 behind 700 59 -> 49; 480 rows alone stay (31 us).
+static uint32_t fill_sections(uint32_t blocks, uint32_t rounds, uint64_t numbers, uint32_t width, uint32_t compute_units) {
+    // NEURA_HIP_FILL_SECTIONS=<sections>: that many (read at every launch: the tests switch it)
+    if (const char *held = getenv("NEURA_HIP_FILL_SECTIONS"); held && atoi(held) > 0) return min((uint32_t)atoi(held), FILL_SECTIONS_MOST);
+    uint32_t best = 1;
+    uint64_t least = UINT64_MAX;
+    for (uint32_t s = 1; s <= FILL_SECTIONS_MOST && s <= rounds; s++) {
+        const uint64_t turns = ((uint64_t)blocks * s + compute_units - 1u) / compute_units;
+        const uint64_t walk = (uint64_t)((rounds + s - 1u) / s) * (width > 64u ? 235u : 185u) + (width > 64u ? 1000u : 650u);
+        const uint64_t cost = turns * walk + (s > 1u ? 400u + numbers / 3500u + numbers * s / 7500u : 0u);
+        if (cost < least) least = cost, best = s;
+    }
+    return best;
+}
+
+template <int WIDTH, int CE, bool SPLIT>
+static int32_t launch_fill(nh_device *d, const AttentionParams &p, dim3 grid, uint32_t rows_per_wave) {
+    constexpr size_t lds = fill_lds_bytes(WIDTH, CE, SPLIT);
+    static bool sized = false;
+    if (!sized) {
+        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_tile_kernel<WIDTH, CE, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        sized = true;
+    }
+    hipLaunchKernelGGL((attention_tile_kernel<WIDTH, CE, SPLIT>), grid, dim3(SPLIT ? 512 : 256), lds, d->stream, p, rows_per_wave);
+    NH_HIP(hipGetLastError());
+    return NH_OK;
+}
+
 int32_t launch_attention(nh_device *d, const AttentionArgs &a) {
     AttentionParams p{};
     p.q = a.q, p.out = a.out;
@@ -1031,18 +1135,32 @@ int32_t launch_attention(nh_device *d, const AttentionArgs &a) {
         // NEURA_HIP_FILL_SPLIT=0 keeps one set
         static const bool split_wanted = [] { const char *v = getenv("NEURA_HIP_FILL_SPLIT"); return !(v && v[0] == '0'); }();
         const bool split = split_wanted && a.cache_element != NH_F32 && a.keys >= 128u;
-#define FILL_TILE(WIDTH)                                                                                                                           \
-    do {                                                                                                                                           \
-        if (a.cache_element == NH_F16 && split) hipLaunchKernelGGL((attention_tile_kernel<WIDTH, NH_F16, true>), grid, dim3(512), 0, d->stream, p, rows_per_wave);   \
-        else if (a.cache_element == NH_BF16 && split) hipLaunchKernelGGL((attention_tile_kernel<WIDTH, NH_BF16, true>), grid, dim3(512), 0, d->stream, p, rows_per_wave); \
-        else if (a.cache_element == NH_F16) hipLaunchKernelGGL((attention_tile_kernel<WIDTH, NH_F16>), grid, dim3(256), 0, d->stream, p, rows_per_wave);   \
-        else if (a.cache_element == NH_BF16) hipLaunchKernelGGL((attention_tile_kernel<WIDTH, NH_BF16>), grid, dim3(256), 0, d->stream, p, rows_per_wave); \
-        else hipLaunchKernelGGL((attention_tile_kernel<WIDTH, NH_F32>), grid, dim3(256), 0, d->stream, p, rows_per_wave);                             \
+        const uint32_t longest = a.longest ? min(a.longest, a.keys) : a.keys;
+        p.sections = fill_sections(grid.x * grid.y, (longest + (split ? 64u : 32u) - 1u) / (split ? 64u : 32u), (uint64_t)units * p.groups * a.width, a.width, (uint32_t)d->compute_units);
+        if (p.sections > 1u) {
+            p.partial = static_cast<float *>(scratch(d, (size_t)p.sections * units * p.groups * (a.width + 2) * sizeof(float)));
+            if (!p.partial) p.sections = 1;  // (a device that holds no more scratch walks every block whole)
+        }
+        grid.z = p.sections;
+        int32_t status;
+#define FILL_TILE(WIDTH)                                                                                                          \
+    do {                                                                                                                          \
+        if (a.cache_element == NH_F16 && split) status = launch_fill<WIDTH, NH_F16, true>(d, p, grid, rows_per_wave);             \
+        else if (a.cache_element == NH_BF16 && split) status = launch_fill<WIDTH, NH_BF16, true>(d, p, grid, rows_per_wave);      \
+        else if (a.cache_element == NH_F16) status = launch_fill<WIDTH, NH_F16, false>(d, p, grid, rows_per_wave);                \
+        else if (a.cache_element == NH_BF16) status = launch_fill<WIDTH, NH_BF16, false>(d, p, grid, rows_per_wave);              \
+        else status = launch_fill<WIDTH, NH_F32, false>(d, p, grid, rows_per_wave);                                               \
     } while (0)
         if (a.width == 64) FILL_TILE(64);
         else FILL_TILE(128);
 #undef FILL_TILE
-        NH_HIP(hipGetLastError());
+        if (status != NH_OK) return status;
+        if (p.sections > 1u) {
+            const dim3 fold((units * p.groups + 3u) / 4u);
+            if (a.width == 64) hipLaunchKernelGGL(attention_fill_fold_kernel<64>, fold, dim3(256), 0, d->stream, p);
+            else hipLaunchKernelGGL(attention_fill_fold_kernel<128>, fold, dim3(256), 0, d->stream, p);
+            NH_HIP(hipGetLastError());
+        }
         return NH_OK;
     }
     // one query row a plane: the group's query heads are the columns of the matrix cores

@@ -295,6 +295,7 @@ struct AttentionArgs {
     const uint16_t *cache_k, *cache_v;
     uint32_t heads, kv_heads, batch, rows, width, capacity, keys;
     const uint32_t *cursor;
+    uint32_t longest = 0;  // where the host knows it: the positions the longest plane holds once the rows are in (0: up to `keys`)
     float scale;
     uint32_t reach = 0;  // 0, or the span of a ring cache of `keys` slots (Cache::windowed): the last `reach` positions are weighed
     int32_t cache_element = NH_F16;  // what the caches hold: NH_F16 (the matrix-core kernels), NH_BF16 or NH_F32 (the kernel for any element)

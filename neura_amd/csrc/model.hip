@@ -125,7 +125,7 @@ GemvArgs narrow(const nh_model *m, int32_t element, const uint8_t *W, uint32_t N
 }
 
 // all layers over T = rows * batch token rows whose inputs are already staged on the device
-int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_only = false) {
+int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_only = false, uint32_t longest = 0) {
     nh_device *d = m->d;
     const nh_model_config &c = m->c;
     const uint32_t B = c.batch, T = rows * B, H = c.hidden, hd = c.head_dim;
@@ -253,7 +253,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
         at.cache_element = c.cache_element;
         at.heads = c.heads, at.kv_heads = c.kv_heads, at.batch = B, at.rows = rows, at.width = hd;
         at.capacity = m->capacity, at.keys = m->window, at.cursor = dev_cursor(m), at.scale = scale;
-        at.reach = m->ring ? m->window : 0u;
+        at.reach = m->ring ? m->window : 0u, at.longest = longest;
         // one row through a product that merges the attention's sections as it stages its row: the attention leaves them unmerged
         SectionSums sums{};
         GemvArgs o{};
@@ -666,15 +666,17 @@ int32_t nh_prefill(nh_model *m, const uint32_t *tokens, uint32_t rows, const uin
     NH_REQUIRE(rows >= 1 && rows * batch <= m->max_tokens, "a fill of %u rows feeds a model built for chunks of %u rows", rows,
                m->max_tokens / m->c.batch);
     bool any_inactive = false;
+    uint32_t longest = 0;  // (positions of the longest active plane: how far the fill's attention walks)
     for (uint32_t b = 0; b < batch; b++) {
         bool active = !mask || mask[b];
         any_inactive |= !active;
+        if (active && cursors[b] + rows > longest) longest = cursors[b] + rows;
         NH_REQUIRE(!active || (uint64_t)cursors[b] + rows <= m->c.context, "plane %u at cursor %u fills %u rows past a context of %u", b,
                    cursors[b], rows, m->c.context);
     }
     int32_t status;
     if ((status = stage_inputs(m, tokens, rows * batch, cursors, mask, batch)) != NH_OK) return status;
-    if ((status = forward(m, rows, any_inactive)) != NH_OK) return status;
+    if ((status = forward(m, rows, any_inactive, false, longest)) != NH_OK) return status;
     return check_refusal(m->d, "a fill");
 }
 

@@ -1016,6 +1016,36 @@ def test_ring_attention_matches_the_oracle(device, heads, kv_heads, batch, width
         origins = origins + rows
 
 
+@pytest.mark.parametrize("sections", [2, 5, 32])
+@pytest.mark.parametrize("element,heads,kv_heads,batch,rows,keys,width,origins,reach", [
+    (1, 28, 4, 2, 5, 300, 128, [0, 295], 0),     # a plane of one round (sections left without keys) beside one of five
+    (1, 14, 2, 1, 37, 260, 64, [223], 0),
+    (30, 12, 2, 1, 20, 200, 128, [150], 0),
+    (0, 12, 2, 2, 17, 200, 64, [100, 7], 0),     # single states: one set of waves, rounds of 32 keys
+    (1, 4, 4, 1, 33, 128, 128, [500], 128),      # a ring that has wrapped
+])
+def test_sections_of_a_fill_walk_meet(device, monkeypatch, sections, element, heads, kv_heads, batch, rows, keys, width, origins, reach):
+    """The walk of a block of query rows shared among workgroups (NEURA_HIP_FILL_SECTIONS), more of them than it has rounds among
+    them: the oracle's rows within the bar of the unshared walk, and rows of NaN scores and infinite values come out as they do unshared."""
+    rng = np.random.default_rng(sections)
+    capacity = keys + rows
+    q = rng.standard_normal((heads, batch, rows, width)).astype(np.float32)
+    K = oracle.cache_cast(rng.standard_normal((kv_heads, batch, capacity, width)).astype(np.float32), element)
+    V = oracle.cache_cast(rng.standard_normal((kv_heads, batch, capacity, width)).astype(np.float32), element)
+    ck, cv = device.upload(K), device.upload(V)
+    scale = 1.0 / np.sqrt(width)
+    monkeypatch.setenv("NEURA_HIP_FILL_SECTIONS", str(sections))
+    got = device.attention(q, ck, cv, kv_heads, capacity, keys, origins, scale, reach=reach, element=element)
+    want = oracle.attention(q, K, V, kv_heads, capacity, keys, origins, scale, reach=reach, element=element)
+    assert np.abs(got - want).max() <= 1e-5
+    q[0, 0, 1, 3], q[1, 0, 2, 5] = np.nan, np.inf
+    got = device.attention(q, ck, cv, kv_heads, capacity, keys, origins, scale, reach=reach, element=element)
+    monkeypatch.setenv("NEURA_HIP_FILL_SECTIONS", "1")
+    want = device.attention(q, ck, cv, kv_heads, capacity, keys, origins, scale, reach=reach, element=element)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.abs(got - want)[~np.isnan(want)].max() <= 1e-5
+
+
 def test_attention_refuses_a_cursor_past_its_keys(device):
     q = np.zeros((2, 1, 1, 64), dtype=np.float32)
     K = np.zeros((2, 1, 8, 64), dtype=np.uint16)
