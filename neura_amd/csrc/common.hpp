@@ -248,6 +248,8 @@ struct GemmArgs {
     // narrow product stacks q|k|v.  end[s] = first output column past matrix s (end[2] == N); unused entries: W_more nullptr.
     const void *W_more[2] = {nullptr, nullptr};
     uint32_t end[2] = {0, 0};
+    // where not null, the columns from end[0] on go there, with the same ldy (the second matrix's first to Y_more[0]); no residual
+    float *Y_more = nullptr;
     // the activations were packed by the launch before this one (same X, M, K, nothing else launched on the device's
     // scratch in between): skip the packing pass
     bool packed = false;

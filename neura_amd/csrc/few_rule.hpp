@@ -1,9 +1,10 @@
-// Which wide products are the product of few rows' (gemm_few.hip) and which the 128 x 128 tiles' (gemm.hip), and which narrow products
-// go there: plain C++, so that the rules can be held to the measured points without a device.
+// Which wide products are the product of few rows' (gemm_few.hip), which the product of shared rows' (gemm_wide.hip) and which the
+// 128 x 128 tiles' (gemm.hip), and which narrow products go to the first: plain C++, so that the rules can be held to the measured points without a device.
 #pragma once
 #include "../../include/neura_hip.h"
 
 #include <cstdint>
+#include <initializer_list>
 
 namespace nh {
 
@@ -39,6 +40,81 @@ inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows,
     const uint64_t groups = (uint64_t)((N + 127u) / 128u) * ((rows + 127u) / 128u), rounds = (groups + compute_units - 1u) / compute_units;
     const uint64_t tiles_cost = 100u * rounds * compute_units + (rounds - 1u) * compute_units * 35000u / K;
     return groups * (few_row_tiles(N, rows, compute_units) == 3u ? share.threes : share.twos) <= tiles_cost;
+}
+
+// How the product of few rows splits the K of a tile of columns: `deep` waves a workgroup, `slices` workgroups; rows in tiles of `mt` a
+// pass, `nt` matrices beside each other (gated).  The split that walks the fewest units: rounds of workgroups times the units of a wave
+// (and what a workgroup takes before its first and after its last, about two units' time).  A matrix of few tiles and deep rows
+// leaves most of the chip idle that way, so K may be shared among workgroups too: their meeting costs a unit's time and the passage of
+// their sums, 2.5 MB in another (eight rows of fp32, with the packing: ffn_down of the 7B shape Q8_0 55 -> 37 us, Q6_K
+// 45 -> 34, Q5_K 37 -> 29, of the 1.5B shape Q8_0 28 -> 18; gate|up of the 7B shape, 592 tiles, is better left alone: Q4_K 34, not 38).
+struct FewSplit {
+    uint32_t deep, slices, cost;  // cost in 64ths of a unit
+};
+constexpr uint32_t FEW_SLICES_MOST = 8, FEW_MEETS_MOST = 1024;
+constexpr uint64_t FEW_SUMS_MOST = 16u << 20;  // bytes
+inline FewSplit few_split(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t mt, uint32_t nt, uint32_t compute_units) {
+    const uint32_t steps = element == NH_Q8_0 ? 2u : 4u, units = (K / 64u + steps - 1u) / steps, tiles = (N + 31u) / 32u, row_tiles = (rows + 31u) / 32u;
+    const uint64_t places = (uint64_t)tiles * ((row_tiles + mt - 1u) / mt);
+    FewSplit best = {1u, 1u, ~0u};
+    for (uint32_t deep = 1; deep <= 8u; deep++)
+        for (uint32_t slices : {1u, 2u, 3u, 4u, 6u, FEW_SLICES_MOST}) {
+            const uint32_t resident = compute_units * (8u / deep);
+            if (slices > 1u && (places > FEW_MEETS_MOST || deep * slices > units || slices * places * mt * nt * 4096u > FEW_SUMS_MOST)) continue;
+            const uint32_t meeting = slices > 1u ? 64u + (uint32_t)((uint64_t)slices * N * nt * rows * 4u * 64u / 2500000u) : 0u;
+            const uint32_t cost = (uint32_t)((places * slices + resident - 1u) / resident) * ((units + deep * slices - 1u) / (deep * slices) + 2u) * 64u + meeting + deep;
+            if (cost < best.cost) best = FewSplit{deep, slices, cost};
+        }
+    return best;
+}
+
+// Where the product of shared rows (gemm_wide.hip) takes over, and in which shape: waves side by side and row tiles a wave (none: the form
+// that few_rows_win picks).  Times in microseconds of all three, each a line fitted to 649 products of the decoder shapes at 20 to
+// 1024 packed rows (mean error 4 % here, 4 % of the tiles, 7 % of the product of few rows): turns of the chip, a base and the units
+// (256 k, Q8_0 128) of each; two workgroups of four waves share a compute unit, and one alone walks faster.  It wants to win by
+// 8 %, so that no line's error makes a product slower: where it is picked it takes 0.87 of the other form's time on average, at most 1.05
+// (7B shape, packed rows, other / here: gate|up Q4_K 128 101 / 74, 200 145 / 106, 1024 392 / 331; Q3_K 1024 455 / 310; Q8_0 200
+// 203 / 143; ffn_down Q4_K 300 119 / 103; 0.5B gate|up Q8_0 800 62 / 47).  Up to two row tiles the walk is latency, not work.
+enum SharedShape { SHARED_NONE = 0, SHARED_42 = 42, SHARED_43 = 43, SHARED_83 = 83, SHARED_84 = 84 };
+inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
+    if (rows <= 64u || !N || !K || !compute_units) return SHARED_NONE;
+    struct Times {
+        double tiles, twos, threes;             // of a 128 x 128 tile's 256 k; of a unit of the product of few rows, two or three row tiles a pass
+        double pair2, one2, pair3, one3, e3, e4;  // of a unit here: 4 x 2 with company and alone, 4 x 3, 8 x 3, 8 x 4
+    };
+    const Times t = element == NH_Q8_0   ? Times{2.73, 2.26, 2.63, 1.82, 1.41, 2.21, 1.55, 0.0, 2.74}
+                    : element == NH_Q6_K ? Times{4.32, 3.41, 4.68, 4.04, 2.41, 4.90, 2.66, 4.26, 0.0}
+                    : element == NH_Q5_K ? Times{2.34, 2.86, 3.74, 2.79, 1.71, 3.36, 1.89, 2.84, 3.28}
+                    : element == NH_Q3_K ? Times{2.72, 2.66, 3.38, 2.47, 1.65, 2.96, 1.87, 2.64, 2.90}
+                                         : Times{1.69, 2.68, 3.56, 2.44, 1.49, 3.11, 1.72, 2.49, 3.04};
+    const uint64_t cu = compute_units, row_tiles = (rows + 31u) / 32u;
+    const uint32_t per = element == NH_Q8_0 ? 128u : 256u, units = (K + per - 1u) / per;
+    const double millions = (double)rows * K * 1e-6;  // (packed, and read again)
+    double other;
+    if (few_rows_win(element, N, K, rows, compute_units)) {
+        const uint32_t mt = few_row_tiles(N, rows, compute_units);
+        const double walk = few_split(element, N, K, rows, mt, 1u, compute_units).cost / 64.0;
+        other = mt == 3u ? 2.2 + t.threes * walk + 5.0 * millions : 3.8 + t.twos * walk + 3.2 * millions;
+    } else {
+        const double rounds = (double)(((uint64_t)((N + 127u) / 128u) * ((rows + 127u) / 128u) + cu - 1u) / cu);
+        other = 3.0 + rounds * (9.5 + t.tiles * K / 256.0) + 3.1 * millions;
+    }
+    SharedShape best = SHARED_NONE;
+    double least = other / 1.08;
+    const auto consider = [&](SharedShape shape, uint32_t waves, uint32_t mt, double pair, double one, double base, double turn, double pack) {
+        if (!(pair > 0.0)) return;
+        const uint64_t workgroups = (uint64_t)((N + 32u * waves - 1u) / (32u * waves)) * ((row_tiles + mt - 1u) / mt), slots = waves == 4u ? 2u * cu : cu;
+        const uint64_t full = workgroups / slots, left = workgroups % slots;
+        const bool lone = waves == 4u && left && left <= cu;
+        const uint64_t turns = full + (left ? 1u : 0u);
+        const double time = base + (double)turns * (turn + units * pair) - (lone ? units * (pair - one) : 0.0) + pack * millions;
+        if (time < least) least = time, best = shape;
+    };
+    consider(SHARED_42, 4u, 2u, t.pair2, t.one2, 5.0, 5.5, 1.7);
+    consider(SHARED_43, 4u, 3u, t.pair3, t.one3, 2.0, 12.0, 1.5);
+    consider(SHARED_83, 8u, 3u, t.e3, t.e3, 1.0, 14.5, 1.4);
+    consider(SHARED_84, 8u, 4u, t.e4, t.e4, 0.0, 18.0, 1.2);
+    return best;
 }
 
 // The same for two to eight rows of a narrow product, against the vector and staged kernels (gemv.hip), which walk the weights once for

@@ -125,7 +125,7 @@ struct GemmQ4Params {
                          // activation row m and row 2m+1 its residue * 2^11
     const _Float16 *S;   // [rows][K / 256][16]: the eight sub-block sums / 64 of a super-block as halves, then their residues * 2^11
     uint32_t rows;       // rows of A
-    float *Y;
+    float *Y, *Y1;       // Y1: where not null, columns from end0 on go there (the second matrix's first to Y1[0])
     const float *residual;
     uint32_t ldy, M;
     int32_t split;
@@ -133,8 +133,11 @@ struct GemmQ4Params {
 };
 
 __device__ __forceinline__ void fetch_parameters(const GemmQ4Params &p) {
-    NH_FETCH(p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, p.split, p.unscale);
+    NH_FETCH(p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.Y1, p.residual, p.ldy, p.M, p.split, p.unscale);
 }
+
+// where column n of a tile from n0 on lies: [n] (a tile lies in one matrix)
+__device__ __forceinline__ float *outputs_of(const GemmQ4Params &p, uint32_t n0) { return p.Y1 && n0 >= p.end0 ? p.Y1 - p.end0 : p.Y; }
 
 // A number (times its row's scale) as PIECES halves whose weights fall by 2^11: two hold 22 of an fp32 number's bits; three hold all 24
 // of every number down to 2^-36 of the row's largest.  Returns what is left over.
@@ -176,7 +179,8 @@ __device__ __forceinline__ void pack_piece(const _Float16 (&pieces)[PIECES][4], 
 #pragma unroll
         for (int j = 0; j < PIECES; j++) {
             // (a sum of 32 is longer than 22 bits, and the minimums' part largely cancels: what a row's sum drops goes into the next's)
-            const float v = j ? fmaf(sums[j], 0.015625f, left) : sums[j] * 0.015625f;
+            constexpr float down = FEW ? 0.0009765625f : 0.015625f;
+            const float v = j ? fmaf(sums[j], down, left) : sums[j] * down;
             const _Float16 h = (_Float16)v;
             const float rest = (v - (float)h) * 2048.0f;
             const _Float16 residue = (_Float16)rest;
@@ -266,10 +270,16 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         }
         return v;
     };
-    if (!HALF_IN) {
+    if (!HALF_IN || FEW) {
         uint32_t top = 0;
         for (uint32_t k = tid * 4u; k < K; k += 1024u) {
-            const float4 v = fetch(k);
+            float4 v;
+            if constexpr (HALF_IN) {
+                const half4_t held = *reinterpret_cast<const half4_t *>(static_cast<const _Float16 *>(X) + (size_t)m * K + k);
+                v = float4{(float)held[0], (float)held[1], (float)held[2], (float)held[3]};
+            } else {
+                v = fetch(k);
+            }
             top = max(max(top, magnitude<WHOLE>(v.x)), magnitude<WHOLE>(v.y));
             top = max(max(top, magnitude<WHOLE>(v.z)), magnitude<WHOLE>(v.w));
         }
@@ -283,6 +293,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         const uint32_t raw = top >> 23, exponent = min(max(raw, 27u), 254u);
         scale = __builtin_bit_cast(float, (267u - exponent) << 23);
         back = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
+        if (HALF_IN && raw == 255u) scale = back = 1.0f;  // (infinities stay)
         if (!WHOLE && tid == 0) unscale[m] = back;
     }
     if constexpr (WHOLE) {
@@ -294,7 +305,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         if (HALF_IN) {
             const half4_t v = *reinterpret_cast<const half4_t *>(static_cast<const _Float16 *>(X) + (size_t)m * K + k);
 #pragma unroll
-            for (int e = 0; e < 4; e++) pieces[0][e] = v[e];
+            for (int e = 0; e < 4; e++) pieces[0][e] = FEW ? (_Float16)((float)v[e] * scale) : v[e];  // (exact: the scale only frees the sums of subnormal halves)
         } else {
             const float4 v = fetch(k);
             const float held[4] = {v.x, v.y, v.z, v.w};
@@ -416,9 +427,8 @@ constexpr size_t PACK_STAGED_LDS_MOST = 152 * 1024;  // the widest row the stage
 constexpr size_t GEMM_Q4K_LDS = sizeof(_Float16) * (2 * GT * GS + 2 * GT * GS + 2 * GT * 8) + sizeof(uint32_t) * 2 * GT;
 
 // What the multiplier waves of a super-block wide product do (waves 0..3 of the workgroup; the stagers fill As, Bs, mns and dds).
-// FLOORS: the weights have minimums (Q4_K, Q5_K), taken off with one more MFMA per four steps over (minimum, activation sum)
-// pairs; SCALE is what the stagers divided the weights' operand by.  Four steps share one (d, dmin) in dds[(step / 4) & 1].
-template <bool FLOORS>
+// The minimums (Q4_K, Q5_K) are taken off with one more MFMA per four steps over (minimum, activation sum) pairs;
+// unscale_weights undoes the power of two the weights' operand was staged with.  Four steps share one (d, dmin) in dds[(step / 4) & 1].
 __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*As)[GT][GS], _Float16 (*Bs)[GT][GS], _Float16 (*mns)[GT][8], uint32_t (*dds)[GT],
                                               const uint32_t wave, const uint32_t lane, const uint32_t n0, const uint32_t m0, const uint32_t steps, const float unscale_weights) {
     typedef const __attribute__((address_space(1))) u32x4 *global_uint4;
@@ -429,7 +439,6 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
     const _Float16 *sums[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) sums[i] = p.S + (size_t)min(m0 + 64u * wm + 32u * i + l32, p.rows - 1u) * nsb * 16u + 8u * part;
-    (void)sums;
 
     f32x16 acc[2][2], tmp[2][2], zero;
 #pragma unroll
@@ -441,11 +450,9 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
 
     for (uint32_t first = 0; first < steps; first += 4) {
         const uint32_t sbuf = (first >> 2) & 1u;
-        u32x4 sraw[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
-        if (FLOORS) {
+        u32x4 sraw[2];
 #pragma unroll
-            for (int i = 0; i < 2; i++) sraw[i] = *(global_uint4)(uintptr_t)(sums[i] + (size_t)(first >> 2) * 16u);  // wanted at the end of the super-block
-        }
+        for (int i = 0; i < 2; i++) sraw[i] = *(global_uint4)(uintptr_t)(sums[i] + (size_t)(first >> 2) * 16u);  // wanted at the end of the super-block
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const uint32_t buf = g & 1u;
@@ -479,10 +486,8 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
             const half2_t dd = __builtin_bit_cast(half2_t, dds[sbuf][64u * wn + 32u * j + l32]);
             dscale[j] = (float)dd.x * unscale_weights;
             mscale[j] = (float)dd.y * -64.0f;  // the sums were packed / 64
-            if (FLOORS) {
-                b2[j] = *reinterpret_cast<const half8_t *>(mns[sbuf][64u * wn + 32u * j + l32]);
-                if (part) b2[j] = b2[j] * (_Float16)0.00048828125f;  // k 8..15: the minimums * 2^-11 against the residues * 2^11
-            }
+            b2[j] = *reinterpret_cast<const half8_t *>(mns[sbuf][64u * wn + 32u * j + l32]);
+            if (part) b2[j] = b2[j] * (_Float16)0.00048828125f;  // k 8..15: the minimums * 2^-11 against the residues * 2^11
         }
 #pragma unroll
         for (int i = 0; i < 2; i++) {
@@ -491,15 +496,14 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
             for (int j = 0; j < 2; j++) {
 #pragma unroll
                 for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(dscale[j], tmp[i][j][e], acc[i][j][e]);
-                if (FLOORS) {
-                    const f32x16 mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b2[j], zero, 0, 0, 0);
+                const f32x16 mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b2[j], zero, 0, 0, 0);
 #pragma unroll
-                    for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(mscale[j], mins[e], acc[i][j][e]);
-                }
+                for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(mscale[j], mins[e], acc[i][j][e]);
             }
         }
     }
     // ---- out: lane (l32, part) holds column n = l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
+    float *const Y = outputs_of(p, n0);
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -516,7 +520,7 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
                         if (m >= p.M) continue;
                         float value = fmaf(acc[i][j][4 * q + 2 * e + 1], 0.00048828125f, acc[i][j][4 * q + 2 * e]) * p.unscale[m];
                         const size_t at = (size_t)m * p.ldy + n;
-                        p.Y[at] = p.residual ? p.residual[at] + value : value;
+                        Y[at] = p.residual ? p.residual[at] + value : value;
                     }
                 } else {
 #pragma unroll
@@ -524,7 +528,7 @@ __device__ __forceinline__ void gemm_multiply(const GemmQ4Params &p, _Float16 (*
                         const uint32_t m = row + e;
                         if (m >= p.M) continue;
                         const size_t at = (size_t)m * p.ldy + n;
-                        p.Y[at] = p.residual ? p.residual[at] + acc[i][j][4 * q + e] : acc[i][j][4 * q + e];
+                        Y[at] = p.residual ? p.residual[at] + acc[i][j][4 * q + e] : acc[i][j][4 * q + e];
                     }
                 }
             }
@@ -646,7 +650,7 @@ __device__ __forceinline__ void gemm_q45k_mfma(const GemmQ4Params &p) {
         return;
     }
 
-    gemm_multiply<true>(p, As, Bs, mns, dds, wave, lane, n0, m0, steps, 16384.0f);  // the weights were staged * 2^-14
+    gemm_multiply(p, As, Bs, mns, dds, wave, lane, n0, m0, steps, 16384.0f);  // the weights were staged * 2^-14
 }
 
 __global__ __launch_bounds__(512) void gemm_q4k_mfma_kernel(GemmQ4Params p) {
@@ -810,6 +814,7 @@ __global__ __launch_bounds__(768) void gemm_q4k_regb_mfma_kernel(GemmQ4Params p)
     // ---- out: lane (l32, part) holds column n = l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
     const uint32_t n = n0 + 32u * wn + l32;
     if (n >= p.N) return;
+    float *const Y = outputs_of(p, n0);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -822,7 +827,7 @@ __global__ __launch_bounds__(768) void gemm_q4k_regb_mfma_kernel(GemmQ4Params p)
                     if (m >= p.M) continue;
                     float value = fmaf(acc[i][4 * q + 2 * e + 1], 0.00048828125f, acc[i][4 * q + 2 * e]) * p.unscale[m];
                     const size_t at = (size_t)m * p.ldy + n;
-                    p.Y[at] = p.residual ? p.residual[at] + value : value;
+                    Y[at] = p.residual ? p.residual[at] + value : value;
                 }
             } else {
 #pragma unroll
@@ -830,7 +835,7 @@ __global__ __launch_bounds__(768) void gemm_q4k_regb_mfma_kernel(GemmQ4Params p)
                     const uint32_t m = row + e;
                     if (m >= p.M) continue;
                     const size_t at = (size_t)m * p.ldy + n;
-                    p.Y[at] = p.residual ? p.residual[at] + acc[i][4 * q + e] : acc[i][4 * q + e];
+                    Y[at] = p.residual ? p.residual[at] + acc[i][4 * q + e] : acc[i][4 * q + e];
                 }
             }
         }
@@ -982,6 +987,7 @@ __global__ __launch_bounds__(512) void gemm_q8_0_mfma_kernel(GemmQ4Params p) {
     }
     weigh(1, late);
     // ---- out: lane (l32, part) holds column n = l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
+    float *const Y = outputs_of(p, n0);
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -998,7 +1004,7 @@ __global__ __launch_bounds__(512) void gemm_q8_0_mfma_kernel(GemmQ4Params p) {
                         if (m >= p.M) continue;
                         float value = fmaf(acc[i][j][4 * q + 2 * e + 1], 0.00048828125f, acc[i][j][4 * q + 2 * e]) * p.unscale[m];
                         const size_t at = (size_t)m * p.ldy + n;
-                        p.Y[at] = p.residual ? p.residual[at] + value : value;
+                        Y[at] = p.residual ? p.residual[at] + value : value;
                     }
                 } else {
 #pragma unroll
@@ -1006,262 +1012,11 @@ __global__ __launch_bounds__(512) void gemm_q8_0_mfma_kernel(GemmQ4Params p) {
                         const uint32_t m = row + e;
                         if (m >= p.M) continue;
                         const size_t at = (size_t)m * p.ldy + n;
-                        p.Y[at] = p.residual ? p.residual[at] + acc[i][j][4 * q + e] : acc[i][j][4 * q + e];
+                        Y[at] = p.residual ? p.residual[at] + acc[i][j][4 * q + e] : acc[i][j][4 * q + e];
                     }
                 }
             }
         }
-}
-
-// ------------------------------------------------------------------- Q6_K on MFMA --------
-//
-// A Q6_K weight is d * sc * (q - 32) with q of six bits and sc a signed byte a 16 weights (crates/neura-precision/src/ggml.rs,
-// the Q6_K reader): sc * (q - 32) reaches +-4064, past the integers a half holds exactly.  The byte splits as
-// sc = 16 * (sc >> 4) + (sc & 15), and (q - 32) * (sc & 15) (below 512) and 16 * (q - 32) * (sc >> 4) (a nine-bit integer times
-// 16) are both exact halves: the weights enter as two operand planes and the matrix cores add the two products in fp32, so
-// tmp holds exactly sum a * sc * (q - 32) however the scales fall.  A step is 32 k: its 64 operand columns are plane one
-// then plane two of those 32 weights, against the step's 32 activations written twice; four steps (half a super-block)
-// are weighed by d together.  The same tiles, packed activation rows, division of the waves and multipliers as the Q4_K
-// kernel; there are no minimums.  Blocks are 210 bytes and start on any half word: a stager reads each 16-byte run it
-// needs as the four aligned words below it and the half word above, and shifts the five into place.
-struct Q6Raw {
-    u32x4 ql[4], qh[2], sc;          // this thread's runs of the low nibbles, of the high bit pairs, and the 16 scales
-    uint32_t qle[4], qhe[2], sce, d;  // the half word above each run; d
-};
-
-__global__ __launch_bounds__(512) void gemm_q6k_mfma_kernel(GemmQ4Params p) {
-    fetch_parameters(p);
-    extern __shared__ __attribute__((aligned(16))) uint8_t gemm_lds[];
-    _Float16(*As)[GT][GS] = reinterpret_cast<_Float16(*)[GT][GS]>(gemm_lds);
-    _Float16(*Bs)[GT][GS] = reinterpret_cast<_Float16(*)[GT][GS]>(gemm_lds + sizeof(_Float16) * 2 * GT * GS);
-    _Float16(*mns)[GT][8] = reinterpret_cast<_Float16(*)[GT][8]>(gemm_lds + sizeof(_Float16) * 4 * GT * GS);  // unused: no minimums
-    uint32_t(*dds)[GT] = reinterpret_cast<uint32_t(*)[GT]>(gemm_lds + sizeof(_Float16) * (4 * GT * GS + 2 * GT * 8));
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t n0 = blockIdx.x * GT, m0 = blockIdx.y * GT;
-    const uint32_t steps = p.K / 32u;  // a multiple of 8: K is whole super-blocks
-    typedef const __attribute__((address_space(1))) u32x4 *global_uint4;
-    typedef const __attribute__((address_space(1))) uint16_t *global_half_word;
-
-    if (wave >= 4) {
-        // ------------------------------------------------------------------ stagers
-        // one row of each tile, one half (16 k: one scale) of the step
-        const uint32_t tid = threadIdx.x - 256u;
-        const uint32_t srow = tid >> 1, sh = tid & 1u;
-        const uint32_t column = min(n0 + srow, p.N - 1u);
-        const uint8_t *wrow = column < p.end0   ? p.W + (size_t)column * p.row_bytes
-                              : column < p.end1 ? p.W1 + (size_t)(column - p.end0) * p.row_bytes
-                                                : p.W2 + (size_t)(column - p.end1) * p.row_bytes;
-        const _Float16 *arow = p.A + (size_t)min(m0 + srow, p.rows - 1u) * p.K + 16u * sh;
-        const uint32_t nsb = steps >> 3;
-        // 16 bytes from `at` (any half word) as the aligned 16 below and the half word at + 14
-        auto run = [&](const uint8_t *at, u32x4 &low, uint32_t &above) {
-            low = *(global_uint4)((uintptr_t)at & ~(uintptr_t)3);
-            above = *(global_half_word)(uintptr_t)(at + 14u);
-        };
-        auto fetch = [&](Q6Raw &raw, uint32_t sb) {
-            const uint8_t *block = wrow + (size_t)min(sb, nsb - 1u) * 210u;  // past the end the last super-block again, dropped
-#pragma unroll
-            for (int r = 0; r < 4; r++) run(block + 64u * (r >> 1) + 32u * (r & 1) + 16u * sh, raw.ql[r], raw.qle[r]);
-#pragma unroll
-            for (int n = 0; n < 2; n++) run(block + 128u + 32u * n + 16u * sh, raw.qh[n], raw.qhe[n]);
-            run(block + 192u, raw.sc, raw.sce);
-            raw.d = *(global_half_word)(uintptr_t)(block + 208u);
-        };
-        // the run as it lies: nothing to do on a word boundary, else every word takes its upper half from the next
-        auto placed = [](const u32x4 &low, uint32_t above, uint32_t shift) -> u32x4 {
-            return u32x4{__builtin_amdgcn_alignbit(low.y, low.x, shift), __builtin_amdgcn_alignbit(low.z, low.y, shift),
-                         __builtin_amdgcn_alignbit(low.w, low.z, shift), __builtin_amdgcn_alignbit(above, low.w, shift)};
-        };
-        u32x4 av[4][2];  // activations by slot = step % 4
-        auto fetch_activations = [&](int slot, uint32_t step) {
-            const _Float16 *at = arow + (size_t)min(step, steps - 1u) * 32u;
-#pragma unroll
-            for (int i = 0; i < 2; i++) av[slot][i] = *(global_uint4)(uintptr_t)(at + 8 * i);
-        };
-        const half2_t bias = {(_Float16)1056.0f, (_Float16)1056.0f};  // 0x6400 | q is the half 1024 + q; the weight is q - 32
-        Q6Raw raws[2];
-        fetch(raws[0], 0);
-        __builtin_amdgcn_sched_barrier(0);  // the first super-block goes out first: the loop waits for the oldest loads only
-#pragma unroll
-        for (int slot = 0; slot < 4; slot++) fetch_activations(slot, slot);
-        fetch(raws[1], 1);
-        __builtin_amdgcn_sched_barrier(0);
-        auto super_block = [&](Q6Raw &raw, const uint32_t sb) {
-            const uint32_t shift = (uint32_t)((uintptr_t)(wrow + (size_t)sb * 210u) & 2u) * 8u;  // 0 or 16: where the block starts in its word
-            const u32x4 scales = placed(raw.sc, raw.sce, shift);
-            const uint32_t scale_words[4] = {scales.x, scales.y, scales.z, scales.w};
-            u32x4 high_pairs = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const uint32_t buf = s & 1u, sbuf = (s >> 2) & 1u;  // steps are whole super-blocks: step 8 sb + s has parity s & 1
-                const int n = s >> 2, quarter = s & 3;
-                if (quarter == 0) high_pairs = placed(raw.qh[n], raw.qhe[n], shift);
-                // group 2 s + sh of the super-block: scale byte 2 (s & 1) + sh of word s / 2
-                const int sc = __builtin_amdgcn_sbfe((int)scale_words[s >> 1], 16u * (s & 1) + 8u * sh, 8u);
-                const _Float16 fine = (_Float16)(float)(sc & 15), coarse = (_Float16)(float)(16 * (sc >> 4));
-                const half2_t fine2 = {fine, fine}, coarse2 = {coarse, coarse};
-                const u32x4 nibbles = placed(raw.ql[2 * n + (quarter & 1)], raw.qle[2 * n + (quarter & 1)], shift);
-                const uint32_t nibble_words[4] = {nibbles.x, nibbles.y, nibbles.z, nibbles.w};
-                const uint32_t pair_words[4] = {high_pairs.x, high_pairs.y, high_pairs.z, high_pairs.w};
-                uint32_t one[8], two[8];
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    const uint32_t low4 = (quarter >= 2 ? nibble_words[w] >> 4 : nibble_words[w]) & 0x0f0f0f0fu;
-                    const uint32_t q4 = low4 | (((pair_words[w] >> (2 * quarter)) & 0x03030303u) << 4);  // four weights' six bits, one a byte
-                    // element order inside a word: 0, 2 then 1, 3, as the activations were packed
-                    const half2_t even = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, q4, 0x0c020c00u) | 0x64006400u) - bias;
-                    const half2_t odd = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, q4, 0x0c030c01u) | 0x64006400u) - bias;
-                    one[2 * w] = __builtin_bit_cast(uint32_t, even * fine2), one[2 * w + 1] = __builtin_bit_cast(uint32_t, odd * fine2);
-                    two[2 * w] = __builtin_bit_cast(uint32_t, even * coarse2), two[2 * w + 1] = __builtin_bit_cast(uint32_t, odd * coarse2);
-                }
-                u32x4 *first = reinterpret_cast<u32x4 *>(&Bs[buf][srow][16u * sh]), *second = reinterpret_cast<u32x4 *>(&Bs[buf][srow][32u + 16u * sh]);
-                first[0] = u32x4{one[0], one[1], one[2], one[3]};
-                first[1] = u32x4{one[4], one[5], one[6], one[7]};
-                second[0] = u32x4{two[0], two[1], two[2], two[3]};
-                second[1] = u32x4{two[4], two[5], two[6], two[7]};
-                if (quarter == 0 && sh == 0) dds[sbuf][srow] = raw.d;  // (d, no dmin) of these four steps
-                u32x4 *once = reinterpret_cast<u32x4 *>(&As[buf][srow][16u * sh]), *again = reinterpret_cast<u32x4 *>(&As[buf][srow][32u + 16u * sh]);
-#pragma unroll
-                for (int i = 0; i < 2; i++) once[i] = av[s & 3][i], again[i] = av[s & 3][i];
-                fetch_activations(s & 3, 8u * sb + (uint32_t)s + 4u);
-                if (s == 7) fetch(raw, sb + 2u);  // these registers are free: the super-block after the next
-                __builtin_amdgcn_sched_barrier(0);
-                __syncthreads();  // step is staged; the multipliers are done with the step before it
-            }
-        };
-        uint32_t sb = 0;
-        for (; sb + 2u <= nsb; sb += 2u) {
-            super_block(raws[0], sb);
-            super_block(raws[1], sb + 1u);
-        }
-        if (sb < nsb) super_block(raws[0], sb);
-        return;
-    }
-    gemm_multiply<false>(p, As, Bs, mns, dds, wave, lane, n0, m0, steps, 1.0f);
-}
-
-// ------------------------------------------------------------------- Q3_K on MFMA --------
-//
-// A Q3_K weight is d * (sc - 32) * c with c in -4..3 (two bits less 4 unless the third bit is set) and sc of six bits a 16
-// weights (crates/neura-precision/src/ggml.rs:224-229, 291-306): (sc - 32) * c stays within +-128 and is an exact half, so the
-// weights are one operand plane, a step is 64 k as in the Q4_K kernel (a stager's 32 weights are two scale groups), a
-// super-block's four steps are weighed by d together, and there are no minimums.  Blocks are 110 bytes and start on any
-// half word; they are read as the Q6_K kernel reads its own.
-struct Q3Raw {
-    u32x4 hm[2], qs[4], sc;           // the third bits of the 32 columns, the bit pairs of both halves, bytes 94..109 (scales, d)
-    uint32_t hme[2], qse[4], sce;     // the half word above each run
-};
-
-__global__ __launch_bounds__(512) void gemm_q3k_mfma_kernel(GemmQ4Params p) {
-    fetch_parameters(p);
-    extern __shared__ __attribute__((aligned(16))) uint8_t gemm_lds[];
-    _Float16(*As)[GT][GS] = reinterpret_cast<_Float16(*)[GT][GS]>(gemm_lds);
-    _Float16(*Bs)[GT][GS] = reinterpret_cast<_Float16(*)[GT][GS]>(gemm_lds + sizeof(_Float16) * 2 * GT * GS);
-    _Float16(*mns)[GT][8] = reinterpret_cast<_Float16(*)[GT][8]>(gemm_lds + sizeof(_Float16) * 4 * GT * GS);  // unused: no minimums
-    uint32_t(*dds)[GT] = reinterpret_cast<uint32_t(*)[GT]>(gemm_lds + sizeof(_Float16) * (4 * GT * GS + 2 * GT * 8));
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t n0 = blockIdx.x * GT, m0 = blockIdx.y * GT;
-    const uint32_t steps = p.K / 64u;  // a multiple of 4: K is whole super-blocks
-    typedef const __attribute__((address_space(1))) u32x4 *global_uint4;
-    typedef const __attribute__((address_space(1))) uint16_t *global_half_word;
-
-    if (wave >= 4) {
-        // ------------------------------------------------------------------ stagers
-        // one row of each tile, one half (32 k: two scales) of the step
-        const uint32_t tid = threadIdx.x - 256u;
-        const uint32_t srow = tid >> 1, sh = tid & 1u;
-        const uint32_t column = min(n0 + srow, p.N - 1u);
-        const uint8_t *wrow = column < p.end0   ? p.W + (size_t)column * p.row_bytes
-                              : column < p.end1 ? p.W1 + (size_t)(column - p.end0) * p.row_bytes
-                                                : p.W2 + (size_t)(column - p.end1) * p.row_bytes;
-        const _Float16 *arow = p.A + (size_t)min(m0 + srow, p.rows - 1u) * p.K + 32u * sh;
-        const uint32_t nsb = steps >> 2;
-        auto run = [&](const uint8_t *at, u32x4 &low, uint32_t &above) {
-            low = *(global_uint4)((uintptr_t)at & ~(uintptr_t)3);
-            above = *(global_half_word)(uintptr_t)(at + 14u);
-        };
-        auto fetch = [&](Q3Raw &raw, uint32_t sb) {
-            const uint8_t *block = wrow + (size_t)min(sb, nsb - 1u) * 110u;  // past the end the last super-block again, dropped
-#pragma unroll
-            for (int r = 0; r < 2; r++) run(block + 16u * r, raw.hm[r], raw.hme[r]);
-#pragma unroll
-            for (int r = 0; r < 4; r++) run(block + 32u + 16u * r, raw.qs[r], raw.qse[r]);
-            run(block + 94u, raw.sc, raw.sce);
-        };
-        auto placed = [](const u32x4 &low, uint32_t above, uint32_t shift) -> u32x4 {
-            return u32x4{__builtin_amdgcn_alignbit(low.y, low.x, shift), __builtin_amdgcn_alignbit(low.z, low.y, shift),
-                         __builtin_amdgcn_alignbit(low.w, low.z, shift), __builtin_amdgcn_alignbit(above, low.w, shift)};
-        };
-        u32x4 av[4][4];  // activations by slot = step % 4
-        auto fetch_activations = [&](int slot, uint32_t step) {
-            const _Float16 *at = arow + (size_t)min(step, steps - 1u) * 64u;
-#pragma unroll
-            for (int i = 0; i < 4; i++) av[slot][i] = *(global_uint4)(uintptr_t)(at + 8 * i);
-        };
-        const half2_t scale_bias = {(_Float16)1056.0f, (_Float16)1056.0f};  // 0x6400 | v is the half 1024 + v; a scale is stored 32 too large
-        const half2_t code_bias = {(_Float16)1028.0f, (_Float16)1028.0f};   // and a code 4 too large
-        Q3Raw raws[2];
-        fetch(raws[0], 0);
-        __builtin_amdgcn_sched_barrier(0);  // the first super-block goes out first: the loop waits for the oldest loads only
-#pragma unroll
-        for (int slot = 0; slot < 4; slot++) fetch_activations(slot, slot);
-        fetch(raws[1], 1);
-        __builtin_amdgcn_sched_barrier(0);
-        auto super_block = [&](Q3Raw &raw, const uint32_t sb) {
-            const uint32_t shift = (uint32_t)((uintptr_t)(wrow + (size_t)sb * 110u) & 2u) * 8u;  // 0 or 16: where the block starts in its word
-            const u32x4 tail = placed(raw.sc, raw.sce, shift ^ 16u);  // bytes 94..109: this run starts on the other half of a word
-            // bytes 96..107: the scales' nibbles (two words) and their top bit pairs (one)
-            const uint32_t nibble_words[2] = {__builtin_amdgcn_alignbit(tail.y, tail.x, 16u), __builtin_amdgcn_alignbit(tail.z, tail.y, 16u)};
-            const uint32_t tops = __builtin_amdgcn_alignbit(tail.w, tail.z, 16u);
-            const u32x4 third0 = placed(raw.hm[0], raw.hme[0], shift), third1 = placed(raw.hm[1], raw.hme[1], shift);
-            const uint32_t third_words[8] = {third0.x, third0.y, third0.z, third0.w, third1.x, third1.y, third1.z, third1.w};
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const uint32_t buf = g & 1u, sbuf = sb & 1u;
-                const int n = g >> 1;
-                // scales 4 g + 2 sh and the one after: nibble 2 sh + t of word g & 1 (low nibbles for the first eight scales), top
-                // bits from byte 2 sh + t of the third word at 2 g
-                const uint32_t two = (nibble_words[g & 1] >> (16u * sh)) & 0xffffu, top = (tops >> (16u * sh)) & 0xffffu;
-                const uint32_t pair = ((g < 2 ? two : two >> 4) & 0x0f0fu) | (((top >> (2 * g)) & 0x0303u) << 4);
-                const half2_t scales = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, pair, 0x0c010c00u) | 0x64006400u) - scale_bias;
-                const half2_t first_scale = {scales.x, scales.x}, second_scale = {scales.y, scales.y};
-                const u32x4 pairs0 = placed(raw.qs[2 * n], raw.qse[2 * n], shift), pairs1 = placed(raw.qs[2 * n + 1], raw.qse[2 * n + 1], shift);
-                const uint32_t pair_words[8] = {pairs0.x, pairs0.y, pairs0.z, pairs0.w, pairs1.x, pairs1.y, pairs1.z, pairs1.w};
-                const uint32_t j = 2u * (g & 1) + sh;  // which bit pair of a byte, and with 4 n which third bit
-                uint32_t out[16];
-#pragma unroll
-                for (int w = 0; w < 8; w++) {
-                    const uint32_t v = ((pair_words[w] >> (2u * j)) & 0x03030303u) | (((third_words[w] >> (4u * n + j)) & 0x01010101u) << 2);  // code + 4, one a byte
-                    // element order inside a word: 0, 2 then 1, 3, as the activations were packed
-                    const half2_t even = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, v, 0x0c020c00u) | 0x64006400u) - code_bias;
-                    const half2_t odd = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, v, 0x0c030c01u) | 0x64006400u) - code_bias;
-                    const half2_t scale = w < 4 ? first_scale : second_scale;
-                    out[2 * w] = __builtin_bit_cast(uint32_t, even * scale), out[2 * w + 1] = __builtin_bit_cast(uint32_t, odd * scale);
-                }
-                u32x4 *to = reinterpret_cast<u32x4 *>(&Bs[buf][srow][32u * sh]);
-#pragma unroll
-                for (int i = 0; i < 4; i++) to[i] = u32x4{out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]};
-                if (g == 0 && sh == 0) dds[sbuf][srow] = tail.w >> 16;  // (d, no dmin)
-                u32x4 *adst = reinterpret_cast<u32x4 *>(&As[buf][srow][32u * sh]);
-#pragma unroll
-                for (int i = 0; i < 4; i++) adst[i] = av[g][i];
-                fetch_activations(g, 4u * sb + (uint32_t)g + 4u);
-                if (g == 3) fetch(raw, sb + 2u);  // these registers are free: the super-block after the next
-                __builtin_amdgcn_sched_barrier(0);
-                __syncthreads();  // step is staged; the multipliers are done with the step before it
-            }
-        };
-        uint32_t sb = 0;
-        for (; sb + 2u <= nsb; sb += 2u) {
-            super_block(raws[0], sb);
-            super_block(raws[1], sb + 1u);
-        }
-        if (sb < nsb) super_block(raws[0], sb);
-        return;
-    }
-    gemm_multiply<false>(p, As, Bs, mns, dds, wave, lane, n0, m0, steps, 1.0f);
 }
 
 // Where a wide product's packed rows lie in the device's scratch: whole tiles of K halves a row, as many of [K / 256][16] sums, M row
@@ -1321,6 +1076,24 @@ static int32_t pack_rows(nh_device *d, const GemmArgs &a, _Float16 *A, _Float16 
     }
 }
 
+// Which form a wide product takes.  `operands`: over rows packed in operand order (the product of few rows, or of shared rows in a
+// shape), else the 128 x 128 tiles.  NEURA_HIP_GEMM_WIDE=0: no shared rows; =42, 43, 83, 84: that shape wherever it can.  Q6_K and
+// Q3_K have no tiles (gate of the 7B shape at 1024 rows 360 and 259 us there, 252 and 190 on shared rows): what few_rows_win
+// leaves, which is what takes whole rounds of them, goes to shared rows.
+struct WideForm {
+    bool operands;
+    SharedShape shape;
+};
+static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows) {
+    const int held = env_int("NEURA_HIP_GEMM_WIDE", -1);
+    if (held == SHARED_42 || held == SHARED_43 || held == SHARED_83 || held == SHARED_84) return WideForm{true, (SharedShape)held};
+    const uint32_t units = (uint32_t)d->compute_units;
+    const SharedShape shape = held == 0 || gemm_few_held() >= 0 ? SHARED_NONE : shared_rows_shape(element, N, K, rows, units);
+    if (shape != SHARED_NONE || gemm_few_takes(d, element, N, K, rows)) return WideForm{true, shape};
+    const bool tiled = element != NH_Q6_K && element != NH_Q3_K;
+    return tiled ? WideForm{false, SHARED_NONE} : WideForm{true, SHARED_43};
+}
+
 static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     GemmQ4Params p{};
     p.W = static_cast<const uint8_t *>(a.W);
@@ -1331,7 +1104,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     p.N = a.N;
     p.K = a.K;
     p.row_bytes = (uint32_t)payload_bytes(a.element, a.K);
-    p.Y = a.Y;
+    p.Y = a.Y, p.Y1 = a.Y_more;
     p.residual = a.residual;
     p.ldy = a.ldy;
     p.M = a.M;
@@ -1339,10 +1112,11 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const uint32_t pieces = half_rows ? 1u : a.whole ? WHOLE_PIECES : 2u;
     p.rows = a.whole ? whole_rows(a.M) : pieces * a.M;
     p.split = half_rows ? 0 : 1;
-    const bool few = a.whole || gemm_few_takes(d, a.element, a.N, a.K, p.rows);
+    const WideForm form = a.whole || a.gated ? WideForm{true, SHARED_NONE} : wide_form(d, a.element, a.N, a.K, p.rows);
+    const bool few = form.operands;
     if (a.whole && (half_rows || gemm_few_held() == 0 || a.M > 65535u * WHOLE_TILE))
         return fail(NH_E_ARGUMENT, "this wide product takes no fp32 rows whole (ask gemm_takes_whole first)");
-    if (a.gated && (!few || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
+    if (a.gated && (!gemm_few_takes(d, a.element, a.N, a.K, p.rows) || !p.W1 || p.W2 || a.residual || p.end0 != a.N))
         return fail(NH_E_ARGUMENT, "this wide product gates no outputs (ask gemm_gates first)");
     const PackedRows at(a.M, a.K, pieces);
     uint8_t *room = static_cast<uint8_t *>(scratch(d, at.bytes));
@@ -1360,24 +1134,22 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
         if (status != NH_OK) return status;
     }
     p.A = A, p.S = S, p.unscale = unscale;
-    if (few)
-        return launch_gemm_few(d, a.element, FewParams{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, pieces, p.unscale, reinterpret_cast<const WholeRow *>(unscale), outside,
-                                                       1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets}, a.gated);
+    if (few) {
+        const FewParams f{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, pieces, p.unscale, reinterpret_cast<const WholeRow *>(unscale), outside,
+                          1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets, a.Y_more};
+        return form.shape != SHARED_NONE ? launch_gemm_wide(d, a.element, f, form.shape) : launch_gemm_few(d, a.element, f, a.gated);
+    }
     static bool sized = false;
     if (!sized) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q8_0_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q8_LDS));
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_regb_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_REGB_LDS));
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q6k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q5k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q3k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
         sized = true;
     }
     dim3 grid((a.N + GT - 1) / GT, (p.rows + GT - 1) / GT);
     if (a.element == NH_Q8_0) hipLaunchKernelGGL(gemm_q8_0_mfma_kernel, grid, dim3(512), GEMM_Q8_LDS, d->stream, p);
-    else if (a.element == NH_Q6_K) hipLaunchKernelGGL(gemm_q6k_mfma_kernel, grid, dim3(512), GEMM_Q4K_LDS, d->stream, p);
     else if (a.element == NH_Q5_K) hipLaunchKernelGGL(gemm_q5k_mfma_kernel, grid, dim3(512), GEMM_Q4K_LDS, d->stream, p);
-    else if (a.element == NH_Q3_K) hipLaunchKernelGGL(gemm_q3k_mfma_kernel, grid, dim3(512), GEMM_Q4K_LDS, d->stream, p);
     else if (const char *held = getenv("NEURA_HIP_GEMM_REGB"); held && held[0] == '0')  // the form that unpacks the weights into LDS
         hipLaunchKernelGGL(gemm_q4k_mfma_kernel, grid, dim3(512), GEMM_Q4K_LDS, d->stream, p);
     else hipLaunchKernelGGL(gemm_q4k_regb_mfma_kernel, grid, dim3(768), GEMM_Q4K_REGB_LDS, d->stream, p);
@@ -1421,7 +1193,7 @@ bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const ui
         return true;
     }
     for (int s = 0; s < 3; s++)
-        if (!mfma_takes(elements[s], K, X, W[s]) || gemm_few_takes(d, elements[s], N[s], K, 2u * M) != gemm_few_takes(d, elements[0], N[0], K, 2u * M)) return false;
+        if (!mfma_takes(elements[s], K, X, W[s]) || wide_form(d, elements[s], N[s], K, 2u * M).operands != wide_form(d, elements[0], N[0], K, 2u * M).operands) return false;
     return true;
 }
 
@@ -1448,7 +1220,7 @@ int32_t launch_gemv_wide(nh_device *d, const GemvArgs &a) {
 
 static int32_t launch_gemm_any(nh_device *d, const GemmArgs &a) {
     if (mfma_takes(a.element, a.K, a.X, a.W)) return launch_gemm_mfma(d, a);
-    if (a.W_more[0] || a.W_more[1] || a.packed || a.norm_w || a.gate || a.gated || a.whole)
+    if (a.W_more[0] || a.W_more[1] || a.Y_more || a.packed || a.norm_w || a.gate || a.gated || a.whole)
         return fail(NH_E_ARGUMENT, "this wide product stacks no matrices, reuses no packed activations and packs rows as they lie (ask gemm_stacks first)");
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM), block(256);
     uint32_t row_bytes = (uint32_t)payload_bytes(a.element, a.K);

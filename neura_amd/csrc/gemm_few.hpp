@@ -1,6 +1,7 @@
 // The wide product of few activation rows (gemm_few.hip), as the wide products' launcher (gemm.hip) reaches it.
 #pragma once
 #include "common.hpp"
+#include "few_rule.hpp"
 
 namespace nh {
 
@@ -64,11 +65,14 @@ struct FewParams {
     uint32_t slices;        // workgroups (blockIdx.z) that share the K of the same tiles
     float *partial;         // FEW_PARTIAL_BYTES of scratch for their sums
     uint32_t *meets;        // FEW_MEETS words, zero between launches: workgroups of a place that have left their sums
+    float *Y1;              // where not null, columns from end0 on go there, with the same ldy (Y's first: Y1[n - end0])
 };
 
 int gemm_few_held();  // NEURA_HIP_GEMM_FEW: 0 never, 1 wherever it can be, -1 by the rule on sizes
 // whether the product of `rows` packed rows is this kernel's, and its launch (the rows are packed)
 bool gemm_few_takes(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows);
-int32_t launch_gemm_few(nh_device *d, int32_t element, FewParams p, bool gated);
+int32_t launch_gemm_few(nh_device *d, int32_t element, const FewParams &p, bool gated);
+// the product of shared rows (gemm_wide.hip), over rows packed the same way
+int32_t launch_gemm_wide(nh_device *d, int32_t element, const FewParams &p, SharedShape shape);
 
 }  // namespace nh

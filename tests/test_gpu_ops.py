@@ -618,6 +618,46 @@ def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, 
     assert (np.abs(device.gemm(element, raw, N, K, X, residual=r) - (exact + r)) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r)) + 1e-30).all()
 
 
+@pytest.mark.parametrize("shape", ["42", "43", "83", "84"])
+@pytest.mark.parametrize("element,M,N,K,half", [
+    (NH_Q4_K, 1, 32, 256, False), (NH_Q4_K, 50, 300, 512, False), (NH_Q4_K, 33, 1056, 1280, False), (NH_Q4_K, 130, 200, 768, True),
+    (NH_Q5_K, 65, 130, 512, False), (NH_Q5_K, 97, 290, 256, True), (NH_Q6_K, 50, 300, 512, False), (NH_Q6_K, 33, 100, 768, True), (NH_Q3_K, 49, 270, 512, False),
+    (NH_Q3_K, 129, 64, 768, True), (NH_Q8_0, 50, 300, 192, False), (NH_Q8_0, 97, 270, 64, True), (NH_Q8_0, 33, 130, 4864, False)])
+def test_wide_products_of_shared_rows(device, monkeypatch, shape, element, M, N, K, half):
+    """The wide product whose workgroups share their rows through LDS, each shape of it forced: columns and row tiles past the last, rows
+    that end inside a tile, one unit and several, an odd number of Q8_0's steps -- against the exact product at the bar of
+    test_both_forms_of_a_wide_product, with random blocks (whose minimums outweigh some scales by more than a half holds), with a
+    block's scale zero and its minimum not, with outliers on zero weights, and with an infinity in one row."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_WIDE", shape)
+    rng = np.random.default_rng(M + N + K + element)
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    per, size = synth.BLOCK_BYTES[element]
+    blocks = raw.reshape(N, K // per, size)
+    if element in (NH_Q4_K, NH_Q5_K):
+        blocks[::3, 0, 0:2] = 0  # d
+        codes = 16 if element == NH_Q4_K else 48
+        blocks[:, -1, 4 + 4] &= 0xC0  # the last block's sub-block 0 without a minimum, and code 0 for its number 5
+        blocks[:, -1, codes + 5] &= 0xF0
+        if element == NH_Q5_K:
+            blocks[:, -1, 16 + 5] &= 0xFE
+    X = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
+    weights = oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64)
+    if element in (NH_Q4_K, NH_Q5_K) and not half:
+        X[:, K - per + 5] *= 1e4
+        assert (weights[:, K - per + 5] == 0).all()
+    exact = X.astype(np.float64) @ weights.T
+    scale = np.sqrt((X.astype(np.float64) ** 2) @ (weights.T ** 2))
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    got = device.gemm(element, raw, N, K, X)
+    assert (np.abs(got - exact) <= 4e-6 * scale + 1e-30).all()
+    assert (np.abs(device.gemm(element, raw, N, K, X, residual=r) - (exact + r)) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r)) + 1e-30).all()
+    X[M // 2, 3] = np.inf
+    bad = device.gemm(element, raw, N, K, X)
+    assert not np.isfinite(bad[M // 2]).any()
+    rest = np.arange(M) != M // 2
+    assert np.array_equal(bad[rest], got[rest])
+
+
 @pytest.mark.parametrize("element,M,N,K", [
     (NH_Q4_K, 8, 96, 8960), (NH_Q4_K, 48, 33, 18944), (NH_Q5_K, 5, 160, 4608), (NH_Q5_K, 17, 64, 2560), (NH_Q6_K, 16, 130, 8960), (NH_Q3_K, 3, 32, 18944),
     (NH_Q3_K, 100, 96, 8960), (NH_Q8_0, 9, 77, 4864), (NH_Q8_0, 33, 256, 8960), (NH_Q8_0, 2, 31, 18944)])
