@@ -820,15 +820,26 @@ __global__ __launch_bounds__(256) void attention_decode_tile_kernel(const uint32
         if (next < last) fetch_keys(next);  // in flight during the rest of this tile
         // ---- weights: register e of block kb is key 16 kb + 4 kq + e of the tile, for this lane's column
         float tile_top = -INFINITY;
+        const bool whole = tile + TK <= last;
+        if (whole && !p.reach) {  // every key is seen (a column past the group may weigh what it likes: it leaves nothing): no mask to work out
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++)
+            for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t key = tile + 16u * kb + 4u * kq + e;
-                const bool seen = held && key < last && (!p.reach || ring.seen(key, origin));
-                scores[kb][e] = seen ? fmaf(fine[kb][e], 1.0f / 2048.0f, scores[kb][e]) * p.scale : -INFINITY;
-                tile_top = fmaxf(tile_top, scores[kb][e]);
-            }
+                for (int e = 0; e < 4; e++) {
+                    scores[kb][e] = fmaf(fine[kb][e], 1.0f / 2048.0f, scores[kb][e]) * p.scale;
+                    tile_top = fmaxf(tile_top, scores[kb][e]);
+                }
+        } else {
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t key = tile + 16u * kb + 4u * kq + e;
+                    const bool seen = held && key < last && (!p.reach || ring.seen(key, origin));
+                    scores[kb][e] = seen ? fmaf(fine[kb][e], 1.0f / 2048.0f, scores[kb][e]) * p.scale : -INFINITY;
+                    tile_top = fmaxf(tile_top, scores[kb][e]);
+                }
+        }
         tile_top = fmaxf(tile_top, __shfl_xor(tile_top, 16, 64));
         tile_top = fmaxf(tile_top, __shfl_xor(tile_top, 32, 64));
         const float newer = fmaxf(top, tile_top);

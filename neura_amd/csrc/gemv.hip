@@ -1571,49 +1571,122 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 3) void gemv_q4k_mfma32_ker
     // ---- activations -> digit planes, 16 elements (half a sub-block) per thread; a row takes at most 256 threads
     // (K <= 4096), so a workgroup of sixteen waves stages four rows side by side
     constexpr uint32_t GROUPS = NT / 256u;
+    constexpr uint32_t PASSES = R2 / GROUPS;
+    static_assert(PASSES * GROUPS == R2, "whole passes of rows");
     const uint32_t chunks = nb * 16u;
     const uint32_t rg = tid >> 8, t = tid & 255u;
-    // a thread's sixteen numbers of row `row0 + rg`, asked for whatever the row and the chunk (past them the last row's, the
-    // last chunk's, dropped by the caller): the next rows' are on their way while these rows become digits
-    auto fetch_rows = [&](uint32_t row0, float4 (&into)[4]) {
-        const float *xr = p.x + (size_t)min(row0 + rg, p.rows - 1u) * p.K + k0 + 16u * min(t, chunks - 1u);
+    // a thread's sixteen numbers of a row of every pass, asked for whatever the row and the chunk (past them the last row's, the
+    // last chunk's, dropped below)
+    float4 held_rows[PASSES][4], w[4];
 #pragma unroll
-        for (int c = 0; c < 4; c++) into[c] = *reinterpret_cast<const float4 *>(xr + 4u * c);
-    };
-    float4 ahead[4], w[4];
-    fetch_rows(0u, ahead);
+    for (uint32_t pass = 0; pass < PASSES; pass++) {
+        const float *xr = p.x + (size_t)min(pass * GROUPS + rg, p.rows - 1u) * p.K + k0 + 16u * min(t, chunks - 1u);
+#pragma unroll
+        for (int c = 0; c < 4; c++) held_rows[pass][c] = *reinterpret_cast<const float4 *>(xr + 4u * c);
+    }
     if (p.norm_w) {
 #pragma unroll
         for (int c = 0; c < 4; c++) w[c] = *reinterpret_cast<const float4 *>(p.norm_w + k0 + 16u * min(t, chunks - 1u) + 4u * c);
     }
+    uint32_t position = 0;  // ROPE: where the plane of this lane's outputs stands
+    if constexpr (ROPE) position = rest.rope_cursor[min(2u * (wave % KS) + (lane >> 5), p.rows - 1u)];
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the weights' first super-block is asked for behind the activations, before they become digits: its way from memory
+    // is covered by that work (a wave's loads come back in order, so the activations are not kept waiting).  A product of one
+    // tile a workgroup is a chain of latencies; with this link, the two barriers a pass of rows and the rotation's loads off the
+    // chain a step of eight planes of the 7B shape went from 22.5 ms for eight to 21.7 (the output projection 11.6 -> 10.4 us)
+    const uint32_t n = lane & 31u, q = lane >> 5;
+    const uint32_t ts = wave / KS, ks = wave % KS;
+    const uint32_t count = ks < nb ? (nb - ks + KS - 1u) / KS : 0u;  // super-blocks ks, ks + KS, ...
+    const uint8_t *const w0 = p.W[0], *const w1 = p.W[1], *const w2 = p.W[2];
+    const uint32_t end0 = p.end[0], end1 = p.end[1];
+    const bool gated = p.swiglu != 0;
+    // ROPE: a tile's first output row -- channel c0 of a head -- and what its rows 16..31 lie further (half a head)
+    const uint32_t rope_tiles_a_head = ROPE ? rest.rope_width / 32u : 1u, rope_half = ROPE ? rest.rope_width / 2u : 0u;
+    // A super-block of the tile is 32 rows x 144 bytes = 288 pieces of 16 bytes.  Lane l fetches pieces l, l + 64, ...: nine
+    // neighbouring lanes read one row's block end to end (a load instruction touches 15 cache lines where one lane per
+    // row would touch 32), and the pieces go through LDS to the lanes that multiply them.
+    const uint8_t *src[5];
+    // (scalars captured by value: a closure by reference would choose between the addresses of w0, w1, w2 in memory)
+    const int64_t to_w1 = w1 - w0, to_w2 = w2 - w0;
+    const uint32_t tiles = p.tiles, row_bytes = p.row_bytes, rope_width = ROPE ? rest.rope_width : 0u;
+    auto aim = [&src, w0, to_w1, to_w2, end0, end1, gated, tiles, row_bytes, blk0, n, q, lane, ts, rope_tiles_a_head, rope_half, rope_width](uint32_t base) __attribute__((always_inline)) {
+        // at the tile of round `base`, or the last one
+        const uint32_t at_tile = min(base + ts, tiles - 1u);
+        // first byte of row `r` of the tile
+        const uint32_t r0 = at_tile * 32u;
+        const bool in0 = r0 < end0, in1 = r0 < end1;
+        const int64_t plain_base = (in0 ? (int64_t)0 : (in1 ? to_w1 : to_w2)) + (int64_t)((size_t)(r0 - (in0 ? 0u : (in1 ? end0 : end1))) * row_bytes);
+        const uint32_t rope_first = ROPE ? (at_tile / rope_tiles_a_head) * rope_width + (at_tile % rope_tiles_a_head) * 16u : 0u;
+        // (a head never straddles two matrices: the tile's first row names the matrix of all its rows)
+        const int64_t rope_base = (rope_first < end0 ? (int64_t)0 : (rope_first < end1 ? to_w1 : to_w2)) +
+                                  (int64_t)((size_t)(rope_first - (rope_first < end0 ? 0u : (rope_first < end1 ? end0 : end1))) * row_bytes);
+        auto row_base = [=](uint32_t r) __attribute__((always_inline)) -> const uint8_t * {
+            const int64_t gated_at = (r < 16u ? (int64_t)0 : to_w1) + (int64_t)((size_t)(at_tile * 16u + (r & 15u)) * row_bytes);
+            const int64_t plain_at = ROPE ? rope_base + (int64_t)((size_t)((r & 15u) + (r >= 16u ? rope_half : 0u)) * row_bytes) : plain_base + (int64_t)((size_t)r * row_bytes);
+            return w0 + (gated && !ROPE ? gated_at : plain_at);
+        };
 #pragma unroll
-    for (uint32_t row0 = 0; row0 < R2; row0 += GROUPS) {
-        const uint32_t row = row0 + rg;  // groups past the staged rows only keep the barriers company
+        for (int i = 0; i < 5; i++) {
+            if (STAGED) {
+                const uint32_t c = lane + 64u * i < 288u ? lane + 64u * i : lane;  // the last 32 pieces do not exist: fetched twice, dropped
+                src[i] = row_base(c / 9u) + (size_t)blk0 * 144u + (c % 9u) * 16u;
+            } else {
+                src[i] = row_base(n) + (size_t)blk0 * 144u + (i == 0 ? 0u : 16u + 32u * (i - 1) + 16u * q);  // this lane's own header and half groups
+            }
+        }
+    };
+    u32x4 ahead[5];
+    auto fetch = [&](uint32_t step) {
+        const size_t off = (size_t)min(ks + KS * step, nb - 1u) * 144u;
+#pragma unroll
+        for (int i = 0; i < 5; i++) ahead[i] = *(global_uint4)(uintptr_t)(src[i] + off);
+    };
+    aim(blockIdx.x * TPW);
+    fetch(0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the whole rows are in registers, 256 threads a row
+    float rms[PASSES];
+    if (p.norm_w) {
+#pragma unroll
+        for (uint32_t pass = 0; pass < PASSES; pass++) {
+            const bool held = t < chunks && pass * GROUPS + rg < p.rows;
+            float square = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float4 a = held ? held_rows[pass][c] : make_float4(0.f, 0.f, 0.f, 0.f);
+                square = __fadd_rn(square, __fmul_rn(a.x, a.x)), square = __fadd_rn(square, __fmul_rn(a.y, a.y));
+                square = __fadd_rn(square, __fmul_rn(a.z, a.z)), square = __fadd_rn(square, __fmul_rn(a.w, a.w));
+            }
+            square = wave_sum(square);
+            if (lane == 0) red[pass * NW + wave] = square;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t pass = 0; pass < PASSES; pass++) {
+            const float *of = red + pass * NW + 4u * rg;
+            rms[pass] = rms_scale_of((of[0] + of[1]) + (of[2] + of[3]), p.K, p.eps);
+        }
+    }
+#pragma unroll
+    for (uint32_t pass = 0; pass < PASSES; pass++) {
+        const uint32_t row = pass * GROUPS + rg;
         const bool real = row < p.rows;
         {
-            const bool held = t < chunks && row < R2;
+            const bool held = t < chunks;
             float v[16];
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const float4 a = held && real ? ahead[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float4 a = held && real ? held_rows[pass][c] : make_float4(0.f, 0.f, 0.f, 0.f);
                 v[4 * c] = a.x, v[4 * c + 1] = a.y, v[4 * c + 2] = a.z, v[4 * c + 3] = a.w;
             }
-            if (row0 + GROUPS < R2) fetch_rows(row0 + GROUPS, ahead);
             if (p.norm_w) {
-                // the whole row is in registers across its 256 threads
-                float square = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 16; i++) square = __fadd_rn(square, __fmul_rn(v[i], v[i]));
-                square = wave_sum(square);
-                if (lane == 0) red[wave] = square;
-                __syncthreads();
-                const float total = (red[4u * rg] + red[4u * rg + 1u]) + (red[4u * rg + 2u] + red[4u * rg + 3u]);
-                __syncthreads();  // red is reused by the next rows
-                const float rms = rms_scale_of(total, p.K, p.eps);
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    v[4 * c] = __fmul_rn(__fmul_rn(v[4 * c], rms), w[c].x), v[4 * c + 1] = __fmul_rn(__fmul_rn(v[4 * c + 1], rms), w[c].y);
-                    v[4 * c + 2] = __fmul_rn(__fmul_rn(v[4 * c + 2], rms), w[c].z), v[4 * c + 3] = __fmul_rn(__fmul_rn(v[4 * c + 3], rms), w[c].w);
+                    v[4 * c] = __fmul_rn(__fmul_rn(v[4 * c], rms[pass]), w[c].x), v[4 * c + 1] = __fmul_rn(__fmul_rn(v[4 * c + 1], rms[pass]), w[c].y);
+                    v[4 * c + 2] = __fmul_rn(__fmul_rn(v[4 * c + 2], rms[pass]), w[c].z), v[4 * c + 3] = __fmul_rn(__fmul_rn(v[4 * c + 3], rms[pass]), w[c].w);
                 }
             }
             uint32_t top = 0;  // largest magnitude as bits: infinities and NaNs sort above every finite value
@@ -1652,13 +1725,6 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 3) void gemv_q4k_mfma32_ker
     __syncthreads();
 
     // ---- tiles of 32 weight rows
-    const uint32_t n = lane & 31u, q = lane >> 5;
-    const uint32_t ts = wave / KS, ks = wave % KS;
-    const uint32_t count = ks < nb ? (nb - ks + KS - 1u) / KS : 0u;  // super-blocks ks, ks + KS, ...
-    const uint32_t last_step = count ? count - 1u : 0u;
-    const uint8_t *const w0 = p.W[0], *const w1 = p.W[1], *const w2 = p.W[2];
-    const uint32_t end0 = p.end[0], end1 = p.end[1];
-    const bool gated = p.swiglu != 0;
     const u32x4 *const a_lane = reinterpret_cast<const u32x4 *>(staged) + (size_t)q * M8 + (lane & 31u);
     const bool a_held = (lane & 31u) < M8;
     uint32_t parity = 0;
@@ -1666,53 +1732,37 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 3) void gemv_q4k_mfma32_ker
         const uint32_t tile = base + ts;
         const bool live = tile < p.tiles;
         const uint32_t at_tile = live ? tile : p.tiles - 1u;
-        // first byte of row `r` of the tile
-        const uint32_t r0 = at_tile * 32u;
-        const bool in0 = r0 < end0, in1 = r0 < end1;
-        const uint8_t *const plain_base = (in0 ? w0 : (in1 ? w1 : w2)) + (size_t)(r0 - (in0 ? 0u : (in1 ? end0 : end1))) * p.row_bytes;
-        // ROPE: the tile's first output row -- channel c0 of a head -- and what its rows 16..31 lie further (half a head)
-        const uint32_t rope_tiles_a_head = ROPE ? rest.rope_width / 32u : 1u, rope_half = ROPE ? rest.rope_width / 2u : 0u;
-        const uint32_t rope_first = ROPE ? (at_tile / rope_tiles_a_head) * rest.rope_width + (at_tile % rope_tiles_a_head) * 16u : 0u;
-        // (a head never straddles two matrices: the tile's first row names the matrix of all its rows)
-        const uint8_t *const rope_base = (rope_first < end0 ? w0 : (rope_first < end1 ? w1 : w2)) +
-                                         (size_t)(rope_first - (rope_first < end0 ? 0u : (rope_first < end1 ? end0 : end1))) * p.row_bytes;
-        auto row_base = [&](uint32_t r) -> const uint8_t * {
-            if (gated) return (r < 16u ? w0 : w1) + (size_t)(at_tile * 16u + (r & 15u)) * p.row_bytes;
-            if constexpr (ROPE) return rope_base + (size_t)((r & 15u) + (r >= 16u ? rope_half : 0u)) * p.row_bytes;
-            return plain_base + (size_t)r * p.row_bytes;
-        };
-        // A super-block of the tile is 32 rows x 144 bytes = 288 pieces of 16 bytes.  Lane l fetches pieces l, l + 64, ...: nine
-        // neighbouring lanes read one row's block end to end (a load instruction touches 15 cache lines where one lane per
-        // row would touch 32), and the pieces go through LDS to the lanes that multiply them.
-        const uint8_t *src[5];
-#pragma unroll
-        for (int i = 0; i < 5; i++) {
-            if (STAGED) {
-                const uint32_t c = lane + 64u * i < 288u ? lane + 64u * i : lane;  // the last 32 pieces do not exist: fetched twice, dropped
-                src[i] = row_base(c / 9u) + (size_t)blk0 * 144u + (c % 9u) * 16u;
-            } else {
-                src[i] = row_base(n) + (size_t)blk0 * 144u + (i == 0 ? 0u : 16u + 32u * (i - 1) + 16u * q);  // this lane's own header and half groups
-            }
+        const uint32_t rope_first = ROPE ? (at_tile / rope_tiles_a_head) * rope_width + (at_tile % rope_tiles_a_head) * 16u : 0u;
+        // what the rotation of this lane's outputs needs is on its way while the tile is multiplied (read from the kernel's own
+        // argument block, `rest`: a member of the local copy chosen by a number would put the whole copy into scratch memory)
+        const uint32_t row_n = rope_first + (n & 15u) + (n >= 16u ? rope_half : 0u);  // the output row among q|k|v's
+        float cosine = 0.0f, sine = 0.0f, bias = 0.0f;
+        bool biased = false;
+        if constexpr (ROPE) {
+            const uint32_t c = (at_tile % rope_tiles_a_head) * 16u + (n & 15u);  // the lane's channel pair
+            const size_t at = (size_t)min(position, rest.rope_positions - 1u) * rope_half + c;
+            cosine = rest.rope_cosines[at], sine = rest.rope_sines[at];
+            const bool first0 = rope_first < end0, first1 = rope_first < end1;  // the tile's matrix: one for all its rows
+            const float *from = first0 ? rest.bias[0] : (first1 ? rest.bias[1] : rest.bias[2]);
+            biased = from != nullptr;
+            bias = *(biased ? from + (row_n - (first0 ? 0u : (first1 ? end0 : end1))) : rest.rope_cosines);
         }
-        u32x4 ahead[5];
-        auto fetch = [&](uint32_t step) {
-            // past the wave's last super-block the last one is fetched again: the waits count on every step issuing its loads
-            const size_t off = (size_t)min(ks + KS * min(step, last_step), nb - 1u) * 144u;
-#pragma unroll
-            for (int i = 0; i < 5; i++) ahead[i] = *(global_uint4)(uintptr_t)(src[i] + off);
-        };
         float acc[J];
 #pragma unroll
         for (int j = 0; j < J; j++) acc[j] = 0.0f;
-        fetch(0);
         for (uint32_t step = 0; step < count; step++) {
             const uint32_t b = min(ks + KS * step, nb - 1u);
+            // behind the wave's last super-block comes the first of its next tile (past the last tile the last again, dropped: the
+            // waits count on every step issuing its loads)
+            const bool closing = step + 1u == count;
+            if (closing) aim(base + gridDim.x * TPW);
+            const uint32_t following = closing ? 0u : step + 1u;
             Tile32Unit u;
             if (STAGED) {
 #pragma unroll
                 for (int i = 0; i < 5; i++)
                     if (i < 4 || lane < 32u) raw[lane + 64u * i] = ahead[i];
-                fetch(step + 1u);
+                fetch(following);
                 __builtin_amdgcn_wave_barrier();  // LDS serves a wave's accesses in order: the reads below see these writes
                 u.hdr = raw[n * 9u];
 #pragma unroll
@@ -1721,7 +1771,7 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 3) void gemv_q4k_mfma32_ker
                 u.hdr = ahead[0];
 #pragma unroll
                 for (int g = 0; g < 4; g++) u.g[g] = ahead[1 + g];
-                fetch(step + 1u);
+                fetch(following);
             }
             // the eight 6-bit scales and minimums (crates/neura-precision/src/ggml.rs:127-136), four to a word
             const uint32_t sc_lo = u.hdr.y & 0x3f3f3f3fu, sc_hi = (u.hdr.w & 0x0f0f0f0fu) | ((u.hdr.y >> 2) & 0x30303030u);
@@ -1767,22 +1817,11 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 3) void gemv_q4k_mfma32_ker
                 for (int k = 0; k < KS; k++) total += from[(size_t)k * J * 64u + j * 64u + lane];
                 const uint32_t arow = 2u * j + q;
                 if constexpr (ROPE) {
-                    // (what the rotation needs is read from the kernel's own argument block, `rest`: a member of the local copy
-                    // chosen by a number would put the whole copy into scratch memory)
-                    const uint32_t row_n = rope_first + (n & 15u) + (n >= 16u ? rope_half : 0u);  // the output row among q|k|v's
-                    const uint32_t c = (at_tile % rope_tiles_a_head) * 16u + (n & 15u);           // its channel pair
-                    const bool first0 = rope_first < end0, first1 = rope_first < end1;            // the tile's matrix: one for all its rows
-                    const float *bias = first0 ? rest.bias[0] : (first1 ? rest.bias[1] : rest.bias[2]);
-                    if (bias) total += bias[row_n - (first0 ? 0u : (first1 ? end0 : end1))];
+                    if (biased) total += bias;
                     const float other = __shfl_xor(total, 16, 64);
                     if (!live || arow >= p.rows) continue;
-                    const uint32_t position = rest.rope_cursor[arow];
                     float value = total;
-                    if (row_n < rest.rope_k_rows) {
-                        const size_t at = (size_t)min(position, rest.rope_positions - 1u) * rope_half + c;
-                        const float cosine = rest.rope_cosines[at], sine = rest.rope_sines[at];
-                        value = n >= 16u ? total * cosine + other * sine : total * cosine - other * sine;
-                    }
+                    if (row_n < rest.rope_k_rows) value = n >= 16u ? total * cosine + other * sine : total * cosine - other * sine;
                     if (row_n < rest.rope_q_rows) {
                         rest.y[(size_t)arow * rest.N + row_n] = value;
                     } else if (position >= rest.rope_positions || (!rest.rope_ring && position >= rest.rope_capacity)) {
@@ -1856,17 +1895,83 @@ __global__ __launch_bounds__(NW * 64) void gemv_q4k_f16_kernel(MFMA_LEAD_PARAMET
     float *const part = reinterpret_cast<float *>(pieces + (size_t)nb * F16_BLOCK_PIECES);  // [TPW][KS][4][64]
     typedef const __attribute__((address_space(1))) u32x4 *global_uint4;
 
-    // ---- activations -> half planes in operand order: row r by threads 128 r .. 128 r + 127, eight neighbours a thread
+    // ---- the activations' loads first: row r by threads 128 r .. 128 r + 127, eight neighbours a thread (past the rows and the
+    // slice the last again, dropped below)
+    const uint32_t staged_row = tid >> 7, t = tid & 127u;
+    const bool real = staged_row < p.rows;
+    float4 raw[4][2], gain[4][2];
     {
-        const uint32_t r = tid >> 7, t = tid & 127u;
-        const bool real = r < p.rows;
-        const float *xr = p.x + (size_t)min(r, p.rows - 1u) * p.K + k0;
+        const float *xr = p.x + (size_t)min(staged_row, p.rows - 1u) * p.K + k0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float *from = xr + min(8u * t + 1024u * c, kn - 8u);
+            raw[c][0] = *reinterpret_cast<const float4 *>(from), raw[c][1] = *reinterpret_cast<const float4 *>(from + 4);
+        }
+        if (p.norm_w) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float *from = p.norm_w + k0 + min(8u * t + 1024u * c, kn - 8u);
+                gain[c][0] = *reinterpret_cast<const float4 *>(from), gain[c][1] = *reinterpret_cast<const float4 *>(from + 4);
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the first super-blocks of the weights are asked for behind them, before the activations become halves: their way from
+    // memory is covered by that work (a wave's loads come back in order, so the activations are not kept waiting).  The staging
+    // is latency, not arithmetic: with half its instructions (packed conversions, sums by dot products) a step of eight planes
+    // took the same time
+    const uint32_t n = lane & 15u, kq = lane >> 4;
+    const uint32_t ts = wave / KS, ks = wave % KS;
+    const uint32_t count = ks < nb ? (nb - ks + KS - 1u) / KS : 0u;  // super-blocks ks, ks + KS, ...
+    const uint32_t last_step = count ? count - 1u : 0u;
+    const uint8_t *const w0 = p.W[0], *const w1 = p.W[1], *const w2 = p.W[2];
+    const uint32_t end0 = p.end[0], end1 = p.end[1];
+    const bool gated = p.swiglu != 0;
+    const half2_t offset = {(_Float16)1024.0f, (_Float16)1024.0f}, powers = {(_Float16)1024.0f, (_Float16)64.0f};
+    const uint32_t shift = 16u * (kq >> 1);  // the group's pair of 6-bit fields inside its scale words
+    // Rounds of tiles: in round i the workgroup's tile slot ts takes tile (blockIdx.x + i * gridDim.x) * TPW + ts.  A wave's loads
+    // run two super-blocks ahead across rounds (the first blocks of the next tile are on their way while this tile's sums meet),
+    // and every fetch issues its three loads: past the last round the last block again, dropped.
+    const uint32_t rounds = (p.tiles > blockIdx.x * TPW) ? (p.tiles - blockIdx.x * TPW + gridDim.x * TPW - 1u) / (gridDim.x * TPW) : 0u;
+    const uint32_t first_round = blockIdx.x, hop = gridDim.x, tiles = p.tiles, row_bytes = p.row_bytes;
+    auto tile_of = [first_round, hop, ts](uint32_t round) __attribute__((always_inline)) -> uint32_t { return (first_round + round * hop) * TPW + ts; };
+    // written with selects over scalars captured by value: nothing here may end up indexed
+    const int64_t to_w1 = w1 - w0, to_w2 = w2 - w0;
+    auto row_of = [w0, to_w1, to_w2, end0, end1, gated, n, tiles, row_bytes, blk0, tile_of](uint32_t round) __attribute__((always_inline)) -> const uint8_t * {
+        const uint32_t at_tile = min(tile_of(round), tiles - 1u);
+        const uint32_t r0 = at_tile * 16u;
+        const bool in0 = r0 < end0, in1 = r0 < end1;
+        const int64_t offset = gated ? (n < 8u ? (int64_t)0 : to_w1) + (int64_t)(at_tile * 8u + (n & 7u)) * row_bytes
+                                     : (in0 ? (int64_t)0 : (in1 ? to_w1 : to_w2)) + (int64_t)(r0 - (in0 ? 0u : (in1 ? end0 : end1)) + n) * row_bytes;
+        return w0 + offset + (size_t)blk0 * 144u;
+    };
+    const uint32_t walked = max(count, 1u);  // a wave with no super-block of its own still keeps the ring's rhythm
+    uint32_t ahead_round = 0, ahead_step = 0;
+    const uint8_t *ahead_row = row_of(0);
+    u32x4 even[3], odd[3];
+    auto fetch = [&](u32x4 (&ahead)[3]) __attribute__((always_inline)) {
+        const uint8_t *block = ahead_row + (size_t)min(ks + KS * min(ahead_step, last_step), nb - 1u) * 144u;
+        ahead[0] = *(global_uint4)(uintptr_t)block;
+        ahead[1] = *(global_uint4)(uintptr_t)(block + 16u + 16u * kq);
+        ahead[2] = *(global_uint4)(uintptr_t)(block + 80u + 16u * kq);
+        if (++ahead_step >= walked) {
+            ahead_step = 0;
+            if (ahead_round + 1u < rounds) ahead_row = row_of(++ahead_round);
+        }
+    };
+    fetch(even);
+    fetch(odd);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- activations -> half planes in operand order
+    {
+        const uint32_t r = staged_row;
         float v[4][8];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const uint32_t k = 8u * t + 1024u * c;
-            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-            if (real && k < kn) a = *reinterpret_cast<const float4 *>(xr + k), b = *reinterpret_cast<const float4 *>(xr + k + 4u);
+            const bool held = real && 8u * t + 1024u * c < kn;
+            const float4 a = held ? raw[c][0] : make_float4(0.f, 0.f, 0.f, 0.f), b = held ? raw[c][1] : make_float4(0.f, 0.f, 0.f, 0.f);
             v[c][0] = a.x, v[c][1] = a.y, v[c][2] = a.z, v[c][3] = a.w, v[c][4] = b.x, v[c][5] = b.y, v[c][6] = b.z, v[c][7] = b.w;
         }
         if (p.norm_w) {  // one slice holds the whole row (the launcher sees to it)
@@ -1881,9 +1986,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_q4k_f16_kernel(MFMA_LEAD_PARAMET
             const float rms = rms_scale_of(red[2u * r] + red[2u * r + 1u], p.K, p.eps);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const uint32_t k = 8u * t + 1024u * c;
-                float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-                if (k < kn) a = *reinterpret_cast<const float4 *>(p.norm_w + k0 + k), b = *reinterpret_cast<const float4 *>(p.norm_w + k0 + k + 4u);
+                const float4 a = gain[c][0], b = gain[c][1];
                 const float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
                 for (int i = 0; i < 8; i++) v[c][i] = __fmul_rn(__fmul_rn(v[c][i], rms), w[i]);
@@ -1943,46 +2046,6 @@ __global__ __launch_bounds__(NW * 64) void gemv_q4k_f16_kernel(MFMA_LEAD_PARAMET
     }
     __syncthreads();
 
-    // ---- tiles of 16 weight rows
-    const uint32_t n = lane & 15u, kq = lane >> 4;
-    const uint32_t ts = wave / KS, ks = wave % KS;
-    const uint32_t count = ks < nb ? (nb - ks + KS - 1u) / KS : 0u;  // super-blocks ks, ks + KS, ...
-    const uint32_t last_step = count ? count - 1u : 0u;
-    const uint8_t *const w0 = p.W[0], *const w1 = p.W[1], *const w2 = p.W[2];
-    const uint32_t end0 = p.end[0], end1 = p.end[1];
-    const bool gated = p.swiglu != 0;
-    const half2_t offset = {(_Float16)1024.0f, (_Float16)1024.0f}, powers = {(_Float16)1024.0f, (_Float16)64.0f};
-    const uint32_t shift = 16u * (kq >> 1);  // the group's pair of 6-bit fields inside its scale words
-    // Rounds of tiles: in round i the workgroup's tile slot ts takes tile (blockIdx.x + i * gridDim.x) * TPW + ts.  A wave's loads
-    // run two super-blocks ahead across rounds (the first blocks of the next tile are on their way while this tile's sums meet),
-    // and every fetch issues its three loads: past the last round the last block again, dropped.
-    const uint32_t rounds = (p.tiles > blockIdx.x * TPW) ? (p.tiles - blockIdx.x * TPW + gridDim.x * TPW - 1u) / (gridDim.x * TPW) : 0u;
-    const uint32_t first_round = blockIdx.x, hop = gridDim.x, tiles = p.tiles, row_bytes = p.row_bytes;
-    auto tile_of = [first_round, hop, ts](uint32_t round) __attribute__((always_inline)) -> uint32_t { return (first_round + round * hop) * TPW + ts; };
-    // written with selects over scalars captured by value: nothing here may end up indexed
-    const int64_t to_w1 = w1 - w0, to_w2 = w2 - w0;
-    auto row_of = [w0, to_w1, to_w2, end0, end1, gated, n, tiles, row_bytes, blk0, tile_of](uint32_t round) __attribute__((always_inline)) -> const uint8_t * {
-        const uint32_t at_tile = min(tile_of(round), tiles - 1u);
-        const uint32_t r0 = at_tile * 16u;
-        const bool in0 = r0 < end0, in1 = r0 < end1;
-        const int64_t offset = gated ? (n < 8u ? (int64_t)0 : to_w1) + (int64_t)(at_tile * 8u + (n & 7u)) * row_bytes
-                                     : (in0 ? (int64_t)0 : (in1 ? to_w1 : to_w2)) + (int64_t)(r0 - (in0 ? 0u : (in1 ? end0 : end1)) + n) * row_bytes;
-        return w0 + offset + (size_t)blk0 * 144u;
-    };
-    const uint32_t walked = max(count, 1u);  // a wave with no super-block of its own still keeps the ring's rhythm
-    uint32_t ahead_round = 0, ahead_step = 0;
-    const uint8_t *ahead_row = row_of(0);
-    u32x4 even[3], odd[3];
-    auto fetch = [&](u32x4 (&ahead)[3]) __attribute__((always_inline)) {
-        const uint8_t *block = ahead_row + (size_t)min(ks + KS * min(ahead_step, last_step), nb - 1u) * 144u;
-        ahead[0] = *(global_uint4)(uintptr_t)block;
-        ahead[1] = *(global_uint4)(uintptr_t)(block + 16u + 16u * kq);
-        ahead[2] = *(global_uint4)(uintptr_t)(block + 80u + 16u * kq);
-        if (++ahead_step >= walked) {
-            ahead_step = 0;
-            if (ahead_round + 1u < rounds) ahead_row = row_of(++ahead_round);
-        }
-    };
     // Two sets of partial sums where the operands leave room (up to fourteen super-blocks staged: what the launcher asked LDS
     // for says so): a tile's parts are read while the next tile's are written, and no wave waits for the readers.  Sixteen
     // super-blocks of operands leave room for one set, and a barrier behind the readers.
@@ -2091,8 +2154,6 @@ __global__ __launch_bounds__(NW * 64) void gemv_q4k_f16_kernel(MFMA_LEAD_PARAMET
 #pragma unroll
             for (int e = 0; e < 4; e++) acc[e] = 0.0f;
         };
-        fetch(even);
-        fetch(odd);
         // every wave walks whole pairs of steps; a tile ends wherever its last step falls, and the steps past the last round
         // multiply what was fetched again and publish nothing
         uint32_t round = 0, step = 0;

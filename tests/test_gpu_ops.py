@@ -267,6 +267,22 @@ def test_q4_k_product_on_32_row_tiles(device, monkeypatch, forced, N, K, rows):
     assert not np.isfinite(device.gemv(NH_Q4_K, raw, N, K, x)[0]).any()
 
 
+@pytest.mark.parametrize("N,K,rows", [(40032, 1280, 2), (40032, 768, 8), (40032, 1280, 5)])
+@pytest.mark.parametrize("forced", ["NEURA_HIP_MFMA32", "NEURA_HIP_F16_TILES"])
+def test_tiles_follow_tiles_in_a_wave(device, monkeypatch, forced, N, K, rows):
+    """1251 tiles of 32 rows (2502 of 16) are several rounds of every workgroup, the last one ragged: a wave asks for the first
+    super-block of its next tile while it multiplies the last of this one, also where a tile has fewer super-blocks than waves.
+    The last rows of
+    weights give what they give in a matrix of one round, within the bar that both keep of the oracle."""
+    monkeypatch.setenv(forced, "2")
+    rng = np.random.default_rng(N + K + rows)
+    raw = synth.q4_k_random(rng, N * K)
+    x = (rng.standard_normal((rows, K)) * np.exp(rng.uniform(-2, 2, (rows, K)))).astype(np.float32)
+    got = device.gemv(NH_Q4_K, raw, N, K, x)
+    close(got, oracle.gemv(NH_Q4_K, raw, N, K, x, threads=8))
+    close(device.gemv(NH_Q4_K, raw[(N - 64) * (K // 256) * 144 :], 64, K, x), got[:, N - 64 :])
+
+
 @pytest.mark.parametrize("tile16", ["1", "0"])
 @pytest.mark.parametrize("N,K", [(16, 256), (64, 3584), (4608, 3584), (3584, 18944), (37888, 3584), (1040, 768), (48, 2048), (272, 8960), (2048, 1536),
                                  (17920, 1536), (1536, 1280)])
