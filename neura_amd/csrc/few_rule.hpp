@@ -25,7 +25,8 @@ inline uint32_t few_row_tiles(uint32_t N, uint32_t rows, uint32_t compute_units)
 // 128 to 8192 packed rows over the 0.5B, 1.5B and 7B shapes (us, tiles / few): Q8_0 18944 x 3584 at 512 rows 157 / 211 and at 1024 262 /
 // 331 (full rounds), 3584 x 3584 at 512 56 / 48 (112 workgroups), 4608 x 3584 at 1024 105 / 87 (288), 4864 x 896 at 1024 47 / 35 (304);
 // Q6_K 221 / 193, 80 / 47, 151 / 96 of the first, third and fourth; Q3_K 155 / 140, 57 / 39, 107 / 71; Q5_K 141 / 150, 51 / 40, 95 / 76; Q4_K
-// 125 / 148, 43 / 39, 82 / 77.  The form it picks is within 8 % of the faster one at those points.
+// 125 / 148, 43 / 39, 82 / 77.  The form it picks is within 8 % of the faster one at those points.  (Q6_K and Q3_K have no tiles since rows
+// are shared below: past their line shared rows serve them, gate at 1024 rows 360 -> 252 and 259 -> 190 us.)
 inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
     if (rows <= 96u) return true;
     if (rows > 65535u * 32u) return false;  // (row tiles are blockIdx.y)

@@ -2629,9 +2629,9 @@ static int32_t launch_mfma32(nh_device *d, const GemvArgs &a) {
 
 // whether the half-precision tile kernel serves this product: NEURA_HIP_F16_TILES = 0 never, 2 wherever it can (two to eight
 // activation rows), 1 (default) where it measured faster than the integer tiles on the 7B shapes -- five to eight rows
-// against a matrix of enough tiles to give every wave several super-blocks (gate|up 36.6 against 42 us, the head 91 against
-// 110, ffn_down 29 against 27 with its fold; q|k|v and the output projection, one super-block a wave, are slower: 16.2 and
-// 12.5 against 11.4 and 11.2)
+// against a matrix of enough tiles to give every wave several super-blocks (eight rows, integer tiles / these: gate|up 36.6 / 25.8 us;
+// ffn_down with its fold 23.2 / 25.5; q|k|v 10.8 / 13.5 and attn_output 10.3 / 12.5, one tile a workgroup: every workgroup stages
+// all rows, and these tiles are twice as many)
 static size_t f16_tiles_lds(uint32_t blocks, uint32_t NW) {
     return (size_t)blocks * F16_BLOCK_PIECES * 16u + (size_t)(blocks <= F16_TWO_SETS_BLOCKS ? 2u : 1u) * NW * 4u * 64u * sizeof(float);
 }
