@@ -179,8 +179,7 @@ __device__ __forceinline__ void pack_piece(const _Float16 (&pieces)[PIECES][4], 
 #pragma unroll
         for (int j = 0; j < PIECES; j++) {
             // (a sum of 32 is longer than 22 bits, and the minimums' part largely cancels: what a row's sum drops goes into the next's)
-            constexpr float down = FEW ? 0.0009765625f : 0.015625f;
-            const float v = j ? fmaf(sums[j], down, left) : sums[j] * down;
+            const float v = j ? fmaf(sums[j], 0.015625f, left) : sums[j] * 0.015625f;
             const _Float16 h = (_Float16)v;
             const float rest = (v - (float)h) * 2048.0f;
             const _Float16 residue = (_Float16)rest;
@@ -270,16 +269,10 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         }
         return v;
     };
-    if (!HALF_IN || FEW) {
+    if (!HALF_IN) {
         uint32_t top = 0;
         for (uint32_t k = tid * 4u; k < K; k += 1024u) {
-            float4 v;
-            if constexpr (HALF_IN) {
-                const half4_t held = *reinterpret_cast<const half4_t *>(static_cast<const _Float16 *>(X) + (size_t)m * K + k);
-                v = float4{(float)held[0], (float)held[1], (float)held[2], (float)held[3]};
-            } else {
-                v = fetch(k);
-            }
+            const float4 v = fetch(k);
             top = max(max(top, magnitude<WHOLE>(v.x)), magnitude<WHOLE>(v.y));
             top = max(max(top, magnitude<WHOLE>(v.z)), magnitude<WHOLE>(v.w));
         }
@@ -293,7 +286,6 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         const uint32_t raw = top >> 23, exponent = min(max(raw, 27u), 254u);
         scale = __builtin_bit_cast(float, (267u - exponent) << 23);
         back = raw == 255u ? __builtin_bit_cast(float, 0x7fc00000u) : __builtin_bit_cast(float, (exponent - 13u) << 23);
-        if (HALF_IN && raw == 255u) scale = back = 1.0f;  // (infinities stay)
         if (!WHOLE && tid == 0) unscale[m] = back;
     }
     if constexpr (WHOLE) {
@@ -305,7 +297,7 @@ __global__ __launch_bounds__(256) void gemm_pack_rows_kernel(const void *__restr
         if (HALF_IN) {
             const half4_t v = *reinterpret_cast<const half4_t *>(static_cast<const _Float16 *>(X) + (size_t)m * K + k);
 #pragma unroll
-            for (int e = 0; e < 4; e++) pieces[0][e] = FEW ? (_Float16)((float)v[e] * scale) : v[e];  // (exact: the scale only frees the sums of subnormal halves)
+            for (int e = 0; e < 4; e++) pieces[0][e] = v[e];
         } else {
             const float4 v = fetch(k);
             const float held[4] = {v.x, v.y, v.z, v.w};

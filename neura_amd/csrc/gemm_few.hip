@@ -350,10 +350,7 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float unscale = p.unscale[min(row + e, p.M - 1u)];
-                leave(row + e, n, v[0][e] * unscale, v[NT - 1][e] * unscale);
-            }
+            for (int e = 0; e < 4; e++) leave(row + e, n, v[0][e], v[NT - 1][e]);
         }
     }
 }

@@ -81,8 +81,8 @@ struct FewQ45 {
         return some | (some - (some >> 7));
     }
     __device__ __forceinline__ float scale() const { return (float)as_halves(header.x).x * 16384.0f; }  // operands are code * sc * 2^-14
-    __device__ __forceinline__ float floor_scale() const { return (float)as_halves(header.x).y * -1024.0f; }  // the sums are packed / 1024
-    __device__ __forceinline__ float centre_scale() const { return (float)as_halves(header.x).x * (1024.0f * CENTRE); }
+    __device__ __forceinline__ float floor_scale() const { return (float)as_halves(header.x).y * -64.0f; }  // the sums are packed / 64
+    __device__ __forceinline__ float centre_scale() const { return (float)as_halves(header.x).x * (64.0f * CENTRE); }
     // the eight minimums (`scales`: the eight scales where the codes are centred) as halves; k 8..15 meet the sums' residues * 2^11
     __device__ __forceinline__ half8_t floors(uint32_t part, bool scales) const {
         const half2_t offset = {(_Float16)1024.0f, (_Float16)1024.0f};
@@ -96,8 +96,8 @@ struct FewQ45 {
         const half2_t downs = {down, down};
         return __builtin_bit_cast(half8_t, u32x4{as_word(m[0] * downs), as_word(m[1] * downs), as_word(m[2] * downs), as_word(m[3] * downs)});
     }
-    // The minimums, and what centring took off, in units of the operands: (CENTRE * sc - dmin / d * m) / 16, in two pieces, to meet the
-    // sums (packed / 1024) where the operands meet the activations: ratio() first, then merged() for either four sub-blocks.  False
+    // The minimums, and what centring took off, in units of the operands: (CENTRE * sc - dmin / d * m) / 256, in two pieces, to meet the
+    // sums (packed / 64) where the operands meet the activations: ratio() first, then merged() for either four sub-blocks.  False
     // where the ratio fits no half (d zero, say): the pieces are zero then and the block's floors() go the long way.
     float down, up;
     __device__ __forceinline__ bool ratio(const u32x4 &header) {
@@ -105,7 +105,7 @@ struct FewQ45 {
         const float inverse = __builtin_amdgcn_rcpf(d);
         const float near = dmin * inverse, ratio = dmin == 0.0f ? 0.0f : fmaf(fmaf(-near, d, dmin), inverse, near);
         const bool fits = fabsf(ratio) <= 8192.0f;
-        down = fits ? ratio * -0.0625f : 0.0f, up = fits ? CENTRE * 0.0625f : 0.0f;
+        down = fits ? ratio * -0.00390625f : 0.0f, up = fits ? CENTRE * 0.00390625f : 0.0f;
         return fits;
     }
     __device__ __forceinline__ void merged(const u32x4 &header, uint32_t part, int four, half8_t &coarse, half8_t &fine) const {

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) scales[i][q][e] = p.unscale[min(((tile0 + i) * 32u + 8u * q + 4u * part + e) / pieces, p.M - 1u)];
+            for (int e = 0; e < 4; e++) scales[i][q][e] = pieces == 2u ? p.unscale[min((tile0 + i) * 16u + 4u * q + 2u * part + e / 2, p.M - 1u)] : 1.0f;  // (halves are packed as they lie)
 #pragma unroll
     for (int i = 0; i < MT; i++) {
         float beside[4][4];

@@ -674,6 +674,25 @@ def test_wide_products_of_shared_rows(device, monkeypatch, shape, element, M, N,
     assert np.array_equal(bad[rest], got[rest])
 
 
+@pytest.mark.parametrize("form,M", [("few", 9), ("few", 40), ("42", 70), ("84", 130)])
+def test_half_activations_keep_their_bits_beside_a_large_one(device, monkeypatch, form, M):
+    """Half activations take part as they lie, down to the smallest normal halves, also where a number near the largest half
+    meets a zero weight: Q8_0, whose codes and halves are exact operands, within the bar of exact products in fp32 sums."""
+    if form != "few":
+        monkeypatch.setenv("NEURA_HIP_GEMM_WIDE", form)
+    N, K = 96, 512
+    rng = np.random.default_rng(M)
+    raw = np.array(synth.q8_0_random(rng, N * K), dtype=np.uint8)
+    raw.reshape(N, K // 32, 34)[:, 3, 2 + 7] = 0
+    X = (rng.standard_normal((M, K)) * 2.0 ** -13).astype(np.float16)
+    X[:, 3 * 32 + 7] = 40000.0
+    weights = oracle.unpack(NH_Q8_0, raw, N * K).reshape(N, K).astype(np.float64)
+    assert (weights[:, 3 * 32 + 7] == 0).all()
+    exact = X.astype(np.float64) @ weights.T
+    scale = np.sqrt((X.astype(np.float64) ** 2) @ (weights.T ** 2))
+    assert (np.abs(device.gemm(NH_Q8_0, raw, N, K, X) - exact) <= 4e-6 * scale).all()
+
+
 @pytest.mark.parametrize("element,M,N,K", [
     (NH_Q4_K, 8, 96, 8960), (NH_Q4_K, 48, 33, 18944), (NH_Q5_K, 5, 160, 4608), (NH_Q5_K, 17, 64, 2560), (NH_Q6_K, 16, 130, 8960), (NH_Q3_K, 3, 32, 18944),
     (NH_Q3_K, 100, 96, 8960), (NH_Q8_0, 9, 77, 4864), (NH_Q8_0, 33, 256, 8960), (NH_Q8_0, 2, 31, 18944)])
