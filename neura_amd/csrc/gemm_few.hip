@@ -192,8 +192,8 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(FewParams p) {
             if constexpr (Weights::FLOORS) {
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    const half8_t b = w[t].floors(part, false), c = w[t].floors(part, true);
-                    const float floor_scale = w[t].floor_scale(), centre_scale = w[t].centre_scale();
+                    const half8_t b = w[t].floors(w[t].header, part, false), c = w[t].floors(w[t].header, part, true);
+                    const float floor_scale = w[t].floor_scale(w[t].header), centre_scale = w[t].centre_scale(w[t].header);
 #pragma unroll
                     for (int i = 0; i < MT; i++) {
                         const f32x16 floors = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], b, zero, 0, 0, 0);

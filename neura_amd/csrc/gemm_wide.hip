@@ -93,7 +93,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
 #pragma unroll
     for (uint32_t i = 0; i <= COPIES; i++) put_piece(0, 0, i), fetch_piece(1u, i);
     __syncthreads();
-    bool unfit = false;
+    bool unfit = false;  // a block whose minimums meet no sums among the products (ratio)
     half8_t a[2][MT], b[2][PLANES], coarse, fine, sums[MT];
     auto read_rows = [&](int into, int r) {
 #pragma unroll
@@ -104,17 +104,10 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
         for (int i = 0; i < MT; i++) sums[i] = *reinterpret_cast<const half8_t *>(sums_lds + (unit & 1u) * (MT * 1024u) + i * 1024u + lane * 16u);
     };
     auto floors = [&](int i) {
-        tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], coarse, zero, 0, 0, 0);
+        tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], coarse, tmp[i], 0, 0, 0);
         tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], fine, tmp[i], 0, 0, 0);
     };
     read_rows(0, 0);
-    if constexpr (FLOORS) {
-        unfit |= !w.ratio(w.header);
-        w.merged(w.header, part, 0, coarse, fine), w.merged(w.header, part, 1, coarse, fine);
-        read_sums(0);
-#pragma unroll
-        for (int i = 0; i < MT; i++) floors(i);
-    }
     ready(w, 0);
     w.step(0);
     w.operand(0, 0, b[0]);
@@ -128,7 +121,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
 #pragma unroll
             for (int r = 0; r < REGIONS; r++) {
                 const int g = h * HALF + r / 4, depth = r & 3, cur = r & 1, nxt = cur ^ 1;
-                const bool last = r == REGIONS - 1, first = BLOCKS ? (depth & 1) == 0 : !FLOORS && g % CLOSED == 0 && depth == 0, end = h == 1 && last;
+                const bool last = r == REGIONS - 1, first = BLOCKS ? (depth & 1) == 0 : g % CLOSED == 0 && depth == 0, end = h == 1 && last;
                 const bool close = BLOCKS ? (depth & 1) == 1 : (g + 1) % CLOSED == 0 && depth == 3;
                 __builtin_amdgcn_sched_barrier(0);
                 if (last) {
@@ -139,11 +132,18 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 read_rows(nxt, last ? 0 : r + 1);
-                if (FLOORS && end) read_sums(unit + 1u);
+                if (FLOORS && end) read_sums(unit);
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
                     tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[cur][i], b[cur][0], first ? zero : tmp[i], 0, 0, 0);
                     if (PLANES > 1) tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[cur][i], b[cur][PLANES - 1], tmp[i], 0, 0, 0);
+                }
+                // (the minimums last: what they outweigh, where they do, meets them once and not at every product)
+                if constexpr (FLOORS) {
+                    if (end) {
+#pragma unroll
+                        for (int i = 0; i < MT; i++) floors(i);
+                    }
                 }
                 float scale;
                 if constexpr (BLOCKS) scale = w.block_scale(2 * g + (depth >> 1));
@@ -156,8 +156,8 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
                 if (depth == 3) w.step(of);
                 w.operand(of, (depth + 1) & 3, b[nxt]);
                 if constexpr (FLOORS) {
-                    if (h == 1 && r == 3) unfit |= !w.ratio(w.header_ahead);
-                    if (h == 1 && (r == 4 || r == 5)) w.merged(w.header_ahead, part, r - 4, coarse, fine);
+                    if (h == 1 && r == 4) unfit = !w.ratio(w.header);
+                    if (h == 1 && (r == 5 || r == 6)) w.merged(w.header, part, r - 5, coarse, fine);
                 }
                 if (!last) {
 #pragma unroll
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
                 if (FLOORS && end) __builtin_amdgcn_sched_group_barrier(0x100, 2 * MT, 0);
                 else __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
 #pragma unroll
-                for (int i = 0; i < MT * PLANES; i++) {
+                for (int i = 0; i < (FLOORS && end ? MT * 3 : MT * PLANES); i++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
                 }
@@ -183,33 +183,27 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
 #pragma unroll
                         for (int e = 0; e < 16; e++) acc[i][e] = fmaf(scale, tmp[i][e], acc[i][e]);
                         asm volatile("" : "+v"(acc[i]));  // (here, not behind the products below: their sums are these registers)
-                        if constexpr (FLOORS) floors(i);
+                    }
+                }
+                if constexpr (FLOORS) {
+                    if (end && __any(unfit)) {  // (few blocks: minimums and centres each in products of their own)
+                        const u32x4 closed = __builtin_amdgcn_raw_buffer_load_b128(weights_at, woff, unit * Weights::BYTES, 0);
+                        read_sums(unit);
+                        const half8_t low = Weights::floors(closed, part, false), centre = Weights::floors(closed, part, true);
+                        const float low_scale = unfit ? Weights::floor_scale(closed) : 0.0f, centre_scale = unfit ? Weights::centre_scale(closed) : 0.0f;
+#pragma unroll
+                        for (int i = 0; i < MT; i++) {
+                            const f32x16 lows = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], low, zero, 0, 0, 0);
+                            const f32x16 centres = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], centre, zero, 0, 0, 0);
+#pragma unroll
+                            for (int e = 0; e < 16; e++) acc[i][e] += fmaf(low_scale, lows[e], centre_scale * centres[e]);
+                        }
                     }
                 }
             }
         }
     }
     __builtin_amdgcn_s_setprio(0);
-
-    if constexpr (FLOORS) {
-        // blocks whose minimums met no sums above (ratio)
-        if (__any(unfit)) {
-            for (uint32_t unit = 0; unit < units; unit++) {
-                w.fetch(wbase + woff, unit, steps, part);
-                const bool fits = w.ratio(w.header);
-                const half8_t low = w.floors(part, false), centre = w.floors(part, true);
-                const float low_scale = fits ? 0.0f : w.floor_scale(), centre_scale = fits ? 0.0f : w.centre_scale();
-#pragma unroll
-                for (int i = 0; i < MT; i++) {
-                    const half8_t own = __builtin_bit_cast(half8_t, *(global_uint4)(uintptr_t)(p.S + ((size_t)min(tile0 + i, last_tile) * nsb + unit) * 512u + lane * 8u));
-                    const f32x16 lows = __builtin_amdgcn_mfma_f32_32x32x16_f16(own, low, zero, 0, 0, 0);
-                    const f32x16 centres = __builtin_amdgcn_mfma_f32_32x32x16_f16(own, centre, zero, 0, 0, 0);
-#pragma unroll
-                    for (int e = 0; e < 16; e++) acc[i][e] += fmaf(low_scale, lows[e], centre_scale * centres[e]);
-                }
-            }
-        }
-    }
 
     // ---- out: lane (l32, part) holds column l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
     const uint32_t n = n0 + l32;

@@ -674,6 +674,30 @@ def test_wide_products_of_shared_rows(device, monkeypatch, shape, element, M, N,
     assert np.array_equal(bad[rest], got[rest])
 
 
+@pytest.mark.parametrize("shape", ["42", "84"])
+@pytest.mark.parametrize("element", [NH_Q4_K, NH_Q5_K])
+@pytest.mark.parametrize("ratio", [1.0, 8.0, 30.0, 63.0, 200.0, 5000.0])
+def test_minimums_of_shared_rows_are_as_exact_as_those_of_the_tiles(device, monkeypatch, shape, element, ratio):
+    """Minimums beside scales of every size (dmin / d from 1 to 5000; the blocks of a file lie around half the largest code): the product
+    of shared rows takes them off among its products up to 64 and in products of their own beyond, and is no further from the product
+    in 64 bits (2-norm over 25600 outputs, which two draws of inputs move by 3 %) than the 128 x 128 tiles, which take them off exactly."""
+    M, N, K = 100, 256, 3584
+    rng = np.random.default_rng(int(ratio) + element)
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    blocks = raw.reshape(N * K // 256, -1)
+    blocks[:, 0:2] = (rng.uniform(0.75, 1.25, len(blocks)) * 1e-3).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    blocks[:, 2:4] = (ratio * 1e-3 * rng.uniform(0.75, 1.0, len(blocks))).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    exact = X.astype(np.float64) @ oracle.unpack(element, raw, N * K).reshape(N, K).astype(np.float64).T
+    errors = []
+    for wide in (shape, "0"):
+        monkeypatch.setenv("NEURA_HIP_GEMM_WIDE", wide)
+        monkeypatch.setenv("NEURA_HIP_GEMM_FEW", "0")
+        errors.append(np.linalg.norm(device.gemm(element, raw, N, K, X) - exact) / np.linalg.norm(exact))
+    print("2-norm: shared rows %.3g, tiles %.3g" % tuple(errors))
+    assert errors[0] <= 1.1 * errors[1]
+
+
 @pytest.mark.parametrize("form,M", [("few", 9), ("few", 40), ("42", 70), ("84", 130)])
 def test_half_activations_keep_their_bits_beside_a_large_one(device, monkeypatch, form, M):
     """Half activations take part as they lie, down to the smallest normal halves, also where a number near the largest half
