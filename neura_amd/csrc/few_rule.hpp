@@ -69,6 +69,17 @@ inline FewSplit few_split(int32_t element, uint32_t N, uint32_t K, uint32_t rows
     return best;
 }
 
+// Units of k a wave of the product of shared rows adds up before its sums leave the accumulators (a chain): as many as a share of the
+// product of few rows has, where that is the form it takes over from, for one chain over all of K adds up less exactly than shares that
+// meet (2-norm from 64 bits, few rows / one chain / here: Q3_K 3584 x 18944 at 600 packed rows 1.15e-7 / 1.75 / 1.16, Q6_K at 800 1.56 /
+// 2.41 / 1.56, Q5_K at 600 1.56 / 1.99 / 1.49, Q8_0 17920 x 1536 at 200 1.10 / 1.38 / 1.10).  The tiles are one chain themselves.
+inline uint32_t shared_rows_chain(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
+    const uint32_t steps = element == NH_Q8_0 ? 2u : 4u, units = (K / 64u + steps - 1u) / steps;
+    if (!few_rows_win(element, N, K, rows, compute_units)) return units;
+    const FewSplit split = few_split(element, N, K, rows, few_row_tiles(N, rows, compute_units), 1u, compute_units);
+    return (units + split.deep * split.slices - 1u) / (split.deep * split.slices);
+}
+
 // Where the product of shared rows (gemm_wide.hip) takes over, and in which shape: waves side by side and row tiles a wave (none: the form
 // that few_rows_win picks).  Times in microseconds of all three, each a line fitted to 649 products of the decoder shapes at 20 to
 // 1024 packed rows (mean error 4 % here, 4 % of the tiles, 7 % of the product of few rows): turns of the chip, a base and the units
@@ -102,13 +113,17 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
     }
     SharedShape best = SHARED_NONE;
     double least = other / 1.08;
+    // places between chains, and the end: two microseconds a turn where the sums go through memory (4608 x 3584 Q3_K at 400 packed rows, 42:
+    // 38.4 -> 41.1; 17920 x 1536 Q8_0 at 400 71.9 -> 80.2, two turns; 84: 37888 x 3584 Q3_K at 200 130.0 -> 137.1)
+    const uint32_t chain = shared_rows_chain(element, N, K, rows, compute_units), places = chain < units ? (units - 1u) / chain + 1u : 0u;
     const auto consider = [&](SharedShape shape, uint32_t waves, uint32_t mt, double pair, double one, double base, double turn, double pack) {
         if (!(pair > 0.0)) return;
         const uint64_t workgroups = (uint64_t)((N + 32u * waves - 1u) / (32u * waves)) * ((row_tiles + mt - 1u) / mt), slots = waves == 4u ? 2u * cu : cu;
         const uint64_t full = workgroups / slots, left = workgroups % slots;
         const bool lone = waves == 4u && left && left <= cu;
         const uint64_t turns = full + (left ? 1u : 0u);
-        const double time = base + (double)turns * (turn + units * pair) - (lone ? units * (pair - one) : 0.0) + pack * millions;
+        const bool spare = mt == 3u && !(element == NH_Q6_K && waves == 4u);  // (gemm_wide.hip: registers for them)
+        const double time = base + (double)turns * (turn + units * pair + (spare ? 0.0 : 2.0 * places)) - (lone ? units * (pair - one) : 0.0) + pack * millions;
         if (time < least) least = time, best = shape;
     };
     consider(SHARED_42, 4u, 2u, t.pair2, t.one2, 5.0, 5.5, 1.7);

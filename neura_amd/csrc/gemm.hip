@@ -1076,8 +1076,9 @@ struct WideForm {
     bool operands;
     SharedShape shape;
 };
-static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows) {
-    const int held = env_int("NEURA_HIP_GEMM_WIDE", -1);
+static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, size_t residuals) {
+    // (`residuals`: bytes of outputs whose place holds residuals; the sums of chains then wait in scratch)
+    const int held = residuals > FEW_PARTIAL_BYTES ? 0 : env_int("NEURA_HIP_GEMM_WIDE", -1);
     if (held == SHARED_42 || held == SHARED_43 || held == SHARED_83 || held == SHARED_84) return WideForm{true, (SharedShape)held};
     const uint32_t units = (uint32_t)d->compute_units;
     const SharedShape shape = held == 0 || gemm_few_held() >= 0 ? SHARED_NONE : shared_rows_shape(element, N, K, rows, units);
@@ -1104,7 +1105,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const uint32_t pieces = half_rows ? 1u : a.whole ? WHOLE_PIECES : 2u;
     p.rows = a.whole ? whole_rows(a.M) : pieces * a.M;
     p.split = half_rows ? 0 : 1;
-    const WideForm form = a.whole || a.gated ? WideForm{true, SHARED_NONE} : wide_form(d, a.element, a.N, a.K, p.rows);
+    const WideForm form = a.whole || a.gated ? WideForm{true, SHARED_NONE} : wide_form(d, a.element, a.N, a.K, p.rows, a.residual ? (size_t)a.M * a.N * sizeof(float) : 0u);
     const bool few = form.operands;
     if (a.whole && (half_rows || gemm_few_held() == 0 || a.M > 65535u * WHOLE_TILE))
         return fail(NH_E_ARGUMENT, "this wide product takes no fp32 rows whole (ask gemm_takes_whole first)");
@@ -1128,7 +1129,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     p.A = A, p.S = S, p.unscale = unscale;
     if (few) {
         const FewParams f{p.W, p.W1, p.W2, p.end0, p.end1, p.N, p.K, p.row_bytes, p.A, p.S, p.rows, p.Y, p.residual, p.ldy, p.M, pieces, p.unscale, reinterpret_cast<const WholeRow *>(unscale), outside,
-                          1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets, a.Y_more};
+                          1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets, 0u, a.Y_more};
         return form.shape != SHARED_NONE ? launch_gemm_wide(d, a.element, f, form.shape) : launch_gemm_few(d, a.element, f, a.gated);
     }
     static bool sized = false;
@@ -1185,7 +1186,7 @@ bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const ui
         return true;
     }
     for (int s = 0; s < 3; s++)
-        if (!mfma_takes(elements[s], K, X, W[s]) || wide_form(d, elements[s], N[s], K, 2u * M).operands != wide_form(d, elements[0], N[0], K, 2u * M).operands) return false;
+        if (!mfma_takes(elements[s], K, X, W[s]) || wide_form(d, elements[s], N[s], K, 2u * M, 0u).operands != wide_form(d, elements[0], N[0], K, 2u * M, 0u).operands) return false;
     return true;
 }
 

@@ -17,6 +17,8 @@
 // 1.3e-7 (tiles 2.3e-7: uncentred).
 #include "gemm_operands.hpp"
 
+#include <type_traits>
+
 namespace nh {
 
 namespace {
@@ -107,6 +109,64 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
         tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], coarse, tmp[i], 0, 0, 0);
         tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], fine, tmp[i], 0, 0, 0);
     };
+    // Where a chain of `chain` units ends, its sums leave the accumulators.  (Rows of residues, 2^11 below the rows they belong to, stay
+    // and run on.)  SPARE: three row tiles leave registers for the sums of whole chains.  Elsewhere they go to the outputs' own place
+    // (or to scratch, where that still holds the residuals), each lane the outputs it writes at the end (18944 x 3584 Q3_K at 200
+    // packed rows, two chains of seven units, against one: 83 60.6 -> 59.5 us, 84 64.5 -> 69.0).
+    constexpr bool SPARE = MT == 3 && !(ELEMENT == NH_Q6_K && WN == 4);
+    const uint32_t pieces = p.pieces;
+    float whole[SPARE ? MT : 1][8] = {};
+    auto keep = [&](auto each, bool first, bool leave) __attribute__((always_inline)) {
+        constexpr int EACH = decltype(each)::value;  // every packed row, or every second
+        if constexpr (SPARE && EACH == 2) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    whole[i][e] += acc[i][2 * e];
+                    acc[i][2 * e] = leave ? 0.0f : whole[i][e];
+                }
+            return;
+        }
+        uint32_t seat = lane, ldk = p.residual ? p.N : p.ldy;
+        asm volatile("" : "+v"(seat), "+v"(ldk));  // (worked out here: kept from before the walk, places and addresses would take its registers)
+        const uint32_t column = n0 + (seat & 31u), rows = column < p.N && column0 < p.N ? p.M : 0u, row0 = tile0 * 32u / EACH + 4u / EACH * (seat >> 5);
+        float *const kept = (p.residual ? p.partial : p.Y1 && n0 >= p.end0 ? p.Y1 - p.end0 : p.Y) + column;
+        // (what the chains before left comes in one round trip, of four tiles in two; a place's sums leave before the next one's address
+        // is made)
+        constexpr int TOGETHER = MT == 4 ? 2 : MT;
+#pragma unroll
+        for (int i0 = 0; i0 < MT; i0 += TOGETHER) {
+            float was[TOGETHER][4][4 / EACH];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < TOGETHER; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t m = row0 + (32 * (i0 + i) + 8 * q) / EACH;
+#pragma unroll
+                    for (int e = 0; e < 4 / EACH; e++) was[i][q][e] = !first && m + e < rows ? kept[(size_t)(m + e) * ldk] : 0.0f;
+                }
+#pragma unroll
+            for (int i = 0; i < TOGETHER; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    const uint32_t m = row0 + (32 * (i0 + i) + 8 * q) / EACH;
+#pragma unroll
+                    for (int e = 0; e < 4 / EACH; e++) {
+                        const float sum = was[i][q][e] + acc[i0 + i][4 * q + EACH * e];
+                        if (leave && m + e < rows) kept[(size_t)(m + e) * ldk] = sum;
+                        acc[i0 + i][4 * q + EACH * e] = leave ? 0.0f : sum;
+                    }
+                }
+        }
+    };
+    auto keep_rows = [&](bool first, bool leave) __attribute__((always_inline)) {
+        if (pieces == 2u) keep(std::integral_constant<int, 2>(), first, leave);
+        else keep(std::integral_constant<int, 1>(), first, leave);
+    };
+    uint32_t until = p.chain;
     read_rows(0, 0);
     ready(w, 0);
     w.step(0);
@@ -185,25 +245,36 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
                         asm volatile("" : "+v"(acc[i]));  // (here, not behind the products below: their sums are these registers)
                     }
                 }
-                if constexpr (FLOORS) {
-                    if (end && __any(unfit)) {  // (few blocks: minimums and centres each in products of their own)
-                        const u32x4 closed = __builtin_amdgcn_raw_buffer_load_b128(weights_at, woff, unit * Weights::BYTES, 0);
-                        read_sums(unit);
-                        const half8_t low = Weights::floors(closed, part, false), centre = Weights::floors(closed, part, true);
-                        const float low_scale = unfit ? Weights::floor_scale(closed) : 0.0f, centre_scale = unfit ? Weights::centre_scale(closed) : 0.0f;
+            }
+        }
+        if constexpr (FLOORS) {
+            if (__any(unfit)) {  // (few blocks: minimums and centres each in products of their own)
+                const u32x4 closed = __builtin_amdgcn_raw_buffer_load_b128(weights_at, woff, unit * Weights::BYTES, 0);
+                read_sums(unit);
+                const half8_t low = Weights::floors(closed, part, false), centre = Weights::floors(closed, part, true);
+                const float low_scale = unfit ? Weights::floor_scale(closed) : 0.0f, centre_scale = unfit ? Weights::centre_scale(closed) : 0.0f;
 #pragma unroll
-                        for (int i = 0; i < MT; i++) {
-                            const f32x16 lows = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], low, zero, 0, 0, 0);
-                            const f32x16 centres = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], centre, zero, 0, 0, 0);
+                for (int i = 0; i < MT; i++) {
+                    const f32x16 lows = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], low, zero, 0, 0, 0);
+                    const f32x16 centres = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], centre, zero, 0, 0, 0);
 #pragma unroll
-                            for (int e = 0; e < 16; e++) acc[i][e] += fmaf(low_scale, lows[e], centre_scale * centres[e]);
-                        }
-                    }
+                    for (int e = 0; e < 16; e++) acc[i][e] += fmaf(low_scale, lows[e], centre_scale * centres[e]);
                 }
             }
         }
+        if (unit + 1u == until && until < units) keep_rows(until == p.chain, true), until += p.chain;
     }
     __builtin_amdgcn_s_setprio(0);
+    // (every scale before the first store, and a tile's residuals before its stores: the compiler cannot tell them from the outputs, and
+    // a chain of loads behind stores is a memory latency each, 16 us a workgroup)
+    float scales[MT][4][4];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) scales[i][q][e] = pieces == 2u ? p.unscale[min((tile0 + i) * 16u + 4u * q + 2u * part + e / 2, p.M - 1u)] : 1.0f;  // (halves are packed as they lie)
+    if (p.chain < units) keep_rows(false, false);
 
     // ---- out: lane (l32, part) holds column l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
     const uint32_t n = n0 + l32;
@@ -211,16 +282,6 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
     // (a second matrix with outputs of its own: the up projection beside the gate's)
     float *const Y = p.Y1 && n >= p.end0 ? p.Y1 + (n - p.end0) : p.Y + n;
     const float *const residual = p.residual ? p.residual + n : nullptr;
-    // (every scale before the first store, and a tile's residuals before its stores: the compiler cannot tell them from the outputs, and
-    // a chain of loads behind stores is a memory latency each, 16 us a workgroup)
-    float scales[MT][4][4];
-    const uint32_t pieces = p.pieces;
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) scales[i][q][e] = pieces == 2u ? p.unscale[min((tile0 + i) * 16u + 4u * q + 2u * part + e / 2, p.M - 1u)] : 1.0f;  // (halves are packed as they lie)
 #pragma unroll
     for (int i = 0; i < MT; i++) {
         float beside[4][4];
@@ -245,7 +306,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
 }
 
 template <int ELEMENT, int WN, int MT>
-int32_t launch_shape(nh_device *d, const FewParams &p) {
+int32_t launch_shape(nh_device *d, FewParams p) {
     typedef typename FewOf<ELEMENT>::type Weights;
     constexpr size_t lds = MT * (3u * (Weights::STEPS / 2u) * 4096u + (Weights::FLOORS ? 2048u : 0u));
     static bool sized = false;
@@ -253,6 +314,8 @@ int32_t launch_shape(nh_device *d, const FewParams &p) {
         NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         sized = true;
     }
+    // (beside residuals the chains' sums wait in scratch: more of them than that holds stay in one chain)
+    p.chain = p.residual && (size_t)p.M * p.N * sizeof(float) > FEW_PARTIAL_BYTES ? ~0u : shared_rows_chain(ELEMENT, p.N, p.K, p.rows, (uint32_t)d->compute_units);
     const uint32_t column_tiles = (p.N + 32u * WN - 1u) / (32u * WN), row_blocks = ((p.rows + 31u) / 32u + MT - 1u) / MT;
     hipLaunchKernelGGL((gemm_wide_kernel<ELEMENT, WN, MT>), dim3((column_tiles * row_blocks + 7u) / 8u * 8u), dim3(64 * WN), lds, d->stream, p, column_tiles, row_blocks);
     NH_HIP(hipGetLastError());

@@ -638,7 +638,8 @@ def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, 
 @pytest.mark.parametrize("element,M,N,K,half", [
     (NH_Q4_K, 1, 32, 256, False), (NH_Q4_K, 50, 300, 512, False), (NH_Q4_K, 33, 1056, 1280, False), (NH_Q4_K, 130, 200, 768, True),
     (NH_Q5_K, 65, 130, 512, False), (NH_Q5_K, 97, 290, 256, True), (NH_Q6_K, 50, 300, 512, False), (NH_Q6_K, 33, 100, 768, True), (NH_Q3_K, 49, 270, 512, False),
-    (NH_Q3_K, 129, 64, 768, True), (NH_Q8_0, 50, 300, 192, False), (NH_Q8_0, 97, 270, 64, True), (NH_Q8_0, 33, 130, 4864, False)])
+    (NH_Q3_K, 129, 64, 768, True), (NH_Q8_0, 50, 300, 192, False), (NH_Q8_0, 97, 270, 64, True), (NH_Q8_0, 33, 130, 4864, False),
+    (NH_Q3_K, 70, 100, 4864, True), (NH_Q5_K, 45, 300, 8960, False)])
 def test_wide_products_of_shared_rows(device, monkeypatch, shape, element, M, N, K, half):
     """The wide product whose workgroups share their rows through LDS, each shape of it forced: columns and row tiles past the last, rows
     that end inside a tile, one unit and several, an odd number of Q8_0's steps -- against the exact product at the bar of
@@ -696,6 +697,31 @@ def test_minimums_of_shared_rows_are_as_exact_as_those_of_the_tiles(device, monk
         errors.append(np.linalg.norm(device.gemm(element, raw, N, K, X) - exact) / np.linalg.norm(exact))
     print("2-norm: shared rows %.3g, tiles %.3g" % tuple(errors))
     assert errors[0] <= 1.1 * errors[1]
+
+
+@pytest.mark.parametrize("element,M,N,K", [
+    (NH_Q3_K, 300, 3584, 18944), (NH_Q3_K, 100, 18944, 3584), (NH_Q6_K, 400, 3584, 18944), (NH_Q6_K, 100, 18944, 3584),
+    (NH_Q8_0, 100, 17920, 1536), (NH_Q5_K, 300, 3584, 18944), (NH_Q4_K, 37, 37888, 3584)])
+@pytest.mark.parametrize("half", [False, True])
+def test_the_picked_form_of_a_wide_product_is_as_exact_as_the_product_of_few_rows(device, monkeypatch, half, element, M, N, K):
+    """Sizes at which the product of shared rows takes over from the product of few rows, whose shares of K meet at the end: a chain of
+    sums over all of K would be up to half as far again from the product in 64 bits.  2-norm over M x 256 outputs, which two draws of
+    inputs move by less than 1 %; with residuals, whose place the chains' sums may not take, the same product plus its residual."""
+    rng = np.random.default_rng(M + element)
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    per, size = synth.BLOCK_BYTES[element]
+    weights = oracle.unpack(element, raw[: 256 * K // per * size], 256 * K).reshape(256, K).astype(np.float64)
+    X = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
+    exact = X.astype(np.float64) @ weights.T
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    picked = device.gemm(element, raw, N, K, X)
+    beside = device.gemm(element, raw, N, K, X, residual=r)
+    monkeypatch.setenv("NEURA_HIP_GEMM_FEW", "1")
+    few = device.gemm(element, raw, N, K, X)
+    errors = [np.linalg.norm(y[:, :256] - exact) / np.linalg.norm(exact) for y in (picked, few)]
+    print("2-norm: picked %.3g, few rows %.3g" % tuple(errors))
+    assert errors[0] <= 1.05 * errors[1]
+    assert np.abs(beside.astype(np.float64) - (picked.astype(np.float64) + r)).max() <= 2.0 ** -22 * (np.abs(picked).max() + np.abs(r).max())
 
 
 @pytest.mark.parametrize("form,M", [("few", 9), ("few", 40), ("42", 70), ("84", 130)])
