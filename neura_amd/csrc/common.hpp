@@ -97,6 +97,8 @@ struct nh_device {
 
 namespace nh {
 
+// hipMalloc, with no error left behind for the next launch to report
+hipError_t allocate(void **held, size_t bytes);
 // grows the device scratch to at least `bytes`; returns nullptr on failure (error recorded)
 void *scratch(nh_device *device, size_t bytes);
 // device table of pow(base, -2c/width), c < width/2, computed on the host in fp32

@@ -87,7 +87,7 @@ void release(nh_model *m) {
 template <typename T>
 bool device_array(T *&out, size_t count) {
     void *held = nullptr;
-    if (hipMalloc(&held, (count ? count : 1) * sizeof(T)) != hipSuccess) return false;
+    if (allocate(&held, (count ? count : 1) * sizeof(T)) != hipSuccess) return false;
     out = static_cast<T *>(held);
     return true;
 }
@@ -730,7 +730,7 @@ static int32_t shared_planes(nh_model *m) {
     const size_t bytes = (size_t)m->c.kv_heads * m->capacity * m->c.head_dim * m->eb;
     for (uint32_t L = 0; L < m->c.layers; L++) {
         uint8_t *k = nullptr, *v = nullptr;
-        if (hipMalloc((void **)&k, bytes) != hipSuccess || hipMalloc((void **)&v, bytes) != hipSuccess) {
+        if (allocate((void **)&k, bytes) != hipSuccess || allocate((void **)&v, bytes) != hipSuccess) {
             if (k) (void)hipFree(k);
             return fail(NH_E_MEMORY, "no room for the %zu bytes a shared prefix of layer %u holds", 2 * bytes, L);
         }
@@ -959,7 +959,7 @@ int32_t nh_sample(nh_device *device, const float *dev_logits, uint32_t rows, uin
     if (!rows) return NH_OK;
     // the draws ride in a small buffer of their own: the scratch belongs to the kernels
     nh_draw *draws = nullptr;
-    NH_HIP(hipMalloc((void **)&draws, (size_t)rows * sizeof(nh_draw)));
+    NH_HIP(allocate((void **)&draws, (size_t)rows * sizeof(nh_draw)));
     hipError_t copied = hipMemcpyAsync(draws, host_draws, (size_t)rows * sizeof(nh_draw), hipMemcpyHostToDevice, device->stream);
     if (copied == hipSuccess) status = launch_sample(device, dev_logits, rows, n, draws, dev_out);
     (void)hipStreamSynchronize(device->stream);

@@ -24,6 +24,12 @@ int32_t hip_fail(hipError_t error, const char *what) {
     return fail(NH_E_DEVICE, "%s failed: %s", what, hipGetErrorString(error));
 }
 
+hipError_t allocate(void **held, size_t bytes) {
+    const hipError_t status = hipMalloc(held, bytes);
+    if (status != hipSuccess) (void)hipGetLastError();  // (a launch does not clear it: the next one would be taken for the failure)
+    return status;
+}
+
 void *scratch(nh_device *device, size_t bytes) {
     if (bytes <= device->scratch_bytes) return device->scratch;
     // The block that is outgrown is kept until nh_close: work already queued on the stream, and any recorded
@@ -32,8 +38,10 @@ void *scratch(nh_device *device, size_t bytes) {
     // It grows to at least twice its size, so that all the retired blocks together stay smaller than the live one.
     size_t wanted = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
     if (wanted < 2 * device->scratch_bytes) wanted = 2 * device->scratch_bytes;
+    // NEURA_HIP_SCRATCH_MOST=<bytes>: the device is asked for more than it can hold past that (read at every growth: the tests switch it)
+    const char *const most = getenv("NEURA_HIP_SCRATCH_MOST");
     void *held = nullptr;
-    if (hipMalloc(&held, wanted) != hipSuccess) {
+    if (allocate(&held, most && wanted > strtoull(most, nullptr, 10) ? (size_t)1 << 60 : wanted) != hipSuccess) {
         fail(NH_E_MEMORY, "device %d holds no %zu bytes of scratch", device->index, wanted);
         return nullptr;
     }
@@ -53,7 +61,7 @@ const float *rope_frequencies(nh_device *device, float base, uint32_t width) {
     std::vector<float> table(width / 2);
     for (uint32_t c = 0; c < width / 2; c++) table[c] = powf(base, -2.0f * (float)c / (float)width);
     float *held = nullptr;
-    if (hipMalloc((void **)&held, table.size() * sizeof(float)) != hipSuccess) {
+    if (allocate((void **)&held, table.size() * sizeof(float)) != hipSuccess) {
         fail(NH_E_MEMORY, "device %d holds no rope table of %u channels", device->index, width);
         return nullptr;
     }
@@ -163,7 +171,7 @@ void *nh_alloc(nh_device *device, size_t bytes) {
     }
     void *held = nullptr;
     size_t wanted = bytes ? bytes : 4;
-    if (hipMalloc(&held, wanted) != hipSuccess) {
+    if (allocate(&held, wanted) != hipSuccess) {
         fail(NH_E_MEMORY, "device %d holds no %zu bytes", device->index, wanted);
         return nullptr;
     }
@@ -279,7 +287,7 @@ nh_weights *nh_weights_create(nh_device *device, size_t bytes) {
     }
     // 256 spare bytes so a 16-byte load that starts inside the last block never leaves the arena
     uint8_t *base = nullptr;
-    if (hipMalloc((void **)&base, bytes + 256) != hipSuccess) {
+    if (allocate((void **)&base, bytes + 256) != hipSuccess) {
         fail(NH_E_MEMORY, "device %d holds no arena of %zu bytes", device->index, bytes);
         return nullptr;
     }

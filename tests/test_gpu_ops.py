@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import cases
+import neura_amd
 import oracle
 from neura_amd import NH_Q3_K, NH_Q4_K, NH_Q5_K, NH_Q6_K, NH_Q8_0, NeuraError, synth
 
@@ -1169,6 +1170,30 @@ def test_sections_of_a_fill_walk_meet(device, monkeypatch, sections, element, he
     want = device.attention(q, ck, cv, kv_heads, capacity, keys, origins, scale, reach=reach, element=element)
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.abs(got - want)[~np.isnan(want)].max() <= 1e-5
+
+
+def test_a_device_that_holds_no_more_scratch_walks_a_fill_whole(monkeypatch):
+    """A fill whose sections find no scratch is walked by one workgroup a block, as exactly; a refused allocation is not
+    reported by the launches behind it."""
+    own = neura_amd.Device(0)
+    rng = np.random.default_rng(9)
+    q = rng.standard_normal((4, 1, 20, 128)).astype(np.float32)
+    states = [own.upload(rng.standard_normal((2, 1, 300, 128)).astype(np.float16).view(np.uint16)) for _ in range(2)]
+
+    def walk():
+        return own.attention(q, *states, 2, 300, 300, [280], 128 ** -0.5)
+
+    monkeypatch.setenv("NEURA_HIP_FILL_SECTIONS", "1")
+    whole = walk()
+    monkeypatch.setenv("NEURA_HIP_SCRATCH_MOST", "0")
+    monkeypatch.setenv("NEURA_HIP_FILL_SECTIONS", "4")
+    assert np.array_equal(walk(), whole)
+    with pytest.raises(NeuraError):
+        own.alloc(1 << 60)
+    assert np.array_equal(walk(), whole)
+    monkeypatch.delenv("NEURA_HIP_SCRATCH_MOST")
+    assert np.abs(walk() - whole).max() <= 1e-5
+    own.close()
 
 
 def test_attention_refuses_a_cursor_past_its_keys(device):
