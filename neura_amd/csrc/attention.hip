@@ -32,11 +32,12 @@ struct AttentionParams {
     float scale;
     uint32_t *refusal;
     uint32_t reach;  // 0, or the span of a ring of `keys` slots
+    const uint32_t *plane_sections;  // a fill's sections plane by plane, `sections` of them at most (null: that many in all)
 };
 
 __device__ __forceinline__ void fetch_parameters(const AttentionParams &p) {
     NH_FETCH(p.q, p.out, p.partial, p.q_sh, p.q_sb, p.q_sr, p.o_sh, p.o_sb, p.o_sr, p.cache_k, p.cache_v, p.heads, p.kv_heads, p.groups, p.batch, p.rows,
-             p.capacity, p.keys, p.sections, p.cursor, p.scale, p.refusal, p.reach);
+             p.capacity, p.keys, p.sections, p.cursor, p.scale, p.refusal, p.reach, p.plane_sections);
 }
 
 // A ring cache (Cache::windowed, crates/neura-decoder/src/cache.rs:311-317, :391-394): once `written` positions have gone
@@ -433,8 +434,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     // the workgroup walks up to the last key its last row sees; a ring is walked whole, every slot asked what it holds
     const uint32_t last_row = min(p.rows, block_row + 4u * rows_per_wave) - 1u;
     const uint32_t span = min(p.keys, p.reach ? origin + p.rows : origin + last_row + 1u);
+    const uint32_t sections = p.plane_sections ? p.plane_sections[b] : p.sections;
+    if (blockIdx.z >= sections) return;  // (a plane of fewer sections than another: a whole workgroup)
     // a section of the walk: whole rounds of tiles, the same number for every section of a block (the last ones may be left without)
-    const uint32_t rounds = (span + SETS * TK - 1u) / (SETS * TK), share = (rounds + p.sections - 1u) / p.sections * (SETS * TK);
+    const uint32_t rounds = (span + SETS * TK - 1u) / (SETS * TK), share = (rounds + sections - 1u) / sections * (SETS * TK);
     const uint32_t begin = blockIdx.z * share, stop = min(span, begin + share);
     const uint32_t wave_first = block_row + wave * rows_per_wave;
     // keys below this are seen by every row of the wave (a column that is not held may weigh what it likes: it leaves nothing)
@@ -624,7 +627,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(Atten
     // register 4j + e of block d is channel 32d + 8j + 4h + e of this lane's column
     float normalized = mass > 0.0f ? 1.0f / (mass * 1024.0f) : 0.0f;
     float *dst = p.out + (uint64_t)(kvh * G + g) * p.o_sh + (uint64_t)b * p.o_sb + (uint64_t)row * p.o_sr;
-    if (p.sections > 1u) {
+    if (sections > 1u) {
         // sums, maximum and mass as they stand; the sums of a section no key of which was seen are left out (attention_fill_fold_kernel)
         const uint64_t place = (((uint64_t)(kvh * p.batch + b) * p.rows + row) * p.sections + blockIdx.z) * G + g;
         if (h == 0u) reinterpret_cast<float2 *>(p.partial + (uint64_t)p.kv_heads * p.batch * p.rows * p.sections * G * WIDTH)[place] = float2{top, mass};
@@ -648,12 +651,15 @@ template <int WIDTH>
 __global__ __launch_bounds__(256) void attention_fill_fold_kernel(AttentionParams p) {
     constexpr uint32_t LANES = WIDTH / 4, STRIPES = 64 / LANES;
     static_assert(FILL_SECTIONS_MOST <= 64, "a lane a section");
-    const uint32_t lane = threadIdx.x & 63u, G = p.groups, S = p.sections;
+    const uint32_t lane = threadIdx.x & 63u, G = p.groups;
     const uint32_t count = p.kv_heads * p.batch * p.rows * G, row_head = blockIdx.x * 4u + (threadIdx.x >> 6);
     if (row_head >= count) return;  // (a whole wave: nothing below meets another)
     const uint32_t unit = row_head / G, g = row_head - unit * G;
-    const uint64_t place = (uint64_t)unit * S * G + g;  // of section 0; a section further is G further
-    const float2 held = reinterpret_cast<const float2 *>(p.partial + (uint64_t)count * S * WIDTH)[place + (uint64_t)min(lane, S - 1u) * G];
+    const uint32_t row = unit % p.rows, b = unit / p.rows % p.batch, kvh = unit / p.rows / p.batch;
+    const uint32_t S = p.plane_sections ? p.plane_sections[b] : p.sections;
+    if (S == 1u) return;  // (a plane walked whole has left its outputs)
+    const uint64_t place = (uint64_t)unit * p.sections * G + g;  // of section 0; a section further is G further
+    const float2 held = reinterpret_cast<const float2 *>(p.partial + (uint64_t)count * p.sections * WIDTH)[place + (uint64_t)min(lane, S - 1u) * G];
     const float top = lane < S ? held.x : -INFINITY;
     const bool empty = lane >= S || (held.x == -INFINITY && held.y == 0.0f);
     const float largest = wave_max(top);
@@ -680,7 +686,6 @@ __global__ __launch_bounds__(256) void attention_fill_fold_kernel(AttentionParam
     for (uint32_t hop = LANES; hop < 64u; hop <<= 1)
         sum.x += __shfl_xor(sum.x, (int)hop, 64), sum.y += __shfl_xor(sum.y, (int)hop, 64), sum.z += __shfl_xor(sum.z, (int)hop, 64), sum.w += __shfl_xor(sum.w, (int)hop, 64);
     if (stripe != 0u) return;
-    const uint32_t row = unit % p.rows, b = unit / p.rows % p.batch, kvh = unit / p.rows / p.batch;
     *reinterpret_cast<float4 *>(p.out + (uint64_t)(kvh * G + g) * p.o_sh + (uint64_t)b * p.o_sb + (uint64_t)row * p.o_sr + c) =
         float4{sum.x * normalized, sum.y * normalized, sum.z * normalized, sum.w * normalized};
 }
@@ -1080,6 +1085,20 @@ static uint32_t fill_sections(uint32_t blocks, uint32_t rounds, uint64_t numbers
     return best;
 }
 
+// Two sets of waves a workgroup where the block's walk is long enough to be worth their meeting (four tiles and more);
+// NEURA_HIP_FILL_SPLIT=0 keeps one set
+static bool fill_splits(const AttentionArgs &a) {
+    static const bool wanted = [] { const char *v = getenv("NEURA_HIP_FILL_SPLIT"); return !(v && v[0] == '0'); }();
+    return wanted && a.cache_element != NH_F32 && a.keys >= 128u;
+}
+
+uint32_t attention_fill_sections(const nh_device *d, const AttentionArgs &a, uint32_t positions) {
+    const uint32_t groups = a.heads / a.kv_heads;
+    if (!groups || groups > (uint32_t)MAX_GROUPS || !a.rows) return 1u;  // (no fill's: launch_attention)
+    const uint32_t block_rows = 4u * (32u / groups), blocks = a.kv_heads * a.batch * ((a.rows + block_rows - 1u) / block_rows), round = fill_splits(a) ? 64u : 32u;
+    return fill_sections(blocks, (min(positions, a.keys) + round - 1u) / round, (uint64_t)a.heads * a.batch * a.rows * a.width, a.width, (uint32_t)d->compute_units);
+}
+
 template <int WIDTH, int CE, bool SPLIT>
 static int32_t launch_fill(nh_device *d, const AttentionParams &p, dim3 grid, uint32_t rows_per_wave) {
     constexpr size_t lds = fill_lds_bytes(WIDTH, CE, SPLIT);
@@ -1141,16 +1160,12 @@ int32_t launch_attention(nh_device *d, const AttentionArgs &a) {
     if (fill_tiles) {
         const uint32_t rows_per_wave = 32u / p.groups;
         dim3 grid(a.kv_heads * a.batch, (a.rows + 4u * rows_per_wave - 1u) / (4u * rows_per_wave));
-        p.sections = 1;
-        // two sets of waves a workgroup where the block's walk is long enough to be worth their meeting (four tiles and more);
-        // NEURA_HIP_FILL_SPLIT=0 keeps one set
-        static const bool split_wanted = [] { const char *v = getenv("NEURA_HIP_FILL_SPLIT"); return !(v && v[0] == '0'); }();
-        const bool split = split_wanted && a.cache_element != NH_F32 && a.keys >= 128u;
-        const uint32_t longest = a.longest ? min(a.longest, a.keys) : a.keys;
-        p.sections = fill_sections(grid.x * grid.y, (longest + (split ? 64u : 32u) - 1u) / (split ? 64u : 32u), (uint64_t)units * p.groups * a.width, a.width, (uint32_t)d->compute_units);
+        const bool split = fill_splits(a);
+        p.sections = a.most_sections ? a.most_sections : attention_fill_sections(d, a, a.keys);
+        p.plane_sections = a.most_sections ? a.plane_sections : nullptr;
         if (p.sections > 1u) {
             p.partial = static_cast<float *>(scratch(d, (size_t)p.sections * units * p.groups * (a.width + 2) * sizeof(float)));
-            if (!p.partial) p.sections = 1;  // (a device that holds no more scratch walks every block whole)
+            if (!p.partial) p.sections = 1, p.plane_sections = nullptr;  // (a device that holds no more scratch walks every block whole)
         }
         grid.z = p.sections;
         int32_t status;

@@ -299,7 +299,10 @@ struct AttentionArgs {
     const uint16_t *cache_k, *cache_v;
     uint32_t heads, kv_heads, batch, rows, width, capacity, keys;
     const uint32_t *cursor;
-    uint32_t longest = 0;  // where the host knows it: the positions the longest plane holds once the rows are in (0: up to `keys`)
+// where the host knows how long each plane is: device words, the sections each plane's walk takes in a fill (attention_fill_sections),
+    // and the most of them (0: as many for every plane as `keys` positions take)
+    const uint32_t *plane_sections = nullptr;
+    uint32_t most_sections = 0;
     float scale;
     uint32_t reach = 0;  // 0, or the span of a ring cache of `keys` slots (Cache::windowed): the last `reach` positions are weighed
     int32_t cache_element = NH_F16;  // what the caches hold: NH_F16 (the matrix-core kernels), NH_BF16 or NH_F32 (the kernel for any element)
@@ -308,6 +311,9 @@ struct AttentionArgs {
     // means `out` holds the merged rows as always.
     SectionSums *unmerged = nullptr;
 };
+// workgroups that share the walk of a block of a fill's rows in a plane of `positions` (the rows among them): by the plane's own length
+// and the launch's shape, whatever the other planes hold
+uint32_t attention_fill_sections(const nh_device *d, const AttentionArgs &a, uint32_t positions);
 int32_t launch_attention(nh_device *d, const AttentionArgs &args);
 
 // fused decode-side step: rope(q,k) + fp16 cache append from a token-major qkv buffer

@@ -33,7 +33,7 @@ struct nh_model {
     // activations; T = rows * batch flattened token rows, t = row * batch + plane
     float *h = nullptr, *xn = nullptr, *qkv = nullptr, *att = nullptr, *act = nullptr, *up = nullptr, *logits = nullptr;
     float *rope_cos = nullptr, *rope_sin = nullptr;  // [capacity][head_dim / 2], for the rotation folded into the q|k|v product
-    uint32_t *inputs_dev = nullptr;  // [tokens T_max | cursors B | draws B x 4 words | mask bytes B]
+    uint32_t *inputs_dev = nullptr;  // [tokens T_max | cursors B | draws B x 4 words, in a fill the planes' sections | mask bytes B]
     uint32_t *chosen_dev = nullptr;
     uint8_t *inputs_host = nullptr;  // pinned mirror of inputs_dev
     uint32_t *chosen_host = nullptr; // pinned [B + 1]: chosen tokens, then the refusal word
@@ -92,7 +92,8 @@ bool device_array(T *&out, size_t count) {
     return true;
 }
 
-// writes tokens / cursors / draws / mask through the pinned staging buffer in one copy
+// writes tokens / cursors / draws (a fill draws nothing: its planes' sections lie there already) / mask through the pinned staging buffer in
+// one copy
 int32_t stage_inputs(nh_model *m, const uint32_t *tokens, uint32_t count, const uint32_t *cursors, const uint8_t *mask, uint32_t batch,
                      const nh_draw *draws = nullptr) {
     static_assert(sizeof(nh_draw) == 16, "a draw is four words");
@@ -110,6 +111,7 @@ int32_t stage_inputs(nh_model *m, const uint32_t *tokens, uint32_t count, const 
 const uint32_t *dev_tokens(const nh_model *m) { return m->inputs_dev; }
 const uint32_t *dev_cursor(const nh_model *m) { return m->inputs_dev + m->max_tokens; }
 const nh_draw *dev_draws(const nh_model *m) { return reinterpret_cast<const nh_draw *>(m->inputs_dev + m->max_tokens + m->c.batch); }
+const uint32_t *dev_sections(const nh_model *m) { return m->inputs_dev + m->max_tokens + m->c.batch; }
 const uint8_t *dev_mask(const nh_model *m) { return reinterpret_cast<const uint8_t *>(m->inputs_dev + m->max_tokens + 5 * (size_t)m->c.batch); }
 
 enum { EMBD = 0, HEAD = 1, Q = 0, K_ = 1, V = 2, O = 3, GATE = 4, UP = 5, DOWN = 6 };
@@ -125,7 +127,7 @@ GemvArgs narrow(const nh_model *m, int32_t element, const uint8_t *W, uint32_t N
 }
 
 // all layers over T = rows * batch token rows whose inputs are already staged on the device
-int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_only = false, uint32_t longest = 0) {
+int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_only = false, uint32_t most_sections = 0) {
     nh_device *d = m->d;
     const nh_model_config &c = m->c;
     const uint32_t B = c.batch, T = rows * B, H = c.hidden, hd = c.head_dim;
@@ -253,7 +255,8 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
         at.cache_element = c.cache_element;
         at.heads = c.heads, at.kv_heads = c.kv_heads, at.batch = B, at.rows = rows, at.width = hd;
         at.capacity = m->capacity, at.keys = m->window, at.cursor = dev_cursor(m), at.scale = scale;
-        at.reach = m->ring ? m->window : 0u, at.longest = longest;
+        at.reach = m->ring ? m->window : 0u;
+        at.plane_sections = dev_sections(m), at.most_sections = most_sections;
         // one row through a product that merges the attention's sections as it stages its row: the attention leaves them unmerged
         SectionSums sums{};
         GemvArgs o{};
@@ -669,18 +672,24 @@ int32_t nh_prefill(nh_model *m, const uint32_t *tokens, uint32_t rows, const uin
     NH_REQUIRE(batch == m->c.batch, "a fill of %u planes feeds a model of %u planes", batch, m->c.batch);
     NH_REQUIRE(rows >= 1 && rows * batch <= m->max_tokens, "a fill of %u rows feeds a model built for chunks of %u rows", rows,
                m->max_tokens / m->c.batch);
+    AttentionArgs shape{};
+    shape.heads = m->c.heads, shape.kv_heads = m->c.kv_heads, shape.batch = batch, shape.rows = rows, shape.width = m->c.head_dim, shape.keys = m->window;
+    shape.cache_element = m->c.cache_element;
+    uint32_t *const sections = reinterpret_cast<uint32_t *>(m->inputs_host) + (dev_sections(m) - m->inputs_dev);
+    uint32_t most_sections = 1;
     bool any_inactive = false;
-    uint32_t longest = 0;  // (positions of the longest active plane: how far the fill's attention walks)
     for (uint32_t b = 0; b < batch; b++) {
         bool active = !mask || mask[b];
         any_inactive |= !active;
-        if (active && cursors[b] + rows > longest) longest = cursors[b] + rows;
         NH_REQUIRE(!active || (uint64_t)cursors[b] + rows <= m->c.context, "plane %u at cursor %u fills %u rows past a context of %u", b,
                    cursors[b], rows, m->c.context);
+        const uint64_t positions = (uint64_t)cursors[b] + rows;  // (an inactive plane's cursor may say anything)
+        sections[b] = attention_fill_sections(m->d, shape, positions < m->window ? (uint32_t)positions : m->window);
+        if (sections[b] > most_sections) most_sections = sections[b];
     }
     int32_t status;
     if ((status = stage_inputs(m, tokens, rows * batch, cursors, mask, batch)) != NH_OK) return status;
-    if ((status = forward(m, rows, any_inactive, false, longest)) != NH_OK) return status;
+    if ((status = forward(m, rows, any_inactive, false, most_sections)) != NH_OK) return status;
     return check_refusal(m->d, "a fill");
 }
 

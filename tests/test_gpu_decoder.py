@@ -342,6 +342,29 @@ def test_sampled_decode_steps_draw_as_the_oracle_draws(device):
     model.release(), weights.release()
 
 
+@pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K)])
+def test_a_plane_s_fill_is_the_same_beside_any_other(device, shape, element):
+    """How many workgroups share the walk of a plane's rows is a matter of that plane's length: its keys, values and logits
+    are bit for bit the same beside a short plane, a long one and an inactive one, while the long one's walk is shared
+    (and stays within the oracle's bar: test_sections_of_a_fill_walk_meet)."""
+    rows, context = 20, 2048
+    held = []
+    for other, mask in ((0, None), (1900, None), (1000, [1, 0])):
+        rng = np.random.default_rng(7)
+        model, _, weights = build(device, shape, element, batch=2, context=context, max_rows=rows, seed=3)
+        states = rng.standard_normal(model.cache_shape).astype(np.float16).view(np.uint16)
+        for layer in range(shape["layers"]):
+            for which in (0, 1):
+                model.cache_write(layer, which, states)
+        prompt = rng.integers(0, shape["vocab"], (rows, 2))
+        model.prefill(prompt.reshape(-1), rows, [80, other], mask=mask)
+        model.decode_step([5, 6], [80 + rows, other + rows], mask=mask)
+        held.append([model.logits()[0]] + [model.cache_read(layer, which)[:, 0, :80 + rows + 1] for layer in range(shape["layers"]) for which in (0, 1)])
+        model.release(), weights.release()
+    for beside in held[1:]:
+        assert all(np.array_equal(one, two) for one, two in zip(held[0], beside))
+
+
 @pytest.mark.parametrize("shape,element,batch", [(TINY, NH_Q8_0, 2), (SMALL_Q4, NH_Q4_K, 1)])
 def test_a_windowed_model_keeps_a_ring_of_its_last_tokens(device, shape, element, batch):
     """BatchSpec::window (crates/neura-generate/src/batch.rs:148-152, :313-325): caches of window + chunk rows written as
