@@ -14,6 +14,7 @@
 // same fold).  The next tile's K/V rows are in flight during the weight and value passes.
 #include "blocks.hpp"
 #include "common.hpp"
+#include "fill_rule.hpp"
 
 #include <cstdlib>
 
@@ -384,7 +385,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float float4_loose __attribute__((ext_vector_type(4), aligned(4)));
 
-constexpr uint32_t FILL_SECTIONS_MOST = 32;
 // two rounds of staged keys and values, a tile of 32 a set of waves (rows padded by eight halves to spread the banks), residues beside single states
 __host__ __device__ constexpr size_t fill_lds_bytes(int width, int element, bool split) { return 2u * 2u * (split ? 2u : 1u) * (element == NH_F32 ? 2u : 1u) * 32u * (width + 8u) * 2u; }
 
@@ -1065,26 +1065,6 @@ static void launch_fold(uint32_t sections, dim3 grid, dim3 block, size_t lds, hi
     else hipLaunchKernelGGL(attention_fold_kernel<32>, grid, block, lds, stream, args...);
 }
 
-// How many workgroups share the walk of a block of query rows in a fill.  A block's walk is a chain of rounds (a tile a set of waves:
-// 2.35 us at width 128, 1.85 at 64) behind some 10 us (6.5) of queries, first tile and meeting; one workgroup runs on a compute unit
-// at a time, so blocks times sections come in turns of the chip; sections leave their sums in memory for a fold of 4 us and
-// more (480 rows of 28 heads in two: 10 us).  In hundredths of a microsecond; over 40 shapes of 5 to 480 rows behind 0 to 1500 kept
-// positions the pick takes 1.005 times the best one's time.  28 heads of 128, one workgroup a block -> here: 37 rows behind 700 kept
-// positions 41 -> 18 us, 100 behind 1500 72 -> 29, 480 behind 700 59 -> 49; 480 rows alone stay (31 us).
-static uint32_t fill_sections(uint32_t blocks, uint32_t rounds, uint64_t numbers, uint32_t width, uint32_t compute_units) {
-    // NEURA_HIP_FILL_SECTIONS=<sections>: that many (read at every launch: the tests switch it)
-    if (const char *held = getenv("NEURA_HIP_FILL_SECTIONS"); held && atoi(held) > 0) return min((uint32_t)atoi(held), FILL_SECTIONS_MOST);
-    uint32_t best = 1;
-    uint64_t least = UINT64_MAX;
-    for (uint32_t s = 1; s <= FILL_SECTIONS_MOST && s <= rounds; s++) {
-        const uint64_t turns = ((uint64_t)blocks * s + compute_units - 1u) / compute_units;
-        const uint64_t walk = (uint64_t)((rounds + s - 1u) / s) * (width > 64u ? 235u : 185u) + (width > 64u ? 1000u : 650u);
-        const uint64_t cost = turns * walk + (s > 1u ? 400u + numbers / 3500u + numbers * s / 7500u : 0u);
-        if (cost < least) least = cost, best = s;
-    }
-    return best;
-}
-
 // Two sets of waves a workgroup where the block's walk is long enough to be worth their meeting (four tiles and more);
 // NEURA_HIP_FILL_SPLIT=0 keeps one set
 static bool fill_splits(const AttentionArgs &a) {
@@ -1095,8 +1075,10 @@ static bool fill_splits(const AttentionArgs &a) {
 uint32_t attention_fill_sections(const nh_device *d, const AttentionArgs &a, uint32_t positions) {
     const uint32_t groups = a.heads / a.kv_heads;
     if (!groups || groups > (uint32_t)MAX_GROUPS || !a.rows) return 1u;  // (no fill's: launch_attention)
+    // NEURA_HIP_FILL_SECTIONS=<sections>: that many (read at every launch: the tests switch it)
+    if (const char *held = getenv("NEURA_HIP_FILL_SECTIONS"); held && atoi(held) > 0) return min((uint32_t)atoi(held), FILL_SECTIONS_MOST);
     const uint32_t block_rows = 4u * (32u / groups), blocks = a.kv_heads * a.batch * ((a.rows + block_rows - 1u) / block_rows), round = fill_splits(a) ? 64u : 32u;
-    return fill_sections(blocks, (min(positions, a.keys) + round - 1u) / round, (uint64_t)a.heads * a.batch * a.rows * a.width, a.width, (uint32_t)d->compute_units);
+    return fill_sections(blocks, (min(positions, a.keys) + round - 1u) / round, (uint64_t)a.heads * a.batch * a.rows * a.width, a.width, a.cache_element == NH_F32, fill_splits(a), (uint32_t)d->compute_units);
 }
 
 template <int WIDTH, int CE, bool SPLIT>
