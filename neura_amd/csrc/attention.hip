@@ -1084,11 +1084,8 @@ uint32_t attention_fill_sections(const nh_device *d, const AttentionArgs &a, uin
 template <int WIDTH, int CE, bool SPLIT>
 static int32_t launch_fill(nh_device *d, const AttentionParams &p, dim3 grid, uint32_t rows_per_wave) {
     constexpr size_t lds = fill_lds_bytes(WIDTH, CE, SPLIT);
-    static bool sized = false;
-    if (!sized) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_tile_kernel<WIDTH, CE, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        sized = true;
-    }
+    static OnceADevice sized;
+    NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(attention_tile_kernel<WIDTH, CE, SPLIT>), lds));
     hipLaunchKernelGGL((attention_tile_kernel<WIDTH, CE, SPLIT>), grid, dim3(SPLIT ? 512 : 256), lds, d->stream, p, rows_per_wave);
     NH_HIP(hipGetLastError());
     return NH_OK;

@@ -8,6 +8,8 @@
 #include <cstdio>
 #include <vector>
 
+#include "once_a_device.hpp"
+
 #include "../../include/neura_hip.h"
 
 namespace nh {
@@ -97,6 +99,17 @@ struct nh_device {
 
 namespace nh {
 
+// the dynamic LDS a kernel may ask for past 64 KB, on the device it is launched on
+inline hipError_t raise_lds(OnceADevice &once, const nh_device *device, const void *kernel, size_t bytes) {
+    return once(device->index, [&] {
+        int current = device->index;
+        hipError_t status = hipGetDevice(&current);
+        if (status == hipSuccess && current != device->index) status = hipSetDevice(device->index);
+        if (status == hipSuccess) status = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (current != device->index) (void)hipSetDevice(current);
+        return status;
+    });
+}
 // hipMalloc, with no error left behind for the next launch to report
 hipError_t allocate(void **held, size_t bytes);
 // grows the device scratch to at least `bytes`; returns nullptr on failure (error recorded)

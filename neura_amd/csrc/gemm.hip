@@ -1030,11 +1030,8 @@ size_t gemm_scratch_bytes(uint32_t M, uint32_t K, uint32_t pieces) { return Pack
 
 template <int PIECES, int PRELUDE, bool FEW, uint32_t THREADS>
 static int32_t pack_staged(nh_device *d, const GemmArgs &a, size_t lds, _Float16 *A, _Float16 *S, float *unscale, const float *aux, float *outside) {
-    static bool roomy = false;
-    if (!roomy) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PIECES, PRELUDE, FEW, THREADS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)PACK_STAGED_LDS_MOST));
-        roomy = true;
-    }
+    static OnceADevice roomy;
+    NH_HIP(raise_lds(roomy, d, reinterpret_cast<const void *>(gemm_pack_rows_staged_kernel<PIECES, PRELUDE, FEW, THREADS>), PACK_STAGED_LDS_MOST));
     hipLaunchKernelGGL((gemm_pack_rows_staged_kernel<PIECES, PRELUDE, FEW, THREADS>), dim3(a.M, PIECES == WHOLE_PIECES ? WHOLE_PARTS : 1u), dim3(THREADS), lds, d->stream, static_cast<const float *>(a.X), a.K, A, S, unscale, aux, a.eps, reinterpret_cast<WholeRow *>(unscale), outside);
     NH_HIP(hipGetLastError());
     return NH_OK;
@@ -1132,14 +1129,11 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
                           1u, 1u, reinterpret_cast<float *>(room + at.partial), d->meets, 0u, a.Y_more};
         return form.shape != SHARED_NONE ? launch_gemm_wide(d, a.element, f, form.shape) : launch_gemm_few(d, a.element, f, a.gated);
     }
-    static bool sized = false;
-    if (!sized) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q8_0_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q8_LDS));
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_regb_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_REGB_LDS));
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q5k_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_Q4K_LDS));
-        sized = true;
-    }
+    static OnceADevice sized[4];
+    NH_HIP(raise_lds(sized[0], d, reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), GEMM_Q4K_LDS));
+    NH_HIP(raise_lds(sized[1], d, reinterpret_cast<const void *>(gemm_q8_0_mfma_kernel), GEMM_Q8_LDS));
+    NH_HIP(raise_lds(sized[2], d, reinterpret_cast<const void *>(gemm_q4k_regb_mfma_kernel), GEMM_Q4K_REGB_LDS));
+    NH_HIP(raise_lds(sized[3], d, reinterpret_cast<const void *>(gemm_q5k_mfma_kernel), GEMM_Q4K_LDS));
     dim3 grid((a.N + GT - 1) / GT, (p.rows + GT - 1) / GT);
     if (a.element == NH_Q8_0) hipLaunchKernelGGL(gemm_q8_0_mfma_kernel, grid, dim3(512), GEMM_Q8_LDS, d->stream, p);
     else if (a.element == NH_Q5_K) hipLaunchKernelGGL(gemm_q5k_mfma_kernel, grid, dim3(512), GEMM_Q4K_LDS, d->stream, p);

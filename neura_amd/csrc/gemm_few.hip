@@ -364,11 +364,8 @@ int32_t launch_few(nh_device *d, FewParams p) {
     const FewSplit split = few_split(ELEMENT, p.N, p.K, p.rows, MT, NT, (uint32_t)d->compute_units);
     p.deep = split.deep, p.slices = split.slices;
     const size_t lds = (size_t)p.deep * NT * MT * 4096u;
-    static bool sized = false;
-    if (!sized) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), hipFuncAttributeMaxDynamicSharedMemorySize, 8 * NT * MT * 4096));
-        sized = true;
-    }
+    static OnceADevice sized;
+    NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), 8 * NT * MT * 4096));
     const dim3 grid(tiles, (row_tiles + MT - 1u) / MT, p.slices);
     hipLaunchKernelGGL((gemm_few_kernel<ELEMENT, MT, GATED, AHEAD>), grid, dim3(64u * p.deep), lds, d->stream, p);
     NH_HIP(hipGetLastError());

@@ -309,11 +309,8 @@ template <int ELEMENT, int WN, int MT>
 int32_t launch_shape(nh_device *d, FewParams p) {
     typedef typename FewOf<ELEMENT>::type Weights;
     constexpr size_t lds = MT * (3u * (Weights::STEPS / 2u) * 4096u + (Weights::FLOORS ? 2048u : 0u));
-    static bool sized = false;
-    if (!sized) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        sized = true;
-    }
+    static OnceADevice sized;
+    NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT>), lds));
     // (beside residuals the chains' sums wait in scratch: more of them than that holds stay in one chain)
     p.chain = p.residual && (size_t)p.M * p.N * sizeof(float) > FEW_PARTIAL_BYTES ? ~0u : shared_rows_chain(ELEMENT, p.N, p.K, p.rows, (uint32_t)d->compute_units);
     const uint32_t column_tiles = (p.N + 32u * WN - 1u) / (32u * WN), row_blocks = ((p.rows + 31u) / 32u + MT - 1u) / MT;

@@ -2394,12 +2394,10 @@ static bool mfma_takes(const GemvArgs &a) {
 
 template <int KS, int NW, int P, int D>
 static hipError_t launch_mfma_instance(nh_device *d, const MfmaParams &p, uint32_t blocks_x, size_t lds) {
-    static bool widened = false;  // past 64 KiB of dynamic LDS a kernel has to be told once
-    if (lds > 64 * 1024 && !widened) {
-        hipError_t status = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<KS, NW, P, D>),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);  // the static arrays take the rest of the 160 KiB
+    static OnceADevice widened;  // past 64 KiB of dynamic LDS a kernel has to be told
+    if (lds > 64 * 1024) {
+        hipError_t status = raise_lds(widened, d, reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<KS, NW, P, D>), 156 * 1024);  // the static arrays take the rest of the 160 KiB
         if (status != hipSuccess) return status;
-        widened = true;
     }
     hipLaunchKernelGGL((gemv_q4k_mfma_kernel<KS, NW, P, D>), dim3(blocks_x, p.splits), dim3(NW * 64), lds, d->stream, MFMA_LEAD(p));
     return hipGetLastError();
@@ -2560,11 +2558,8 @@ static bool mfma32_takes(const nh_device *d, const GemvArgs &a) {
 
 template <int J, int NW, int KS, bool ROPE = false>
 static int32_t launch_mfma32_instance(nh_device *d, const MfmaParams &p, size_t lds) {
-    static bool widened = false;  // past 64 KiB of dynamic LDS a kernel has to be told once
-    if (lds > 64 * 1024 && !widened) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_q4k_mfma32_kernel<J, NW, KS, ROPE>), hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024));
-        widened = true;
-    }
+    static OnceADevice widened;  // past 64 KiB of dynamic LDS a kernel has to be told
+    if (lds > 64 * 1024) NH_HIP(raise_lds(widened, d, reinterpret_cast<const void *>(&gemv_q4k_mfma32_kernel<J, NW, KS, ROPE>), 158 * 1024));
     // one resident round of workgroups, as many as LDS and registers let a compute unit hold
     uint32_t resident = (uint32_t)((159 * 1024) / (lds + 1280));
     const uint32_t by_waves = NW == 16 ? 1u : 12u / NW;
@@ -2652,11 +2647,8 @@ static bool f16_tiles_take(const nh_device *d, const GemvArgs &a) {
 
 template <int NW, int KS>
 static int32_t launch_f16_tiles_instance(nh_device *d, const MfmaParams &p, size_t lds) {
-    static bool widened = false;  // past 64 KiB of dynamic LDS a kernel has to be told once
-    if (lds > 64 * 1024 && !widened) {
-        NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_q4k_f16_kernel<NW, KS>), hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024));
-        widened = true;
-    }
+    static OnceADevice widened;  // past 64 KiB of dynamic LDS a kernel has to be told
+    if (lds > 64 * 1024) NH_HIP(raise_lds(widened, d, reinterpret_cast<const void *>(&gemv_q4k_f16_kernel<NW, KS>), 158 * 1024));
     uint32_t resident = (uint32_t)((159 * 1024) / (lds + 1280));
     if (resident > 1) resident = 1;  // sixteen waves a workgroup
     if (resident < 1) resident = 1;
@@ -2742,11 +2734,8 @@ static int32_t launch_staged_rows(nh_device *d, const GemvArgs &a, const float *
     if (blocks_x > most) blocks_x = most;
     profile_mark(d);
     if (lds > 64u * 1024u) {
-        static bool widened = false;  // past 64 KiB of dynamic LDS a kernel has to be told once
-        if (!widened) {
-            NH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_staged_kernel<ELEMENT, RB>), hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024));
-            widened = true;
-        }
+        static OnceADevice widened;  // past 64 KiB of dynamic LDS a kernel has to be told
+        NH_HIP(raise_lds(widened, d, reinterpret_cast<const void *>(&gemv_staged_kernel<ELEMENT, RB>), 158 * 1024));
     }
     hipLaunchKernelGGL((gemv_staged_kernel<ELEMENT, RB>), dim3(blocks_x, p.splits), dim3(256), lds, d->stream, GEMV_LEAD(p));
     NH_HIP(hipGetLastError());

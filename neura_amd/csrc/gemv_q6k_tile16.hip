@@ -56,11 +56,10 @@ bool q6k_tile16_takes(const GemvArgs &a) {
 
 template <int NW, bool HANDED, bool SWIGLU = false, int ELEMENT = NH_Q6_K, bool ROPE = false>
 static hipError_t launch_q6k_tile16_instance(nh_device *d, const GemvParams &p, uint32_t grid, size_t lds) {
-    static bool raised = false;  // a workgroup may hold more than the default 64 KiB of LDS once the kernel says so
-    if (!raised && lds > 64u * 1024u) {
-        hipError_t error = hipFuncSetAttribute((const void *)gemv_q6k_tile16_kernel<NW, HANDED, SWIGLU, ELEMENT, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static OnceADevice raised;  // a workgroup may hold more than the default 64 KiB of LDS once the kernel says so
+    if (lds > 64u * 1024u) {
+        hipError_t error = raise_lds(raised, d, (const void *)gemv_q6k_tile16_kernel<NW, HANDED, SWIGLU, ELEMENT, ROPE>, 160 * 1024);
         if (error != hipSuccess) return error;
-        raised = true;
     }
     hipLaunchKernelGGL((gemv_q6k_tile16_kernel<NW, HANDED, SWIGLU, ELEMENT, ROPE>), dim3(grid), dim3(NW * 64), lds, d->stream, p.W[0],
                        HANDED ? static_cast<const void *>(p.digits_in) : static_cast<const void *>(p.x), p.norm_w, p.row_bytes, grid, p.row_groups,

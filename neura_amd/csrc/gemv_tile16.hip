@@ -1296,11 +1296,10 @@ bool rows4_takes(const GemvArgs &a) {
 
 template <int NW, int MODE, int P>
 static hipError_t launch_rows4_instance(nh_device *d, const GemvParams &p, uint32_t grid, size_t lds) {
-    static bool raised = false;
-    if (!raised && lds > 64u * 1024u) {
-        hipError_t error = hipFuncSetAttribute((const void *)gemv_q4k_rows4_kernel<NW, 2, MODE, P>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static OnceADevice raised;
+    if (lds > 64u * 1024u) {
+        hipError_t error = raise_lds(raised, d, (const void *)gemv_q4k_rows4_kernel<NW, 2, MODE, P>, 160 * 1024);
         if (error != hipSuccess) return error;
-        raised = true;
     }
     hipLaunchKernelGGL((gemv_q4k_rows4_kernel<NW, 2, MODE, P>), dim3(grid), dim3(NW * 64), lds, d->stream, GEMV_LEAD(p));
     return hipGetLastError();
@@ -1354,11 +1353,10 @@ int32_t launch_rows4(nh_device *d, const GemvArgs &a) {
 
 template <int NW, int D, int MODE, int R, bool HANDED = false, bool FIFTH = false>
 static hipError_t launch_tile16_instance(nh_device *d, const GemvParams &p, uint32_t grid, size_t lds) {
-    static bool raised = false;  // a workgroup may hold more than the default 64 KiB of LDS once the kernel says so
-    if (!raised && lds > 64u * 1024u) {
-        hipError_t error = hipFuncSetAttribute((const void *)gemv_q4k_tile16_kernel<NW, D, MODE, R, HANDED, FIFTH>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static OnceADevice raised;  // a workgroup may hold more than the default 64 KiB of LDS once the kernel says so
+    if (lds > 64u * 1024u) {
+        hipError_t error = raise_lds(raised, d, (const void *)gemv_q4k_tile16_kernel<NW, D, MODE, R, HANDED, FIFTH>, 160 * 1024);
         if (error != hipSuccess) return error;
-        raised = true;
     }
     hipLaunchKernelGGL((gemv_q4k_tile16_kernel<NW, D, MODE, R, HANDED, FIFTH>), dim3(grid), dim3(NW * 64), lds, d->stream, p.W[0],
                        HANDED ? static_cast<const void *>(p.digits_in) : static_cast<const void *>(p.x), p.norm_w, (int32_t)((p.W[1] - p.W[0]) / 16),
@@ -1531,11 +1529,10 @@ __global__ __launch_bounds__(NW * 64) void gemv_q4k_rope_beside_q6k_kernel(const
 template <int NW, bool FIFTH>
 static hipError_t launch_pair_instance(nh_device *d, const Tile16Launch &first, const Q6kLaunch &second) {
     const size_t lds = first.lds > second.lds ? first.lds : second.lds;
-    static bool raised = false;
-    if (!raised && lds > 64u * 1024u) {
-        hipError_t error = hipFuncSetAttribute((const void *)gemv_q4k_rope_beside_q6k_kernel<NW, FIFTH>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static OnceADevice raised;
+    if (lds > 64u * 1024u) {
+        hipError_t error = raise_lds(raised, d, (const void *)gemv_q4k_rope_beside_q6k_kernel<NW, FIFTH>, 160 * 1024);
         if (error != hipSuccess) return error;
-        raised = true;
     }
     const GemvParams &p = first.p;
     Q6kBeside beside{second.p.W[0], second.p.norm_w, second.p.row_bytes, second.grid, second.p.row_groups, second.p.tile_rows, second.p};
@@ -1691,12 +1688,8 @@ bool gemv_chains(nh_device *d, const GemvArgs *lead, const GemvArgs &gate_up, co
 
 template <int PROGRAM>
 static hipError_t launch_chain_program(nh_device *d, const ChainParams &c, uint32_t grid, size_t lds) {
-    static bool raised = false;
-    if (!raised) {
-        hipError_t error = hipFuncSetAttribute((const void *)gemv_q4k_chain_kernel<PROGRAM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (error != hipSuccess) return error;
-        raised = true;
-    }
+    static OnceADevice raised;
+    if (hipError_t error = raise_lds(raised, d, (const void *)gemv_q4k_chain_kernel<PROGRAM>, 160 * 1024); error != hipSuccess) return error;
     hipLaunchKernelGGL((gemv_q4k_chain_kernel<PROGRAM>), dim3(grid), dim3(512), lds, d->stream, c);
     return hipGetLastError();
 }
