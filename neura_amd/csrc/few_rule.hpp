@@ -24,20 +24,16 @@ inline uint32_t few_row_tiles(uint32_t N, uint32_t rows, uint32_t compute_units)
 // weights serves.  A round costs the tiles 350 k more than it walks (filling and draining).  Shares are fitted to both forms timed at
 // 128 to 8192 packed rows over the 0.5B, 1.5B and 7B shapes (us, tiles / few): Q8_0 18944 x 3584 at 512 rows 157 / 211 and at 1024 262 /
 // 331 (full rounds), 3584 x 3584 at 512 56 / 48 (112 workgroups), 4608 x 3584 at 1024 105 / 87 (288), 4864 x 896 at 1024 47 / 35 (304);
-// Q6_K 221 / 193, 80 / 47, 151 / 96 of the first, third and fourth; Q3_K 155 / 140, 57 / 39, 107 / 71; Q5_K 141 / 150, 51 / 40, 95 / 76; Q4_K
-// 125 / 148, 43 / 39, 82 / 77.  The form it picks is within 8 % of the faster one at those points.  (Q6_K and Q3_K have no tiles since rows
-// are shared below: past their line shared rows serve them, gate at 1024 rows 360 -> 252 and 259 -> 190 us.)
+// Q5_K 141 / 150, 51 / 40, 95 / 76 of the first, third and fourth; Q4_K 125 / 148, 43 / 39, 82 / 77.  The form it picks is within 8 % of the
+// faster one at those points.  Q6_K and Q3_K have no tiles: few rows up to the height of a grid, and shared rows below.
 inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
     if (rows <= 96u) return true;
     if (rows > 65535u * 32u) return false;  // (row tiles are blockIdx.y)
+    if (element == NH_Q6_K || element == NH_Q3_K) return true;
     struct Share {
         uint32_t twos, threes;
     };
-    const Share share = element == NH_Q8_0   ? Share{195u, 145u}
-                        : element == NH_Q6_K ? Share{105u, 95u}
-                        : element == NH_Q5_K ? Share{180u, 140u}
-                        : element == NH_Q3_K ? Share{120u, 109u}
-                                             : Share{200u, 170u};
+    const Share share = element == NH_Q8_0 ? Share{195u, 145u} : element == NH_Q5_K ? Share{180u, 140u} : Share{200u, 170u};
     const uint64_t groups = (uint64_t)((N + 127u) / 128u) * ((rows + 127u) / 128u), rounds = (groups + compute_units - 1u) / compute_units;
     const uint64_t tiles_cost = 100u * rounds * compute_units + (rounds - 1u) * compute_units * 35000u / K;
     return groups * (few_row_tiles(N, rows, compute_units) == 3u ? share.threes : share.twos) <= tiles_cost;
@@ -91,13 +87,13 @@ enum SharedShape { SHARED_NONE = 0, SHARED_42 = 42, SHARED_43 = 43, SHARED_83 = 
 inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
     if (rows <= 64u || !N || !K || !compute_units) return SHARED_NONE;
     struct Times {
-        double tiles, twos, threes;             // of a 128 x 128 tile's 256 k; of a unit of the product of few rows, two or three row tiles a pass
+        double tiles, twos, threes;             // of a 128 x 128 tile's 256 k (Q6_K, Q3_K: none); of a unit of the product of few rows, two or three row tiles a pass
         double pair2, one2, pair3, one3, e3, e4;  // of a unit here: 4 x 2 with company and alone, 4 x 3, 8 x 3, 8 x 4
     };
     const Times t = element == NH_Q8_0   ? Times{2.73, 2.26, 2.63, 1.82, 1.41, 2.21, 1.55, 0.0, 2.74}
-                    : element == NH_Q6_K ? Times{4.32, 3.41, 4.68, 4.04, 2.41, 4.90, 2.66, 4.26, 0.0}
+                    : element == NH_Q6_K ? Times{0.0, 3.41, 4.68, 4.04, 2.41, 4.90, 2.66, 4.26, 0.0}
                     : element == NH_Q5_K ? Times{2.34, 2.86, 3.74, 2.79, 1.71, 3.36, 1.89, 2.84, 3.28}
-                    : element == NH_Q3_K ? Times{2.72, 2.66, 3.38, 2.47, 1.65, 2.96, 1.87, 2.64, 2.90}
+                    : element == NH_Q3_K ? Times{0.0, 2.66, 3.38, 2.47, 1.65, 2.96, 1.87, 2.64, 2.90}
                                          : Times{1.69, 2.68, 3.56, 2.44, 1.49, 3.11, 1.72, 2.49, 3.04};
     const uint64_t cu = compute_units, row_tiles = (rows + 31u) / 32u;
     const uint32_t per = element == NH_Q8_0 ? 128u : 256u, units = (K + per - 1u) / per;

@@ -1067,8 +1067,8 @@ static int32_t pack_rows(nh_device *d, const GemmArgs &a, _Float16 *A, _Float16 
 
 // Which form a wide product takes.  `operands`: over rows packed in operand order (the product of few rows, or of shared rows in a
 // shape), else the 128 x 128 tiles.  NEURA_HIP_GEMM_WIDE=0: no shared rows; =42, 43, 83, 84: that shape wherever it can.  Q6_K and
-// Q3_K have no tiles (gate of the 7B shape at 1024 rows 360 and 259 us there, 252 and 190 on shared rows): what few_rows_win
-// leaves, which is what takes whole rounds of them, goes to shared rows.
+// Q3_K have no tiles: past the height of the product of few rows' grid, and where NEURA_HIP_GEMM_FEW=0 keeps them from it, they go to shared
+// rows whatever is held.
 struct WideForm {
     bool operands;
     SharedShape shape;

@@ -619,7 +619,7 @@ def test_q6_k_q5_k_and_q3_k_wide_products_on_the_matrix_cores(device, element, M
     (NH_Q3_K, 42, 4130, 512, False), (NH_Q3_K, 65, 4130, 768, True), (NH_Q8_0, 48, 4130, 192, False), (NH_Q5_K, 33, 4224, 1280, False)])
 def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, K, half):
     """The wide product of few rows (operands in registers, the K shares of a workgroup's waves meeting in LDS) and the one of 128 x 128
-    tiles, each forced: single tiles, ragged columns and rows, one and two row tiles a wave, three (more than 128 column
+    tiles (of Q6_K and Q3_K, which have none, shared rows), each forced: single tiles, ragged columns and rows, one and two row tiles a wave, three (more than 128 column
     tiles, three row tiles or five of them, the last ones ragged) and more passes, K of one unit, of fewer units than
     waves and of half a Q8_0 unit -- against the exact product.  Bar: 22 bits of every activation take part and fp32 sums of K terms
     in any order stay within a few rounding errors of the sum of magnitudes' root (1e-6 of the outputs' scale at these depths)."""
