@@ -342,6 +342,31 @@ def test_sampled_decode_steps_draw_as_the_oracle_draws(device):
     model.release(), weights.release()
 
 
+# (83 of Q8_0 and 84 of Q6_K are another shape's kernel)
+@pytest.mark.parametrize("element,form", [(element, form) for element in (NH_Q8_0, NH_Q6_K, NH_Q5_K, NH_Q4_K, NH_Q3_K) for form in ("42", "43", "83", "84")
+                                          if (element, form) not in ((NH_Q8_0, "83"), (NH_Q6_K, "84"))])
+def test_a_fill_on_shared_rows_stacks_its_matrices(device, monkeypatch, form, element):
+    """A fill whose wide products all go to one shape of the product of shared rows: q|k|v as three stacked matrices, gate|up as two
+    with outputs of their own, the projections back onto the residual stream (whose chains of sums wait in scratch), for
+    every format, 45 rows ending inside a row tile."""
+    monkeypatch.setenv("NEURA_HIP_GEMM_WIDE", form)
+    rows = 45
+    model, ref, weights = build(device, dict(SMALL_Q4, layers=2), element, batch=1, context=64, max_rows=rows, seed=element)
+    prompt = np.random.default_rng(8).integers(0, SMALL_Q4["vocab"], rows)
+    model.prefill(prompt, rows, [0])
+    ref.forward(prompt, rows, [0], want_logits=False)
+    want_logits, want = ref.forward([3], 1, [rows])
+    got = model.decode_step([3], [rows])
+    assert np.abs(model.logits() - want_logits).max() <= 1e-3 * np.abs(want_logits).max()
+    assert list(got) == list(want), margins(want_logits)
+    for layer in range(2):
+        for which, held in ((0, ref.cache_k), (1, ref.cache_v)):
+            got_cache = oracle.f16_to_f32(model.cache_read(layer, which).reshape(-1))
+            want_cache = oracle.f16_to_f32(held[layer])
+            assert np.abs(got_cache - want_cache).max() <= 2e-3 * max(1.0, np.abs(want_cache).max())
+    model.release(), weights.release()
+
+
 @pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K)])
 def test_a_plane_s_fill_is_the_same_beside_any_other(device, shape, element):
     """How many workgroups share the walk of a plane's rows is a matter of that plane's length: its keys, values and logits
