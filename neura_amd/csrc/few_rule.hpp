@@ -65,15 +65,22 @@ inline FewSplit few_split(int32_t element, uint32_t N, uint32_t K, uint32_t rows
     return best;
 }
 
+// units of K: 256 numbers, 128 of Q8_0
+inline uint32_t shared_rows_units(int32_t element, uint32_t K) { return element == NH_Q8_0 ? (K / 64u + 1u) / 2u : (K / 64u + 3u) / 4u; }
+
 // Units of k a wave of the product of shared rows adds up before its sums leave the accumulators (a chain): as many as a share of the
 // product of few rows has, where that is the form it takes over from, for one chain over all of K adds up less exactly than shares that
 // meet (2-norm from 64 bits, few rows / one chain / here: Q3_K 3584 x 18944 at 600 packed rows 1.15e-7 / 1.75 / 1.16, Q6_K at 800 1.56 /
 // 2.41 / 1.56, Q5_K at 600 1.56 / 1.99 / 1.49, Q8_0 17920 x 1536 at 200 1.10 / 1.38 / 1.10).  The tiles are one chain themselves.
 inline uint32_t shared_rows_chain(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
-    const uint32_t steps = element == NH_Q8_0 ? 2u : 4u, units = (K / 64u + steps - 1u) / steps;
+    const uint32_t units = shared_rows_units(element, K);
     if (!few_rows_win(element, N, K, rows, compute_units)) return units;
     const FewSplit split = few_split(element, N, K, rows, few_row_tiles(N, rows, compute_units), 1u, compute_units);
     return (units + split.deep * split.slices - 1u) / (split.deep * split.slices);
+}
+// Beside residuals, whose place is the outputs', the sums of chains wait in scratch: whether they do, and are more than that holds
+inline bool shared_rows_overflow(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint64_t residual_bytes, uint32_t compute_units) {
+    return residual_bytes > FEW_SUMS_MOST && shared_rows_chain(element, N, K, rows, compute_units) < shared_rows_units(element, K);
 }
 
 // Where the product of shared rows (gemm_wide.hip) takes over, and in which shape: waves side by side and row tiles a wave (none: the form

@@ -1078,10 +1078,10 @@ struct WideForm {
     SharedShape shape;
 };
 static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, size_t residuals) {
-    // (`residuals`: bytes of outputs whose place holds residuals; the sums of chains then wait in scratch)
-    const int held = residuals > FEW_PARTIAL_BYTES ? 0 : env_int("NEURA_HIP_GEMM_WIDE", -1);
-    if (held == SHARED_42 || held == SHARED_43 || held == SHARED_83 || held == SHARED_84) return WideForm{true, (SharedShape)held};
+    // (`residuals`: bytes of outputs whose place holds residuals)
     const uint32_t units = (uint32_t)d->compute_units;
+    const int held = shared_rows_overflow(element, N, K, rows, residuals, units) ? 0 : env_int("NEURA_HIP_GEMM_WIDE", -1);
+    if (held == SHARED_42 || held == SHARED_43 || held == SHARED_83 || held == SHARED_84) return WideForm{true, (SharedShape)held};
     const SharedShape shape = held == 0 || gemm_few_held() >= 0 ? SHARED_NONE : shared_rows_shape(element, N, K, rows, units);
     if (shape != SHARED_NONE || gemm_few_takes(d, element, N, K, rows)) return WideForm{true, shape};
     const bool tiled = element != NH_Q6_K && element != NH_Q3_K;

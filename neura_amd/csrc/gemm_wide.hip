@@ -23,7 +23,6 @@ namespace nh {
 
 namespace {
 
-// MT tiles of 32 packed rows by NT x 32 columns a wave
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t *at, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(at), 0, bytes, 0x00020000); }
 
 // WN: waves side by side, 32 columns each; MT: tiles of 32 packed rows a wave multiplies its unpacked weights by.
@@ -312,7 +311,9 @@ int32_t launch_shape(nh_device *d, FewParams p) {
     static OnceADevice sized;
     NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT>), lds));
     // (beside residuals the chains' sums wait in scratch: more of them than that holds stay in one chain)
-    p.chain = p.residual && (size_t)p.M * p.N * sizeof(float) > FEW_PARTIAL_BYTES ? ~0u : shared_rows_chain(ELEMENT, p.N, p.K, p.rows, (uint32_t)d->compute_units);
+    const uint32_t compute_units = (uint32_t)d->compute_units;
+    const uint64_t residuals = p.residual ? (uint64_t)p.M * p.N * sizeof(float) : 0u;
+    p.chain = shared_rows_overflow(ELEMENT, p.N, p.K, p.rows, residuals, compute_units) ? ~0u : shared_rows_chain(ELEMENT, p.N, p.K, p.rows, compute_units);
     const uint32_t column_tiles = (p.N + 32u * WN - 1u) / (32u * WN), row_blocks = ((p.rows + 31u) / 32u + MT - 1u) / MT;
     hipLaunchKernelGGL((gemm_wide_kernel<ELEMENT, WN, MT>), dim3((column_tiles * row_blocks + 7u) / 8u * 8u), dim3(64 * WN), lds, d->stream, p, column_tiles, row_blocks);
     NH_HIP(hipGetLastError());

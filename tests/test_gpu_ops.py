@@ -700,6 +700,26 @@ def test_minimums_of_shared_rows_are_as_exact_as_those_of_the_tiles(device, monk
     assert errors[0] <= 1.1 * errors[1]
 
 
+@pytest.mark.parametrize("element,M,N,K", [(NH_Q4_K, 1200, 3584, 1792), (NH_Q8_0, 1200, 3584, 1792), (NH_Q6_K, 1200, 3584, 3584), (NH_Q3_K, 4200, 1024, 1536)])
+def test_wide_products_beside_more_residuals_than_scratch_holds(device, element, M, N, K):
+    """More than 16 MB of outputs whose place holds residuals: forms whose sums run in one chain, and a product that goes back to few rows
+    because its chains' sums have no room to wait in -- against the exact product of the first and the last columns, at the bar of
+    test_both_forms_of_a_wide_product."""
+    assert M * N * 4 > 16 << 20
+    rng = np.random.default_rng(M + N + element)
+    raw = np.array(synth.RANDOM[element](rng, N * K), dtype=np.uint8)
+    per, size = synth.BLOCK_BYTES[element]
+    bytes_ = 64 * K // per * size
+    weights = np.concatenate([oracle.unpack(element, raw[part], 64 * K).reshape(64, K) for part in (slice(0, bytes_), slice(-bytes_, None))]).astype(np.float64)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    exact = X.astype(np.float64) @ weights.T
+    scale = np.sqrt((X.astype(np.float64) ** 2) @ (weights.T ** 2))
+    got = device.gemm(element, raw, N, K, X, residual=r)
+    ends = np.r_[0:64, N - 64 : N]
+    assert (np.abs(got[:, ends] - (exact + r[:, ends])) <= 4e-6 * scale + 2.0 ** -23 * (np.abs(exact) + np.abs(r[:, ends])) + 1e-30).all()
+
+
 @pytest.mark.parametrize("element,M,N,K", [
     (NH_Q3_K, 300, 3584, 18944), (NH_Q3_K, 100, 18944, 3584), (NH_Q6_K, 400, 3584, 18944), (NH_Q6_K, 100, 18944, 3584),
     (NH_Q8_0, 100, 17920, 1536), (NH_Q5_K, 300, 3584, 18944), (NH_Q4_K, 37, 37888, 3584)])
