@@ -78,6 +78,9 @@ inline uint32_t shared_rows_chain(int32_t element, uint32_t N, uint32_t K, uint3
     const FewSplit split = few_split(element, N, K, rows, few_row_tiles(N, rows, compute_units), 1u, compute_units);
     return (units + split.deep * split.slices - 1u) / (split.deep * split.slices);
 }
+// Sums of chains that registers hold, of a row tile's sixteen a lane: of two tiles all, of three the eight of whole rows (every second row
+// holds residues, whose sums run on in one chain), which Q6_K in four waves, two planes of operands, leaves no room for.
+constexpr int shared_rows_spare(int32_t element, uint32_t waves, uint32_t mt) { return mt == 2u ? 16 : mt == 3u && !(element == NH_Q6_K && waves == 4u) ? 8 : 0; }
 // Beside residuals, whose place is the outputs', the sums of chains wait in scratch: whether they do, and are more than that holds
 inline bool shared_rows_overflow(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint64_t residual_bytes, uint32_t compute_units) {
     return residual_bytes > FEW_SUMS_MOST && shared_rows_chain(element, N, K, rows, compute_units) < shared_rows_units(element, K);
@@ -91,7 +94,7 @@ inline bool shared_rows_overflow(int32_t element, uint32_t N, uint32_t K, uint32
 // (7B shape, packed rows, other / here: gate|up Q4_K 128 101 / 74, 200 145 / 106, 1024 392 / 331; Q3_K 1024 455 / 310; Q8_0 200
 // 203 / 143; ffn_down Q4_K 300 119 / 103; 0.5B gate|up Q8_0 800 62 / 47).  Up to two row tiles the walk is latency, not work.
 enum SharedShape { SHARED_NONE = 0, SHARED_42 = 42, SHARED_43 = 43, SHARED_83 = 83, SHARED_84 = 84 };
-inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
+inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, uint32_t rows, bool halves, uint32_t compute_units) {
     if (rows <= 64u || !N || !K || !compute_units) return SHARED_NONE;
     struct Times {
         double tiles, twos, threes;             // of a 128 x 128 tile's 256 k (Q6_K, Q3_K: none); of a unit of the product of few rows, two or three row tiles a pass
@@ -116,8 +119,11 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
     }
     SharedShape best = SHARED_NONE;
     double least = other / 1.08;
-    // places between chains, and the end: two microseconds a turn where the sums go through memory (4608 x 3584 Q3_K at 400 packed rows, 42:
-    // 38.4 -> 41.1; 17920 x 1536 Q8_0 at 400 71.9 -> 80.2, two turns; 84: 37888 x 3584 Q3_K at 200 130.0 -> 137.1)
+    // Places between chains, and the end: nothing where three row tiles keep whole rows' sums in registers, 1.5 microseconds a turn for two, 2
+    // through memory (84: 37888 x 3584 Q3_K at 200 packed rows 130.0 -> 137.1) and 5 of half rows there, which have twice the sums.
+    // `halves`: rows of half activations.  Their outputs are twice as many too, 5 us here and not in few rows, whose shares meet
+    // in LDS: over 400 products of 70 to 1024 of them the pick takes 1.003 times the fastest form's time, at most 1.07 times the other
+    // form's; with the line of whole rows up to 1.26 (17920 x 1536 at 200 Q3_K few rows 32.9, 83 41.4; 18944 x 3584 at 512 135.7, 42 123.6).
     const uint32_t chain = shared_rows_chain(element, N, K, rows, compute_units), places = chain < units ? (units - 1u) / chain + 1u : 0u;
     const auto consider = [&](SharedShape shape, uint32_t waves, uint32_t mt, double pair, double one, double base, double turn, double pack) {
         if (!(pair > 0.0)) return;
@@ -125,8 +131,8 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
         const uint64_t full = workgroups / slots, left = workgroups % slots;
         const bool lone = waves == 4u && left && left <= cu;
         const uint64_t turns = full + (left ? 1u : 0u);
-        const bool spare = mt == 3u && !(element == NH_Q6_K && waves == 4u);  // (gemm_wide.hip: registers for them)
-        const double time = base + (double)turns * (turn + units * pair + (spare ? 0.0 : 2.0 * places)) - (lone ? units * (pair - one) : 0.0) + pack * millions;
+        const double place = mt == 2u ? 1.5 : halves ? 5.0 : shared_rows_spare(element, waves, mt) ? 0.0 : 2.0;
+        const double time = base + (halves ? 5.0 : 0.0) + (double)turns * (turn + units * pair + place * places) - (lone ? units * (pair - one) : 0.0) + pack * millions;
         if (time < least) least = time, best = shape;
     };
     consider(SHARED_42, 4u, 2u, t.pair2, t.one2, 5.0, 5.5, 1.7);

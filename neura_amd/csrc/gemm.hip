@@ -1077,12 +1077,12 @@ struct WideForm {
     bool operands;
     SharedShape shape;
 };
-static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, size_t residuals) {
+static WideForm wide_form(const nh_device *d, int32_t element, uint32_t N, uint32_t K, uint32_t rows, bool halves, size_t residuals) {
     // (`residuals`: bytes of outputs whose place holds residuals)
     const uint32_t units = (uint32_t)d->compute_units;
     const int held = shared_rows_overflow(element, N, K, rows, residuals, units) ? 0 : env_int("NEURA_HIP_GEMM_WIDE", -1);
     if (held == SHARED_42 || held == SHARED_43 || held == SHARED_83 || held == SHARED_84) return WideForm{true, (SharedShape)held};
-    const SharedShape shape = held == 0 || gemm_few_held() >= 0 ? SHARED_NONE : shared_rows_shape(element, N, K, rows, units);
+    const SharedShape shape = held == 0 || gemm_few_held() >= 0 ? SHARED_NONE : shared_rows_shape(element, N, K, rows, halves, units);
     if (shape != SHARED_NONE || gemm_few_takes(d, element, N, K, rows)) return WideForm{true, shape};
     const bool tiled = element != NH_Q6_K && element != NH_Q3_K;
     return tiled ? WideForm{false, SHARED_NONE} : WideForm{true, SHARED_43};
@@ -1106,7 +1106,7 @@ static int32_t launch_gemm_mfma(nh_device *d, const GemmArgs &a) {
     const uint32_t pieces = half_rows ? 1u : a.whole ? WHOLE_PIECES : 2u;
     p.rows = a.whole ? whole_rows(a.M) : pieces * a.M;
     p.split = half_rows ? 0 : 1;
-    const WideForm form = a.whole || a.gated ? WideForm{true, SHARED_NONE} : wide_form(d, a.element, a.N, a.K, p.rows, a.residual ? (size_t)a.M * a.N * sizeof(float) : 0u);
+    const WideForm form = a.whole || a.gated ? WideForm{true, SHARED_NONE} : wide_form(d, a.element, a.N, a.K, p.rows, half_rows, a.residual ? (size_t)a.M * a.N * sizeof(float) : 0u);
     const bool few = form.operands;
     if (a.whole && (half_rows || gemm_few_held() == 0 || a.M > 65535u * WHOLE_TILE))
         return fail(NH_E_ARGUMENT, "this wide product takes no fp32 rows whole (ask gemm_takes_whole first)");
@@ -1184,7 +1184,7 @@ bool gemm_shares_rows(const nh_device *d, const int32_t (&elements)[3], const ui
         return true;
     }
     for (int s = 0; s < 3; s++)
-        if (!mfma_takes(elements[s], K, X, W[s]) || wide_form(d, elements[s], N[s], K, 2u * M, 0u).operands != wide_form(d, elements[0], N[0], K, 2u * M, 0u).operands) return false;
+        if (!mfma_takes(elements[s], K, X, W[s]) || wide_form(d, elements[s], N[s], K, 2u * M, false, 0u).operands != wide_form(d, elements[0], N[0], K, 2u * M, false, 0u).operands) return false;
     return true;
 }
 

@@ -109,21 +109,22 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
         tmp[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[i], fine, tmp[i], 0, 0, 0);
     };
     // Where a chain of `chain` units ends, its sums leave the accumulators.  (Rows of residues, 2^11 below the rows they belong to, stay
-    // and run on.)  SPARE: three row tiles leave registers for the sums of whole chains.  Elsewhere they go to the outputs' own place
-    // (or to scratch, where that still holds the residuals), each lane the outputs it writes at the end (18944 x 3584 Q3_K at 200
-    // packed rows, two chains of seven units, against one: 83 60.6 -> 59.5 us, 84 64.5 -> 69.0).
-    constexpr bool SPARE = MT == 3 && !(ELEMENT == NH_Q6_K && WN == 4);
+    // and run on.)  SPARE: so many of a tile's sixteen registers hold on.  Sums that find none go to the outputs' own place (or to
+    // scratch, where that still holds the residuals), each lane the outputs it writes at the end (18944 x 3584 Q3_K at 200 packed
+    // rows, two chains of seven units, against one: 83 60.6 -> 59.5 us, 84 64.5 -> 69.0; 512 half rows, chains of four: 42 in registers 123.6
+    // us, 83 through memory 113.7 -> 129.4).
+    constexpr int SPARE = shared_rows_spare(ELEMENT, WN, MT);
     const uint32_t pieces = p.pieces;
-    float whole[SPARE ? MT : 1][8] = {};
+    float whole[SPARE ? MT : 1][SPARE ? SPARE : 1] = {};
     auto keep = [&](auto each, bool first, bool leave) __attribute__((always_inline)) {
         constexpr int EACH = decltype(each)::value;  // every packed row, or every second
-        if constexpr (SPARE && EACH == 2) {
+        if constexpr (SPARE * EACH >= 16) {
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    whole[i][e] += acc[i][2 * e];
-                    acc[i][2 * e] = leave ? 0.0f : whole[i][e];
+                for (int e = 0; e < 16 / EACH; e++) {
+                    whole[i][e] += acc[i][EACH * e];
+                    acc[i][EACH * e] = leave ? 0.0f : whole[i][e];
                 }
             return;
         }
