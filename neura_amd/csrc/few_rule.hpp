@@ -119,11 +119,12 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
     }
     SharedShape best = SHARED_NONE;
     double least = other / 1.08;
-    // Places between chains, and the end: nothing where three row tiles keep whole rows' sums in registers, 1.5 microseconds a turn for two, 2
-    // through memory (84: 37888 x 3584 Q3_K at 200 packed rows 130.0 -> 137.1) and 5 of half rows there, which have twice the sums.
-    // `halves`: rows of half activations.  Their outputs are twice as many too, 5 us here and not in few rows, whose shares meet
-    // in LDS: over 400 products of 70 to 1024 of them the pick takes 1.003 times the fastest form's time, at most 1.07 times the other
-    // form's; with the line of whole rows up to 1.26 (17920 x 1536 at 200 Q3_K few rows 32.9, 83 41.4; 18944 x 3584 at 512 135.7, 42 123.6).
+    // Places between chains, and the end: nothing where three row tiles keep whole rows' sums in registers, 2 microseconds a turn for two
+    // (which leave a compute unit two workgroups in place of three: 18944 x 3584 Q3_K at 400 packed rows 108 -> 120) and through memory (84:
+    // 37888 x 3584 Q3_K at 200 130.0 -> 137.1), 7 of half rows there, which have twice the sums.
+    // `halves`: rows of half activations.  Their outputs are twice as many too, 2 us here and not in few rows, whose shares meet
+    // in LDS: over 400 products of 70 to 1024 of them the pick takes 1.003 times the fastest form's time, at most 1.01 times the other
+    // form's; with the line of whole rows up to 1.26 (17920 x 1536 at 200 Q3_K few rows 32.9, 83 41.4).
     const uint32_t chain = shared_rows_chain(element, N, K, rows, compute_units), places = chain < units ? (units - 1u) / chain + 1u : 0u;
     const auto consider = [&](SharedShape shape, uint32_t waves, uint32_t mt, double pair, double one, double base, double turn, double pack) {
         if (!(pair > 0.0)) return;
@@ -131,8 +132,8 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
         const uint64_t full = workgroups / slots, left = workgroups % slots;
         const bool lone = waves == 4u && left && left <= cu;
         const uint64_t turns = full + (left ? 1u : 0u);
-        const double place = mt == 2u ? 1.5 : halves ? 5.0 : shared_rows_spare(element, waves, mt) ? 0.0 : 2.0;
-        const double time = base + (halves ? 5.0 : 0.0) + (double)turns * (turn + units * pair + place * places) - (lone ? units * (pair - one) : 0.0) + pack * millions;
+        const double place = mt == 2u ? 2.0 : halves ? 7.0 : shared_rows_spare(element, waves, mt) ? 0.0 : 2.0;
+        const double time = base + (halves ? 2.0 : 0.0) + (double)turns * (turn + units * pair + place * places) - (lone ? units * (pair - one) : 0.0) + pack * millions;
         if (time < least) least = time, best = shape;
     };
     consider(SHARED_42, 4u, 2u, t.pair2, t.one2, 5.0, 5.5, 1.7);

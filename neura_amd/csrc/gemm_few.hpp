@@ -65,7 +65,7 @@ struct FewParams {
     uint32_t slices;        // workgroups (blockIdx.z) that share the K of the same tiles
     float *partial;         // FEW_PARTIAL_BYTES of scratch for their sums
     uint32_t *meets;        // FEW_MEETS words, zero between launches: workgroups of a place that have left their sums
-    uint32_t chain;         // of shared rows: units after which sums leave the registers (no fewer than all of K: never)
+    uint32_t chain;         // of shared rows: units after which sums leave the accumulators
     float *Y1;              // where not null, columns from end0 on go there, with the same ldy (Y's first: Y1[n - end0])
 };
 

@@ -25,8 +25,9 @@ namespace {
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t *at, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(at), 0, bytes, 0x00020000); }
 
-// WN: waves side by side, 32 columns each; MT: tiles of 32 packed rows a wave multiplies its unpacked weights by.
-template <int ELEMENT, int WN, int MT>
+// WN: waves side by side, 32 columns each; MT: tiles of 32 packed rows a wave multiplies its unpacked weights by; CHAINED: sums leave the
+// accumulators every p.chain units (a kernel of one chain is one of fewer registers).
+template <int ELEMENT, int WN, int MT, bool CHAINED>
 __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint32_t column_tiles, uint32_t row_blocks) {
     typedef typename FewOf<ELEMENT>::type Weights;
     constexpr int STEPS = Weights::STEPS, PLANES = Weights::PLANES, CLOSED = Weights::CLOSED, HALF = STEPS / 2, REGIONS = 4 * HALF;
@@ -111,8 +112,9 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
     // Where a chain of `chain` units ends, its sums leave the accumulators.  (Rows of residues, 2^11 below the rows they belong to, stay
     // and run on.)  SPARE: so many of a tile's sixteen registers hold on.  Sums that find none go to the outputs' own place (or to
     // scratch, where that still holds the residuals), each lane the outputs it writes at the end (18944 x 3584 Q3_K at 200 packed
-    // rows, two chains of seven units, against one: 83 60.6 -> 59.5 us, 84 64.5 -> 69.0; 512 half rows, chains of four: 42 in registers 123.6
-    // us, 83 through memory 113.7 -> 129.4).
+    // rows, two chains of seven units, against one: 83 60.6 -> 59.5 us, 84 64.5 -> 69.0; 512 half rows: 42 in registers 123.6, 83 through
+    // memory 113.7 -> 129.4).  Kernels of one chain do without, in 20 to 40 registers fewer (18944 x 3584 Q4_K at 400 packed rows 43 111 ->
+    // 108 us; 42, of which a compute unit then holds three workgroups, 118 -> 108).
     constexpr int SPARE = shared_rows_spare(ELEMENT, WN, MT);
     const uint32_t pieces = p.pieces;
     float whole[SPARE ? MT : 1][SPARE ? SPARE : 1] = {};
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
         if (pieces == 2u) keep(std::integral_constant<int, 2>(), first, leave);
         else keep(std::integral_constant<int, 1>(), first, leave);
     };
-    uint32_t until = p.chain;
+    uint32_t until = CHAINED ? p.chain : 0u;
     read_rows(0, 0);
     ready(w, 0);
     w.step(0);
@@ -262,7 +264,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
                 }
             }
         }
-        if (unit + 1u == until && until < units) keep_rows(until == p.chain, true), until += p.chain;
+        if (CHAINED && unit + 1u == until && until < units) keep_rows(until == p.chain, true), until += p.chain;
     }
     __builtin_amdgcn_s_setprio(0);
     // (every scale before the first store, and a tile's residuals before its stores: the compiler cannot tell them from the outputs, and
@@ -274,7 +276,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
         for (int q = 0; q < 4; q++)
 #pragma unroll
             for (int e = 0; e < 4; e++) scales[i][q][e] = pieces == 2u ? p.unscale[min((tile0 + i) * 16u + 4u * q + 2u * part + e / 2, p.M - 1u)] : 1.0f;  // (halves are packed as they lie)
-    if (p.chain < units) keep_rows(false, false);
+    if (CHAINED && p.chain < units) keep_rows(false, false);
 
     // ---- out: lane (l32, part) holds column l32 of a 32 x 32 block; register 4q + e is row 8q + 4 part + e
     const uint32_t n = n0 + l32;
@@ -305,20 +307,26 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_wide_kernel(FewParams p, uint
     }
 }
 
-template <int ELEMENT, int WN, int MT>
-int32_t launch_shape(nh_device *d, FewParams p) {
+template <int ELEMENT, int WN, int MT, bool CHAINED>
+int32_t launch_chained(nh_device *d, const FewParams &p) {
     typedef typename FewOf<ELEMENT>::type Weights;
     constexpr size_t lds = MT * (3u * (Weights::STEPS / 2u) * 4096u + (Weights::FLOORS ? 2048u : 0u));
     static OnceADevice sized;
-    NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT>), lds));
+    NH_HIP(raise_lds(sized, d, reinterpret_cast<const void *>(gemm_wide_kernel<ELEMENT, WN, MT, CHAINED>), lds));
+    const uint32_t column_tiles = (p.N + 32u * WN - 1u) / (32u * WN), row_blocks = ((p.rows + 31u) / 32u + MT - 1u) / MT;
+    hipLaunchKernelGGL((gemm_wide_kernel<ELEMENT, WN, MT, CHAINED>), dim3((column_tiles * row_blocks + 7u) / 8u * 8u), dim3(64 * WN), lds, d->stream, p, column_tiles, row_blocks);
+    NH_HIP(hipGetLastError());
+    return NH_OK;
+}
+
+template <int ELEMENT, int WN, int MT>
+int32_t launch_shape(nh_device *d, FewParams p) {
     // (beside residuals the chains' sums wait in scratch: more of them than that holds stay in one chain)
     const uint32_t compute_units = (uint32_t)d->compute_units;
     const uint64_t residuals = p.residual ? (uint64_t)p.M * p.N * sizeof(float) : 0u;
-    p.chain = shared_rows_overflow(ELEMENT, p.N, p.K, p.rows, residuals, compute_units) ? ~0u : shared_rows_chain(ELEMENT, p.N, p.K, p.rows, compute_units);
-    const uint32_t column_tiles = (p.N + 32u * WN - 1u) / (32u * WN), row_blocks = ((p.rows + 31u) / 32u + MT - 1u) / MT;
-    hipLaunchKernelGGL((gemm_wide_kernel<ELEMENT, WN, MT>), dim3((column_tiles * row_blocks + 7u) / 8u * 8u), dim3(64 * WN), lds, d->stream, p, column_tiles, row_blocks);
-    NH_HIP(hipGetLastError());
-    return NH_OK;
+    p.chain = shared_rows_chain(ELEMENT, p.N, p.K, p.rows, compute_units);
+    if (p.chain >= shared_rows_units(ELEMENT, p.K) || shared_rows_overflow(ELEMENT, p.N, p.K, p.rows, residuals, compute_units)) return launch_chained<ELEMENT, WN, MT, false>(d, p);
+    return launch_chained<ELEMENT, WN, MT, true>(d, p);
 }
 
 // (eight waves copy a step of Q8_0 in whole pieces only for two row tiles and four; two planes of Q6_K leave no registers for four)
