@@ -25,7 +25,9 @@ constexpr int MAX_GROUPS = 8;
 struct AttentionParams {
     const float *q;
     float *out;
-    float *partial;      // [unit][section][group][width + 2] when sections > 1
+    // when sections > 1.  Steps: [unit][section][group][width + 2], a section's sums, maximum and mass together.  Fills:
+    // [unit][section][group][width] sums, then [unit][section][group] pairs of maximum and mass
+    float *partial;
     uint64_t q_sh, q_sb, q_sr, o_sh, o_sb, o_sr;
     const uint16_t *cache_k, *cache_v;  // as bytes of another element for attention_any_kernel
     uint32_t heads, kv_heads, groups, batch, rows, capacity, keys, sections;
@@ -379,8 +381,9 @@ __device__ __forceinline__ void states_as_halves(const u32x4 (&raw)[WORDS], u32x
 //           and sum never leave its two lanes.
 //   values  O^T[channel][column] += V^T[channel][key] . P^T[key][column]: the weights go back in as the B operand
 //           straight from the registers C left them in (again as value and residue planes), and the value tile, which
-//           the workgroup wrote to LDS transposed, is the A operand in that same key order.
-// The running maximum, sum and the 32 x 64 accumulators of a column live in its two lanes; nothing is folded afterwards.
+//           lies in LDS as it is stored and is transposed on its way out, is the A operand in that same key order.
+// The running maximum, sum and the accumulators of a column live in its two lanes.  Where several workgroups share a block's walk each
+// leaves them in memory and attention_fill_fold_kernel adds them up.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float float4_loose __attribute__((ext_vector_type(4), aligned(4)));
@@ -396,7 +399,7 @@ __host__ __device__ constexpr size_t fill_lds_bytes(int width, int element, bool
 template <int WIDTH, int CE = NH_F16, bool SPLIT = false>
 __global__ __launch_bounds__(SPLIT ? 512 : 256) void attention_tile_kernel(AttentionParams p, uint32_t rows_per_wave) {
     fetch_parameters(p);
-    static_assert(!SPLIT || CE != NH_F32, "two sets of staged tiles of single states do not fit the static LDS");
+    static_assert(!SPLIT || CE != NH_F32, "two sets of staged tiles of single states do not fit the LDS");
     constexpr int SETS = SPLIT ? 2 : 1;
     constexpr int TK = 32;                       // keys per tile
     constexpr int STEPS = WIDTH / 16;            // MFMA steps over the channels of a score

@@ -312,7 +312,7 @@ struct AttentionArgs {
     const uint16_t *cache_k, *cache_v;
     uint32_t heads, kv_heads, batch, rows, width, capacity, keys;
     const uint32_t *cursor;
-// where the host knows how long each plane is: device words, the sections each plane's walk takes in a fill (attention_fill_sections),
+    // where the host knows how long each plane is: device words, the sections each plane's walk takes in a fill (attention_fill_sections),
     // and the most of them (0: as many for every plane as `keys` positions take)
     const uint32_t *plane_sections = nullptr;
     uint32_t most_sections = 0;

@@ -90,9 +90,11 @@ inline bool shared_rows_overflow(int32_t element, uint32_t N, uint32_t K, uint32
 // that few_rows_win picks).  Times in microseconds of all three, each a line fitted to 649 products of the decoder shapes at 20 to
 // 1024 packed rows (mean error 4 % here, 4 % of the tiles, 7 % of the product of few rows): turns of the chip, a base and the units
 // (256 k, Q8_0 128) of each; two workgroups of four waves share a compute unit, and one alone walks faster.  It wants to win by
-// 8 %, so that no line's error makes a product slower: where it is picked it takes 0.87 of the other form's time on average, at most 1.05
-// (7B shape, packed rows, other / here: gate|up Q4_K 128 101 / 74, 200 145 / 106, 1024 392 / 331; Q3_K 1024 455 / 310; Q8_0 200
-// 203 / 143; ffn_down Q4_K 300 119 / 103; 0.5B gate|up Q8_0 800 62 / 47).  Up to two row tiles the walk is latency, not work.
+// 8 %, so that no line's error makes a product slower: where it is picked it takes 0.9 of the other form's time on average, at most 1.05
+// (7B shape, packed rows, other / here: gate|up Q4_K 74 56 / 50, 128 76 / 65, 400 208 / 188, 1024 406 / 344; Q3_K 1024 436 / 329;
+// Q8_0 200 and ffn_down Q4_K 300 tie).  The lines are of one matrix again and again, which the Infinity Cache holds; over matrices from
+// HBM every form takes 2 to 15 % longer in the same order (gate|up Q4_K 74 63 / 58, 128 82 / 67, 1024 407 / 352).  Up to two row tiles the
+// walk is latency, not work.
 enum SharedShape { SHARED_NONE = 0, SHARED_42 = 42, SHARED_43 = 43, SHARED_83 = 83, SHARED_84 = 84 };
 inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, uint32_t rows, bool halves, uint32_t compute_units) {
     if (rows <= 64u || !N || !K || !compute_units) return SHARED_NONE;

@@ -12,9 +12,9 @@
 // accumulators, in units of the operands, where products of their own took three instructions an output; 32-bit offsets from
 // uniform buffer descriptors; the next region's operands made and read while this one's products run, matrix and vector
 // instructions by turns.  A region of four products and 22 vector instructions takes 36 cycles a product with two waves a SIMD.
-// At full occupancy the card's clock gives way (2.3 to 1.8 GHz): 37888 x 3584 at 1024 packed rows, Q4_K, 331 us with the packing = 840
-// TFLOP/s, two launches of the 128 x 128 tiles 392; at 200 rows 106, the product of few rows twice 145; 2-norm from 64 bits
-// 1.3e-7 (tiles 2.3e-7: uncentred).
+// At full occupancy the card's clock gives way (2.3 to 1.8 GHz): 37888 x 3584 at 1024 packed rows, Q4_K, 344 us with the packing over one
+// matrix again and again = 810 TFLOP/s (the 128 x 128 tiles 406), 352 over matrices from HBM, 351 to 366 without it in a fill; at 128 rows 65
+// (few rows 76, tiles 77), at 74 rows 50, and 58 from HBM (few rows 56 and 63); 2-norm from 64 bits 1.2e-7 (tiles 1.7e-7 and more: uncentred).
 #include "gemm_operands.hpp"
 
 #include <type_traits>

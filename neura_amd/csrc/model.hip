@@ -281,7 +281,7 @@ int32_t forward(nh_model *m, uint32_t rows, bool any_inactive, bool products_onl
             if (paired || both) g.norm_w = m->ffn_norm[L], g.eps = c.eps, u.packed = true;
             if (both) g.gated = true, g.W_more[0] = m->ffn_up[L], g.end[0] = g.end[1] = F;
             // the two as one product with outputs of their own, where the tiles end together: twice the columns leave a smaller part of the
-            // chip's last turn empty (7B shape, 74 packed rows 65 -> 49 us, 1024 rows 400 -> 331)
+            // chip's last turn empty (7B shape in a fill, 74 packed rows 73 -> 56 us, 1024 rows 418 -> 351 to 366)
             const bool joined = paired && gemm_stacks(element_at(m, L, GATE), H, m->h, m->ffn_gate[L], m->ffn_up[L], nullptr, F, 0);
             if (joined) g.N = 2 * F, g.W_more[0] = m->ffn_up[L], g.end[0] = F, g.end[1] = 2 * F, g.Y_more = m->up;
             if ((status = launch_gemm(d, g)) != NH_OK) return status;
