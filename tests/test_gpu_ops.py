@@ -642,7 +642,8 @@ def test_both_forms_of_a_wide_product(device, monkeypatch, form, element, M, N, 
     (NH_Q3_K, 129, 64, 768, True), (NH_Q8_0, 50, 300, 192, False), (NH_Q8_0, 97, 270, 64, True), (NH_Q8_0, 33, 130, 4864, False),
     (NH_Q3_K, 70, 100, 4864, True), (NH_Q5_K, 45, 300, 8960, False)])
 def test_wide_products_of_shared_rows(device, monkeypatch, shape, element, M, N, K, half):
-    """The wide product whose workgroups share their rows through LDS, each shape of it forced: columns and row tiles past the last, rows
+    """The wide product whose workgroups share their rows through LDS, each shape of it forced (83 of Q8_0 is 43, 84 of Q6_K is 83: they have
+    no kernels of their own): columns and row tiles past the last, rows
     that end inside a tile, one unit and several, an odd number of Q8_0's steps -- against the exact product at the bar of
     test_both_forms_of_a_wide_product, with random blocks (whose minimums outweigh some scales by more than a half holds), with a
     block's scale zero and its minimum not, with outliers on zero weights, and with an infinity in one row."""
