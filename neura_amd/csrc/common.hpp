@@ -225,7 +225,8 @@ struct GemvArgs {
     void *pairs_out = nullptr;
 };
 int32_t launch_gemv(nh_device *d, const GemvArgs &args);
-// whether launch_gemv takes this product at more rows than eight (nine to sixteen, where one workgroup holds the rows it norms)
+// whether launch_gemv walks the matrix once for this product's nine to sixteen rows (where one workgroup holds the rows it norms); it takes any
+// number of rows of a plain product, a few at a time where no form takes more
 bool gemv_takes_many(const GemvArgs &args);
 // whether launch_gemv can merge attention sections of `width` channels a head into the activation row of this product
 bool gemv_merges_sections(const GemvArgs &args, uint32_t width);

@@ -1441,7 +1441,6 @@ bool gemv_appends_value(const GemvArgs &a) {
 bool gemv_takes_many(const GemvArgs &a) { return a.rows > 8 && (!a.norm_w || a.K <= 1792u) && rows_takes(a); }
 
 int32_t launch_gemv(nh_device *d, const GemvArgs &a) {
-    if (a.rows > 8 && !rows_takes(a)) return fail(NH_E_ARGUMENT, "a narrow product takes one to eight rows, not %u (ask gemv_takes_many first)", a.rows);
     if (!a.rope && !a.append_value && (a.bias[0] || a.bias[1] || a.bias[2]))
         return fail(NH_E_ARGUMENT, "a product adds a bias only where it folds the rotation in or appends value rows");
     if (a.append_value && !gemv_appends_value(a))

@@ -529,6 +529,28 @@ def test_nine_to_sixteen_planes_on_the_half_precision_tiles(device, batch, shape
     one.release(), one_weights.release(), model.release(), weights.release()
 
 
+@pytest.mark.parametrize("planes,shape,element,few", [
+    (9, dict(layers=2, hidden=96, heads=3, kv_heads=1, head_dim=32, ffn=160, vocab=320, tied=True), NH_Q8_0, None),
+    (17, dict(layers=2, hidden=96, heads=3, kv_heads=1, head_dim=32, ffn=160, vocab=320, tied=True), NH_Q8_0, None),
+    (17, TINY, NH_Q8_0, "0"), (9, SMALL_Q4, NH_Q6_K, "0"), (17, SMALL_Q4, NH_Q4_K, "0"), (17, dict(SMALL_Q4, layers=1, vocab=1003), NH_Q4_K, "0")])
+def test_heads_of_more_planes_that_no_wide_product_takes(device, monkeypatch, planes, shape, element, few):
+    """A head whose rows the wide product does not take whole (Q8_0 rows of an odd number of blocks, here three; NEURA_HIP_GEMM_FEW=0) is a narrow
+    product of more than eight rows, walked a few at a time: logits and tokens of steps as the oracle's, and the products can be timed."""
+    if few:
+        monkeypatch.setenv("NEURA_HIP_GEMM_FEW", few)
+    model, ref, weights = build(device, shape, element, batch=planes, context=16, seed=planes)
+    tokens = np.random.default_rng(planes).integers(0, shape["vocab"], planes)
+    for step in range(3):
+        want_logits, want = ref.forward(tokens, 1, [step] * planes)
+        got = model.decode_step(tokens, [step] * planes)
+        assert np.abs(model.logits() - want_logits).max() <= 1e-3 * np.abs(want_logits).max(), step
+        clear = margins(want_logits) > 2e-3 * np.abs(want_logits).max()
+        assert (np.asarray(got)[clear] == np.asarray(want)[clear]).all(), (step, margins(want_logits))
+        tokens = want
+    assert model.time_products(1)[1] > 0
+    model.release(), weights.release()
+
+
 def test_decode_refuses_what_the_reference_refuses(device):
     model, ref, weights = build(device, TINY, NH_Q8_0, batch=1, context=8)
     with pytest.raises(NeuraError):   # cursor at the context (batch.rs:1627-1632)
