@@ -429,14 +429,41 @@ def test_q4_k_products_of_several_rows_at_the_edges_of_their_plans(device, N, K,
     x[0, 7] = 1e10
     raw = blocks.reshape(-1)
     exact = x[0].astype(np.float64) @ oracle.unpack(NH_Q4_K, raw, N * K).reshape(N, K).astype(np.float64).T
-    if K == 256:  # (the outlier's super-block holds its neighbours below its scale: two half pieces, 2^-22 of their own size down to 2^-27 of it)
-        return
+    # (the outlier's super-block holds its neighbours to 2^-23 of their own size, or 2^-48 of the outlier where that is more)
     ours = device.gemv(NH_Q4_K, raw, N, K, x)[0]
-    others = np.abs(x[0]).astype(np.float64)
-    others[7] = 0.0
-    others[:256] = 0.0
-    lost = 1e10 * 2.0 ** -36 * np.abs(oracle.unpack(NH_Q4_K, raw, N * K).reshape(N, K)[:, :256]).astype(np.float64).sum(axis=1)
+    lost = 1e10 * 2.0 ** -48 * np.abs(oracle.unpack(NH_Q4_K, raw, N * K).reshape(N, K)[:, :256]).astype(np.float64).sum(axis=1)
     assert (np.abs(ours - exact) <= 1e-5 * np.abs(exact).max() + lost).all()
+
+
+@pytest.mark.parametrize("N,K,rows", [(64, 256, 3), (512, 3584, 3), (512, 3584, 8), (16416, 1536, 4), (16416, 3584, 8), (256, 18944, 5)])
+def test_rows_with_a_mean_keep_their_bits_beside_weights_without_one(device, N, K, rows):
+    """Several rows of mean 0, 1 and 8 (and magnitudes alone) against matrices whose minimums centre their values, as a quantized matrix's do:
+    what the codes add up to and what the minimums take off again are 60 to 500 times the result.  Every plan of the half-precision tiles
+    stays within four half units in the last place of an fp32 number, 2^-22, of the exact product (2-norm; an activation is held to
+    2^-23, and the sums' roundings are as large again: 1.2 to 1.9e-7 measured; minimums and codes weighed apart are 5 to 25e-7 away)."""
+    rng = np.random.default_rng(N + K + rows)
+    blocks = np.array(synth.q4_k_random(rng, N * K), copy=True).reshape(-1, 144)
+    d = (1e-3 * (0.75 + 0.5 * rng.random(len(blocks)))).astype(np.float16)
+    blocks[:, 0:2] = d.view(np.uint8).reshape(-1, 2)
+    blocks[:, 2:4] = (d.astype(np.float32) * 7.5).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    sc = 32 + (rng.integers(0, 32, (len(blocks), 8))).astype(np.uint8)  # scales and minimums alike
+    blocks[:, 4:8] = blocks[:, 8:12] = sc[:, :4] | ((sc[:, 4:] >> 4) << 6)
+    blocks[:, 12:16] = (sc[:, 4:] & 15) | ((sc[:, 4:] & 15) << 4)
+    raw = blocks.reshape(-1)
+    weights = oracle.unpack(NH_Q4_K, raw, N * K).reshape(N, K).astype(np.float64)
+    assert np.abs(weights.mean()) < 0.05 * weights.std()
+    # (the oracle's weights are fp32 numbers: exact ones, d sc q - dmin m in 64 bits)
+    scales = (d.astype(np.float64)[:, None] * sc, np.frombuffer(blocks[:, 2:4].tobytes(), np.float16).astype(np.float64)[:, None] * sc)
+    codes = np.stack([blocks[:, 16:].reshape(-1, 4, 32) & 15, blocks[:, 16:].reshape(-1, 4, 32) >> 4], axis=2).reshape(-1, 8, 32)
+    exact_weights = (scales[0][:, :, None] * codes - scales[1][:, :, None]).reshape(N, K)
+    assert np.abs(exact_weights - weights).max() <= 2e-6 * np.abs(weights).max()
+    normal = rng.standard_normal((rows, K))
+    for x in (normal, normal + 1.0, normal + 8.0, np.abs(normal)):
+        x = x.astype(np.float32)
+        exact = x.astype(np.float64) @ exact_weights.T
+        apart = np.linalg.norm(device.gemv(NH_Q4_K, raw, N, K, x) - exact) / np.linalg.norm(exact)
+        print("%d x %d, %d rows: %.3g" % (N, K, rows, apart))
+        assert apart <= 2.0 ** -22, apart
 
 
 def test_q4_k_product_on_the_matrix_cores_keeps_non_finite_inputs_visible(device, monkeypatch):
