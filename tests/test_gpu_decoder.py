@@ -483,11 +483,11 @@ def test_decode_on_half_precision_tiles_matches_the_oracle(device, monkeypatch, 
     model.release(), weights.release()
 
 
-@pytest.mark.parametrize("batch", [3, 8])
-def test_planes_of_a_decoder_whose_rows_are_two_slices(device, batch):
-    """A hidden width of 3840 is two slices of the half-precision tiles: q|k|v and gate|up leave the norm's scalar to the fold that adds
-    their slices up, and the rotation to its own kernel; against the oracle's logits and tokens."""
-    shape = dict(layers=1, hidden=3840, heads=4, kv_heads=2, head_dim=64, ffn=512, vocab=320, tied=False)
+@pytest.mark.parametrize("batch,hidden", [(3, 3840), (8, 3840), (3, 4352), (8, 4352)])
+def test_planes_of_a_decoder_whose_rows_are_two_slices(device, batch, hidden):
+    """A hidden width of 4352 is two slices of the half-precision tiles: q|k|v and gate|up leave the norm's scalar to the fold that adds
+    their slices up, and the rotation to its own kernel; one of 3840 is one, the rotation in it; against the oracle's logits and tokens."""
+    shape = dict(layers=1, hidden=hidden, heads=4, kv_heads=2, head_dim=64, ffn=512, vocab=320, tied=False)
     model, ref, weights = build(device, shape, NH_Q4_K, batch=batch, context=8, seed=12)
     tokens = np.random.default_rng(13).integers(0, shape["vocab"], batch)
     for step in range(3):

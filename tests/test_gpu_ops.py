@@ -398,10 +398,12 @@ def test_q4_k_products_of_several_rows_four_rows_to_an_mfma(device, N, K, rows):
     assert np.array_equal(device.gemv(NH_Q4_K, raw, N, K, np.zeros((rows, K), np.float32)), np.zeros((rows, N), np.float32))
 
 
-@pytest.mark.parametrize("N,K,rows", [(16, 256, 3), (16, 3584, 8), (32, 3840, 7), (1536, 2048, 5), (1536, 2304, 8), (16384, 512, 3), (16400, 768, 6), (16400, 2304, 8), (240, 7680, 4)])
+@pytest.mark.parametrize("N,K,rows", [(16, 256, 3), (16, 3584, 8), (32, 3840, 7), (1536, 2048, 5), (1536, 2304, 8), (16384, 512, 3), (16400, 768, 6), (16400, 2304, 8), (240, 7680, 4),
+                                      (4096, 512, 3), (4112, 768, 8), (64, 4096, 8), (4112, 4096, 4), (16400, 4096, 5), (48, 4352, 6)])
 def test_q4_k_products_of_several_rows_at_the_edges_of_their_plans(device, N, K, rows):
     """Three to eight activation rows on the half-precision tiles where their plans change: one tile, the most and the fewest super-blocks of
-    a slice, slices that a fold adds up, eight super-blocks and nine, tall matrices with a last round that few workgroups take.  Half of
+    a slice (sixteen; seventeen are two slices), slices that a fold adds up, eight super-blocks and nine, as many tiles as compute units and one more,
+    tall matrices with a last round that few workgroups take.  Half of
     the sub-blocks have no minimum and column 7 meets codes of zero there: an outlier of 1e10 leaves the other numbers' products whole
     (codes that a kernel centres keep exact zeros exact).  N(0, 1) rows and 10^+-6 either side are held to the exact product: at most
     four times the oracle's own fp32 distance, or 2e-6 of the largest output."""
@@ -435,7 +437,7 @@ def test_q4_k_products_of_several_rows_at_the_edges_of_their_plans(device, N, K,
     assert (np.abs(ours - exact) <= 1e-5 * np.abs(exact).max() + lost).all()
 
 
-@pytest.mark.parametrize("N,K,rows", [(64, 256, 3), (512, 3584, 3), (512, 3584, 8), (16416, 1536, 4), (16416, 3584, 8), (256, 18944, 5)])
+@pytest.mark.parametrize("N,K,rows", [(64, 256, 3), (512, 3584, 3), (512, 3584, 8), (16416, 1536, 4), (16416, 3584, 8), (256, 18944, 5), (512, 4096, 6)])
 def test_rows_with_a_mean_keep_their_bits_beside_weights_without_one(device, N, K, rows):
     """Several rows of mean 0, 1 and 8 (and magnitudes alone) against matrices whose minimums centre their values, as a quantized matrix's do:
     what the codes add up to and what the minimums take off again are 60 to 500 times the result.  Every plan of the half-precision tiles
