@@ -25,7 +25,8 @@ inline uint32_t few_row_tiles(uint32_t N, uint32_t rows, uint32_t compute_units)
 // 128 to 8192 packed rows over the 0.5B, 1.5B and 7B shapes (us, tiles / few): Q8_0 18944 x 3584 at 512 rows 157 / 211 and at 1024 262 /
 // 331 (full rounds), 3584 x 3584 at 512 56 / 48 (112 workgroups), 4608 x 3584 at 1024 105 / 87 (288), 4864 x 896 at 1024 47 / 35 (304);
 // Q5_K 141 / 150, 51 / 40, 95 / 76 of the first, third and fourth; Q4_K 125 / 148, 43 / 39, 82 / 77.  The form it picks is within 8 % of the
-// faster one at those points.  Q6_K and Q3_K have no tiles: few rows up to the height of a grid, and shared rows below.
+// faster one at those points.  (`share` goes by few_row_tiles: threes that few_pass_tiles takes beyond it are at few columns, where the shares of twos
+// decide as well; asked for them the rule moves 4 of 1368 points of such matrices, 3 % slower.)  Q6_K and Q3_K have no tiles: few rows up to the height of a grid, and shared rows below.
 inline bool few_rows_win(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
     if (rows <= 96u) return true;
     if (rows > 65535u * 32u) return false;  // (row tiles are blockIdx.y)
@@ -69,8 +70,9 @@ inline FewSplit few_split(int32_t element, uint32_t N, uint32_t K, uint32_t rows
 // passes, split as they are best split, cost less: fewer workgroups, each a longer walk, and where twos start a second round or leave a
 // slice to meet, the shorter one (us, twos / threes: 896 x 4864 Q8_0 at 800 packed rows 37.0 / 29.1, at 960 38.0 / 43.5; 3584 x 18944 Q8_0 at 74
 // 55.1 / 44.6, Q6_K 53.0 / 46.0, Q4_K 42.2 / 39.3, at 104 43.1 / 54.0; 3584 x 3584 Q6_K at 140 24.4 / 20.2; 1536 x 8960 Q8_0 at 400 47.4 / 39.5).  Over
-// 239 products of the decoder shapes at 74 to 960 packed rows it takes 0.975 times the twos' time, at most 1.017.  Never with fewer shares
-// of K: those add up less exactly.
+// 239 products of the decoder shapes at 74 to 960 packed rows it takes 0.975 times the twos' time, at most 1.017; over 1368 of matrices of up to
+// 4096 columns at 66 to 1024 the pass it picks takes 1.007 times the faster one's time, with a ratio of each element's own (1.16 to 1.37 for 6 / 5)
+// 1.009.  Never with fewer shares of K: those add up less exactly.
 inline uint32_t few_pass_tiles(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
     const uint32_t mt = few_row_tiles(N, rows, compute_units);
     if (mt != 2u || rows <= 64u || (N + 31u) / 32u > compute_units / 2u) return mt;
@@ -83,7 +85,7 @@ inline uint32_t few_pass_tiles(int32_t element, uint32_t N, uint32_t K, uint32_t
 inline uint32_t shared_rows_units(int32_t element, uint32_t K) { return element == NH_Q8_0 ? (K / 64u + 1u) / 2u : (K / 64u + 3u) / 4u; }
 
 // Units of k a wave of the product of shared rows adds up before its sums leave the accumulators (a chain): as many as a share of the
-// product of few rows has, where that is the form it takes over from, for one chain over all of K adds up less exactly than shares that
+// product of few rows has in the passes of few_row_tiles (threes by cost have as many or more), where that is the form it takes over from, for one chain over all of K adds up less exactly than shares that
 // meet (2-norm from 64 bits, few rows / one chain / here: Q3_K 3584 x 18944 at 600 packed rows 1.15e-7 / 1.75 / 1.16, Q6_K at 800 1.56 /
 // 2.41 / 1.56, Q5_K at 600 1.56 / 1.99 / 1.49, Q8_0 17920 x 1536 at 200 1.10 / 1.38 / 1.10).  The tiles are one chain themselves.
 inline uint32_t shared_rows_chain(int32_t element, uint32_t N, uint32_t K, uint32_t rows, uint32_t compute_units) {
@@ -106,7 +108,8 @@ inline bool shared_rows_overflow(int32_t element, uint32_t N, uint32_t K, uint32
 // (256 k, Q8_0 128) of each; two workgroups of four waves share a compute unit, and one alone walks faster.  It wants to win by
 // 8 %, so that no line's error makes a product slower: where it is picked it takes 0.9 of the other form's time on average, at most 1.05
 // (7B shape, packed rows, other / here: gate|up Q4_K 74 56 / 50, 128 76 / 65, 400 208 / 188, 1024 406 / 344; Q3_K 1024 436 / 329;
-// Q8_0 200 and ffn_down Q4_K 300 tie).  The lines are of one matrix again and again, which the Infinity Cache holds; over matrices from
+// Q8_0 200 and ffn_down Q4_K 300 tie).  Over 1368 products of matrices of up to 4096 columns at 66 to 1024 packed rows what is picked takes 1.005 times the
+// fastest form's time.  The lines are of one matrix again and again, which the Infinity Cache holds; over matrices from
 // HBM every form takes 2 to 15 % longer in the same order (gate|up Q4_K 74 63 / 58, 128 82 / 67, 1024 407 / 352).  Up to two row tiles the
 // walk is latency, not work.
 enum SharedShape { SHARED_NONE = 0, SHARED_42 = 42, SHARED_43 = 43, SHARED_83 = 83, SHARED_84 = 84 };
@@ -126,7 +129,7 @@ inline SharedShape shared_rows_shape(int32_t element, uint32_t N, uint32_t K, ui
     const double millions = (double)rows * K * 1e-6;  // (packed, and read again)
     double other;
     if (few_rows_win(element, N, K, rows, compute_units)) {
-        const uint32_t mt = few_row_tiles(N, rows, compute_units);
+        const uint32_t mt = few_pass_tiles(element, N, K, rows, compute_units);  // (the passes that are launched)
         const double walk = few_split(element, N, K, rows, mt, 1u, compute_units).cost / 64.0;
         other = mt == 3u ? 2.2 + t.threes * walk + 5.0 * millions : 3.8 + t.twos * walk + 3.2 * millions;
     } else {
