@@ -228,6 +228,8 @@ int32_t launch_gemv(nh_device *d, const GemvArgs &args);
 // whether launch_gemv walks the matrix once for this product's nine to sixteen rows (where one workgroup holds the rows it norms); it takes any
 // number of rows of a plain product, a few at a time where no form takes more
 bool gemv_takes_many(const GemvArgs &args);
+// scratch that a product of these sizes takes in whatever form, one to `rows` rows
+size_t gemv_scratch_bytes(uint32_t N, uint32_t K, uint32_t rows);
 // whether launch_gemv can merge attention sections of `width` channels a head into the activation row of this product
 bool gemv_merges_sections(const GemvArgs &args, uint32_t width);
 constexpr uint32_t MERGED_SECTIONS_MOST = 16;  // sections such a product merges at most

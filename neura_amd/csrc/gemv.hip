@@ -27,6 +27,7 @@
 #include "blocks.hpp"
 #include "common.hpp"
 #include "gemv_shared.hpp"
+#include "rows_rule.hpp"
 
 #include <cstdlib>
 
@@ -1439,6 +1440,13 @@ bool gemv_appends_value(const GemvArgs &a) {
 }
 
 bool gemv_takes_many(const GemvArgs &a) { return a.rows > 8 && (!a.norm_w || a.K <= 1792u) && rows_takes(a); }
+
+// (the vector and staged forms walk four rows at most at a time, in slices of 2048 numbers at least)
+size_t gemv_scratch_bytes(uint32_t N, uint32_t K, uint32_t rows) {
+    size_t most = K > 2048u ? (size_t)((K + 2047u) / 2048u) * min(rows, 4u) * N * sizeof(float) : 0u;
+    for (uint32_t r = 2; r <= min(rows, 16u) && K % 256u == 0; r++) most = max(most, rows_scratch_bytes(N, K, r));
+    return most;
+}
 
 int32_t launch_gemv(nh_device *d, const GemvArgs &a) {
     if (!a.rope && !a.append_value && (a.bias[0] || a.bias[1] || a.bias[2]))

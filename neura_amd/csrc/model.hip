@@ -541,11 +541,14 @@ nh_model *nh_model_create(nh_device *device, const nh_model_config *config, nh_w
          hipHostMalloc((void **)&m->chosen_host, ((size_t)c.batch + 1) * 4, hipHostMallocDefault) == hipSuccess;
     if (const char *held = getenv("NEURA_HIP_PUBLISH"); ok && !(held && held[0] == '0')) ok = hipHostGetDevicePointer((void **)&m->chosen_mapped, m->chosen_host, 0) == hipSuccess;
     // everything a captured step touches exists before the capture: the split partials of the
-    // products (at most 5 slices x 4 rows), of the attention (at most 256 sections) and of the
-    // greedy choice, and the rope table
+    // products, of the attention (at most 256 sections) and of the greedy choice, and the rope table
     {
-        size_t widest = (size_t)(2 * F > c.vocab ? 2 * F : c.vocab);
-        size_t products = 8 * 4 * widest * sizeof(float);
+        const uint32_t narrow_rows = (uint32_t)(T < 16 ? T : 16), sizes[5][2] = {{QW + 2 * KW, H}, {H, QW}, {2 * F, H}, {H, F}, {c.vocab, H}};
+        size_t products = 8 * 4 * (size_t)(2 * F > c.vocab ? 2 * F : c.vocab) * sizeof(float);  // (what most shapes take, and operator calls beside them)
+        for (const auto &[N, K] : sizes) {
+            const size_t bytes = gemv_scratch_bytes(N, K, narrow_rows);
+            if (bytes > products) products = bytes;
+        }
         size_t sections = (size_t)256 * c.heads * T * (c.head_dim + 2) * sizeof(float);
         size_t choice = (size_t)c.batch * 1024 * 8;
         // the wide product packs its fp32 activations as two half rows each, with their sub-block sums and a scale per row; the narrow
