@@ -59,8 +59,8 @@ def test_decode_steps_match_oracle_logits_and_tokens(device, shape, element):
 @pytest.mark.parametrize("shape,element", [(TINY, NH_Q8_0), (SMALL_Q4, NH_Q4_K), (SMALL_Q4, NH_Q6_K), (dict(SMALL_Q4, layers=1, vocab=4400), NH_Q5_K)],
                          ids=["q8_0", "q4_k", "q6_k", "q5_k-more-than-128-tiles"])
 def test_steps_of_more_planes_than_a_narrow_product_takes(device, shape, element, planes):
-    """Every product of a step runs as the wide product of few rows, the head over the whole vocabulary too; up to sixteen planes the
-    gate and the up projection share a launch that gates its outputs.  The head's rows are whole: ten to a tile, one, two and three tiles of
+    """Every product of a step runs as the wide product of few rows (a Q4_K layer's up to sixteen planes on the half-precision tiles), the head over
+    the whole vocabulary too; up to sixteen planes the gate and the up projection share a launch that gates its outputs.  The head's rows are whole: ten to a tile, one, two and three tiles of
     them (three a wave over more than 128 column tiles).  Eager, recorded and replayed steps at cursors of their own."""
     model, ref, weights = build(device, shape, element, batch=planes, context=40, seed=planes)
     rng = np.random.default_rng(planes)
@@ -518,6 +518,7 @@ def test_nine_to_sixteen_planes_on_the_half_precision_tiles(device, batch, shape
         mask = [1] * (batch - 1) + [0]
         beside = twin.decode_step(tokens, cursors + step, mask=mask)
         assert list(beside[:-1]) == list(got[:-1]) and np.array_equal(twin.logits()[:-1], model.logits()[:-1]), step
+    same_cache_rows(model, ref, shape["layers"], [list(range(at, at + 3)) for at in cursors], "rows the planes' steps appended")
     twin.release()
     one, oracle_one, one_weights = build(device, shape, NH_Q4_K, batch=1, context=40, max_rows=batch, seed=21)
     prompt = rng.integers(0, shape["vocab"], batch)
@@ -896,11 +897,21 @@ def test_rotation_folded_into_the_product_matches_the_separate_kernel(device, mo
         held.release()
 
 
-@pytest.mark.parametrize("shape,biased", [(SMALL_Q4, False), (SMALL_Q4, True), (WIDE_CUT, False)], ids=["small", "small-biased", "3584"])
-@pytest.mark.parametrize("batch", [5, 8])
-def test_rotation_folded_into_the_product_of_several_planes(device, monkeypatch, shape, biased, batch):
-    """Five to eight planes of one token each: the q|k|v product of a Q4_K decoder (the 32-row integer tiles) rotates q and k
-    and appends k and v in its epilogue, every plane at its own cursor.  The twin with the rotation as a kernel of its own runs
+# (320 tiles of 16 rows: more than a compute unit each, of short rows; 4096 numbers a row: the deepest slice there is)
+MANY_HEADS = dict(layers=1, hidden=512, heads=32, kv_heads=4, head_dim=128, ffn=512, vocab=500, tied=False)
+WIDE_4096 = dict(layers=1, hidden=4096, heads=16, kv_heads=4, head_dim=128, ffn=512, vocab=512, tied=False)
+NARROW_HEADS, BROAD_HEADS = dict(SMALL_Q4, layers=2, heads=16, kv_heads=4, head_dim=32), dict(SMALL_Q4, layers=2, heads=4, kv_heads=2, head_dim=256)
+
+
+@pytest.mark.parametrize("shape,biased,batch,window,cache_element", [
+    *((shape, biased, batch, None, 1) for batch in (5, 8) for shape, biased in ((SMALL_Q4, False), (SMALL_Q4, True), (WIDE_CUT, False))),
+    *((SMALL_Q4, True, batch, None, 1) for batch in (3, 4, 9, 13, 16)), (WIDE_CUT, True, 3, None, 1), (WIDE_4096, True, 7, None, 1), (MANY_HEADS, True, 6, None, 1),
+    (SMALL_Q4, True, 4, 12, 1), (SMALL_Q4, True, 13, 12, 0), (SMALL_Q4, True, 3, None, 0), (SMALL_Q4, True, 9, None, 30), (SMALL_Q4, False, 16, 12, 30),
+    (NARROW_HEADS, True, 5, None, 1), (NARROW_HEADS, True, 11, None, 1), (BROAD_HEADS, True, 3, None, 1)])
+def test_rotation_folded_into_the_product_of_several_planes(device, monkeypatch, shape, biased, batch, window, cache_element):
+    """Three to sixteen planes of one token each: the q|k|v product of a Q4_K decoder (the half-precision tiles; nine planes and more in two sets of
+    rows) rotates q and k and appends k and v in its epilogue, every plane at its own cursor, into states of any element, round a ring too.
+    The twin with the rotation as a kernel of its own runs
     the same product kernel and the same table of cosines and sines, so logits and caches agree bit for bit; both are held to
     the oracle (logits, tokens, and the rows the steps appended).  With q, k and v biases the twin's stacked product leaves
     them to the rotation's kernel, which adds them first as the folded epilogue does: the same sums, and the same bits."""
@@ -911,11 +922,11 @@ def test_rotation_folded_into_the_product_of_several_planes(device, monkeypatch,
         rng = np.random.default_rng(31)
         tensors = list(synth.model_tensors(shape, NH_Q4_K, rng, mode="normal" if shape is not WIDE_CUT else "blocks", biases=layers))
         weights = Weights(device, tensors)
-        return Model(device, weights, shape, NH_Q4_K, batch, 40, 1), weights, {name: (raw.view(np.float32) if name.endswith(".bias") else raw) for name, _, _, raw in tensors}
+        return Model(device, weights, shape, NH_Q4_K, batch, 64, 1, window=window, cache_element=cache_element), weights, {name: (raw.view(np.float32) if name.endswith(".bias") else raw) for name, _, _, raw in tensors}
 
     folded, weights_a, host = pair()
     apart, weights_b, _ = pair()
-    ref = oracle.Model(shape, NH_Q4_K, host, batch, 40, 1)
+    ref = oracle.Model(shape, NH_Q4_K, host, batch, 64, 1, window=window, cache_element=cache_element)
     tokens = [3 + 7 * plane for plane in range(batch)]
     first = [3 * plane for plane in range(batch)]  # every plane at a cursor of its own
     steps = 5
@@ -930,16 +941,19 @@ def test_rotation_folded_into_the_product_of_several_planes(device, monkeypatch,
         want_logits, want = ref.forward(tokens, 1, cursors)
         assert np.array_equal(logits_a, logits_b), step
         assert np.abs(logits_a - want_logits).max() <= 1e-3 * np.abs(want_logits).max()
-        assert list(got_a) == list(got_b) == list(want), (step, margins(want_logits))
+        clear = margins(want_logits) > 2e-3 * np.abs(want_logits).max()
+        assert list(got_a) == list(got_b) and (np.asarray(got_a)[clear] == np.asarray(want)[clear]).all(), (step, margins(want_logits))
         tokens = [int(t) for t in got_a]
     for layer in range(shape["layers"]):
         for which in (0, 1):
             assert np.array_equal(folded.cache_read(layer, which), apart.cache_read(layer, which)), (layer, which)
-    same_cache_rows(folded, ref, shape["layers"], [list(range(at, at + steps)) for at in first], "rows the planes' steps appended")
+    if cache_element == 1:
+        seats = [[(at + step) % window if window else at + step for step in range(steps)] for at in first]
+        same_cache_rows(folded, ref, shape["layers"], seats, "rows the planes' steps appended")
     # a cursor past the window is refused by the folded form as by the separate kernel
     monkeypatch.setenv("NEURA_HIP_FUSE_ROPE", "1")
     with pytest.raises(NeuraError):
-        folded.decode_step(tokens, [folded.capacity + 3] * batch)
+        folded.decode_step(tokens, [67] * batch)
     for held in (folded, apart, weights_a, weights_b):
         held.release()
 
