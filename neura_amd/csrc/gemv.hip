@@ -1,9 +1,9 @@
-// Narrow products (1..8 activation rows) over raw GGUF blocks: y[r][n] = sum_k x[r][k] * W[n][k].
+// Narrow products (one to eight activation rows, of Q4_K to sixteen; any count a few at a time) over raw GGUF blocks: y[r][n] = sum_k x[r][k] * W[n][k].
 //
 // Which Q4_K form a product reaches with no switch set (launch_gemv asks them in this order):
 //
-//   gemv_q4k_rows_kernel       3 to 8 activation rows, matrices that end on 16-row tiles, any K (deep rows in slices, which a fold adds up);
-//                              q|k|v of three to eight planes with the rotation and the cache append in its epilogue (gemv_rows.hip)
+//   gemv_q4k_rows_kernel       3 to 16 activation rows, matrices that end on 16-row tiles, any K (deep rows in slices, which a fold adds up);
+//                              q|k|v of three to sixteen planes with the rotation and the cache append in its epilogue (gemv_rows.hip)
 //   gemv_q4k_tile16_kernel     1 row, any K of whole super-blocks, matrices that end on 16-row tiles: every product of a
 //                              batch-1 decode step of the 0.5B .. 7B shapes; 2 rows where their digits fit LDS (ffn_down's 18944 columns
 //                              included; the form above takes the rest) (gemv_tile16.hip)
@@ -12,8 +12,7 @@
 //                              boundary (odd vocabularies and widths: the small decoders of the tests); the vector form
 //   gemv_q4k_kernel            the same refusals with K > 4096 or several rows: the LDS-tile vector form
 //
-// NEURA_HIP_TILE16=0, NEURA_HIP_ROWS4=0 (three and four rows stay on the one-row tiles), NEURA_HIP_MFMA=0 (the vector forms at several rows)
-// and NEURA_HIP_F16_TILES=0|2 push a product down (or up) this list so that the tests can hold the forms to each other on the same shapes.
+// NEURA_HIP_TILE16=0, NEURA_HIP_MFMA=0 (the vector forms throughout) and NEURA_HIP_F16_TILES=0|2 push a product down (or up) this list so that the tests can hold the forms to each other on the same shapes.
 //
 // The vector form, Q4_K: a super-block is 144 B = a 16 B header (d, dmin, 12 scale bytes) + 128 B of nibbles.
 // One lane owns one 64-element group of one super-block: it loads the header and its 32
@@ -1361,7 +1360,6 @@ bool gemv_fuses_rope(const GemvArgs &a, const RopeFusion &rope) {
         if (a.element != NH_Q4_K || a.K % 256u != 0 || a.K > 4096u) return false;
         if (a.N >= 16384u || a.N < 2u || (uint64_t)a.N * (a.K / 256u * 144u) >= (1ull << 32)) return false;
     }
-    if (env_int("NEURA_HIP_MFMA", 1) == 2) return false;
     const uint32_t width = rope.width;
     if (width < 2 || (width & (width - 1u)) != 0) return false;
     if (rope.q_rows % width || rope.k_rows % width || a.N % width || rope.q_rows > rope.k_rows || rope.k_rows > a.N) return false;
@@ -1457,12 +1455,12 @@ int32_t launch_gemv(nh_device *d, const GemvArgs &a) {
                     (a.K / a.merge->width) % a.merge->groups))
         return fail(NH_E_ARGUMENT, "this product merges no attention sections (ask gemv_merges_sections first)");
     if (a.merge) return launch_rows<1>(d, a, a.x, a.y, a.residual);
-    if ((a.rows > 4 || a.rope || (a.rows > 2 && env_int("NEURA_HIP_ROWS4", 1) != 0)) && rows_takes(a)) return launch_rows(d, a);
+    if (a.rows > 2 && rows_takes(a)) return launch_q4k_rows(d, a);
     if (tile16_takes(a)) return launch_tile16(d, a);
     if (q6k_tile16_takes(a)) return launch_q6k_tile16(d, a);
     if (a.digits_out || a.digits_in) return fail(NH_E_ARGUMENT, "this product hands over no digit planes (ask gemv_hands_digits first)");
     if (a.rope && a.rows != 1) return fail(NH_E_ARGUMENT, "this product cannot fold the rotation in (ask gemv_fuses_rope first)");
-    if (rows_takes(a)) return launch_rows(d, a);
+    if (rows_takes(a)) return launch_q4k_rows(d, a);
     if (gemv_wide_takes(d, a)) return launch_gemv_wide(d, a);
     // activation rows are taken four, two or one at a time
     uint32_t outputs = a.swiglu ? a.N / 2 : a.N;

@@ -234,9 +234,9 @@ constexpr uint32_t TILE16_BLOCK_HANDED = 1024;
 // the 16-row tile kernel (gemv_tile16.hip): whether it serves this product, and its launch
 bool tile16_takes(const GemvArgs &args);
 int32_t launch_tile16(nh_device *d, const GemvArgs &args);
-// two to eight activation rows of Q4_K on half-precision tiles (gemv_rows.hip)
+// two to sixteen activation rows of Q4_K on half-precision tiles (gemv_rows.hip)
 bool rows_takes(const GemvArgs &args);
-int32_t launch_rows(nh_device *d, const GemvArgs &args);
+int32_t launch_q4k_rows(nh_device *d, const GemvArgs &args);
 // several activation rows as a wide product of few rows (gemm.hip)
 bool gemv_wide_takes(const nh_device *d, const GemvArgs &args);
 int32_t launch_gemv_wide(nh_device *d, const GemvArgs &args);

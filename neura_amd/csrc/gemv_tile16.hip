@@ -879,16 +879,15 @@ TILE16_KERNEL(8, 2, TILE16_PLAIN, 1, true, false);
 
 // ---------------------------------------------------------------------------------------------------------------------
 // ---- the 16-row tile kernel (one activation row, Q4_K)
-// NEURA_HIP_TILE16=0 keeps it out (the vector and the other matrix-core forms then take one row as before), as does a forced
-// NEURA_HIP_MFMA form.  Otherwise it takes every Q4_K product of one row whose matrices end on tile boundaries, and of two
-// to four rows (NEURA_HIP_TILE16_ROWS lowers that) where all their digit planes fit the workgroup's LDS.  From three rows on
-// the MFMAs and the weighing, both paid once a row, cost more than the weights' bytes: gemv_rows.hip takes those (unless NEURA_HIP_ROWS4=0).
-constexpr uint32_t TILE16_MOST_ROWS = 4;
-static uint32_t tile16_row_form(uint32_t rows) { return rows <= 1u ? 1u : (rows <= 2u ? 2u : 4u); }
+// NEURA_HIP_TILE16=0 keeps it out (the vector and the other matrix-core forms then take one row as before), as does NEURA_HIP_MFMA=0.
+// Otherwise it takes every Q4_K product of one row whose matrices end on tile boundaries, and of two (NEURA_HIP_TILE16_ROWS=1: not) where
+// both rows' digit planes fit the workgroup's LDS.  From three rows on the MFMAs and the weighing, both paid once a row, cost more than
+// the weights' bytes: gemv_rows.hip takes those (three rows, us here / there: q|k|v of the 7B shape 8.7 / 6.9, gate|up 22.3 / 20.6, ffn_down 23.8 / 15.5).
+constexpr uint32_t TILE16_MOST_ROWS = 2;
 
 bool tile16_takes(const GemvArgs &a) {
     if ((a.element != NH_Q4_K && a.element != NH_Q5_K) || a.rows < 1 || a.rows > TILE16_MOST_ROWS || a.K % 256u != 0 || a.K == 0) return false;
-    if (env_int("NEURA_HIP_TILE16", 1) == 0 || env_int("NEURA_HIP_MFMA", 1) != 1) return false;
+    if (env_int("NEURA_HIP_TILE16", 1) == 0 || env_int("NEURA_HIP_MFMA", 1) == 0) return false;
     // Q5_K (one row): the same tiles with the fifth bit beside the nibble; NEURA_HIP_Q5K_TILE16=0 leaves it to the staged kernel
     if (a.element == NH_Q5_K && (a.rows != 1 || a.merge || env_int("NEURA_HIP_Q5K_TILE16", 1) == 0)) return false;
     // a value projection that casts its rows into the value state: one row, whole heads, no other epilogue
@@ -898,7 +897,7 @@ bool tile16_takes(const GemvArgs &a) {
     for (int m = 0; m < 3; m++)
         if (a.W[m] && ((uintptr_t)a.W[m] & 15u)) return false;
     if (a.rows > 1 && (a.rope || a.rows > (uint32_t)env_int("NEURA_HIP_TILE16_ROWS", (int)TILE16_MOST_ROWS))) return false;
-    if (a.rows > 1 && (env_int("NEURA_HIP_MFMA32", 1) == 2 || env_int("NEURA_HIP_F16_TILES", 1) == 2)) return false;  // another form is forced
+    if (a.rows > 1 && env_int("NEURA_HIP_F16_TILES", 1) == 2) return false;  // another form is forced
     if (((uintptr_t)a.x & 15u) || (a.norm_w && ((uintptr_t)a.norm_w & 15u))) return false;
     if (a.N < 16u || a.N % 16u != 0) return false;
     if (a.swiglu) {
@@ -919,7 +918,7 @@ bool tile16_takes(const GemvArgs &a) {
     if (a.digits_out && (!a.swiglu || a.rows != 1 || a.N % 512u != 0 || ((uintptr_t)a.digits_out & 63u))) return false;
     if (a.digits_in && (a.swiglu || a.rope || a.norm_w || a.rows != 1 || ((uintptr_t)a.digits_in & 15u))) return false;
     const uint32_t nblk = a.K / 256u;
-    return tile16_lds(nblk, nblk > 32u ? 16u : 8u, tile16_row_form(a.rows), a.digits_in != nullptr) <= 160u * 1024u;
+    return tile16_lds(nblk, nblk > 32u ? 16u : 8u, a.rows, a.digits_in != nullptr) <= 160u * 1024u;
 }
 
 // A SwiGLU product of one row ends with a chunk's sixteen outputs in sixteen lanes of one wave: it can leave them as the digit
@@ -980,11 +979,7 @@ static hipError_t launch_tile16_rows(nh_device *d, const GemvParams &p, uint32_t
 template <int MODE>
 static hipError_t launch_tile16_mode(nh_device *d, const GemvParams &p, uint32_t waves, uint32_t grid, size_t lds) {
     if constexpr (MODE != TILE16_ROPE) {
-        switch (tile16_row_form(p.rows)) {
-        case 1: break;
-        case 2: return launch_tile16_rows<MODE, 2>(d, p, waves, grid, lds);
-        default: return launch_tile16_rows<MODE, 4>(d, p, waves, grid, lds);
-        }
+        if (p.rows == 2u) return launch_tile16_rows<MODE, 2>(d, p, waves, grid, lds);
     }
     return launch_tile16_rows<MODE, 1>(d, p, waves, grid, lds);
 }
@@ -1042,7 +1037,7 @@ static Tile16Launch tile16_plan(nh_device *d, const GemvArgs &a, uint32_t fixed_
     plan.waves = fixed_waves ? fixed_waves : (p.nblk <= 8u ? 4u : (p.nblk <= 14u ? 7u : (p.nblk <= 32u || a.digits_in ? 8u : 16u)));
     // one row against short rows (the 1.5B shape's 1536 columns are six super-blocks): a wave a super-block keeps more bytes in
     // flight a compute unit than four waves of two steps -- measured on that shape, a decode step 0.963 -> 0.898 ms
-    // (two to four rows take the same waves: a row of theirs is then, bit for bit, what the one-row product gives)
+    // (two rows take the same waves: a row of theirs is then, bit for bit, what the one-row product gives)
     if (!fixed_waves && !a.digits_in && p.nblk > 4u && p.nblk <= 8u) plan.waves = p.nblk <= 6u ? 6u : 8u;
     // units of work: tiles, or with SwiGLU pairs (a gate tile and the up tile behind it); every workgroup takes the same
     // number of them, one workgroup a compute unit when there are that many
@@ -1063,7 +1058,7 @@ static Tile16Launch tile16_plan(nh_device *d, const GemvArgs &a, uint32_t fixed_
     p.row_groups = units;
     const uint32_t rounds = (units + (uint32_t)d->compute_units - 1u) / (uint32_t)d->compute_units;
     plan.grid = (units + rounds - 1u) / rounds;
-    plan.lds = tile16_lds(p.nblk, plan.waves, tile16_row_form(a.rows), a.digits_in != nullptr);
+    plan.lds = tile16_lds(p.nblk, plan.waves, a.rows, a.digits_in != nullptr);
     return plan;
 }
 

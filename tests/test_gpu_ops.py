@@ -217,13 +217,13 @@ def test_gemv_epilogues(device, element, N, K):
         close(device.gemv(element, raw, N, K, x, swiglu=True), want, rel=1e-4, abs_=1e-4 * np.abs(want).max())
 
 
-@pytest.mark.parametrize("mode", ["0", "2"])
+@pytest.mark.parametrize("switch,mode", [("NEURA_HIP_MFMA", "0"), ("NEURA_HIP_F16_TILES", "2")])
 @pytest.mark.parametrize("N,K,rows", [(16, 256, 1), (48, 512, 3), (272, 3584, 1), (64, 1536, 8), (32, 18944, 1), (32, 18944, 5), (1040, 768, 2)])
-def test_q4_k_products_agree_in_every_form(device, monkeypatch, mode, N, K, rows):
-    """NEURA_HIP_MFMA=0 forces the vector kernels, =2 the matrix-core kernel (integer MFMA over four-digit activations);
+def test_q4_k_products_agree_in_every_form(device, monkeypatch, switch, mode, N, K, rows):
+    """NEURA_HIP_MFMA=0 forces the vector kernels, NEURA_HIP_F16_TILES=2 the half-precision tiles from two rows on (one row is on the integer tiles);
     both sit within fp32 reordering of the order-faithful oracle, plain, with a residual and with SwiGLU, for 1..8
     activation rows, rows deeper than one LDS stage, and activations that span many orders of magnitude."""
-    monkeypatch.setenv("NEURA_HIP_MFMA", mode)
+    monkeypatch.setenv(switch, mode)
     rng = np.random.default_rng(N + K + rows)
     raw = synth.q4_k_random(rng, N * K)
     x = (rng.standard_normal((rows, K)) * np.exp(rng.uniform(-6, 6, (rows, K)))).astype(np.float32)  # wide dynamic range
@@ -243,14 +243,11 @@ def test_q4_k_products_agree_in_every_form(device, monkeypatch, mode, N, K, rows
 
 @pytest.mark.parametrize("N,K,rows", [(64, 3584, 1), (96, 2048, 4), (128, 256, 2), (2048, 3584, 7), (64, 4096, 3), (64, 1536, 8), (160, 768, 5),
                                       (64, 18944, 8), (96, 8960, 2), (32, 18944, 5)])
-@pytest.mark.parametrize("forced", ["NEURA_HIP_MFMA32", "NEURA_HIP_F16_TILES"])
-def test_q4_k_product_on_32_row_tiles(device, monkeypatch, forced, N, K, rows):
-    """NEURA_HIP_MFMA32=2 forces the 32 x 32 x 32 integer MFMA kernel (weights as the B operand, the digit planes of up to
-    eight activation rows as A, digits scaled per sub-block): plain, with a residual and with SwiGLU, for every count of
-    activation rows, against the oracle and an fp64 product (the decoder tests run it with the fused norm).
-    NEURA_HIP_F16_TILES=2 forces, for two rows and more, the 16-row tiles on half-precision MFMA (weights as exact halves
-    code * sc, activations as value and residue half rows) through the same cases."""
-    monkeypatch.setenv(forced, "2")
+def test_q4_k_product_on_half_precision_tiles(device, monkeypatch, N, K, rows):
+    """NEURA_HIP_F16_TILES=2 forces, for two rows and more, the 16-row tiles on half-precision MFMA (weights as exact halves
+    code * sc, activations as value and residue half rows): plain, with a residual and with SwiGLU, for every count of
+    activation rows, against the oracle and an fp64 product (the decoder tests run it with the fused norm)."""
+    monkeypatch.setenv("NEURA_HIP_F16_TILES", "2")
     rng = np.random.default_rng(N + K + rows)
     raw = synth.q4_k_random(rng, N * K)
     x = (rng.standard_normal((rows, K)) * np.exp(rng.uniform(-6, 6, (rows, K)))).astype(np.float32)  # wide dynamic range
@@ -269,13 +266,12 @@ def test_q4_k_product_on_32_row_tiles(device, monkeypatch, forced, N, K, rows):
 
 
 @pytest.mark.parametrize("N,K,rows", [(40032, 1280, 2), (40032, 768, 8), (40032, 1280, 5)])
-@pytest.mark.parametrize("forced", ["NEURA_HIP_MFMA32", "NEURA_HIP_F16_TILES"])
-def test_tiles_follow_tiles_in_a_wave(device, monkeypatch, forced, N, K, rows):
-    """1251 tiles of 32 rows (2502 of 16) are several rounds of every workgroup, the last one ragged: a wave asks for the first
+def test_tiles_follow_tiles_in_a_wave(device, monkeypatch, N, K, rows):
+    """2502 tiles of 16 rows are several rounds of every workgroup, the last one ragged: a wave asks for the first
     super-block of its next tile while it multiplies the last of this one, also where a tile has fewer super-blocks than waves.
     The last rows of weights give what they give in a matrix of one round: each is within 1e-5 of its largest output of the
     oracle (a wrong block would be off by a tenth of it), the two within that of one another."""
-    monkeypatch.setenv(forced, "2")
+    monkeypatch.setenv("NEURA_HIP_F16_TILES", "2")
     rng = np.random.default_rng(N + K + rows)
     raw = synth.q4_k_random(rng, N * K)
     x = (rng.standard_normal((rows, K)) * np.exp(rng.uniform(-2, 2, (rows, K)))).astype(np.float32)
@@ -321,15 +317,13 @@ def test_q4_k_one_row_product_on_16_row_tiles(device, monkeypatch, tile16, N, K)
     assert np.array_equal(device.gemv(NH_Q4_K, raw, N, K, np.zeros((1, K), np.float32)), np.zeros((1, N), np.float32))
 
 
-@pytest.mark.parametrize("N,K,rows", [(16, 256, 2), (64, 3584, 4), (4608, 3584, 4), (3584, 3584, 3), (4608, 3584, 2), (1040, 768, 4), (48, 2048, 3),
-                                      (272, 8960, 4), (96, 18944, 2), (37888, 3584, 4), (64, 10240, 3), (152064, 3584, 2)])
-def test_q4_k_products_of_a_few_rows_on_16_row_tiles(device, monkeypatch, N, K, rows):
-    """(NEURA_HIP_ROWS4=0: the form that serves where the kernel with four rows to an MFMA does not fit.)
-    Two to four activation rows against Q4_K rows in one pass of the 16-row tiles (every row its own digit planes, the
+@pytest.mark.parametrize("N,K,rows", [(16, 256, 2), (64, 3584, 2), (4608, 3584, 2), (3584, 3584, 2), (1040, 768, 2), (48, 2048, 2),
+                                      (272, 8960, 2), (96, 18944, 2), (37888, 3584, 2), (64, 10240, 2), (152064, 3584, 2)])
+def test_q4_k_products_of_a_few_rows_on_16_row_tiles(device, N, K, rows):
+    """Two activation rows against Q4_K rows in one pass of the 16-row tiles (every row its own digit planes, the
     weights unpacked once a step): each row is, bit for bit, what the one-row product gives for it alone, plain, with a
     residual and with SwiGLU (the decoders' batches run it with the norm folded in); and the whole sits as close to the exact
     product as the oracle does.  A non-finite number stays in its own row."""
-    monkeypatch.setenv("NEURA_HIP_ROWS4", "0")
     rng = np.random.default_rng(N + K + rows)
     raw = synth.q4_k_random(rng, N * K)
     x = (rng.standard_normal((rows, K)) * np.exp(rng.uniform(-2, 2, (rows, K)))).astype(np.float32)
@@ -357,9 +351,9 @@ def test_q4_k_products_of_a_few_rows_on_16_row_tiles(device, monkeypatch, N, K, 
 
 @pytest.mark.parametrize("N,K,rows", [(16, 256, 3), (64, 3584, 4), (4608, 3584, 4), (3584, 3584, 3), (4608, 3584, 3), (1040, 768, 4), (48, 2048, 3),
                                       (272, 8960, 4), (37888, 3584, 4), (37888, 3584, 3), (64, 10240, 3), (152064, 3584, 3)])
-def test_q4_k_products_of_several_rows_four_rows_to_an_mfma(device, N, K, rows):
-    """Three and four activation rows against Q4_K rows, four activation rows in an MFMA's sixteen operand rows and the
-    sub-block scales inside the weight operand: within the product's bar of the oracle and as close to the exact product as the oracle is, plain, with a residual
+def test_q4_k_products_of_three_and_four_rows(device, N, K, rows):
+    """Three and four activation rows against Q4_K rows on the half-precision tiles, a value and a residue each among an MFMA's sixteen
+    operand rows and the sub-block scales inside the weight operand: within the product's bar of the oracle and as close to the exact product as the oracle is, plain, with a residual
     and with SwiGLU; a row's numbers do not depend on the rows beside it (bit for bit what it gives next to rows of zeros),
     and a non-finite number stays in its own row."""
     rng = np.random.default_rng(N + K + rows)
@@ -376,8 +370,7 @@ def test_q4_k_products_of_several_rows_four_rows_to_an_mfma(device, N, K, rows):
     if small:
         plain = oracle.gemv(NH_Q4_K, raw, N, K, x, threads=8)
         exact = oracle.unpack(NH_Q4_K, raw, N * K).reshape(N, K).astype(np.float64) @ x.astype(np.float64).T
-        # the digits' scale is a super-block's here: an outlier costs its 255 neighbours the bits it stands above them
-        as_exact_as_the_oracle(got, plain, exact.T, 8e-6)
+        as_exact_as_the_oracle(got, plain, exact.T, 2e-6)
         if N % 32 == 0:
             gate, up = plain[:, : N // 2].astype(np.float64), plain[:, N // 2 :].astype(np.float64)
             want = gate / (1.0 + np.exp(-gate)) * up
@@ -469,7 +462,8 @@ def test_rows_with_a_mean_keep_their_bits_beside_weights_without_one(device, N, 
 
 
 def test_q4_k_product_on_the_matrix_cores_keeps_non_finite_inputs_visible(device, monkeypatch):
-    monkeypatch.setenv("NEURA_HIP_MFMA", "2")
+    """two rows on the half-precision tiles, one on the integer tiles"""
+    monkeypatch.setenv("NEURA_HIP_F16_TILES", "2")
     rng = np.random.default_rng(2)
     N, K = 32, 512
     raw = synth.q4_k_random(rng, N * K)
